@@ -12,104 +12,137 @@ namespace tcpx {
 
 DataPipe::DataPipe()
     // 2048 control messages of CMSG_SPACE(sizeof(struct iovec)) bytes (src/devcomm/unpack_defs1.h:32-36).
-    : ctrl_data(static_cast<size_t>(kSlotPages) * CMSG_SPACE(sizeof(struct iovec))), scatter_list(kSlotPages) {}
+    : ctrl_data(static_cast<size_t>(kSlotPages) * CMSG_SPACE(sizeof(struct iovec))), scatter_list(kSlotPages),
+      list(scatter_list.data()), list_room(kSlotPages) {}
 
 void DevmemSocket::push(const tcpxSynthFrag* frags, size_t n) {
   std::lock_guard<std::mutex> lock(mu);
   arrived.insert(arrived.end(), frags, frags + n);
 }
 
+bool PageLedger::open(size_t arena_pages) {
+  pages = static_cast<Page*>(calloc(arena_pages, sizeof(Page)));
+  n_pages = pages ? arena_pages : 0;
+  return pages != nullptr;
+}
+
+namespace {
+
+// One control message as it lies in the buffer: the fields of struct cmsghdr, the vector, and the padding that the
+// kernel zeroes too.
+struct WireCmsg {
+  size_t len;
+  int level, type;
+  DevmemVec v;
+  uint32_t pad;
+};
+static_assert(sizeof(WireCmsg) == CMSG_SPACE(sizeof(DevmemVec)) && offsetof(WireCmsg, v) == CMSG_LEN(0) &&
+                  offsetof(WireCmsg, level) == offsetof(struct cmsghdr, cmsg_level) &&
+                  offsetof(WireCmsg, type) == offsetof(struct cmsghdr, cmsg_type),
+              "one control message: header, 12 bytes, 4 of padding");
+
+constexpr size_t kPrefetchFrags = 8;  // page entries asked for ahead: the pages of a message lie anywhere in the arena
+
+}  // namespace
+
 ssize_t DevmemSocket::recvmsg(struct msghdr* msg, size_t max_bytes) {
   msg->msg_flags = 0;
   if (head == rx.size()) {  // everything taken over earlier has been received: look for new arrivals
     rx.clear();
     head = 0;
-    {
-      std::lock_guard<std::mutex> lock(mu);
-      rx.swap(arrived);
-    }
-    for (const tcpxSynthFrag& f : rx) payload_frags += f.frag_size != 0;
+    std::lock_guard<std::mutex> lock(mu);
+    rx.swap(arrived);
   }
   // A recvmsg that returns no bytes means "peer closed" to the caller, so empty fragments (which the adversarial
   // workload contains) only ever travel together with a non-empty one.
-  if (payload_frags == 0 && head < rx.size()) {
+  auto payload_ahead = [&] {
+    for (size_t i = head; i < rx.size(); ++i)
+      if (rx[i].frag_size != 0) return true;
+    return false;
+  };
+  bool payload = payload_ahead();  // (looks at one fragment unless empty ones are next)
+  if (!payload && head < rx.size()) {
     // Only empty fragments are left on this side: the payload they travel with may have arrived meanwhile.
-    std::lock_guard<std::mutex> lock(mu);
-    for (const tcpxSynthFrag& f : arrived) payload_frags += f.frag_size != 0;
-    rx.insert(rx.end(), arrived.begin(), arrived.end());
-    arrived.clear();
+    {
+      std::lock_guard<std::mutex> lock(mu);
+      rx.insert(rx.end(), arrived.begin(), arrived.end());
+      arrived.clear();
+    }
+    payload = payload_ahead();
   }
-  if (payload_frags == 0 || max_bytes == 0) {
+  if (!payload || max_bytes == 0) {
     msg->msg_controllen = 0;
     errno = EAGAIN;
     return -1;
   }
-  const uint32_t frag_limit = max_frags_per_recvmsg.load(std::memory_order_relaxed);
-  const size_t room = msg->msg_controllen;
-  const size_t per_cmsg = CMSG_SPACE(sizeof(DevmemVec));
-  static_assert(CMSG_SPACE(sizeof(DevmemVec)) == CMSG_LEN(sizeof(DevmemVec)) + 4, "one control message: header, 12 bytes, 4 of padding");
-  char* out = static_cast<char*>(msg->msg_control);
-  size_t used = 0;
+  const uint32_t limit = max_frags_per_recvmsg.load(std::memory_order_relaxed);
+  uint32_t payload_left = limit != 0 ? limit : UINT32_MAX;
+  WireCmsg* const first = static_cast<WireCmsg*>(msg->msg_control);
+  WireCmsg* out = first;
+  WireCmsg* const out_end = first + msg->msg_controllen / sizeof(WireCmsg);
   size_t bytes = 0;
-  uint32_t n_payload = 0;
   uint64_t refs = 0;
-  while (head < rx.size()) {
-    tcpxSynthFrag& f = rx[head];
-    if (f.frag_size != 0) {
-      if (bytes >= max_bytes) break;
-      if (frag_limit != 0 && n_payload >= frag_limit) break;
+  tcpxSynthFrag* f = rx.data() + head;
+  tcpxSynthFrag* const end = rx.data() + rx.size();
+  for (; f != end; ++f) {
+    if (f->frag_size != 0) {
+      if (bytes >= max_bytes || payload_left == 0) break;
+      --payload_left;
     }
-    if (used + per_cmsg > room) {
+    if (out == out_end) {
       msg->msg_flags |= MSG_CTRUNC;
       break;
     }
-    const uint32_t take = static_cast<uint32_t>(std::min<size_t>(f.frag_size, max_bytes - bytes));
-    // One control message: the header's three fields, the vector, and the padding that the kernel zeroes too.
-    struct cmsghdr* cm = reinterpret_cast<struct cmsghdr*>(out + used);
-    cm->cmsg_len = CMSG_LEN(sizeof(DevmemVec));
-    cm->cmsg_level = SOL_SOCKET;
-    cm->cmsg_type = kScmDevmemOffset;
-    const DevmemVec v{f.frag_offset, take, f.frag_token};
-    memcpy(CMSG_DATA(cm), &v, sizeof v);
-    memset(CMSG_DATA(cm) + sizeof v, 0, 4);
-    used += per_cmsg;
+    const uint32_t take = static_cast<uint32_t>(std::min<size_t>(f->frag_size, max_bytes - bytes));
+    *out++ = WireCmsg{CMSG_LEN(sizeof(DevmemVec)), SOL_SOCKET, kScmDevmemOffset, {f->frag_offset, take, f->frag_token}, 0};
     bytes += take;
-    if (f.frag_size != 0) ++n_payload;
     // Every control message hands one page reference to the receiver.
-    if (device && f.frag_token < device->n_pages) {
-      device->page_refs[f.frag_token].fetch_add(1, std::memory_order_relaxed);
+    if (f->frag_token < ledger->n_pages) {
+      ledger->give(f->frag_token);
       ++refs;
     }
-    if (take == f.frag_size) {
-      payload_frags -= f.frag_size != 0;
-      ++head;
-    } else {  // byte budget ended inside the fragment: the rest stays queued
-      f.frag_offset += take;
-      f.frag_size -= take;
+    if (end - f > static_cast<ptrdiff_t>(kPrefetchFrags)) __builtin_prefetch(&ledger->pages[f[kPrefetchFrags].frag_token], 1);
+    if (take != f->frag_size) {  // byte budget ended inside the fragment: the rest stays queued
+      f->frag_offset += take;
+      f->frag_size -= take;
       break;
     }
   }
-  if (refs) device->pages_outstanding.fetch_add(refs, std::memory_order_relaxed);
-  msg->msg_controllen = used;
+  head = static_cast<size_t>(f - rx.data());
+  ledger->given.store(ledger->given.load(std::memory_order_relaxed) + refs, std::memory_order_relaxed);
+  msg->msg_controllen = static_cast<size_t>(out - first) * sizeof(WireCmsg);
   return static_cast<ssize_t>(bytes);
 }
 
 int DevmemSocket::dontneed(const PageToken* tokens, size_t n) {
-  if (!device) return 0;
   uint64_t given_back = 0;
   int rc = 0;
   for (size_t i = 0; i < n && rc == 0; ++i) {
+    if (i + kPrefetchFrags < n) __builtin_prefetch(&ledger->pages[tokens[i + kPrefetchFrags].token_start], 1);
     for (uint32_t k = 0; k < tokens[i].token_count; ++k) {
       const uint32_t page = tokens[i].token_start + k;
-      if (page >= device->n_pages || device->page_refs[page].fetch_sub(1, std::memory_order_relaxed) <= 0) {
+      if (page >= ledger->n_pages || !ledger->take_back(page)) {
         rc = -1;  // no such page, or freed twice
         break;
       }
       ++given_back;
     }
   }
-  device->pages_outstanding.fetch_sub(given_back, std::memory_order_relaxed);
+  ledger->back.store(ledger->back.load(std::memory_order_relaxed) + given_back, std::memory_order_relaxed);
   return rc;
+}
+
+// The control message after `cm`, or null: the bounds of CMSG_NXTHDR, without the call into the C library that the
+// macro makes for every message.
+static inline struct cmsghdr* next_cmsg(const struct msghdr* msg, struct cmsghdr* cm) {
+  const size_t at = static_cast<size_t>(reinterpret_cast<char*>(cm) - static_cast<char*>(msg->msg_control));
+  const size_t left = msg->msg_controllen - at;
+  if (cm->cmsg_len < sizeof(struct cmsghdr) || CMSG_ALIGN(cm->cmsg_len) > left ||
+      left - CMSG_ALIGN(cm->cmsg_len) < sizeof(struct cmsghdr))
+    return nullptr;
+  struct cmsghdr* next = reinterpret_cast<struct cmsghdr*>(reinterpret_cast<char*>(cm) + CMSG_ALIGN(cm->cmsg_len));
+  if (CMSG_ALIGN(next->cmsg_len) > left - CMSG_ALIGN(cm->cmsg_len)) return nullptr;  // runs past the end of the buffer
+  return next;
 }
 
 ssize_t process_recv_cmsg(struct msghdr* msg, DataPipe* p, int offset, uint64_t dst_base_offset,
@@ -117,7 +150,16 @@ ssize_t process_recv_cmsg(struct msghdr* msg, DataPipe* p, int offset, uint64_t 
   int num_cm = 0;
   size_t host_bytes = 0;
   ssize_t dst_offset = 0;
-  for (struct cmsghdr* cm = CMSG_FIRSTHDR(msg); cm; cm = CMSG_NXTHDR(msg, cm)) {
+  // What changes per fragment stays in registers: through `p` the compiler reads it back after every store.
+  union loadMeta* const list = p->list;
+  uint64_t cnt = p->cnt_cache;
+  const uint64_t cnt_end = p->list_room;
+  PageToken* const toks = p->pgtoks;
+  size_t n_toks = *p->pgtok_cnt;
+  uint32_t next_token = 0;  // the page that would continue the last run
+  if (n_toks > 0) next_token = toks[n_toks - 1].token_start + toks[n_toks - 1].token_count;
+  const uint64_t dst_base = static_cast<uint64_t>(offset) + dst_base_offset;
+  for (struct cmsghdr* cm = CMSG_FIRSTHDR(msg); cm; cm = next_cmsg(msg, cm)) {
     if (cm->cmsg_level != SOL_SOCKET || (cm->cmsg_type != kScmDevmemOffset && cm->cmsg_type != kScmDevmemHeader)) {
       INFO(NCCL_NET, "cmsg: unknown %u.%u", cm->cmsg_level, cm->cmsg_type);
       continue;
@@ -134,39 +176,45 @@ ssize_t process_recv_cmsg(struct msghdr* msg, DataPipe* p, int offset, uint64_t 
       }
       continue;
     }
+    // Page tokens, run-length coded (src/sock/tcpx.h:190-199).
+    if (n_toks > 0 && next_token == v.frag_token) {
+      toks[n_toks - 1].token_count++;
+    } else if (n_toks < static_cast<size_t>(kSlotPages)) {
+      toks[n_toks++] = PageToken{v.frag_token, 1};
+    } else {
+      // The token list is the slot's, one per flow, and a request may put several chunks on one flow: it is full
+      // when it holds as many runs as a slot holds descriptors.  (The reference zeroes the count per task and so
+      // never gets here; it also forgets the earlier chunks' pages.)
+      WARN("flow holds %zu page-token runs for one request, the most a slot records; failstop", n_toks);
+      *p->pgtok_cnt = n_toks;
+      *result = fail_stop("too many page-token runs on one flow of a request");
+      return -1;
+    }
+    next_token = v.frag_token + 1u;
+    if (cnt == cnt_end) {  // (a list that does not start at the slot's first descriptor; src/net_tcpx.cc:1350-1353)
+      WARN("request too many pages, %lu more than its slot had room for, failstop", static_cast<unsigned long>(cnt + 1 - cnt_end));
+      *p->pgtok_cnt = n_toks;
+      *result = fail_stop("request needs more descriptors than a slot holds");
+      return -1;
+    }
     // src/sock/tcpx.h:178-181: where the fragment lies in the bounce buffer, how long it is, and where in the
     // request's buffer it belongs: bytes of this recvmsg so far + bytes of the task so far + the task's offset in
     // the request.
-    union loadMeta& d = p->scatter_list[p->cnt_cache];
+    union loadMeta& d = list[cnt];
     d.src_off = v.frag_offset;
     d.len = v.frag_size;
-    d.dst_off = static_cast<uint64_t>(dst_offset) + static_cast<uint64_t>(offset) + dst_base_offset;
-    p->cnt_cache++;
-    if (p->cnt_cache >= static_cast<uint64_t>(kSlotPages)) {  // src/sock/tcpx.h:183-187
-      WARN("received %lu/%d segs, failstop", static_cast<unsigned long>(p->cnt_cache), kSlotPages);
+    d.dst_off = static_cast<uint64_t>(dst_offset) + dst_base;
+    cnt++;
+    if (cnt >= static_cast<uint64_t>(kSlotPages)) {  // src/sock/tcpx.h:183-187
+      WARN("received %lu/%d segs, failstop", static_cast<unsigned long>(cnt), kSlotPages);
+      *p->pgtok_cnt = n_toks;
       *result = fail_stop("too many fragments in one task");
       return -1;
     }
     dst_offset += v.frag_size;
-    // Page tokens, run-length coded (src/sock/tcpx.h:190-199).
-    if (*p->pgtok_cnt > 0) {
-      PageToken& prev = p->pgtoks[*p->pgtok_cnt - 1];
-      if (prev.token_start + prev.token_count == v.frag_token) {
-        prev.token_count++;
-        continue;
-      }
-    }
-    // The token list is the slot's, one per flow, and a request may put several chunks on one flow: it is full
-    // when it holds as many runs as a slot holds descriptors.  (The reference zeroes the count per task and so
-    // never gets here; it also forgets the earlier chunks' pages.)
-    if (*p->pgtok_cnt >= static_cast<size_t>(kSlotPages)) {
-      WARN("flow holds %zu page-token runs for one request, the most a slot records; failstop", *p->pgtok_cnt);
-      *result = fail_stop("too many page-token runs on one flow of a request");
-      return -1;
-    }
-    p->pgtoks[*p->pgtok_cnt] = PageToken{v.frag_token, 1};
-    (*p->pgtok_cnt)++;
   }
+  p->cnt_cache = cnt;
+  *p->pgtok_cnt = n_toks;
   if (num_cm == 0) {  // src/sock/tcpx.h:202-209
     WARN("fatal, no cmsg");
     *result = fail_stop("recvmsg returned data without control messages");

@@ -710,8 +710,8 @@ ncclResult_t tcpxFinalize(void) {
   for (int d = 0; d < g.n_devices; ++d) {
     DeviceState* ds = &g.devices[d];
     std::lock_guard<std::mutex> dl(ds->mu);
-    if (ds->comms != 0) {
-      WARN("device %d still has %d open comm(s)", d, ds->comms);
+    if (!ds->comms.empty()) {
+      WARN("device %d still has %zu open comm(s)", d, ds->comms.size());
       rc = ncclInvalidUsage;
       continue;
     }
@@ -731,9 +731,7 @@ ncclResult_t tcpxFinalize(void) {
     if (ds->arena) g.ops->arena_destroy(d, ds->arena);
     ds->arena = nullptr;
     ds->arena_bytes = 0;
-    ds->page_refs.reset();
-    ds->n_pages = 0;
-    ds->pages_outstanding = 0;
+    ds->pages_never_returned = 0;
   }
   if (rc == ncclSuccess) g.initialized = false;
   return rc;
@@ -776,10 +774,7 @@ ncclResult_t tcpxSynthArenaCreate(int dev, size_t bytes, void** base) {
   }
   TCPXCHECK(device_result(g.ops->arena_create(dev, bytes, &ds->arena), "arena_create"));
   ds->arena_bytes = bytes;
-  ds->n_pages = bytes / SLICE_PAGE_SIZE;
-  ds->page_refs.reset(new std::atomic<int32_t>[ds->n_pages]);
-  for (size_t i = 0; i < ds->n_pages; ++i) ds->page_refs[i] = 0;
-  ds->pages_outstanding = 0;
+  ds->pages_never_returned = 0;
   *base = ds->arena;
   return ncclSuccess;
 }
@@ -812,7 +807,7 @@ static ncclResult_t new_comm(int dev, bool passive, Comm** out) {
   c->num_flows = g.flows_per_comm;
   c->use_helper = g.use_helper_thread != 0;
   c->sched.reset(new_flow_scheduler(g.sched_alg));  // src/net_tcpx.cc:1101-1112 (there: at the first progress call)
-  for (int f = 0; f < kMaxFlows; ++f) c->flows[f].sock.device = c->device;
+  for (int f = 0; f < kMaxFlows; ++f) c->flows[f].sock.ledger = &c->ledger;
   c->ctrl_watch.configure(static_cast<uint64_t>(g.timeout_threshold_ns), static_cast<uint64_t>(g.timeout_frequency_ns));
   if (g.task_stats || g.request_stats) c->trace.reset(new TraceBuffer(kTraceEvents));
   *out = c;
@@ -872,7 +867,8 @@ ncclResult_t tcpxAccept_v5(void* listenComm, void** recvComm, ncclNetDeviceHandl
     l->backlog.fetch_add(1, std::memory_order_release);  // the connection stays in the backlog
     return rc;
   }
-  rc = g.device_type == kDeviceHost ? ensure_engine(ds) : ncclSuccess;
+  if (!c->ledger.open(ds->arena_bytes / SLICE_PAGE_SIZE)) rc = ncclSystemError;
+  if (rc == ncclSuccess && g.device_type == kDeviceHost) rc = ensure_engine(ds);
   if (rc == ncclSuccess) rc = unpack_queue_new(l->dev, true, &c->queue);  // tcpxGetDeviceHandle, src/net_tcpx.cc:1452-1471
   if (rc != ncclSuccess) {
     delete c;
@@ -881,7 +877,7 @@ ncclResult_t tcpxAccept_v5(void* listenComm, void** recvComm, ncclNetDeviceHandl
   }
   {
     std::lock_guard<std::mutex> lock(ds->mu);
-    ds->comms++;
+    ds->comms.push_back(c);
   }
   if (c->use_helper) c->helper = std::thread(helper_main, c);
   if (recvDevHandle && *recvDevHandle) {
@@ -1127,7 +1123,9 @@ ncclResult_t tcpxClose(void* oComm) {
            static_cast<unsigned long>(comm->queue->tail));
     unpack_queue_free(comm->queue);
     std::lock_guard<std::mutex> lock(comm->device->mu);
-    comm->device->comms--;
+    std::vector<Comm*>& open = comm->device->comms;
+    open.erase(std::remove(open.begin(), open.end(), comm), open.end());
+    comm->device->pages_never_returned += comm->ledger.outstanding();
   }
   delete comm;
   return ncclSuccess;
@@ -1171,7 +1169,10 @@ ncclResult_t tcpxSynthSetRecvmsgLimit(void* recvComm, uint32_t max_frags_per_rec
 ncclResult_t tcpxSynthOutstandingPages(void* recvComm, uint64_t* pages) {
   Comm* comm = static_cast<Comm*>(recvComm);
   if (!comm || !pages) return ncclInvalidArgument;
-  *pages = comm->device->pages_outstanding.load();
+  DeviceState* ds = comm->device;
+  std::lock_guard<std::mutex> lock(ds->mu);
+  *pages = ds->pages_never_returned;
+  for (const Comm* c : ds->comms) *pages += c->ledger.outstanding();
   return ncclSuccess;
 }
 

@@ -170,6 +170,8 @@ struct DevmemVec {  // struct devmemvec, src/sock/tcpx.h:130-134
 struct DataPipe {  // struct tcpxDataPipe, src/sock/datapipe.h:25-46
   std::vector<char> ctrl_data;           // control-message buffer handed to recvmsg
   std::vector<union loadMeta> scatter_list;  // [kSlotPages]
+  union loadMeta* list;                      // where descriptors go: scatter_list
+  uint64_t list_room;                        // how many fit there
   uint64_t cnt_cache = 0;
   int bytes_cnt = 0;
   size_t* pgtok_cnt = nullptr;
@@ -177,7 +179,44 @@ struct DataPipe {  // struct tcpxDataPipe, src/sock/datapipe.h:25-46
   DataPipe();
 };
 
+struct Comm;
 struct DeviceState;
+
+// The page references that the synthetic kernel keeps for one comm's sockets: each control message hands one to the
+// receiver, SO_DEVMEM_DONTNEED gives it back (devmem TCP keeps a frag's reference with the socket that received it).
+// The thread that receives writes `given`, the thread that consumes writes `back`, so a reference costs a load and a
+// store and no locked instruction (with one counter per page and GPU that both threads and all comms updated, two
+// locked ones per fragment were 9 of the 18.6 ns that a fragment of a bulk message cost the host).  Counted modulo 2^16:
+// a comm holds at most kMaxRequests x kSlotPages = 2^15 references.
+struct PageLedger {
+  struct Page {
+    uint16_t given, back;
+  };
+  Page* pages = nullptr;  // calloc'ed: a page of the arena that is never used costs nothing
+  size_t n_pages = 0;
+  // Both sides' totals, a line each for the thread that counts.
+  alignas(64) std::atomic<uint64_t> given{0};
+  alignas(64) std::atomic<uint64_t> back{0};
+
+  bool open(size_t arena_pages);
+  ~PageLedger() { free(pages); }
+  uint64_t outstanding() const {
+    const uint64_t returned = back.load(std::memory_order_acquire);  // (first: a page is given before it comes back)
+    return given.load(std::memory_order_relaxed) - returned;
+  }
+  // (Relaxed accesses to the two halves of an entry: a page comes back after the request that received it has gone
+  // from one thread to the other through a task ring, which orders the two.)
+  void give(uint32_t page) {
+    uint16_t* g = &pages[page].given;
+    __atomic_store_n(g, static_cast<uint16_t>(__atomic_load_n(g, __ATOMIC_RELAXED) + 1u), __ATOMIC_RELAXED);
+  }
+  bool take_back(uint32_t page) {  // false: not held, freed twice
+    const uint16_t b = __atomic_load_n(&pages[page].back, __ATOMIC_RELAXED);
+    if (b == __atomic_load_n(&pages[page].given, __ATOMIC_RELAXED)) return false;
+    __atomic_store_n(&pages[page].back, static_cast<uint16_t>(b + 1u), __ATOMIC_RELAXED);
+    return true;
+  }
+};
 
 // One data flow's receive queue: what the kernel has for this socket.  recvmsg() hands out at most `max_bytes`
 // and at most the control buffer's worth of fragments, one SCM_DEVMEM_OFFSET control message each, splitting a
@@ -190,9 +229,8 @@ struct DevmemSocket {
   std::vector<tcpxSynthFrag> arrived;
   std::vector<tcpxSynthFrag> rx;
   size_t head = 0;                     // read position in rx
-  size_t payload_frags = 0;            // fragments in rx[head..] with frag_size != 0
   std::atomic<uint32_t> max_frags_per_recvmsg{0};  // 0 = no extra limit
-  DeviceState* device = nullptr;       // page accounting
+  PageLedger* ledger = nullptr;        // the comm's page references
   void push(const tcpxSynthFrag* frags, size_t n);  // takes the lock
   ssize_t recvmsg(struct msghdr* msg, size_t max_bytes);
   // setsockopt(SO_DEVMEM_DONTNEED): gives page references back (src/sock/tcpx.h:299-307).
@@ -209,7 +247,6 @@ ssize_t devmem_recv(DevmemSocket* sock, int size, int offset, DataPipe* pipe, ui
                     ncclResult_t* result);
 
 // ---- requests and tasks -------------------------------------------------------------------------------------------
-struct Comm;
 struct Request;
 
 // A task goes from the proxy thread (which fills it in) to the thread that serves its socket and back (descriptor
@@ -295,6 +332,7 @@ struct Comm {  // struct tcpxComm, src/common.h:159-216
   int num_flows = 0;
   int end_flow_idx = 0;
   FlowData flows[kMaxFlows];
+  PageLedger ledger;  // for the sockets of all flows
   std::unique_ptr<FlowScheduler> sched;  // tcpxComm::flow_mapper: the flows whose task ring has room
   std::mutex ctrl_mu;
   std::deque<CtrlMessage> ctrl_rx;  // the control socket's receive queue: what has arrived (under ctrl_mu)
@@ -349,14 +387,10 @@ struct DeviceState {
   std::mutex mu;
   void* arena = nullptr;
   size_t arena_bytes = 0;
-  std::unique_ptr<std::atomic<int32_t>[]> page_refs;  // references held by the plugin, per arena page
-  size_t n_pages = 0;
-  // Counted up by whoever receives (every recvmsg) and down by whoever consumes: a cache line of its own, or every
-  // count would take the line with the fields around it away from the thread that reads those at every poll.
-  alignas(64) std::atomic<uint64_t> pages_outstanding{0};
-  alignas(64) tcpxuEngine* engine = nullptr;
+  tcpxuEngine* engine = nullptr;
   bool engine_started = false;
-  int comms = 0;
+  std::vector<Comm*> comms;           // open receive comms
+  uint64_t pages_never_returned = 0;  // page references that comms still held when they were closed
   std::vector<QueueBlock> free_blocks;
 };
 
