@@ -10,14 +10,23 @@
 
 namespace tcpx {
 
-DataPipe::DataPipe()
+DataPipe::DataPipe(bool own_list)
     // 2048 control messages of CMSG_SPACE(sizeof(struct iovec)) bytes (src/devcomm/unpack_defs1.h:32-36).
-    : ctrl_data(static_cast<size_t>(kSlotPages) * CMSG_SPACE(sizeof(struct iovec))), scatter_list(kSlotPages),
-      list(scatter_list.data()), list_room(kSlotPages) {}
+    : ctrl_data(static_cast<size_t>(kSlotPages) * CMSG_SPACE(sizeof(struct iovec))), scatter_list(own_list ? kSlotPages : 0),
+      list(scatter_list.data()), list_room(scatter_list.size()) {}
 
 void DevmemSocket::push(const tcpxSynthFrag* frags, size_t n) {
   std::lock_guard<std::mutex> lock(mu);
-  arrived.insert(arrived.end(), frags, frags + n);
+  push_locked(frags, n);
+}
+
+void DevmemSocket::push_locked(const tcpxSynthFrag* frags, size_t n) {
+  if (n < 4) {  // (a range insert costs more than a few appends)
+    for (size_t i = 0; i < n; ++i) arrived.push_back(frags[i]);
+  } else {
+    arrived.insert(arrived.end(), frags, frags + n);
+  }
+  any_arrived.store(!arrived.empty(), std::memory_order_release);
 }
 
 bool PageLedger::open(size_t arena_pages) {
@@ -50,8 +59,11 @@ ssize_t DevmemSocket::recvmsg(struct msghdr* msg, size_t max_bytes) {
   if (head == rx.size()) {  // everything taken over earlier has been received: look for new arrivals
     rx.clear();
     head = 0;
-    std::lock_guard<std::mutex> lock(mu);
-    rx.swap(arrived);
+    if (any_arrived.load(std::memory_order_acquire)) {
+      std::lock_guard<std::mutex> lock(mu);
+      rx.swap(arrived);
+      any_arrived.store(false, std::memory_order_relaxed);
+    }
   }
   // A recvmsg that returns no bytes means "peer closed" to the caller, so empty fragments (which the adversarial
   // workload contains) only ever travel together with a non-empty one.
@@ -67,6 +79,7 @@ ssize_t DevmemSocket::recvmsg(struct msghdr* msg, size_t max_bytes) {
       std::lock_guard<std::mutex> lock(mu);
       rx.insert(rx.end(), arrived.begin(), arrived.end());
       arrived.clear();
+      any_arrived.store(false, std::memory_order_relaxed);
     }
     payload = payload_ahead();
   }
@@ -265,7 +278,7 @@ ssize_t devmem_recv(DevmemSocket* sock, int size, int offset, DataPipe* p, uint6
 
 TaskRing::TaskRing() {
   for (int i = 0; i < kMaxTasks; ++i) {
-    items[i].pipe = new DataPipe;
+    items[i].pipe = new DataPipe(true);
     scatter[i] = items[i].pipe->scatter_list.data();
   }
 }

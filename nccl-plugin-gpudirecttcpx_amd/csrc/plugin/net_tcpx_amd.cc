@@ -222,11 +222,12 @@ ncclResult_t flow_progress(Comm* comm, int flow) {
   for (int served = 0; served < kMaxTasks; ++served) {
     if (tasks->has(kTaskActive)) {
       Task* t = tasks->first(kTaskActive);
-      if (t->offset == 0) {
-        // Nothing received for this task yet: its pipe starts empty.  (Done here, by the thread that serves the
+      if (!t->started) {
+        // Its pipe starts empty, at the byte the task starts at.  (Done here, by the thread that serves the
         // socket, where the reference has the thread that enqueues do it: the pipe then never leaves this thread.)
+        t->started = true;
         t->pipe->cnt_cache = 0;
-        t->pipe->bytes_cnt = 0;
+        t->pipe->bytes_cnt = t->offset;
         t->pipe->pgtoks = t->pgtoks;
         t->pipe->pgtok_cnt = t->pgtok_cnt;
       }
@@ -310,18 +311,60 @@ void helper_main(Comm* comm) {  // persistentSocketThread, src/net_tcpx.cc:252-3
   }
 }
 
-// enqueueTask, src/net_tcpx.cc:1037-1097 (receive part)
-void enqueue_task(Comm* comm, Request* r) {
-  const int flow = r->next_flow;
+// The pending chunk has been taken over, whole or as a task; the request's last one completes its description.
+void chunk_taken(Comm* comm, Request* r) {
   r->next_flow = -1;  // RESET_CTRL
+  r->offset += r->next_size;
+  if (r->size == r->offset) {
+    if (g.device_type == kDeviceHost && r->size != 0) ++comm->to_submit;
+    request_advance(comm, kReqActive);  // REQUEST_INACTIVE -> finish_active
+  }
+}
+
+// A chunk whose control message has been read and whose bytes are there already: received at once, its descriptors
+// written where the GPU will read them, without a task, its ring and a copy from a task's list in between (8 MiB of
+// fragments that are a chunk each: 88 -> 55 us of host time, with the driver's feeding in one pass).  For a flow on which nothing is queued -- a socket
+// delivers in order -- and where the proxy thread serves the sockets itself; with task-level statistics on every chunk
+// is a task, because tasks are what those count.  *got receives the bytes that were there: fewer than the chunk has
+// mean that a task waits for the rest.
+ncclResult_t receive_chunk(Comm* comm, Request* r, int* got) {
+  const int flow = r->next_flow;
+  FlowData* fd = &comm->flows[flow];
+  UnpackSlot* u = &r->slot;
+  DataPipe* p = &comm->direct;
+  u->flows[flow] = flow;
+  p->list = u->mem + u->cnt_cache;
+  p->list_room = static_cast<uint64_t>(kSlotPages) - u->cnt_cache;
+  p->cnt_cache = 0;
+  p->bytes_cnt = 0;
+  p->pgtoks = &u->pgtoks[static_cast<size_t>(flow) * kSlotPages];
+  p->pgtok_cnt = &u->pgtok_cnts[flow];
+  int at = 0;
+  while (at < r->next_size) {
+    ncclResult_t res = ncclSuccess;
+    const ssize_t bytes = devmem_recv(&fd->sock, r->next_size, at, p, static_cast<uint64_t>(r->offset), &res);
+    if (res != ncclSuccess) return res;
+    if (bytes <= 0) break;
+    at += static_cast<int>(bytes);
+  }
+  u->cnt_cache += p->cnt_cache;
+  fd->bytes += static_cast<uint64_t>(at);
+  *got = at;
+  return ncclSuccess;
+}
+
+// enqueueTask, src/net_tcpx.cc:1037-1097 (receive part); the first `received` bytes of the chunk have been received.
+void enqueue_task(Comm* comm, Request* r, int received) {
+  const int flow = r->next_flow;
   const int sz = r->next_size;
   TaskRing* tasks = &comm->flows[flow].tasks;
   Task* t = tasks->next_free();
-  t->op = static_cast<uint16_t>(r->op);
+  t->op = static_cast<uint8_t>(r->op);
   t->data = static_cast<char*>(r->data) + r->offset;
   t->r = r;
   t->result = ncclSuccess;
-  t->offset = 0;
+  t->started = false;
+  t->offset = received;
   t->request_offset = r->offset;
   t->size = sz;
   t->flow = static_cast<uint16_t>(flow);
@@ -339,8 +382,8 @@ void enqueue_task(Comm* comm, Request* r) {
   }
   tp_task(comm, t, kTaskActiveTs);
   tasks->enqueue();  // FREE -> ACTIVE
-  r->offset += sz;
-  if (r->size == r->offset) request_advance(comm, kReqActive);  // REQUEST_INACTIVE -> finish_active
+  ++comm->tasks_live;
+  chunk_taken(comm, r);
 }
 
 // Reaps finished tasks: their descriptors move into the request's slot (src/net_tcpx.cc:1119-1151), and the flows
@@ -377,6 +420,7 @@ ncclResult_t reap_tasks(Comm* comm) {
         u->cnt_cache += t->cnt;
       }
       task_advance(comm, tasks, kTaskInactive);  // INACTIVE -> FREE
+      --comm->tasks_live;
     }
     // Priority = task slots in use: the emptiest flow is served first (src/net_tcpx.cc:1152-1155).
     if (tasks->has_free()) comm->sched->schedule(idx, kMaxTasks - static_cast<int>(tasks->num_free()));
@@ -384,34 +428,40 @@ ncclResult_t reap_tasks(Comm* comm) {
   return ncclSuccess;
 }
 
-ncclResult_t take_control_messages(Comm* comm, bool* enqueued);
+ncclResult_t take_control_messages(Comm* comm, bool* progress);
 ncclResult_t submit_ready_requests(Comm* comm);
 
 // tcpxCommProgress, src/net_tcpx.cc:1099-1308 (receive branch)
 ncclResult_t comm_progress(Comm* comm) {
   if (comm->rq.empty()) return ncclSuccess;
   // One call makes up to kProgressPasses passes of: sockets, reap, control messages.  The reference makes one and
-  // is called again by the next test(); a pass that has just started tasks is followed by another at once here,
-  // because the bytes of a chunk whose control message has been read have usually arrived already and the tasks
-  // they finish make room for the next control messages.
+  // is called again by the next test(); a pass that has just started tasks or received chunks is followed by another at
+  // once here, because the bytes of a chunk whose control message has been read have usually arrived already and the
+  // tasks they finish make room for the next control messages.
   constexpr int kProgressPasses = 4;
-  for (int pass = 0; pass < kProgressPasses; ++pass) {
-    if (!comm->use_helper) {
-      for (int f = 0; f < comm->num_flows; ++f) TCPXCHECK(flow_progress(comm, f));
+  bool progress = true;
+  for (int pass = 0; progress && pass < kProgressPasses; ++pass) {
+    if (comm->tasks_live != 0) {
+      if (!comm->use_helper) {
+        for (int f = 0; f < comm->num_flows; ++f) TCPXCHECK(flow_progress(comm, f));
+      }
+      TCPXCHECK(reap_tasks(comm));
     }
-    TCPXCHECK(reap_tasks(comm));
-    TCPXCHECK(submit_ready_requests(comm));
-    bool enqueued = false;
-    TCPXCHECK(take_control_messages(comm, &enqueued));
-    if (!enqueued || comm->use_helper) break;
+    if (comm->to_submit != 0) TCPXCHECK(submit_ready_requests(comm));
+    progress = false;
+    TCPXCHECK(take_control_messages(comm, &progress));
+    if (comm->use_helper) return ncclSuccess;
   }
+  // What the last pass received whole need not wait for the next call.
+  if (progress && comm->to_submit != 0) TCPXCHECK(submit_ready_requests(comm));
   return ncclSuccess;
 }
 
-ncclResult_t take_control_messages(Comm* comm, bool* enqueued) {
+ncclResult_t take_control_messages(Comm* comm, bool* progress) {
   if (comm->rq.has(kReqPosted)) request_advance(comm, kReqPosted);  // POSTED -> ACTIVE (src/net_tcpx.cc:1158-1180)
 
-  if (!comm->rq.has(kReqActive) || !comm->sched->has_flow()) return ncclSuccess;
+  // (With no task anywhere every flow has room, whatever the scheduler was last told.)
+  if (!comm->rq.has(kReqActive) || (comm->tasks_live != 0 && !comm->sched->has_flow())) return ncclSuccess;
   Request* ar = comm->rq.first(kReqActive);
   if (ar->op != kOpRecv) return ncclSuccess;
 
@@ -419,13 +469,16 @@ ncclResult_t take_control_messages(Comm* comm, bool* enqueued) {
     if (!ctrl_done(ar)) {
       CtrlMessage ctrl;
       bool got_ctrl = false;
-      if (comm->ctrl_local.empty()) {  // take over everything that has arrived: one lock per burst, not per message
+      if (comm->ctrl_next == comm->ctrl_local.size() && comm->ctrl_arrived.load(std::memory_order_acquire)) {
+        // take over everything that has arrived: one lock per burst, not per message
+        comm->ctrl_local.clear();
+        comm->ctrl_next = 0;
         std::lock_guard<std::mutex> lock(comm->ctrl_mu);
         comm->ctrl_local.swap(comm->ctrl_rx);
+        comm->ctrl_arrived.store(false, std::memory_order_relaxed);
       }
-      if (!comm->ctrl_local.empty()) {
-        ctrl = comm->ctrl_local.front();
-        comm->ctrl_local.pop_front();
+      if (comm->ctrl_next < comm->ctrl_local.size()) {
+        ctrl = comm->ctrl_local[comm->ctrl_next++];
         got_ctrl = true;
       }
       // Every look at the control socket counts towards its slowness watch; a message resets it
@@ -472,7 +525,7 @@ ncclResult_t take_control_messages(Comm* comm, bool* enqueued) {
           WARN("no more unpack queue slot, head %lu tail %lu", static_cast<unsigned long>(comm->queue->head),
                static_cast<unsigned long>(comm->queue->tail));
           // The control message is consumed and cannot be re-read: put it back so that a later poll retries.
-          comm->ctrl_local.push_front(ctrl);
+          --comm->ctrl_next;
           ar->next_flow = -1;
           break;
         }
@@ -501,9 +554,19 @@ ncclResult_t take_control_messages(Comm* comm, bool* enqueued) {
     }
     TaskRing* tasks = &comm->flows[ar->next_flow].tasks;
     if (!tasks->has_free()) break;  // "No free space for recv task": retried at the next poll
+    int received = 0;
+    if (comm->receive_at_once && tasks->empty() && ar->next_size > 0) {
+      TCPXCHECK(receive_chunk(comm, ar, &received));
+      if (received == ar->next_size) {
+        ar->size_pending -= received;
+        chunk_taken(comm, ar);
+        *progress = true;
+        continue;
+      }
+    }
     comm->end_flow_idx = ar->next_flow;
-    enqueue_task(comm, ar);
-    *enqueued = true;
+    enqueue_task(comm, ar, received);
+    *progress = true;
   } while (ar->offset < ar->size);
   return ncclSuccess;
 }
@@ -579,6 +642,7 @@ ncclResult_t publish_to_engine(Comm* comm, Request* r, bool* submitted) {
   }
   TCPXCHECK(device_result(rc, "engine_submit"));
   r->published = true;
+  --comm->to_submit;
   r->published_ns = g.clock();
   r->unpack_watch.configure(static_cast<uint64_t>(g.timeout_threshold_ns), static_cast<uint64_t>(g.timeout_frequency_ns));
   comm->unpack_cnt++;
@@ -595,12 +659,22 @@ ncclResult_t publish_to_engine(Comm* comm, Request* r, bool* submitted) {
 // keeps that many slots at the GPU.  Completion is still reported strictly in posting order, by tcpxTest.
 ncclResult_t submit_ready_requests(Comm* comm) {
   if (g.device_type != kDeviceHost) return ncclSuccess;
-  for (uint32_t i = comm->rq.stage_begin(kReqTransmitting), end = comm->rq.stage_end(kReqTransmitting); i != end; ++i) {
+  // (Empty messages pass through this stage without being given to the engine.)
+  const uint32_t begin = comm->rq.stage_begin(kReqTransmitting);
+  if (static_cast<int32_t>(begin - comm->submit_from) > 0) comm->submit_from = begin;
+  bool all_so_far = true;
+  for (uint32_t i = comm->submit_from, end = comm->rq.stage_end(kReqTransmitting); i != end; ++i) {
     Request* r = &comm->rq.items[i % kMaxRequests];
-    if (r->published || r->op != kOpRecv || r->size == 0 || !request_done(r)) continue;
-    bool submitted = false;
-    TCPXCHECK(publish_to_engine(comm, r, &submitted));
-    if (!submitted) break;  // ring full: the younger ones wait behind this one
+    if (!r->published && r->size != 0) {
+      if (!request_done(r)) {
+        all_so_far = false;
+        continue;
+      }
+      bool submitted = false;
+      TCPXCHECK(publish_to_engine(comm, r, &submitted));
+      if (!submitted) break;  // ring full: the younger ones wait behind this one
+    }
+    if (all_so_far) comm->submit_from = i + 1;
   }
   return ncclSuccess;
 }
@@ -616,21 +690,7 @@ int sched_alg_from_name(const char* name, bool* valid) {
 void ctrl_send_batch(Comm* comm, const CtrlMessage* messages, size_t n) {
   std::lock_guard<std::mutex> lock(comm->ctrl_mu);
   comm->ctrl_rx.insert(comm->ctrl_rx.end(), messages, messages + n);
-}
-
-ncclResult_t deliver_fragments(Comm* comm, uint32_t flow, const tcpxSynthFrag* frags, uint32_t n_frags) {
-  const size_t arena = comm->device->arena_bytes;
-  for (uint32_t i = 0; i < n_frags; ++i) {
-    const tcpxSynthFrag& f = frags[i];
-    // The devmem contract: a fragment lies inside the arena and inside one 4 KiB page.
-    if (static_cast<size_t>(f.frag_offset) + f.frag_size > arena ||
-        (f.frag_offset % SLICE_PAGE_SIZE) + f.frag_size > SLICE_PAGE_SIZE) {
-      WARN("fragment %u (offset %u, size %u) breaks the devmem contract", i, f.frag_offset, f.frag_size);
-      return ncclInvalidArgument;
-    }
-  }
-  comm->flows[flow].sock.push(frags, n_frags);
-  return ncclSuccess;
+  comm->ctrl_arrived.store(!comm->ctrl_rx.empty(), std::memory_order_release);
 }
 
 FlowScheduler* new_flow_scheduler(int alg) {
@@ -806,6 +866,7 @@ static ncclResult_t new_comm(int dev, bool passive, Comm** out) {
   c->device = &g.devices[dev];
   c->num_flows = g.flows_per_comm;
   c->use_helper = g.use_helper_thread != 0;
+  c->receive_at_once = !c->use_helper && !g.task_stats;
   c->sched.reset(new_flow_scheduler(g.sched_alg));  // src/net_tcpx.cc:1101-1112 (there: at the first progress call)
   for (int f = 0; f < kMaxFlows; ++f) c->flows[f].sock.ledger = &c->ledger;
   c->ctrl_watch.configure(static_cast<uint64_t>(g.timeout_threshold_ns), static_cast<uint64_t>(g.timeout_frequency_ns));
@@ -1148,15 +1209,22 @@ ncclResult_t tcpxSynthCtrlSend(void* recvComm, uint16_t type, uint16_t flow, uin
                                uint32_t total) {
   Comm* comm = static_cast<Comm*>(recvComm);
   if (!comm || !comm->passive || type > TCPX_CTRL_INLINE) return ncclInvalidArgument;
-  std::lock_guard<std::mutex> lock(comm->ctrl_mu);
-  comm->ctrl_rx.push_back(CtrlMessage{type, flow, size, offset, total});
+  const CtrlMessage message{type, flow, size, offset, total};
+  ctrl_send_batch(comm, &message, 1);
   return ncclSuccess;
 }
 
 ncclResult_t tcpxSynthDeliver(void* recvComm, uint32_t flow, const tcpxSynthFrag* frags, uint32_t n_frags) {
   Comm* comm = static_cast<Comm*>(recvComm);
   if (!comm || !comm->passive || flow >= static_cast<uint32_t>(comm->num_flows) || (!frags && n_frags)) return ncclInvalidArgument;
-  return deliver_fragments(comm, flow, frags, n_frags);
+  for (uint32_t i = 0; i < n_frags; ++i) {
+    if (!keeps_devmem_contract(frags[i], comm->device->arena_bytes)) {
+      WARN("fragment %u (offset %u, size %u) breaks the devmem contract", i, frags[i].frag_offset, frags[i].frag_size);
+      return ncclInvalidArgument;
+    }
+  }
+  comm->flows[flow].sock.push(frags, n_frags);
+  return ncclSuccess;
 }
 
 ncclResult_t tcpxSynthSetRecvmsgLimit(void* recvComm, uint32_t max_frags_per_recvmsg) {

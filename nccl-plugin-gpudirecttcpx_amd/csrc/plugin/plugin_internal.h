@@ -24,7 +24,6 @@
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
-#include <deque>
 #include <memory>
 #include <mutex>
 #include <thread>
@@ -176,7 +175,7 @@ struct DataPipe {  // struct tcpxDataPipe, src/sock/datapipe.h:25-46
   int bytes_cnt = 0;
   size_t* pgtok_cnt = nullptr;
   PageToken* pgtoks = nullptr;
-  DataPipe();
+  explicit DataPipe(bool own_list);  // false: without a scatter_list, for a pipe that is pointed at a slot
 };
 
 struct Comm;
@@ -227,11 +226,13 @@ struct DevmemSocket {
   // the two -- once per burst of deliveries instead of once per recvmsg.
   std::mutex mu;
   std::vector<tcpxSynthFrag> arrived;
+  std::atomic<bool> any_arrived{false};  // `arrived` is not empty: a look at a quiet socket takes no lock
   std::vector<tcpxSynthFrag> rx;
   size_t head = 0;                     // read position in rx
   std::atomic<uint32_t> max_frags_per_recvmsg{0};  // 0 = no extra limit
   PageLedger* ledger = nullptr;        // the comm's page references
-  void push(const tcpxSynthFrag* frags, size_t n);  // takes the lock
+  void push(const tcpxSynthFrag* frags, size_t n);         // takes the lock
+  void push_locked(const tcpxSynthFrag* frags, size_t n);  // the caller holds it
   ssize_t recvmsg(struct msghdr* msg, size_t max_bytes);
   // setsockopt(SO_DEVMEM_DONTNEED): gives page references back (src/sock/tcpx.h:299-307).
   int dontneed(const PageToken* tokens, size_t n);
@@ -257,7 +258,8 @@ struct alignas(64) Task {  // struct tcpxTask, src/work_queue.h:38-59 (receive-s
   int size = 0;
   int offset = 0;
   int request_offset = 0;
-  uint16_t op = 0;
+  uint8_t op = 0;
+  bool started = false;  // its pipe has been set up
   uint16_t flow = 0;
   void* data = nullptr;
   Request* r = nullptr;
@@ -335,9 +337,17 @@ struct Comm {  // struct tcpxComm, src/common.h:159-216
   PageLedger ledger;  // for the sockets of all flows
   std::unique_ptr<FlowScheduler> sched;  // tcpxComm::flow_mapper: the flows whose task ring has room
   std::mutex ctrl_mu;
-  std::deque<CtrlMessage> ctrl_rx;  // the control socket's receive queue: what has arrived (under ctrl_mu)
-  std::deque<CtrlMessage> ctrl_local;  // ... and what the proxy thread has taken over from it, to read without the lock
+  std::vector<CtrlMessage> ctrl_rx;  // the control socket's receive queue: what has arrived (under ctrl_mu)
+  std::atomic<bool> ctrl_arrived{false};  // ctrl_rx is not empty: a look at a quiet control socket takes no lock
+  std::vector<CtrlMessage> ctrl_local;  // ... and what the proxy thread has taken over from it, to read without the lock
+  size_t ctrl_next = 0;                 // the first message of ctrl_local not yet read
   RequestRing rq;
+  // The proxy thread's own view of what there is to do, so that a poll that finds nothing looks at nothing.
+  uint32_t tasks_live = 0;    // tasks enqueued and not yet reaped, all flows
+  uint32_t to_submit = 0;     // transmitting requests that the engine has not been given
+  uint32_t submit_from = 0;   // ring position: every transmitting request before it has been given to the engine
+  bool receive_at_once = false;  // chunks whose bytes are there go straight into the slot (see receive_chunk)
+  DataPipe direct{false};        // the pipe for that
   UnpackQueue* queue = nullptr;
   DeviceState* device = nullptr;
   uint64_t done_seq = 0;
@@ -438,10 +448,13 @@ extern Global g;
 FlowScheduler* new_flow_scheduler(int alg);  // kSchedKaty, or round robin for anything else
 int sched_alg_from_name(const char* name, bool* valid);  // "RR" / "KATY" (exact); anything else is round robin
 
-// The synthetic peer and kernel, for drivers inside the library: many control messages under one lock, and
-// fragments that the caller has already checked against the devmem contract.
+// The synthetic peer and kernel, for drivers inside the library: many control messages under one lock, and the devmem
+// contract (a fragment lies inside the arena and inside one 4 KiB page).
 void ctrl_send_batch(Comm* comm, const CtrlMessage* messages, size_t n);
-ncclResult_t deliver_fragments(Comm* comm, uint32_t flow, const tcpxSynthFrag* frags, uint32_t n_frags);
+inline bool keeps_devmem_contract(const tcpxSynthFrag& f, size_t arena_bytes) {
+  return static_cast<size_t>(f.frag_offset) + f.frag_size <= arena_bytes &&
+         (f.frag_offset % SLICE_PAGE_SIZE) + f.frag_size <= SLICE_PAGE_SIZE;
+}
 
 const tcpxDeviceOps* default_device_ops();  // binds libtcpxu_hip.so, or nullptr (reason logged)
 ncclResult_t device_result(int rc, const char* what);

@@ -7,7 +7,7 @@
 // flight.  Used by tests and by the benchmark to drive the plugin without an interpreter in the loop.
 #include <time.h>
 
-#include <deque>
+#include <mutex>
 #include <vector>
 
 #include "plugin_internal.h"
@@ -15,35 +15,49 @@
 namespace tcpx {
 namespace {
 
-struct Chunk {
-  uint32_t flow, first, count, bytes;
-};
-
-// Runs of consecutive fragments on the same flow.  An empty fragment cannot travel alone (recvmsg reports it
-// together with payload), so it joins the run of the payload fragment before it, or after it at the very start.
-void chunks_of(const tcpxSynthFrag* frags, uint32_t n, uint32_t n_flows, std::vector<Chunk>* out) {
-  out->clear();
-  std::vector<uint32_t> flow(n);
-  int64_t last_payload = -1;
-  uint32_t first_payload_flow = 0;
-  bool any = false;
-  for (uint32_t i = 0; i < n && !any; ++i) {
-    if (frags[i].frag_size > 0) {
-      first_payload_flow = frags[i].flow % n_flows;
-      any = true;
+// The peer and the NIC for one posted request: the fragments of each flow's socket in arrival order (a socket keeps
+// order only within itself, so handing each flow its fragments in one go is what many small deliveries come to), and
+// one control message per chunk, in chunk order.  A chunk is a run of consecutive fragments on the same flow; an empty
+// fragment cannot travel alone (recvmsg reports it together with payload), so it joins the run of the payload fragment
+// before it, or after it at the very start.  One pass, each socket's lock taken once.
+ncclResult_t feed_request(Comm* comm, const tcpxSynthFrag* frags, uint32_t n, uint32_t total, std::vector<CtrlMessage>* ctrl) {
+  const uint32_t n_flows = static_cast<uint32_t>(comm->num_flows);
+  const size_t arena = comm->device->arena_bytes;
+  auto flow_of = [n_flows](const tcpxSynthFrag& f) { return f.flow < n_flows ? f.flow : f.flow % n_flows; };
+  uint32_t first_payload = 0;
+  while (first_payload < n && frags[first_payload].frag_size == 0) ++first_payload;
+  if (first_payload == n) return ncclSuccess;
+  ctrl->clear();
+  {
+    std::unique_lock<std::mutex> locks[kMaxFlows];
+    uint32_t offset = 0, first = 0, bytes = 0;
+    uint32_t flow = flow_of(frags[first_payload]);
+    auto close_chunk = [&](uint32_t end) {
+      DevmemSocket& sock = comm->flows[flow].sock;
+      if (!locks[flow].owns_lock()) locks[flow] = std::unique_lock<std::mutex>(sock.mu);
+      sock.push_locked(frags + first, end - first);
+      ctrl->push_back(CtrlMessage{TCPX_CTRL_NORMAL, static_cast<uint16_t>(flow), bytes, offset, total});
+      offset += bytes;
+    };
+    for (uint32_t i = 0; i < n; ++i) {
+      const tcpxSynthFrag& f = frags[i];
+      if (!keeps_devmem_contract(f, arena)) {
+        WARN("fragment %u (offset %u, size %u) breaks the devmem contract", i, f.frag_offset, f.frag_size);
+        return ncclInvalidArgument;
+      }
+      const uint32_t on = f.frag_size != 0 ? flow_of(f) : flow;
+      if (on != flow) {
+        close_chunk(i);
+        flow = on;
+        first = i;
+        bytes = 0;
+      }
+      bytes += f.frag_size;
     }
+    close_chunk(n);
   }
-  if (!any) return;
-  for (uint32_t i = 0; i < n; ++i) {
-    if (frags[i].frag_size > 0) last_payload = i;
-    flow[i] = last_payload >= 0 ? frags[last_payload].flow % n_flows : first_payload_flow;
-  }
-  for (uint32_t i = 0; i < n;) {
-    uint32_t j = i + 1, bytes = frags[i].frag_size;
-    while (j < n && flow[j] == flow[i]) bytes += frags[j++].frag_size;
-    out->push_back(Chunk{flow[i], i, j - i, bytes});
-    i = j;
-  }
+  ctrl_send_batch(comm, ctrl->data(), ctrl->size());
+  return ncclSuccess;
 }
 
 double now_s() {
@@ -68,71 +82,58 @@ extern "C" ncclResult_t tcpxSynthRunRequests(void* recvComm, const tcpxSynthFrag
   TCPXCHECK(tcpxRegMr(comm, dst_base, static_cast<int>(dst_bytes), NCCL_PTR_CUDA, &mhandle));
   struct Posted {
     void* request;
-    uint32_t index;
     double fed;
   };
-  std::deque<Posted> posted;
-  std::vector<Chunk> chunks;
+  Posted posted[kMaxRequests];  // request i of the call at i % kMaxRequests
   std::vector<CtrlMessage> ctrl;
-  std::vector<tcpxSynthFrag> by_flow[kMaxFlows];
-  uint32_t next = 0;
+  uint32_t next = 0, oldest = 0;
   ncclResult_t rc = ncclSuccess;
   const double t0 = now_s();
-  double deadline = t0 + 1e-3 * timeout_ms;
-  const uint32_t n_flows = static_cast<uint32_t>(comm->num_flows);
-  while (rc == ncclSuccess && (next < n_requests || !posted.empty())) {
-    while (rc == ncclSuccess && next < n_requests && posted.size() < window) {
+  // The clock is looked at once in kPollsPerLook polls that find nothing; a look costs as much as a poll.
+  constexpr uint32_t kPollsPerLook = 64;
+  uint32_t polls = 0;
+  double waiting_since = 0;
+  while (rc == ncclSuccess && oldest < n_requests) {
+    while (rc == ncclSuccess && next < n_requests && next - oldest < window) {
       const tcpxSynthRequest& r = requests[next];
       void* data = static_cast<char*>(dst_base) + r.dst_off;
       int size = static_cast<int>(r.bytes), tag = 0;
-      void* request = nullptr;
-      if ((rc = tcpxIrecv_v5(comm, 1, &data, &size, &tag, &mhandle, &request)) != ncclSuccess) break;
-      const tcpxSynthFrag* f = frags + r.first_desc;
-      if (r.bytes == 0) {
-        rc = tcpxSynthCtrlSend(comm, TCPX_CTRL_INLINE, 0, 0, 0, 0);
-      } else {
-        // The peer's control messages, one per chunk, in chunk order; then what the kernel has for each flow: the
-        // flow's fragments in arrival order (a socket keeps order only within itself, so handing each flow its
-        // fragments in one piece is what many small deliveries come to).
-        chunks_of(f, r.n_descs, n_flows, &chunks);
-        ctrl.clear();
-        for (uint32_t k = 0; k < n_flows; ++k) by_flow[k].clear();
-        uint32_t offset = 0;
-        for (const Chunk& c : chunks) {
-          ctrl.push_back(CtrlMessage{TCPX_CTRL_NORMAL, static_cast<uint16_t>(c.flow), c.bytes, offset, r.bytes});
-          offset += c.bytes;
-          by_flow[c.flow].insert(by_flow[c.flow].end(), f + c.first, f + c.first + c.count);
-        }
-        ctrl_send_batch(comm, ctrl.data(), ctrl.size());
-        for (uint32_t k = 0; rc == ncclSuccess && k < n_flows; ++k)
-          if (!by_flow[k].empty()) rc = deliver_fragments(comm, k, by_flow[k].data(), static_cast<uint32_t>(by_flow[k].size()));
-      }
-      posted.push_back(Posted{request, next, now_s()});
+      Posted& p = posted[next % kMaxRequests];
+      if ((rc = tcpxIrecv_v5(comm, 1, &data, &size, &tag, &mhandle, &p.request)) != ncclSuccess) break;
+      rc = r.bytes == 0 ? tcpxSynthCtrlSend(comm, TCPX_CTRL_INLINE, 0, 0, 0, 0)
+                        : feed_request(comm, frags + r.first_desc, r.n_descs, r.bytes, &ctrl);
+      if (latency_s) p.fed = now_s();
       ++next;
     }
-    if (rc != ncclSuccess || posted.empty()) break;
+    if (rc != ncclSuccess) break;
     int done = 0, size = 0;
-    if ((rc = tcpxTest(posted.front().request, &done, &size)) != ncclSuccess) break;
+    void* request = posted[oldest % kMaxRequests].request;
+    if ((rc = tcpxTest(request, &done, &size)) != ncclSuccess) break;
     if (done) {
-      if (latency_s) latency_s[posted.front().index] = now_s() - posted.front().fed;
+      if (latency_s) latency_s[oldest] = now_s() - posted[oldest % kMaxRequests].fed;
       // NCCL's proxy flushes a finished receive before it hands the buffer on (iflush takes the request in the
       // request slot and answers with its size, src/net_tcpx.cc:946-954), then reports the slot consumed.
-      const tcpxSynthRequest& fr = requests[posted.front().index];
+      const tcpxSynthRequest& fr = requests[oldest];
       void* fdata = static_cast<char*>(dst_base) + fr.dst_off;
       int fsize = -1;
-      void* freq = posted.front().request;
+      void* freq = request;
       if ((rc = tcpxIflush_v5(comm, 1, &fdata, &fsize, &mhandle, &freq)) != ncclSuccess) break;
       if (fsize != static_cast<int>(fr.bytes)) {
         WARN("iflush answered size %d for a request of %u bytes", fsize, fr.bytes);
         rc = ncclInternalError;
         break;
       }
-      if ((rc = tcpxIrecvConsumed(comm, 1, posted.front().request)) != ncclSuccess) break;
-      posted.pop_front();
-      deadline = now_s() + 1e-3 * timeout_ms;
-    } else if (now_s() > deadline) {
-      WARN("request %u did not complete within %u ms", posted.front().index, timeout_ms);
-      rc = ncclInternalError;
+      if ((rc = tcpxIrecvConsumed(comm, 1, request)) != ncclSuccess) break;
+      ++oldest;
+      polls = 0;
+    } else if (++polls % kPollsPerLook == 0) {
+      const double now = now_s();
+      if (polls == kPollsPerLook) {
+        waiting_since = now;
+      } else if (now > waiting_since + 1e-3 * timeout_ms) {
+        WARN("request %u did not complete within %u ms", oldest, timeout_ms);
+        rc = ncclInternalError;
+      }
     }
   }
   if (seconds) *seconds = now_s() - t0;
