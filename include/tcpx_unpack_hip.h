@@ -223,20 +223,17 @@ int tcpxuEngineRunning(tcpxuEngine* engine, int* running);
 /* tcpxuEngineSubmit for callers that cannot allocate and cannot keep a persistent kernel: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the reference.
  * Unpacks one slot -- `n_descs` descriptors (at most TCPXU_SLOT_PAGES = 2048; more is TCPXU_INVALID_ARGUMENT and
- * nothing is launched) at `descs_dev`, from `bounce_base` into `dst_base` -- with ordinary launches on `stream`
- * (a hipStream_t, NULL = the default stream): the engine's worker workgroups over tickets that a small kernel
- * writes first, and the workgroup that finishes the slot's last ticket stores `done_value` to `*done_flag_dev`
- * (device-visible 8-byte word, e.g. the alias of mapped host memory; may be NULL when stream order is all the
- * caller needs).  Asynchronous.  It calls no hipMalloc, hipFree or other allocating routine: ticket records,
- * ticket cursor and done counters live in a fixed array of device memory inside the library (17 KiB, held by
- * every GPU the library runs on until the process ends), which every call on a GPU shares and which each call
- * clears with its own first kernel.  Calls that overlap on one GPU (two streams, two threads) race on that
- * array: issue them on one stream, or order them otherwise.  (A workgroup that finds its ticket overwritten by
- * such a race gives up after 65536 looks and stores the complement of `done_value` to the completion word, so that
- * a poller is not left waiting; the slot's bytes are then not all there.)
+ * nothing is launched) at `descs_dev`, from `bounce_base` into `dst_base` -- with an ordinary launch on `stream`
+ * (a hipStream_t, NULL = the default stream): one kernel, whose last workgroup to finish stores `done_value` to
+ * `*done_flag_dev` (device-visible 8-byte word, e.g. the alias of mapped host memory; may be NULL when stream order is
+ * all the caller needs: the call is then tcpxuUnpackBatch).  Asynchronous.  It calls no hipMalloc, hipFree or other
+ * allocating routine: what counts the workgroups lives in a fixed array of device memory inside the library (72 KiB,
+ * held by every GPU the library runs on until the process ends), a set of counters for each of 64 calls in turn, which
+ * a call leaves as it found it.  Calls may overlap on a GPU (two streams, two threads, a replayed graph beside an
+ * ordinary call) as long as fewer than 64 calls after a call are made while it is under way.
  * Under HIP graph capture: make one ordinary call on the device first -- it looks up the array's address and loads
- * the kernels' code, which do not belong under capture -- then capture; a replay launches the same two kernels
- * with the same arguments. */
+ * the kernels' code, which do not belong under capture -- then capture; a replay launches the same kernel with the
+ * same arguments. */
 int tcpxuUnpackSlotNoAlloc(int device, const void* bounce_base, void* dst_base, const void* descs_dev,
                            uint32_t n_descs, void* done_flag_dev, uint64_t done_value, void* stream);
 

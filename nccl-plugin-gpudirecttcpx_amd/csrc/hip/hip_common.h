@@ -14,7 +14,27 @@ constexpr int kMaxDevices = 64;
 void set_error(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
 int use_device(int device);            // hipSetDevice + cache properties
 int device_compute_units(int device);  // valid after use_device
-void batch_geometry(int device, uint64_t n_descs, uint32_t* descs_per_wg, uint64_t* n_batches, uint32_t* grid);
+
+// Engine calls arrive on threads that belong to somebody else (NCCL's proxy thread calls tcpxTest, which may have
+// to relaunch the kernel): the calling thread's current device is put back when the call returns.
+class DeviceScope {
+ public:
+  explicit DeviceScope(int device) {
+    if (hipGetDevice(&saved_) != hipSuccess) saved_ = -1;
+    rc_ = use_device(device);
+    if (saved_ == device) saved_ = -1;  // nothing to put back
+  }
+  ~DeviceScope() {
+    if (saved_ >= 0) (void)hipSetDevice(saved_);
+  }
+  int rc() const { return rc_; }
+  DeviceScope(const DeviceScope&) = delete;
+  DeviceScope& operator=(const DeviceScope&) = delete;
+
+ private:
+  int saved_ = -1;
+  int rc_ = TCPXU_SUCCESS;
+};
 
 }  // namespace tcpxu
 

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -28,64 +29,86 @@ void set_error(const char* fmt, ...) {
 
 namespace {
 
-constexpr uint32_t kMaxDescsPerWg = 64;
-// Twelve wavefronts to a workgroup, one fragment each: 128 chunks of 8 MiB in one launch move 70.3 % of the HBM
-// roofline this way, 69.6 % with eight wavefronts and eight descriptors, 67-68 % with four wavefronts taking two to
-// four fragments each in turn, 65-68 % with sixteen.
-#ifndef TCPXU_BATCH_THREADS
-#define TCPXU_BATCH_THREADS 768
-#endif
-constexpr int kBatchThreads = TCPXU_BATCH_THREADS;
-constexpr int kBatchWaves = kBatchThreads / kWaveLanes;
-
-// Launch-per-batch unpack.  A workgroup takes `descs_per_wg` consecutive descriptors at a time, stages them in
-// LDS with one 16-byte load per thread, then its twelve wavefronts take one fragment each (a short list is cut into
-// batches of four or eight).  The descriptors of the workgroup's next batch are fetched into registers before the
-// current batch is copied and go into the other of two LDS stages, so that a batch costs one barrier and no exposed
-// descriptor fetch.
-__global__ __launch_bounds__(kBatchThreads) void unpack_batch_kernel(const uint8_t* __restrict__ bounce,
-                                                                   uint8_t* __restrict__ dst,
-                                                                   const tcpxuLoadMeta* __restrict__ descs,
-                                                                   uint64_t n_descs, uint32_t descs_per_wg,
-                                                                   uint64_t n_batches) {
-  // A stage holds the batch at [1, cnt] and, around it, the last descriptor of the batch before and the first of the
-  // batch after (where the list has them): the fragments at the two ends of a batch share destination lines with
-  // them like any other neighbours, and the workgroup that copies the neighbouring batch sees the same pairs.
-  __shared__ tcpxuLoadMeta staged[2][kMaxDescsPerWg + 2];
-  const uint32_t tid = threadIdx.x;
-  const uint32_t lane = tid & (kWaveLanes - 1);
-  const uint32_t wave = tid / kWaveLanes;
-  const uint64_t n_slots = (n_batches + 7) / 8 * 8;  // work-item indices, some of which name no batch
-
-  // Batch number and descriptor count of work item `wg` (count 0: none), and this thread's descriptor of it.
-  auto batch_of = [&](uint64_t wg, uint64_t* first) -> uint32_t {
-    if (wg >= n_slots) return 0;
-    const uint64_t batch = xcd_contiguous_index(wg, n_batches);
-    if (batch >= n_batches) return 0;
-    *first = batch * descs_per_wg;
-    return static_cast<uint32_t>(std::min<uint64_t>(descs_per_wg, n_descs - *first));
-  };
-  auto fetch = [&](uint64_t first, uint32_t cnt) -> u32x4 {  // thread t: descriptor first - 1 + t
-    const uint64_t one_past = first + tid;
-    const bool there = cnt != 0 && tid < cnt + 2 && one_past >= 1 && one_past <= n_descs;
-    return there ? *reinterpret_cast<const u32x4*>(descs + one_past - 1) : u32x4{0, 0, 0, 0};
-  };
-
-  uint64_t wg = blockIdx.x, first = 0;
-  uint32_t cnt = batch_of(wg, &first);
-  u32x4 raw = fetch(first, cnt);
-  for (uint32_t stage = 0; wg < n_slots; stage ^= 1u) {
-    if (tid < cnt + 2) *reinterpret_cast<u32x4*>(&staged[stage][tid]) = raw;
-    const uint32_t cnt_now = cnt;
-    const bool has_before = first > 0, has_after = first + cnt < n_descs;
-    wg += gridDim.x;
-    cnt = batch_of(wg, &first);
-    raw = fetch(first, cnt);  // in flight while this batch is copied
-    __syncthreads();          // the stage is complete; every wavefront has left the stage written two batches ago
-    wave_copy_descriptors(staged[stage] + 1, cnt_now, wave, kBatchWaves, cnt_now, bounce, dst, lane, [] {}, has_before,
-                          has_after);
-  }
+// Launch-per-batch unpack: one wavefront per descriptor, four to a workgroup, as many workgroups as it takes.
+//
+// What bounds a short list is the chain launch -> descriptor -> payload -> store, each link a trip to memory; what
+// bounds a long one is the memory system, and for short fragments how many wavefronts keep loads in flight.  Hence no
+// LDS, no barrier and nothing carried from one fragment to the next: the descriptors go from the load into scalar
+// registers, every wavefront of the 32 that a compute unit holds has a fragment of its own, and the dispatcher hands
+// out new ones as they finish.  (Against workgroups of twelve wavefronts that staged their batch's descriptors in LDS,
+// where a list of up to 8192 kept four of the twelve busy: 16 fragments 2.9 -> 2.4 us a launch (what the host needs for
+// one), 4 MiB of wire fragments 5.1 -> 4.3 us, 8 MiB 6.6 -> 5.0, 16 MiB 10.0 -> 7.0, 64 MiB 23.6 -> 22.4; 256 MiB of
+// 1.8 KiB fragments 126-140 -> 99 us = 5.4 TB/s r+w, which wants all 32 wavefronts: with 16 resident it takes 136 us.
+// Whole pages by the half GiB move 2 % faster with 16 resident, 190 against 194 us; the list does not say which they
+// are.  Half a fragment per wavefront, or two wavefronts to a workgroup, measured no better for short lists.)
+constexpr uint32_t kBatchWaves = 4;
+constexpr uint32_t kBatchThreads = kBatchWaves * kWaveLanes;
+__global__ __launch_bounds__(kBatchThreads) __attribute__((amdgpu_waves_per_eu(8))) void unpack_batch_kernel(
+    const uint8_t* __restrict__ bounce, uint8_t* __restrict__ dst, const tcpxuLoadMeta* __restrict__ descs,
+    uint64_t n_descs, uint64_t first_group, uint32_t n_groups) {
+  const uint32_t lane = threadIdx.x & (kWaveLanes - 1);
+  const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWaveLanes)));
+  // Neighbouring groups go to the same XCD: they share a destination line and, in mapped memory, the line that their
+  // descriptors come in.
+  const uint64_t group = xcd_contiguous_index(blockIdx.x, n_groups);
+  if (group >= n_groups) return;
+  const uint64_t i = (first_group + group) * kBatchWaves + wave;
+  if (i < n_descs) copy_descriptor(bounce, dst, descs, n_descs, i, lane);
 }
+
+// One slot with a completion word (tcpxuUnpackSlotNoAlloc): the same, and the workgroup that finishes last writes the
+// word.  Counting is two more trips to memory at the end of the chain; they are kept short by counting per workgroup in
+// LDS first and, where many workgroups would queue up at one counter, in eight counters before the last (270 workgroups
+// of a 4 MiB slot: 7.9 us a call with one counter, 6.4 with eight and one; 16 fragments: 4.5 and 4.9).  The last one at
+// a counter sets it back to zero, so that the next call finds it as this one did.
+constexpr uint32_t kSlotSubCounters = 8;
+constexpr uint32_t kSlotOneCounterGroups = 64;  // workgroups up to which one counter is the faster way (69: even)
+struct SlotCounters {
+  struct alignas(128) Line {
+    uint32_t count;
+  };
+  Line sub[kSlotSubCounters];
+  Line top;
+};
+__global__ __launch_bounds__(kBatchThreads) __attribute__((amdgpu_waves_per_eu(8))) void unpack_slot_kernel(
+    const uint8_t* __restrict__ bounce, uint8_t* __restrict__ dst, const tcpxuLoadMeta* __restrict__ descs,
+    uint32_t n_descs, uint32_t n_groups, uint64_t* done_flag, uint64_t done_value, SlotCounters* counters) {
+  __shared__ uint32_t waves_done;
+  const uint32_t lane = threadIdx.x & (kWaveLanes - 1);
+  const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWaveLanes)));
+  if (threadIdx.x == 0) waves_done = 0;
+  __syncthreads();
+  const uint32_t group = static_cast<uint32_t>(xcd_contiguous_index(blockIdx.x, n_groups));
+  const uint32_t i = group * kBatchWaves + wave;
+  if (group < n_groups && i < n_descs) copy_descriptor(bounce, dst, descs, n_descs, i, lane);
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // this wavefront's write-through stores are acknowledged
+  if (lane != 0) return;
+  // Every count is a read-modify-write at agent scope that follows the acknowledgement of the stores it stands for.
+  auto last_at = [](uint32_t* counter, uint32_t of) {
+    if (__hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u != of) return false;
+    __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+  };
+  if (__hip_atomic_fetch_add(&waves_done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) + 1u != kBatchWaves) return;
+  uint32_t at_top = gridDim.x;
+  if (n_groups > kSlotOneCounterGroups) {
+    // The grid is a multiple of eight workgroups, so each of the eight counters has an eighth of them.
+    static_assert(kSlotSubCounters == 8, "the grid is rounded up to a multiple of eight");
+    if (!last_at(&counters->sub[blockIdx.x % kSlotSubCounters].count, gridDim.x / kSlotSubCounters)) return;
+    at_top = kSlotSubCounters;
+  }
+  if (last_at(&counters->top.count, at_top)) __hip_atomic_store(done_flag, done_value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// An empty slot: nothing to copy, only the word.
+__global__ void complete_empty_slot_kernel(uint64_t* done_flag, uint64_t done_value) {
+  __hip_atomic_store(done_flag, done_value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The counters, in a fixed array of device memory: a set for each of kSlotCalls calls in turn, so that calls may overlap
+// on a GPU (two streams, a call beside a replayed graph) as long as fewer than that many are under way.  In host code
+// the name is only a handle for hipGetSymbolAddress; kernels get the address it returns.
+constexpr uint32_t kSlotCalls = 64;
+static __device__ SlotCounters slot_counters[kSlotCalls];
 
 struct DeviceProps {
   bool valid = false;
@@ -93,12 +116,6 @@ struct DeviceProps {
   char name[256] = "";
 };
 DeviceProps g_props[kMaxDevices];
-
-int env_int(const char* name, int fallback) {
-  const char* v = getenv(name);
-  if (!v || !*v) return fallback;
-  return atoi(v);
-}
 
 }  // namespace
 
@@ -119,29 +136,6 @@ int use_device(int device) {
 }
 
 int device_compute_units(int device) { return g_props[device].compute_units; }
-
-// Grid geometry of the launch-per-batch kernel: enough descriptors per workgroup to amortise the staging
-// barrier, few enough that a small slot still spreads over the whole GPU.
-void batch_geometry(int device, uint64_t n_descs, uint32_t* descs_per_wg, uint64_t* n_batches, uint32_t* grid) {
-  const uint64_t cus = static_cast<uint64_t>(std::max(1, g_props[device].compute_units));
-  uint32_t dpw = static_cast<uint32_t>(env_int("TCPXU_DESCS_PER_WG", 0));
-  if (dpw == 0) {
-    // Aim for about 8 workgroups per compute unit, and at most one fragment per wavefront.
-    const uint64_t want_wgs = cus * 8;
-    const uint64_t d = (n_descs + want_wgs - 1) / want_wgs;
-    dpw = d <= 4 ? 4 : d <= 8 ? 8 : static_cast<uint32_t>(kBatchWaves);
-  }
-  dpw = std::min(std::max(dpw, 1u), kMaxDescsPerWg);
-  const uint64_t batches = (n_descs + dpw - 1) / dpw;
-  const uint64_t per_xcd = (batches + 7) / 8;
-  // One batch per workgroup up to 128 workgroups per compute unit; beyond that workgroups take several batches in
-  // turn.  Letting the dispatcher hand out batches balances the compute units better than a grid that just fills
-  // them and strides (1 GiB of 4 KiB fragments: 5.34 against 5.09 TB/s r+w with 16 workgroups per compute unit).
-  const uint64_t max_grid = cus * static_cast<uint64_t>(std::max(1, env_int("TCPXU_BATCH_WGS_PER_CU", 128)));
-  *descs_per_wg = dpw;
-  *n_batches = batches;
-  *grid = static_cast<uint32_t>(std::min<uint64_t>(per_xcd * 8, std::max<uint64_t>(max_grid, 8)));
-}
 
 }  // namespace tcpxu
 
@@ -307,7 +301,7 @@ int tcpxuVisibleFree(int device, void* host_ptr) {
 
 void tcpxuVisibleFlush(void) { __builtin_ia32_sfence(); }
 
-static int launch_batch(int device, const void* bounce_base, void* dst_base, const tcpxuLoadMeta* descs,
+static int launch_batch(const void* bounce_base, void* dst_base, const tcpxuLoadMeta* descs,
                         uint64_t n_descs, hipStream_t stream) {
   if (n_descs == 0) return TCPXU_SUCCESS;
   if (!bounce_base || !dst_base || !descs) {
@@ -318,20 +312,73 @@ static int launch_batch(int device, const void* bounce_base, void* dst_base, con
     set_error("descriptor array must be 16-byte aligned");
     return TCPXU_INVALID_ARGUMENT;
   }
-  uint32_t dpw, grid;
-  uint64_t batches;
-  batch_geometry(device, n_descs, &dpw, &batches, &grid);
-  hipLaunchKernelGGL(unpack_batch_kernel, dim3(grid), dim3(kBatchThreads), 0, stream,
-                     static_cast<const uint8_t*>(bounce_base), static_cast<uint8_t*>(dst_base), descs, n_descs, dpw,
-                     batches);
-  TCPXU_HIP(hipGetLastError());
+  uint64_t groups = (n_descs + kBatchWaves - 1) / kBatchWaves;
+  // (A launch holds fewer than 2^32 threads: a list of more than 32 Mi descriptors takes several.)
+  constexpr uint64_t kGroupsPerLaunch = 1ull << 23;
+  for (uint64_t first = 0; first < groups; first += kGroupsPerLaunch) {
+    uint32_t here = static_cast<uint32_t>(std::min(groups - first, kGroupsPerLaunch));
+    void* args[] = {&bounce_base, &dst_base, &descs, &n_descs, &first, &here};
+    TCPXU_HIP(hipLaunchKernel(reinterpret_cast<const void*>(unpack_batch_kernel), dim3((here + 7) / 8 * 8), dim3(kBatchThreads), args, 0, stream));
+  }
   return TCPXU_SUCCESS;
 }
 
 int tcpxuUnpackBatch(int device, const void* bounce_base, void* dst_base, const tcpxuLoadMeta* descs,
                      uint64_t n_descs, void* stream) {
   TCPXU_TRY(use_device(device));
-  return launch_batch(device, bounce_base, dst_base, descs, n_descs, static_cast<hipStream_t>(stream));
+  return launch_batch(bounce_base, dst_base, descs, n_descs, static_cast<hipStream_t>(stream));
+}
+
+// The address of the counters on each device, asked for once per device with that device current.
+static std::atomic<SlotCounters*> g_slot_counters[kMaxDevices];
+static std::atomic<uint32_t> g_slot_calls[kMaxDevices];
+
+static int next_slot_counters(int device, SlotCounters** out) {
+  SlotCounters* all = g_slot_counters[device].load(std::memory_order_acquire);
+  if (!all) {  // (two threads may both ask; they get the same answer)
+    void* p = nullptr;
+    TCPXU_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(slot_counters)));
+    if (!p) {
+      set_error("the slot counters have no address on device %d", device);
+      return TCPXU_INTERNAL_ERROR;
+    }
+    all = static_cast<SlotCounters*>(p);
+    g_slot_counters[device].store(all, std::memory_order_release);
+  }
+  *out = all + g_slot_calls[device].fetch_add(1, std::memory_order_relaxed) % kSlotCalls;
+  return TCPXU_SUCCESS;
+}
+
+int tcpxuUnpackSlotNoAlloc(int device, const void* bounce_base, void* dst_base, const void* descs_dev,
+                           uint32_t n_descs, void* done_flag_dev, uint64_t done_value, void* stream) {
+  if (n_descs > TCPXU_SLOT_PAGES) {
+    set_error("%u descriptors exceed the %d of one slot, the most this entry point serves", n_descs, TCPXU_SLOT_PAGES);
+    return TCPXU_INVALID_ARGUMENT;
+  }
+  if (reinterpret_cast<uintptr_t>(done_flag_dev) % 8 != 0 || (done_flag_dev && done_value == 0)) {
+    set_error("the completion word must be 8-byte aligned and its value nonzero");
+    return TCPXU_INVALID_ARGUMENT;
+  }
+  if (n_descs > 0 && (!bounce_base || !dst_base || !descs_dev || reinterpret_cast<uintptr_t>(descs_dev) % 16 != 0)) {
+    set_error("unpack needs bounce, destination and a 16-byte aligned descriptor address");
+    return TCPXU_INVALID_ARGUMENT;
+  }
+  DeviceScope scope(device);
+  TCPXU_TRY(scope.rc());
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  // Without a completion word the end of the launch says everything.
+  if (!done_flag_dev) return launch_batch(bounce_base, dst_base, static_cast<const tcpxuLoadMeta*>(descs_dev), n_descs, s);
+  if (n_descs == 0) {
+    void* args[] = {&done_flag_dev, &done_value};
+    TCPXU_HIP(hipLaunchKernel(reinterpret_cast<const void*>(complete_empty_slot_kernel), dim3(1), dim3(1), args, 0, s));
+    return TCPXU_SUCCESS;
+  }
+  SlotCounters* counters = nullptr;
+  TCPXU_TRY(next_slot_counters(device, &counters));
+  uint32_t groups = (n_descs + kBatchWaves - 1) / kBatchWaves;
+  void* args[] = {&bounce_base, &dst_base, &descs_dev, &n_descs, &groups, &done_flag_dev, &done_value, &counters};
+  TCPXU_HIP(hipLaunchKernel(reinterpret_cast<const void*>(unpack_slot_kernel), dim3((groups + 7) / 8 * 8), dim3(kBatchThreads), args, 0, s));
+  return TCPXU_SUCCESS;
 }
 
 }  // extern "C"

@@ -331,136 +331,45 @@ __device__ __forceinline__ CopyRound first_round_of(const uint8_t* src, uint8_t*
   return c;
 }
 
-// Splits a fragment that is not tiny (all arguments wave-uniform) into rounds of 1..kVecPerRound vectors.
-// Fragments of the wire format (at most 4 KiB) have exactly one round; the first round of a longer fragment
-// copies its edge bytes and its shared line.
-struct FragmentRounds {
-  uint32_t nvec_left = 0;  // vectors not yet handed out
-
-  __device__ __forceinline__ CopyRound first_round(const uint8_t* src, uint8_t* dst, uint32_t len, bool share_prev,
-                                                   bool share_next, const uint8_t* src_next, uint32_t lane) {
-    const FragmentPlan p = plan_fragment(reinterpret_cast<uintptr_t>(dst), len, share_prev, share_next);
-    return first_round_of(src, dst, src_next, len, share_next, p.start_off, p.end_off, p.head, p.tail, p.nvec, lane,
-                          &nvec_left);
+// Copies descriptor i of a list of n with the calling wavefront (all arguments wave-uniform but `lane`): what the
+// kernels that are launched per list do.  Lanes 0 to 2 read the descriptor before it, its own and the one after it,
+// one load for the three, and hand them over through scalar registers: nothing is staged, nobody waits at a barrier.
+// A fragment that is longer than a round takes several, the first with its edges and its shared line.
+__device__ __forceinline__ void copy_descriptor(const uint8_t* bounce, uint8_t* dst, const tcpxuLoadMeta* descs, uint64_t n,
+                                                uint64_t i, uint32_t lane) {
+  u32x4 d = {0u, 0u, 0u, 0u};
+  const uint64_t at = i + lane - 1u;  // (wraps around before the first: not below n either)
+  if (lane < 3 && at < n) d = *reinterpret_cast<const u32x4*>(descs + at);
+  auto word = [&](int of, int k) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(d[k]), of)); };
+  auto place = [&](int of) { return reinterpret_cast<uint64_t>(dst) + ((static_cast<uint64_t>(word(of, 3)) << 32) | word(of, 2)); };
+  constexpr int kPrev = 0, kOwn = 1, kNext = 2;
+  const uint32_t len = word(kOwn, 1);
+  if (len == 0) return;
+  const uint64_t to = place(kOwn);
+  const uint8_t* from = bounce + word(kOwn, 0);
+  uint8_t* const to_ptr = reinterpret_cast<uint8_t*>(to);
+  if (fragment_is_tiny(to_ptr, len)) {
+    copy_tiny_fragment(from, to_ptr, len, lane);
+    return;
   }
-  __device__ __forceinline__ bool more() const { return nvec_left != 0; }
-  __device__ __forceinline__ CopyRound next_round(const CopyRound& prev) {
-    CopyRound c = prev;
-    c.has_edge = false;  // the first round has copied the edge bytes and the shared line
-    c.share_next = false;
-    c.src_vec = prev.src_vec + (static_cast<size_t>(prev.nvec) << 4);
-    c.dst_vec = prev.dst_vec + (static_cast<size_t>(prev.nvec) << 4);
-    c.nvec = nvec_left < kVecPerRound ? nvec_left : kVecPerRound;
-    nvec_left -= c.nvec;
-    return c;
-  }
-};
-
-// A wavefront's position in its share of a descriptor list staged in LDS: descriptors j, j + stride, ... < end of
-// a list of n.  Neighbours in the list (whoever copies them) decide which destination lines are shared.
-// Everything that describes a fragment is wave-uniform; saying so keeps it in scalar registers and leaves the
-// vector registers to the payload in flight.  `bounce` and `dst` must be wave-uniform.
-// `before` / `after`: the list has a valid descriptor at index -1 / at index n (the last of the batch before, the
-// first of the batch after, staged with it), which the first and the last fragment of the list may share a line with:
-// the wavefront that copies the neighbouring batch looks at the same pair from the other side.
-struct ShareCursor {
-  const tcpxuLoadMeta* descs;
-  uint32_t n, j, end, stride;
-  bool before, after;
-  const uint8_t* bounce;
-  uint8_t* dst;
-  FragmentRounds fr;
-
-  static __device__ __forceinline__ uint32_t uniform(uint32_t v) {
-    return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(v));
-  }
-  static __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
-    return (static_cast<uint64_t>(uniform(static_cast<uint32_t>(v >> 32))) << 32) | uniform(static_cast<uint32_t>(v));
-  }
-  __device__ __forceinline__ void open(const tcpxuLoadMeta* list, uint32_t count, uint32_t first, uint32_t step,
-                                       uint32_t stop, const uint8_t* bounce_base, uint8_t* dst_base,
-                                       bool has_before, bool has_after) {
-    descs = list;
-    n = count;
-    before = has_before;
-    after = has_after;
-    j = uniform(first);
-    end = uniform(stop);
-    stride = step;
-    bounce = bounce_base;
-    dst = dst_base;
-    fr.nvec_left = 0;
-  }
-  // Next round of the share, or false when there is none.  `prev` is the round before it (read only while a
-  // fragment longer than one round is being continued).  `on_take()` runs after each descriptor has been taken
-  // off the share, with j already advanced.  Fragments too short for a round are copied here, at once.
-  template <typename OnTake>
-  __device__ __forceinline__ bool produce(CopyRound& out, const CopyRound& prev, uint32_t lane, OnTake&& on_take) {
-    if (fr.more()) {
-      out = fr.next_round(prev);
-      return true;
-    }
-    const uint64_t dst_addr = reinterpret_cast<uint64_t>(dst);
-    while (j < end) {
-      const uint32_t cur = j;
-      j += stride;
-      on_take();
-      const tcpxuLoadMeta d = descs[cur];
-      const uint32_t len = uniform(d.len);
-      if (len == 0) continue;
-      const uint32_t so = uniform(d.src_off);
-      const uint64_t doff = uniform64(d.dst_off);
-      const uint8_t* fsrc = bounce + so;
-      uint8_t* fdst = dst + doff;
-      if (fragment_is_tiny(fdst, len)) {
-        copy_tiny_fragment(fsrc, fdst, len, lane);
-        continue;
-      }
-      bool share_prev = false, share_next = false;
-      const uint8_t* src_next = fsrc;
-      if (cur > 0 || before) {
-        const tcpxuLoadMeta p = descs[static_cast<int32_t>(cur) - 1];
-        share_prev = shares_line(dst_addr + uniform64(p.dst_off), uniform(p.len), dst_addr + doff, len);
-      }
-      if (cur + 1 < n || after) {
-        const tcpxuLoadMeta q = descs[cur + 1];
-        share_next = shares_line(dst_addr + doff, len, dst_addr + uniform64(q.dst_off), uniform(q.len));
-        if (share_next) src_next = bounce + uniform(q.src_off);
-      }
-      out = fr.first_round(fsrc, fdst, len, share_prev, share_next, src_next, lane);
-      return true;
-    }
-    return false;
-  }
-};
-
-// Copies descriptors first, first + stride, ... < end of a descriptor list of n staged in LDS with the calling
-// wavefront, one round (at most 4 KiB) in flight at a time.
-// `on_last_fragment()` is called exactly once, when the wavefront turns to the last descriptor of its share (at
-// once if it has none): a caller that feeds the wavefront can use it to start fetching more work.
-template <typename OnLastFragment>
-__device__ __forceinline__ void wave_copy_descriptors(const tcpxuLoadMeta* descs, uint32_t n, uint32_t first,
-                                                      uint32_t stride, uint32_t end, const uint8_t* bounce,
-                                                      uint8_t* dst, uint32_t lane,
-                                                      OnLastFragment&& on_last_fragment, bool has_before = false,
-                                                      bool has_after = false) {
-  ShareCursor cursor;
-  cursor.open(descs, n, first, stride, end, bounce, dst, has_before, has_after);
-  if (cursor.j >= cursor.end) on_last_fragment();
-  auto on_take = [&] {
-    if (cursor.j >= cursor.end) on_last_fragment();
-  };
-  CopyRound r;
+  // (Past either end of the list the neighbour reads as empty, and an empty fragment shares nothing.)
+  const bool share_prev = shares_line(place(kPrev), word(kPrev, 1), to, len);
+  const bool share_next = shares_line(to, len, place(kNext), word(kNext, 1));
+  const FragmentPlan p = plan_fragment(to, len, share_prev, share_next);
+  uint32_t left;
+  CopyRound r = first_round_of(from, to_ptr, share_next ? bounce + word(kNext, 0) : from, len, share_next, p.start_off, p.end_off,
+                               p.head, p.tail, p.nvec, lane, &left);
   CopyRegs x;
-  if (!cursor.produce(r, r, lane, on_take)) return;
   for (;;) {
     round_load(r, x, lane);
-    // The next round is worked out while this one's loads are on their way.
-    CopyRound nxt;
-    const bool more = cursor.produce(nxt, r, lane, on_take);
     round_store(r, x, lane);
-    if (!more) return;
-    r = nxt;
+    if (left == 0) return;
+    r.has_edge = false;
+    r.share_next = false;
+    r.src_vec += static_cast<size_t>(r.nvec) << 4;
+    r.dst_vec += static_cast<size_t>(r.nvec) << 4;
+    r.nvec = left < kVecPerRound ? left : kVecPerRound;
+    left -= r.nvec;
   }
 }
 
