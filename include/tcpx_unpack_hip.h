@@ -135,7 +135,9 @@ int tcpxuEngineStop(tcpxuEngine* engine, double* elapsed_us);
 int tcpxuEngineDestroy(tcpxuEngine* engine);
 
 /* Publishes one slot: `n_descs` descriptors at `descs_dev` (device-visible address, normally the device
- * alias of a slot of the mapped queue), gathered from `bounce_base` into `dst_base`.  When the GPU has
+ * alias of a slot of the mapped queue), gathered from `bounce_base` into `dst_base`.  A list of at most 16 in memory
+ * from tcpxuMappedAlloc is read by the call itself, any other by the GPU until the completion word is written; either
+ * way it stays as it is until then.  When the GPU has
  * written every byte it stores `done_value` (nonzero) to `*done_flag_dev` (device alias of a mapped 8-byte
  * word that the host poller reads).  Returns TCPXU_IN_PROGRESS if the ring is full (caller retries).
  * This is the publish of src/net_tcpx.cc:1354-1357 made explicit: count, then a release, then the tail. */

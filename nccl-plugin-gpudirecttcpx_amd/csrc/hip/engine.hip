@@ -93,6 +93,7 @@ __host__ __device__ __forceinline__ uint32_t tickets_for(uint32_t n, uint32_t pe
 // the copy wavefronts' shares come out even, up to 64 (full_ticket_size).  Written as comparisons: the leader runs
 // this for every submission and a division costs it forty instructions.
 constexpr uint32_t kManyInFlight = 8, kSmallSubmission = 32;
+constexpr uint32_t kCarriedDescs = 16;  // descriptors that travel with a submission, and then with its one ticket (see below)
 constexpr uint32_t kLaneTickets = 32;  // tickets of one submission that the lanes holding its entry still write themselves
 constexpr uint32_t kLeaderBehind = 8;  // entries waiting in one poll from which the leader counts as the bottleneck
 constexpr uint32_t kFullTicket = 16;
@@ -107,7 +108,8 @@ __host__ __device__ __forceinline__ uint32_t full_ticket_size(uint32_t bytes, ui
   return bytes == 0 || b >= 2731ull * n ? 16u : b >= 2048ull * n ? 32u : b >= 1366ull * n ? 48u : 64u;
 }
 __host__ __device__ __forceinline__ uint32_t ticket_size_for_submission(uint32_t in_flight, uint32_t n,
-                                                                        uint32_t bytes, uint32_t workers) {
+                                                                        uint32_t bytes, uint32_t workers, bool burst) {
+  if (n <= kCarriedDescs) return kCarriedDescs;
   if (in_flight >= kManyInFlight && n <= kSmallSubmission) return kSmallSubmission;
   const uint64_t all = static_cast<uint64_t>(in_flight) * n;
   const uint32_t backlog = all > (1u << 20) ? (1u << 20) : static_cast<uint32_t>(all);
@@ -119,7 +121,7 @@ __host__ __device__ __forceinline__ uint32_t ticket_size_for_submission(uint32_t
   // workgroup: every workgroup holds a ticket and has the next one staged, and hardly any wait unclaimed): tickets
   // of 14 make a seventh more of them, and the workgroups run dry less often -- one comm 71.1 -> 72.2 % of the
   // roofline, two to four comms the same as with 16 (72.4-72.5 %).
-  return backlog < kDeepBacklog * workers ? 14u : kFullTicket;
+  return backlog < kDeepBacklog * workers && !burst ? 14u : kFullTicket;
 }
 constexpr uint32_t kMaxDescsPerSubmission = 1u << 20;
 constexpr uint32_t kSmallestAdaptiveTicket = 8;  // the least ticket_size_for_submission returns
@@ -158,6 +160,34 @@ __host__ __device__ constexpr int payload_slot(int i) { return (i / 3) * 4 + (i 
 // to decide whether the destination line at that end of the ticket is shared with the neighbouring ticket).
 constexpr uint32_t kOnlyTicket = 1u << 31;
 constexpr uint32_t kMoreAfter = 1u << 30, kMoreBefore = 1u << 29;
+// Descriptors that travel with the submission.  A small request's descriptors lie in memory that the GPU reaches over
+// PCIe (1.7 us from the ticket's record to the last of them, 0.8 if the caller has put a copy into the GPU's memory, which
+// costs the caller a microsecond of waiting for its write-combining buffers).  The host has them at hand when it submits:
+// where it can see that they are host memory it copies them beside the ring's entry, the leader fetches those of the
+// next few entries in the round trip that fetches the entries, and writes them beside the ticket, where the fetcher that
+// polls the ticket reads them in the same round trip as the record: 0.5 us.  (A lone request of 16 whole pages, publish ->
+// done: 7.7 us -> 6.5 with the looks below.)  Each is one 16-byte sector of three words and the stamp of its entry or
+// ticket, like the records' own: source offset, length, the destination offset's low word (a list with a destination
+// offset of 4 GiB or more is not carried).  Sixteen, a ticket of which is a quarter of a look's lanes; only the first four
+// of a call, and only while the leader keeps up, because only the first four entries of a look bring theirs and the copy
+// costs the host 50 ns each (2048 requests in one call: 1 us in 67).
+constexpr uint32_t kCarriedEntry = 1u << 31;   // in a submission's payload word 10, beside the count
+// There too: how many more submissions the same call hands over.  The leader looks at the ring faster than the host
+// writes it, so the first submissions of a burst would be cut up as if each came alone (eleven requests of 2000 short
+// fragments in one call: 28.4 -> 26.2 us).
+// And whether that call handed over kManyInFlight or more: a burst does not go on as a stream does, so the tickets of 14
+// that keep a stream's workgroups from running dry only leave it an uneven last round (sixteen requests of 4 MiB: 33.9 us
+// in tickets of 14, 32.1 in tickets of 16).
+constexpr uint32_t kBurstEntry = 1u << 30;
+constexpr uint32_t kFollowShift = 21, kMostFollow = 0x1FF;
+constexpr uint32_t kCountMask = (1u << kFollowShift) - 1u;  // 1 .. 2^20 descriptors
+__device__ __forceinline__ uint32_t following(uint32_t count_word) { return (count_word >> kFollowShift) & kMostFollow; }
+constexpr uint32_t kCarriedTicket = 1u << 28;  // in a ticket's
+constexpr uint32_t kCarriedEntries = 4;        // entries of a poll whose descriptors it fetches as well: 64 lanes' worth
+constexpr uint32_t kCarryBehind = 16;          // entries the leader is behind from which the host carries no more
+struct alignas(64) CarriedList {
+  uint32_t w[kCarriedDescs][4];
+};
 __host__ __device__ __forceinline__ uint32_t neighbour_bits(uint32_t i, uint32_t nt, bool across) {
   return (nt == 1 ? kOnlyTicket : 0u) | (across && i != 0 ? kMoreBefore : 0u) | (across && i + 1 < nt ? kMoreAfter : 0u);
 }
@@ -185,7 +215,7 @@ struct HostCtl {  // mapped host memory
   alignas(64) uint64_t leader_polls;
   uint64_t leader_entries;
   uint64_t leader_deep_polls;
-  alignas(64) Record ring[1];      // ring_entries follow
+  alignas(64) Record ring[1];      // ring_entries follow, then as many CarriedLists
 };
 
 struct alignas(256) StopWord {
@@ -203,6 +233,7 @@ struct DevState {  // device memory
   uint32_t exit_reason;
   alignas(256) StopWord stop[kStopReplicas];
   alignas(64) Record tickets[kTicketRing];
+  CarriedList carried[kTicketRing];  // of the tickets that say so
   // uint32_t jobs_done[ring_entries], then uint32_t job_target[ring_entries] follow
 };
 
@@ -233,6 +264,45 @@ __device__ __forceinline__ uint64_t bcast64(uint64_t v, uint32_t src_lane) {
   return (static_cast<uint64_t>(bcast(static_cast<uint32_t>(v >> 32), src_lane)) << 32) |
          bcast(static_cast<uint32_t>(v), src_lane);
 }
+// ---- looks at the ring ----------------------------------------------------------------------------------------------
+// A look brings sixteen entries, the descriptors that travel with the first four, and what is known of the entries' job
+// slots, straight into LDS.  kLooks of them are under way at a time, so that an entry waits half the round trip to the
+// host's memory (1.2 us) less for the look that sees it, and going through one look hides behind the next; in LDS because a
+// look that is still under way when the leader leaves this way of polling would otherwise land in registers that have found
+// another use.  A lone request of 16 pages, submit -> done: 9.3 us with one, 8.6 with two, 9.4 with three (going through a
+// look takes 0.4 us, so more than two under way only grow old before their turn comes), and 10.5 with four.
+// (A look asked for before an earlier one was gone through shows the job slots' counters as they were then.  That is safe:
+// a ring has sixteen entries or more, so none of a look's entries shares its slot with another of them, and what was
+// issued for the slot's last tenant was written before the look was asked for.)
+constexpr uint32_t kLooks = 2;  // (a power of two: places are counted modulo it)
+struct alignas(16) Look {
+  uint32_t sect[kWaveLanes][4];     // lane 4k+j: sector j of entry base+k
+  uint32_t carried[kWaveLanes][4];  // lane 16k+j: descriptor j of entry base+k
+  uint32_t aux[kWaveLanes];         // see leader_loop
+  uint32_t base, pad[3];            // low word of the first entry's number
+};
+constexpr int kLookSleep = 2;  // in 64 clocks; 0 to 4 measured alike
+constexpr uint32_t kLookLoads = 3;  // vector memory instructions of a look
+constexpr uint32_t kManyAtOnce = 3;  // see where it is used
+#define TCPXU_LDS __attribute__((address_space(3)))
+typedef TCPXU_LDS Look LdsLook;
+typedef TCPXU_LDS u32x4 lds_u32x4;
+__device__ __forceinline__ uint32_t lds_address(const TCPXU_LDS void* p) {
+  return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(reinterpret_cast<uintptr_t>(p))));
+}
+// The loads of a look (one address each per lane).  Instructions, because the compiler would wait for everything under way
+// before the next read of LDS; m0 holds where in LDS lane 0's share goes.
+__device__ __forceinline__ void ask_for_look(LdsLook* look, const void* aux, const uint8_t* carried, const uint8_t* sect) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\ts_nop 1\n\tglobal_load_lds_dword %3, off sc0 sc1\n\t"
+      "s_mov_b32 m0, %1\n\ts_nop 1\n\tglobal_load_lds_dwordx4 %4, off sc0 sc1\n\t"
+      "s_mov_b32 m0, %2\n\ts_nop 1\n\tglobal_load_lds_dwordx4 %5, off sc0 sc1"
+      :
+      : "s"(lds_address(look->aux)), "s"(lds_address(look->carried)), "s"(lds_address(look->sect)),
+        "v"(reinterpret_cast<uint64_t>(aux)), "v"(reinterpret_cast<uint64_t>(carried)), "v"(reinterpret_cast<uint64_t>(sect))
+      : "memory");
+}
+
 // ---- leader -------------------------------------------------------------------------------------------------------
 // Runs on wavefront 0 of workgroup 0.  All control flow is wave-uniform.
 __device__ __forceinline__ uint32_t lane_value(uint32_t v, uint32_t src_lane) {
@@ -249,18 +319,25 @@ __device__ __forceinline__ uint64_t clock_now() { return wall_clock64(); }
 // What the four lanes of an entry know about it, for the sixteen entries of one group at once.
 struct EntryView {
   uint32_t n, bytes, per_ticket, target_prev, in_flight, slot;
+  uint32_t ticket_bits;  // kCarriedTicket where the entry's descriptors go along, else 0
   bool sane, slot_free;
 };
 
+// How many of a group's entries, from the first, can become tickets now, one each; `room` is what the ticket ring still
+// takes.
+__device__ __forceinline__ uint32_t single_tickets_run(const EntryView& v, uint32_t room) {
+  const uint64_t not_now = ~__ballot(v.sane && v.slot_free);
+  const uint32_t run = not_now == 0 ? kPollEntries : static_cast<uint32_t>(__builtin_ctzll(not_now)) >> 2;
+  return std::min(run, room);
+}
+
 // Every entry of a group fits one ticket (a storm of small requests): the leading run of them becomes tickets in
-// one store instruction.  Returns the length of the run; `room` is what the ticket ring still takes.
+// one store instruction.  Returns the length of the run.
 __device__ __forceinline__ uint32_t write_single_tickets_of_group(DevState* st, uint32_t* job_target, uint64_t* stamps,
                                                                   uint64_t& tickets_out, uint32_t lane, const EntryView& v,
                                                                   const u32x4& sc, uint32_t room) {
   const uint32_t k_of_lane = lane >> 2;
-  const uint64_t not_now = ~__ballot(v.sane && v.slot_free);
-  uint32_t run = not_now == 0 ? kPollEntries : static_cast<uint32_t>(__builtin_ctzll(not_now)) >> 2;
-  run = std::min(run, room);
+  const uint32_t run = single_tickets_run(v, room);
   if (run != 0) {
     if (k_of_lane < run) {
       const uint64_t t = tickets_out + k_of_lane;
@@ -268,7 +345,7 @@ __device__ __forceinline__ uint32_t write_single_tickets_of_group(DevState* st, 
       const uint32_t target = v.target_prev + 1u;
       u32x4 out{sc.x, sc.y, sc.z, stamp};
       if ((lane & 3u) == 3) {
-        out.y = v.n | (v.slot << 8) | kOnlyTicket;
+        out.y = v.n | (v.slot << 8) | kOnlyTicket | v.ticket_bits;
         out.z = target;
         sys_store_global(&job_target[v.slot], target);
         if (stamps) sys_store_global(&stamps[kStampsPerJob * v.slot], clock_now());
@@ -280,6 +357,10 @@ __device__ __forceinline__ uint32_t write_single_tickets_of_group(DevState* st, 
   return run;
 }
 
+// Where lanes that took different ways meet again, said as a statement of its own: where they meet at the end of a loop,
+// the compiler would take whatever else meets there -- the leader's positions -- for different from lane to lane.
+__device__ __forceinline__ void lanes_together() { asm volatile(""); }
+
 // Every lane takes the value that lane q of its own group of four holds: one move, no trip through the LDS.
 template <int q>
 __device__ __forceinline__ uint32_t quad_value(uint32_t v) {
@@ -287,6 +368,9 @@ __device__ __forceinline__ uint32_t quad_value(uint32_t v) {
   return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), q * 0x55, 0xF, 0xF, false));
 }
 
+__device__ __forceinline__ uint32_t same_in_all_lanes32(uint32_t v) {
+  return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
+}
 __device__ __forceinline__ uint64_t same_in_all_lanes64(uint64_t v) {
   return (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v >> 32)))) << 32) |
          static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
@@ -413,7 +497,8 @@ __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevS
       // flight: 5.8 -> 33 M requests/s).  No sizing here, and a group with a larger one ends the storm and goes the
       // ordinary way.
       EntryView more;
-      more.n = quad_value<3>(sc.y);  // payload word 10 sits in .y of sector 3
+      more.n = quad_value<3>(sc.y) & kCountMask;  // payload word 10 sits in .y of sector 3
+      more.ticket_bits = 0;  // (whoever takes the ticket fetches the descriptors: they are nobody's wait with a deep queue)
       more.bytes = 0, more.per_ticket = 0, more.in_flight = 0;  // (not looked at by write_single_tickets_of_group)
       more.target_prev = quad_value<1>(ax);
       more.sane = ((okm >> (4 * k_of_lane)) & 0xFull) == 0xFull && more.n - 1u < kMaxDescsPerSubmission;
@@ -473,7 +558,8 @@ __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevS
 }
 
 __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uint32_t* job_target,
-                            uint32_t ring_mask, uint32_t fixed_per_ticket, uint32_t spin_limit, uint64_t* stamps) {
+                            uint32_t ring_mask, uint32_t fixed_per_ticket, uint32_t spin_limit, uint64_t* stamps,
+                            LdsLook* looks) {
   // The leader's positions are the same in every lane: said outright, so that they stay in scalar registers (in
   // vector registers the compiler waits for the leader's own stores at the top of every pass).
   auto same_in_all_lanes = [](uint64_t v) {
@@ -482,14 +568,17 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
   };
   uint64_t s = same_in_all_lanes(sys_load(&st->sub_head));
   uint64_t tickets_out = same_in_all_lanes(sys_load(&st->tickets_out));
-  uint64_t mirrored = ~0ull;
+  uint64_t mirrored = same_in_all_lanes(sys_load(&st->jobs_completed));  // completed submissions, as the host was last told
   // Read once: the grid's size comes from the dispatch packet, a scalar load with a wait behind it wherever it is asked.
   const uint32_t workers = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(gridDim.x - 1)));
   uint64_t idle = 0;
   uint32_t reason = 0;
   uint32_t polls = 0, entries = 0, deep_polls = 0;  // of this launch; added to the running totals at the end
-  // The next poll fetches 64 entries.  (A ring of fewer entries than that never has them.)
-  bool deep = false;
+  uint32_t wide = 0;       // the last entry taken was one of several tickets and the last of its call
+  uint32_t direct = 0;     // the next poll brings its entries into registers (flags in scalar registers, like the positions)
+  uint32_t deep = 0;       // and so many as 64 of them (a ring of fewer never has them)
+  uint32_t under_way = 0;  // looks asked for and not gone through
+  uint32_t look = 0;       // the next to ask for, modulo kLooks
   bool storm_next = false;
   uint32_t storm_backoff = 0, storm_backoff_len = 4;  // polls until the rolling loop is next tried from the several-tickets way
   const bool ring_allows_deep = ring_mask + 1u >= (kDeepGroups + 1) * kPollEntries;
@@ -510,14 +599,16 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
       const StormEnd end = leader_storm(ctl, st, jobs_done, stamps, ring_mask, fixed_per_ticket, s, tickets_out);
       s = same_in_all_lanes(end.s);
       tickets_out = same_in_all_lanes(end.tickets_out);
-      entries += end.entries;
-      polls += (end.entries + (kDeepGroups + 1) * kPollEntries - 1) / ((kDeepGroups + 1) * kPollEntries);
-      deep_polls += (end.entries + (kDeepGroups + 1) * kPollEntries - 1) / ((kDeepGroups + 1) * kPollEntries);
-      deep = ring_allows_deep;
+      const uint32_t taken = same_in_all_lanes32(end.entries);
+      entries += taken;
+      polls += (taken + (kDeepGroups + 1) * kPollEntries - 1) / ((kDeepGroups + 1) * kPollEntries);
+      deep_polls += (taken + (kDeepGroups + 1) * kPollEntries - 1) / ((kDeepGroups + 1) * kPollEntries);
+      deep = ring_allows_deep ? 1u : 0u;
+      direct = deep;
       // Nothing taken: the queue was not deep, or what waits is not for that loop.  Wait longer each time before
       // asking again (an attempt costs a round trip), and start over once it has worked.
-      storm_backoff_len = end.entries != 0 ? 4u : std::min(2u * storm_backoff_len, 256u);
-      storm_backoff = end.entries != 0 ? 0u : storm_backoff_len;
+      storm_backoff_len = taken != 0 ? 4u : std::min(2u * storm_backoff_len, 256u);
+      storm_backoff = taken != 0 ? 0u : storm_backoff_len;
     } else if (storm_backoff != 0) {
       --storm_backoff;
     }
@@ -530,13 +621,15 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     // One round trip fetches entries s .. s+15: lane 4k+j reads sector j (three payload words and the stamp) of
     // entry s+k.
     const uint32_t k_of_lane = lane >> 2;
-    const u32x4 sect = load_vec_sys(reinterpret_cast<const uint8_t*>(&ctl->ring[(s + k_of_lane) & ring_mask]) + 16 * (lane & 3));
+    const uint8_t* const sect_of_lane = reinterpret_cast<const uint8_t*>(&ctl->ring[(s + k_of_lane) & ring_mask]) + 16 * (lane & 3);
     const uint32_t* aux_addr = host_stop_lo;
     if (lane < kPollEntries) aux_addr = &jobs_done[(s + lane) & ring_mask];
     else if (lane < 2 * kPollEntries) aux_addr = &job_target[(s + lane - kPollEntries) & ring_mask];
     else if (lane == kAuxTicketsDone) aux_addr = tickets_done_lo;
     else if (lane == kAuxJobsCompleted) aux_addr = jobs_completed_lo;
-    const uint32_t aux = sys_load(aux_addr);
+    u32x4 sect;
+    uint32_t aux;
+    uint32_t gone = 0;  // entries of this look's sixteen that an earlier look has brought
     // A deep poll: entries s+16 .. s+63 and their job slots' counters ride along in the same round trip.
     u32x4 sect_more[kDeepGroups];
     uint32_t aux_more[kDeepGroups];
@@ -545,19 +638,55 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
       sect_more[g] = u32x4{0u, 0u, 0u, 0u};
       aux_more[g] = 0;
     }
-    if (deep) {
+    if (direct != 0) {
+      under_way = 0;  // (what has been asked for lands in LDS and is not looked at)
+      sect = load_vec_sys(sect_of_lane);
+      aux = sys_load(aux_addr);
+      if (deep != 0) {
+        ++deep_polls;
 #pragma unroll
-      for (uint32_t g = 0; g < kDeepGroups; ++g) {
-        const uint64_t s_g = s + (g + 1) * kPollEntries;
-        sect_more[g] = load_vec_sys(reinterpret_cast<const uint8_t*>(&ctl->ring[(s_g + k_of_lane) & ring_mask]) + 16 * (lane & 3));
-        // (The upper lanes of the last group's load read the stamp of the entry kStormBacklog beyond the poll's 64.)
-        if (lane < 2 * kPollEntries || g == kDeepGroups - 1)
-          aux_more[g] = sys_load(lane < kPollEntries       ? &jobs_done[(s_g + lane) & ring_mask]
-                                 : lane < 2 * kPollEntries ? &job_target[(s_g + lane - kPollEntries) & ring_mask]
-                                                           : &ctl->ring[(s_g + kPollEntries + kStormBacklog - 1) & ring_mask].w[15]);
+        for (uint32_t g = 0; g < kDeepGroups; ++g) {
+          const uint64_t s_g = s + (g + 1) * kPollEntries;
+          sect_more[g] = load_vec_sys(reinterpret_cast<const uint8_t*>(&ctl->ring[(s_g + k_of_lane) & ring_mask]) + 16 * (lane & 3));
+          // (The upper lanes of the last group's load read the stamp of the entry kStormBacklog beyond the poll's 64.)
+          if (lane < 2 * kPollEntries || g == kDeepGroups - 1)
+            aux_more[g] = sys_load(lane < kPollEntries       ? &jobs_done[(s_g + lane) & ring_mask]
+                                   : lane < 2 * kPollEntries ? &job_target[(s_g + lane - kPollEntries) & ring_mask]
+                                                             : &ctl->ring[(s_g + kPollEntries + kStormBacklog - 1) & ring_mask].w[15]);
+        }
       }
-      ++deep_polls;
+      // All of it waited for here: left to the places where it is used, which looks reach as well, the compiler would
+      // wait there for what looks have under way.
+      asm volatile("" : "+v"(sect), "+v"(aux));
+#pragma unroll
+      for (uint32_t g = 0; g < kDeepGroups; ++g) asm volatile("" : "+v"(sect_more[g]), "+v"(aux_more[g]));
+    } else {
+      // Ask for looks from s on until kLooks are under way, then wait for the oldest: a wavefront's vector memory
+      // instructions complete in the order issued, and at least kLookLoads for each of the others (stores on top of them)
+      // have been issued since its own.
+      const uint8_t* const carried_of_lane = reinterpret_cast<const uint8_t*>(&ctl->ring[ring_mask + 1u]) +
+                                             ((s + lane / kCarriedDescs) & ring_mask) * sizeof(CarriedList) + 16 * (lane % kCarriedDescs);
+#pragma unroll 1
+      for (; under_way != kLooks; under_way = same_in_all_lanes32(under_way + 1u)) {
+        LdsLook* l = &looks[look];
+        if (lane == 0) l->base = static_cast<uint32_t>(s);
+        ask_for_look(l, aux_addr, carried_of_lane, sect_of_lane);
+        look = same_in_all_lanes32((look + 1u) % kLooks);
+      }
+      asm volatile("s_waitcnt vmcnt(%0)" : : "n"((kLooks - 1) * kLookLoads) : "memory");
+      LdsLook* l = &looks[(look - under_way) % kLooks];
+      under_way = same_in_all_lanes32(under_way - 1u);
+      gone = static_cast<uint32_t>(s) - static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(l->base)));
+      // Entry s sits `gone` places from the front.  What lies beyond the sixteen is not in this look: its stamp is made
+      // one that it cannot have, below.
+      const uint32_t from = (lane + 4 * gone) & (kWaveLanes - 1), from_list = (lane + kCarriedDescs * gone) & (kWaveLanes - 1);
+      sect = *reinterpret_cast<lds_u32x4*>(l->sect[from]);
+      sect_more[0] = *reinterpret_cast<lds_u32x4*>(l->carried[from_list]);
+      aux = l->aux[lane < 2 * kPollEntries ? (lane & kPollEntries) | ((lane + gone) & (kPollEntries - 1)) : lane];
     }
+    // (After the two ways have met: a choice per lane at the end of one of them would make the compiler take everything
+    // that differs between them for different from lane to lane.)
+    if (k_of_lane + gone >= kPollEntries) sect.w = static_cast<uint32_t>(s + k_of_lane);
     ++polls;
 
     const uint32_t expect = static_cast<uint32_t>(s + k_of_lane + 1);
@@ -588,17 +717,21 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     // them, and what is worked out per lane first would only add to their latency.)
     uint32_t consumed = 0;
     bool deep_next = false;
-    const uint32_t n_first = lane_value(sect.y, 3);
+    const uint32_t n_first = lane_value(sect.y, 3) & kCountMask;
     const uint32_t lane_tickets_hold = kLaneTickets * (fixed_per_ticket != 0 ? fixed_per_ticket : full_ticket_size(lane_value(sect.z, 3), n_first));
     auto view_entries = [&](const u32x4& sc, uint32_t ax, uint64_t s0, uint64_t okm) {
       EntryView v;
       v.n = bcast(sc.y, lane | 3u);      // payload word 10 sits in .y of sector 3
+      v.ticket_bits = v.n & kCarriedEntry;  // (made a ticket's below, or cleared)
+      const uint32_t follow = following(v.n);
+      const bool burst = (v.n & kBurstEntry) != 0;
+      v.n &= kCountMask;
       v.bytes = bcast(sc.z, lane | 3u);  // payload word 11 sits in .z of sector 3
       const bool all_sectors = ((okm >> (4 * k_of_lane)) & 0xFull) == 0xFull;
       const uint32_t done_now = bcast(ax, k_of_lane);
       v.target_prev = bcast(ax, kPollEntries + k_of_lane);
-      v.in_flight = static_cast<uint32_t>(s0 + k_of_lane) - jobs_completed + 1u;
-      v.per_ticket = fixed_per_ticket != 0 ? fixed_per_ticket : ticket_size_for_submission(v.in_flight, v.n, v.bytes, workers);
+      v.in_flight = static_cast<uint32_t>(s0 + k_of_lane) - jobs_completed + 1u + follow;
+      v.per_ticket = fixed_per_ticket != 0 ? fixed_per_ticket : ticket_size_for_submission(v.in_flight, v.n, v.bytes, workers, burst);
       if (fixed_per_ticket == 0 && leader_behind && v.per_ticket < kFullTicket) v.per_ticket = kFullTicket;  // see below
       v.sane = all_sectors && v.n - 1u < kMaxDescsPerSubmission;  // 1 .. 2^20 descriptors
       v.slot_free = done_now == v.target_prev;  // every ticket ever issued for the job slot has been counted
@@ -610,7 +743,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     };
     if ((ok_mask & 0xFull) == 0xFull &&  // entry s is there
         (n_first <= kMaxDescsPerTicket || (ready >= 2 && n_first <= lane_tickets_hold))) {
-      const EntryView ev = view_entries(sect, aux, s, ok_mask);
+      EntryView ev = view_entries(sect, aux, s, ok_mask);
       const uint32_t n = ev.n, bytes = ev.bytes, per_ticket = ev.per_ticket, target_prev = ev.target_prev;
       const uint32_t in_flight = ev.in_flight, slot = ev.slot;
       const bool sane = ev.sane, slot_free = ev.slot_free;
@@ -618,8 +751,33 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
       const uint32_t room = kTicketRing - (static_cast<uint32_t>(tickets_out) - tickets_done);
       const uint32_t sector = lane & 3u;
       if (__ballot(sane && n > per_ticket) == 0) {
+        const uint64_t says_so = __ballot(ev.ticket_bits != 0);
+        ev.ticket_bits = 0;
+        if (direct == 0 && (says_so & ((1ull << (4 * kCarriedEntries)) - 1ull)) != 0) {
+          // Of the entries that carry descriptors, those whose sectors have all arrived (the others' are fetched by
+          // their workgroups) and which become tickets now (a list left beside a ticket's place without the ticket
+          // would be taken for that of the one that comes there later).
+          static_assert(kCarriedEntries * kCarriedDescs == kWaveLanes, "a lane to a descriptor");
+          const uint32_t of = lane / kCarriedDescs, at = lane % kCarriedDescs;
+          const uint32_t count = bcast(n, 4 * of);
+          const uint64_t t = tickets_out + of;
+          const uint32_t stamp = static_cast<uint32_t>(t + 1);
+          const bool mine = at < count;
+          const uint32_t run = single_tickets_run(ev, room);  // (all lanes ask)
+          u32x4 carried = sect_more[0];
+          const uint64_t there = __ballot(!mine || carried.w == static_cast<uint32_t>(s + of + 1));
+          const bool whole_list = of + gone < kCarriedEntries && ((there >> (kCarriedDescs * of)) & 0xFFFFull) == 0xFFFFull && ((says_so >> (4 * of)) & 1u) != 0 &&
+                                  count <= kCarriedDescs && stamp != 0 && of < run;
+          if (whole_list && mine) {
+            carried.w = stamp;
+            store_vec_sys(reinterpret_cast<uint8_t*>(&st->carried[t & (kTicketRing - 1)]) + 16 * at, carried);
+          }
+          const uint64_t lists = __ballot(whole_list);
+          if (k_of_lane < kCarriedEntries && ((lists >> (kCarriedDescs * k_of_lane)) & 1u) != 0) ev.ticket_bits = kCarriedTicket;
+        }
         consumed = write_single_tickets(ev, sect, room);
-        if (deep && consumed == kPollEntries) {
+        wide = 0;
+        if (deep != 0 && consumed == kPollEntries) {
           // The groups that rode along, in order, each as long as the one before it went through whole.  One loop
           // body that the groups pass through in turn (the registers rotate), so that the three are not worked out
           // side by side in three times the registers: the kernel must stay within 80 for two workgroups per
@@ -634,7 +792,8 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
             const uint64_t okm = __ballot(sc0.w == static_cast<uint32_t>(s_g + k_of_lane + 1));
             uint32_t run = 0;
             if ((okm & 0xFull) == 0xFull) {
-              const EntryView more = view_entries(sc0, ax0, s_g, okm);
+              EntryView more = view_entries(sc0, ax0, s_g, okm);
+              more.ticket_bits = 0;
               if (__ballot(more.sane && more.n > more.per_ticket) == 0) run = write_single_tickets(more, sc0, left);
             }
             consumed += run;
@@ -644,7 +803,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
             ax0 = ax1, ax1 = ax2;
           }
         }
-        deep_next = ring_allows_deep && consumed >= kPollEntries;
+        deep_next = ring_allows_deep && consumed + gone >= kPollEntries;  // everything that the look could show was there
         // All 64 entries of a deep poll became tickets and the entry kStormBacklog beyond them is published (entries
         // are published in order, so everything up to it is there): a storm, taken from the top of the next pass.  How
         // far the host has got is read off the ring itself: the host's tail word is a line that the host writes with
@@ -675,7 +834,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
         const uint32_t total = run != 0 ? lane_value(upto, 4 * run - 4) : 0u;
         // Taken when the run has some width (`most` is over the regular run, which the room may have cut: an upper
         // bound, good enough for the choice): a lone entry of many tickets is written faster by the loop below.
-        if (run != 0 && total >= 2 * most) {
+        if (run != 0 && total >= 2 * same_in_all_lanes32(most)) {
           const uint32_t target = target_prev + nt;
           const bool across = shares_across_tickets(in_flight, n, bytes, bcast(sect.z, lane & ~3u));  // dst_lo: .z of sector 0
           const uint64_t first_ticket = tickets_out + (upto - mine);
@@ -704,6 +863,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
           }
           tickets_out += static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(total)));
           consumed = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(run)));
+          wide = following(lane_value(sect.y, 4 * consumed - 1)) == 0 ? 1u : 0u;
           // Sixteen entries of a few tickets each, the first of them of no more descriptors than one ticket holds: if
           // hundreds more wait, the rolling loop makes one ticket of each such entry (asked once in a while).
           storm_next = consumed == kPollEntries && n_first <= kMaxDescsPerTicket && ring_allows_storm && storm_backoff == 0;
@@ -714,21 +874,22 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     for (uint32_t k = consumed; k < kPollEntries; ++k) {
       if (((ok_mask >> (4 * k)) & 0xFull) != 0xFull) break;
       const uint32_t fl = 4 * k;  // first lane of entry k
-      const uint32_t n = payload_of(fl, 10);
+      const uint32_t count_word = payload_of(fl, 10), n = count_word & kCountMask;
       if (n == 0) {
         const uint32_t flag_lo = payload_of(fl, 6), flag_hi = payload_of(fl, 7);
         const uint32_t val_lo = payload_of(fl, 8), val_hi = payload_of(fl, 9);
         if (lane == 0) {
-          sys_store(reinterpret_cast<uint64_t*>((static_cast<uint64_t>(flag_hi) << 32) | flag_lo),
+          sys_store_global(reinterpret_cast<uint64_t*>((static_cast<uint64_t>(flag_hi) << 32) | flag_lo),
                     (static_cast<uint64_t>(val_hi) << 32) | val_lo);
           __hip_atomic_fetch_add(&st->jobs_completed, 1ull, __ATOMIC_RELAXED, SYS);
         }
+        lanes_together();
       } else {
-        // Submissions not yet completed, this one included, taken to be as long as this one.
-        const uint32_t in_flight = static_cast<uint32_t>(s + k) - jobs_completed + 1u;
+        // Submissions not yet completed, this one and those on their way included, taken to be as long as this one.
+        const uint32_t in_flight = static_cast<uint32_t>(s + k) - jobs_completed + 1u + following(count_word);
         uint32_t per_ticket = fixed_per_ticket != 0
                                   ? fixed_per_ticket
-                                  : ticket_size_for_submission(in_flight, n, payload_of(fl, 11), workers);
+                                  : ticket_size_for_submission(in_flight, n, payload_of(fl, 11), workers, (count_word & kBurstEntry) != 0);
         // Small tickets spread a small backlog over many workgroups, at the price of more tickets to write.  When
         // submissions queue up at the leader, its time per submission is what limits the engine, not the spread:
         // a stream of 1 MiB requests of 256 whole pages, 64 in flight, is served at 1.44 M/s in tickets of 8 (which
@@ -788,17 +949,25 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
           left -= kPerPass * per_ticket;
           at += kPerPass;
         }
+        lanes_together();
         tickets_out += nt;
+        wide = nt > 1 && following(count_word) == 0 ? 1u : 0u;
       }
       ++consumed;
     }
-    deep = deep_next;
+    deep = same_in_all_lanes32(deep_next ? 1u : 0u);
+    // Several entries of several tickets each in one pass, and no more known to be on their way: a stream that keeps the
+    // leader busy.  It is served better by a poll that waits until now to ask and so brings more entries, which become
+    // tickets at a stroke, than by a look that was asked for a pass ago (1 MiB requests, 64 in flight: 3.4 M/s by looks
+    // alone, with some runs at 2.1; 3.57 with this rule, the same with 2 or 4 for the 3).
+    direct = same_in_all_lanes32(deep_next || (wide != 0 && consumed >= kManyAtOnce) ? 1u : 0u);
     if (consumed != 0) {
       consumed = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(consumed)));
       s += consumed;
       entries += consumed;
       idle = 0;
       if (lane == 0) sys_store(&ctl->head, s);
+      lanes_together();
       continue;
     }
 
@@ -809,20 +978,20 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
       // read now bounds what is still to come.
       uint64_t tail_now = 0;
       if (lane == 0) tail_now = sys_load(&ctl->tail);
-      if (s >= bcast64(tail_now, 0)) {
+      if (s >= same_in_all_lanes64(tail_now)) {  // (lane 0's)
         reason = 1;
         break;
       }
       continue;
     }
-    if (lane == 0) {
-      const uint64_t c = sys_load(&st->jobs_completed);
-      if (c != mirrored) {
-        sys_store(&ctl->completed, c);
-        mirrored = c;
-      }
+    if (jobs_completed != static_cast<uint32_t>(mirrored)) {
+      // (the look brings the count's low word; the host is told the whole)
+      mirrored += jobs_completed - static_cast<uint32_t>(mirrored);
+      if (lane == 0) sys_store(&ctl->completed, mirrored);
+      lanes_together();
     }
-    if (spin_limit != kNeverIdleOut && nothing_there && ++idle > spin_limit) {
+    // (kLooks of them go into the round trip that spin_limit counts)
+    if (spin_limit != kNeverIdleOut && nothing_there && ++idle > static_cast<uint64_t>(spin_limit) * kLooks) {
       // Idle for long enough: leave, so that a device-wide synchronize by anybody returns.  The host relaunches
       // the kernel with its next submission.  A submission must not fall between "the leader stopped looking"
       // and "the host thinks the kernel is running": the leader announces that it is leaving, then looks once
@@ -834,13 +1003,15 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
       const bool there = ((lane & 3) == 3 && lane < 16) ? (again == static_cast<uint32_t>(s + 1)) : true;
       if (__all(there)) {
         if (lane == 0) sys_store(&ctl->exiting, static_cast<uint64_t>(0));
+        lanes_together();
         idle = 0;
         continue;
       }
       reason = 2;
       break;
     }
-    __builtin_amdgcn_s_sleep(1);
+    // (leaves the compute unit's issue slots to its copy wavefronts)
+    __builtin_amdgcn_s_sleep(kLookSleep);
   }
 
   // Every ticket written must be visible before any stop word is.
@@ -898,13 +1069,16 @@ struct Stage {
 
 // The stages live in LDS, and every access says so: through a plain pointer the compiler loses track of that and
 // reads the records with flat instructions (a 64-bit address in vector registers each, and slower).
-#define TCPXU_LDS __attribute__((address_space(3)))
 typedef TCPXU_LDS Stage LdsStage;
 typedef TCPXU_LDS uint32_t lds_u32;
-typedef TCPXU_LDS u32x4 lds_u32x4;
 
 __device__ __forceinline__ uint32_t lane_shift(uint32_t v, uint32_t from_lane) {
   return static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(static_cast<int>((from_lane & 63u) << 2), static_cast<int>(v)));
+}
+
+// The value of the lane above (the last lane's own in the last).
+__device__ __forceinline__ uint32_t lane_above(uint32_t v) {
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v), kDppWaveShiftLeft1, 0xF, 0xF, false));
 }
 
 // Fetcher: look once at the slot of ticket number `ticket` (one 64-byte read, with this workgroup's stop word in
@@ -916,9 +1090,16 @@ __device__ uint32_t try_fetch_ticket(DevState* st, const uint32_t* stop_word, ui
   uint32_t word = 0;
   if (lane < 16) word = sys_load(&rec->w[lane]);
   else if (lane == 16) word = sys_load(stop_word);
-  *stop_up = bcast(word, 16) != 0;
+  // (asked for with every look: a ticket that brings its descriptors along is there whole after one round trip)
+  u32x4 d = {0u, 0u, 0u, 0u};
+  if (lane < kCarriedDescs) d = load_vec_sys(reinterpret_cast<const uint8_t*>(&st->carried[ticket & (kTicketRing - 1)]) + 16 * lane);
+  *stop_up = lane_value(word, 16) != 0;
   const bool stamp_ok = (lane < 16 && (lane & 3) == 3) ? (word == expect) : true;
   if (!__all(stamp_ok)) return 0;
+  const uint32_t ticket_bits = lane_value(word, payload_slot(10));
+  const uint32_t n = ticket_bits & 0xFFu;
+  const bool carried = (ticket_bits & kCarriedTicket) != 0;
+  if (carried && !__all(lane >= n || d[3] == expect)) return 0;  // its descriptors are still on their way
   const uint64_t fetched_at = stamps ? clock_now() : 0;
   // Lane broadcasts need the whole wavefront: gather first, then let 12 lanes store.
   const uint32_t pl = lane < kPayloadWords ? lane : 0u;
@@ -926,15 +1107,14 @@ __device__ uint32_t try_fetch_ticket(DevState* st, const uint32_t* stop_word, ui
   if (lane < kPayloadWords) stage->payload[lane] = gathered;
   if (lane == 0) stage->go = 1;
   auto word64 = [&](int lo) {
-    return (static_cast<uint64_t>(bcast(word, payload_slot(lo + 1))) << 32) | bcast(word, payload_slot(lo));
+    return (static_cast<uint64_t>(lane_value(word, payload_slot(lo + 1))) << 32) | lane_value(word, payload_slot(lo));
   };
   const uint64_t bounce = word64(0), dst = word64(2), descs_addr = word64(4);
-  const uint32_t ticket_bits = bcast(word, payload_slot(10));
-  const uint32_t n = ticket_bits & 0xFFu;
   // One 16-byte descriptor per lane straight from where the submission keeps them (system scope: never a cached
   // copy); lanes past the end repeat the last one and write no record.
   const uint32_t mine = lane < n ? lane : (n != 0 ? n - 1u : 0u);  // a ticket has at least one descriptor
-  const u32x4 d = load_vec_sys(reinterpret_cast<const uint8_t*>(descs_addr) + 16 * mine);
+  if (carried) d[3] = 0;  // (the stamp's place is the high word of the destination offset)
+  else d = load_vec_sys(reinterpret_cast<const uint8_t*>(descs_addr) + 16 * mine);
   const uint32_t so = d[0], len = d[1];
   const uint64_t doff = (static_cast<uint64_t>(d[3]) << 32) | d[2];
   // The descriptor before the ticket's first and the one after its last, where the submission has them (lanes 0
@@ -952,54 +1132,51 @@ __device__ uint32_t try_fetch_ticket(DevState* st, const uint32_t* stop_word, ui
     after_so = from_lane(outer[0], 1), after_len = from_lane(outer[1], 1);
     after_dlo = from_lane(outer[2], 1), after_dhi = from_lane(outer[3], 1);
   }
-  // The neighbours' descriptors decide which destination lines are shared with them.  A fragment's neighbours are
-  // the nearest descriptors of the ticket that are not empty: an empty descriptor between two fragments (a
-  // zero-length control message's, a fragment cut to nothing) leaves them back to back in the destination.
-  const uint64_t live = __ballot(lane < n && len != 0);
-  const uint64_t below = live & ((1ull << lane) - 1ull);
-  const uint64_t above = lane < 63u ? live & ~((2ull << lane) - 1ull) : 0ull;
-  const bool prev_inside = below != 0, next_inside = above != 0;
-  // Across a ticket's ends only the very first and the very last descriptor have a neighbour, and only one that
-  // is not empty: that is the pair the other ticket sees too.
-  const bool prev_outside = !prev_inside && lane == 0 && before_len != 0;
-  const bool next_outside = !next_inside && lane + 1 == n && after_len != 0;
-  const bool has_prev = prev_inside || prev_outside, has_next = next_inside || next_outside;
-  const uint32_t prev_lane = prev_inside ? 63u - static_cast<uint32_t>(__builtin_clzll(below)) : lane;
-  const uint32_t next_lane = next_inside ? static_cast<uint32_t>(__builtin_ctzll(above)) : lane;
-  uint32_t p_len = lane_shift(len, prev_lane), p_dlo = lane_shift(d[2], prev_lane), p_dhi = lane_shift(d[3], prev_lane);
-  uint32_t q_len = lane_shift(len, next_lane), q_dlo = lane_shift(d[2], next_lane), q_dhi = lane_shift(d[3], next_lane);
-  uint32_t q_so = lane_shift(so, next_lane);
-  if (prev_outside) p_len = before_len, p_dlo = before_dlo, p_dhi = before_dhi;
-  if (next_outside) q_len = after_len, q_dlo = after_dlo, q_dhi = after_dhi, q_so = after_so;
   const uint64_t fdst = dst + doff, fsrc = bounce + so;
-  const uint64_t p_dst = dst + ((static_cast<uint64_t>(p_dhi) << 32) | p_dlo);
-  const uint64_t q_dst = dst + ((static_cast<uint64_t>(q_dhi) << 32) | q_dlo);
   uint32_t kind = kRecRounds;
-  if (len == 0) kind = kRecSkip;
-  else if (fragment_is_tiny(reinterpret_cast<const uint8_t*>(fdst), len)) kind = kRecTiny;
-  const bool share_prev = kind == kRecRounds && has_prev && shares_line(p_dst, p_len, fdst, len);
-  const bool share_next = kind == kRecRounds && has_next && shares_line(fdst, len, q_dst, q_len);
-  FragmentPlan plan = {0, 0, 0, 0, 1};
-  if (kind == kRecRounds) plan = plan_fragment(fdst, len, share_prev, share_next);
-  const uint64_t next_src = share_next ? bounce + q_so : fsrc;
+  FragmentPlan plan = {0, len, 0, 0, len >> 4};
+  uint64_t next_src = fsrc;
+  bool share_next = false;
+  // Fragments of whole destination lines (a message of whole pages into an aligned buffer) share none of them and have
+  // no edges: what follows would find just that.
+  const uint32_t off_line = (static_cast<uint32_t>(fdst) | len) & (kLineBytes - 1);
+  if (__any(lane < n && (off_line != 0 || len == 0))) {
+    // The neighbours' descriptors decide which destination lines are shared with them.  A fragment's neighbours are
+    // the nearest descriptors of the ticket that are not empty: an empty descriptor between two fragments (a
+    // zero-length control message's, a fragment cut to nothing) leaves them back to back in the destination.
+    const uint64_t live = __ballot(lane < n && len != 0);
+    const uint64_t below = live & ((1ull << lane) - 1ull);
+    const uint64_t above = lane < 63u ? live & ~((2ull << lane) - 1ull) : 0ull;
+    // Across a ticket's ends only the very first and the very last descriptor have a neighbour, and only one that
+    // is not empty: that is the pair the other ticket sees too.
+    const bool next_inside = above != 0, next_outside = !next_inside && lane + 1 == n && after_len != 0;
+    uint32_t q_len, q_dlo, q_dhi, q_so;
+    if (live == (n < 64 ? (1ull << n) - 1ull : ~0ull)) {  // (no empty ones: the next lane's)
+      q_len = lane_above(len), q_dlo = lane_above(d[2]), q_dhi = lane_above(d[3]), q_so = lane_above(so);
+    } else {
+      const uint32_t next_lane = next_inside ? static_cast<uint32_t>(__builtin_ctzll(above)) : lane;
+      q_len = lane_shift(len, next_lane), q_dlo = lane_shift(d[2], next_lane), q_dhi = lane_shift(d[3], next_lane);
+      q_so = lane_shift(so, next_lane);
+    }
+    if (next_outside) q_len = after_len, q_dlo = after_dlo, q_dhi = after_dhi, q_so = after_so;
+    const uint64_t q_dst = dst + ((static_cast<uint64_t>(q_dhi) << 32) | q_dlo);
+    share_next = lane < n && len != 0 && (next_inside || next_outside) && shares_line(fdst, len, q_dst, q_len);
+    // The line that a fragment shares with the one before it is the one that that one shares with it.
+    const uint64_t sharing = __ballot(share_next);
+    const uint64_t nearest = below != 0 ? 1ull << (63u - static_cast<uint32_t>(__builtin_clzll(below))) : 0ull;
+    bool share_prev = (sharing & nearest) != 0;
+    if (more_before && below == 0 && lane == 0 && before_len != 0 && len != 0)
+      share_prev = shares_line(dst + ((static_cast<uint64_t>(before_dhi) << 32) | before_dlo), before_len, fdst, len);
+    if (len == 0) kind = kRecSkip;
+    else if (fragment_is_tiny(reinterpret_cast<const uint8_t*>(fdst), len)) kind = kRecTiny;
+    if (kind == kRecRounds) plan = plan_fragment(fdst, len, share_prev, share_next);
+    if (share_next) next_src = bounce + q_so;
+  }
   if (lane < n) {
-    RoundRec r;
-    r.src_lo = static_cast<uint32_t>(fsrc);
-    r.src_hi = static_cast<uint32_t>(fsrc >> 32);
-    r.dst_lo = static_cast<uint32_t>(fdst);
-    r.dst_hi = static_cast<uint32_t>(fdst >> 32);
-    r.next_lo = static_cast<uint32_t>(next_src);
-    r.next_hi = static_cast<uint32_t>(next_src >> 32);
-    r.start_off = plan.start_off;
-    r.end_off = plan.end_off;
-    r.len = len;
-    r.nvec = plan.nvec;
-    r.bits = plan.head | (plan.tail << 8) | (share_next ? 1u << 16 : 0u) | (kind << 24);
-    r.pad = 0;
     lds_u32x4* out = reinterpret_cast<lds_u32x4*>(&stage->rec[lane]);
-    out[0] = u32x4{r.src_lo, r.src_hi, r.dst_lo, r.dst_hi};
-    out[1] = u32x4{r.next_lo, r.next_hi, r.start_off, r.end_off};
-    out[2] = u32x4{r.len, r.nvec, r.bits, r.pad};
+    out[0] = u32x4{static_cast<uint32_t>(fsrc), static_cast<uint32_t>(fsrc >> 32), static_cast<uint32_t>(fdst), static_cast<uint32_t>(fdst >> 32)};
+    out[1] = u32x4{static_cast<uint32_t>(next_src), static_cast<uint32_t>(next_src >> 32), plan.start_off, plan.end_off};
+    out[2] = u32x4{len, plan.nvec, plan.head | (plan.tail << 8) | (share_next ? 1u << 16 : 0u) | (kind << 24), 0u};
   }
   if (stamps) {
     const uint32_t job = (ticket_bits >> 8) & 0xFFFFu;
@@ -1205,7 +1382,9 @@ __global__ __launch_bounds__(kEngineThreads) __attribute__((amdgpu_waves_per_eu(
                                                                    uint32_t per_ticket, uint32_t spin_limit,
                                                                    uint32_t flags, uint64_t* stamps) {
   if (blockIdx.x == 0) {
-    if (threadIdx.x < kWaveLanes) leader_loop(ctl, st, jobs_done, job_target, ring_mask, per_ticket, spin_limit, stamps);
+    __shared__ Look looks[kLooks];
+    if (threadIdx.x < kWaveLanes)
+      leader_loop(ctl, st, jobs_done, job_target, ring_mask, per_ticket, spin_limit, stamps, (LdsLook*)&looks[0]);
   } else {
     worker_loop(st, jobs_done, flags, stamps);
   }
@@ -1248,11 +1427,14 @@ struct tcpxuEngine {
   bool failed = false;    // the kernel stopped answering (see tcpxuEngineSubmitSized); nothing more is accepted
   uint64_t launches = 0;
   uint64_t submissions = 0;
+  MappedView mapped;           // what mapped host memory there is (see carry_descriptors)
   uint64_t* stamps = nullptr;  // device memory, kStampsPerJob per ring entry, or null (tcpxuEngineEnableStamps)
   std::mutex mu;
 };
 
-static size_t ctl_bytes(uint32_t ring_entries) { return offsetof(HostCtl, ring) + sizeof(Record) * ring_entries; }
+static size_t ctl_bytes(uint32_t ring_entries) {
+  return offsetof(HostCtl, ring) + (sizeof(Record) + sizeof(CarriedList)) * ring_entries;
+}
 
 extern "C" {
 
@@ -1347,6 +1529,12 @@ int tcpxuEngineCreate(int device, const tcpxuEngineConfig* config, tcpxuEngine**
     const char* vc = getenv("TCPXU_ENGINE_COUNT_FROM");
     if (vc && *vc) {
       const uint64_t from = strtoull(vc, nullptr, 0);
+      const uint32_t to_wrap = 0u - static_cast<uint32_t>(from);
+      if (to_wrap != 0 && to_wrap <= std::max(kTicketRing, e->ring_entries)) {
+        set_error("TCPXU_ENGINE_COUNT_FROM: %u is less than a lap of the rings below 2^32", to_wrap);
+        rc = TCPXU_INVALID_ARGUMENT;
+        break;
+      }
       uint64_t* const counts[] = {&e->st->ticket_head, &e->st->tickets_done, &e->st->jobs_completed, &e->st->sub_head,
                                   &e->st->tickets_out};  // device addresses: only computed here, never read
       for (uint64_t* c : counts) {
@@ -1449,7 +1637,7 @@ int tcpxuEngineDestroy(tcpxuEngine* e) {
   if (e->stream) (void)hipStreamDestroy(e->stream);
   if (e->st) (void)hipFree(e->st);
   if (e->stamps) (void)hipFree(e->stamps);
-  if (e->ctl) (void)hipHostFree(e->ctl);
+  if (e->ctl) (void)tcpxuMappedFree(e->device, e->ctl);
   delete e;
   return TCPXU_SUCCESS;
 }
@@ -1487,6 +1675,23 @@ static int check_submission(const tcpxuEngine* e, const tcpxuSubmission& s) {
   return TCPXU_SUCCESS;
 }
 
+// Copies a small list's descriptors beside the ring's entry, if they lie in memory that tcpxuMappedAlloc gave out (where
+// the host has them too) and their destination offsets fit.  Caller holds e->mu.
+static bool carry_descriptors(tcpxuEngine* e, const tcpxuSubmission& sub, uint32_t stamp) {
+  const tcpxuLoadMeta* from = static_cast<const tcpxuLoadMeta*>(mapped_host_address(&e->mapped, sub.descs_dev, sizeof(tcpxuLoadMeta) * sub.n_descs));
+  if (!from) return false;
+  CarriedList* lists = reinterpret_cast<CarriedList*>(&e->ctl->ring[e->ring_entries]);
+  CarriedList* list = &lists[e->tail & (e->ring_entries - 1)];
+  uint64_t high = 0;
+  for (uint32_t i = 0; i < sub.n_descs; ++i) {
+    const tcpxuLoadMeta d = from[i];
+    high |= d.dst_off >> 32;
+    typedef uint32_t host_u32x4 __attribute__((ext_vector_type(4)));
+    *reinterpret_cast<volatile host_u32x4*>(list->w[i]) = host_u32x4{d.src_off, d.len, static_cast<uint32_t>(d.dst_off), stamp};
+  }
+  return high == 0;
+}
+
 int tcpxuEngineSubmitMany(tcpxuEngine* e, const tcpxuSubmission* subs, uint32_t n, uint32_t* accepted) {
   if (accepted) *accepted = 0;
   if (!e || (!subs && n != 0)) {
@@ -1519,8 +1724,12 @@ int tcpxuEngineSubmitMany(tcpxuEngine* e, const tcpxuSubmission* subs, uint32_t 
       p[2 * i] = static_cast<uint32_t>(v[i]);
       p[2 * i + 1] = static_cast<uint32_t>(v[i] >> 32);
     }
-    p[10] = sub.n_descs;
+    p[10] = sub.n_descs | std::min(take - 1 - k, kMostFollow) << kFollowShift | (take >= kManyInFlight ? kBurstEntry : 0u);
+
     p[11] = sub.payload_bytes;
+    if (k < kCarriedEntries && sub.n_descs != 0 && sub.n_descs <= kCarriedDescs && stamp != 0 && e->tail - head < kCarryBehind &&
+        carry_descriptors(e, sub, stamp))
+      p[10] |= kCarriedEntry;
     for (int sct = 0; sct < 4; ++sct) {
       w[4 * sct] = p[3 * sct];
       w[4 * sct + 1] = p[3 * sct + 1];
@@ -1648,7 +1857,7 @@ int tcpxuEngineTicketPlan(uint32_t workgroups, uint32_t descs_per_ticket, uint32
   }
   const uint32_t bytes = payload_bytes > 0xFFFFFFFFull ? 0xFFFFFFFFu : static_cast<uint32_t>(payload_bytes);
   const uint32_t per = descs_per_ticket != 0 ? descs_per_ticket
-                                             : ticket_size_for_submission(in_flight, n_descs, bytes, workgroups - 1);
+                                             : ticket_size_for_submission(in_flight, n_descs, bytes, workgroups - 1, false);
   if (per_ticket) *per_ticket = per;
   if (n_tickets) *n_tickets = (n_descs + per - 1) / per;
   return TCPXU_SUCCESS;

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 #include "tcpx_unpack_hip.h"
 
 namespace tcpxu {
@@ -14,6 +16,19 @@ constexpr int kMaxDevices = 64;
 void set_error(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
 int use_device(int device);            // hipSetDevice + cache properties
 int device_compute_units(int device);  // valid after use_device
+
+// The blocks that tcpxuMappedAlloc has given out, as one caller last saw them: it looks an address up in its own copy
+// and takes a new one only when blocks have come or gone since.
+struct MappedView {
+  struct Block {
+    uintptr_t dev, host;
+    size_t bytes;
+  };
+  uint64_t generation = 0;
+  std::vector<Block> blocks;  // by device address
+};
+// The host's address of `bytes` bytes at a device address inside one of those blocks, or null.
+const void* mapped_host_address(MappedView* view, const void* dev, size_t bytes);
 
 // Engine calls arrive on threads that belong to somebody else (NCCL's proxy thread calls tcpxTest, which may have
 // to relaunch the kernel): the calling thread's current device is put back when the call returns.

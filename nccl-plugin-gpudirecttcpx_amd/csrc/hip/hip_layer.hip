@@ -137,6 +137,39 @@ int use_device(int device) {
 
 int device_compute_units(int device) { return g_props[device].compute_units; }
 
+namespace {
+std::mutex g_mapped_mu;
+std::vector<MappedView::Block> g_mapped;  // by device address
+std::atomic<uint64_t> g_mapped_generation{1};
+
+void mapped_block_added(void* host, void* dev, size_t bytes) {
+  std::lock_guard<std::mutex> lock(g_mapped_mu);
+  const MappedView::Block b{reinterpret_cast<uintptr_t>(dev), reinterpret_cast<uintptr_t>(host), bytes};
+  g_mapped.insert(std::upper_bound(g_mapped.begin(), g_mapped.end(), b, [](const auto& x, const auto& y) { return x.dev < y.dev; }), b);
+  g_mapped_generation.fetch_add(1, std::memory_order_release);
+}
+void mapped_block_removed(void* host) {
+  std::lock_guard<std::mutex> lock(g_mapped_mu);
+  const uintptr_t h = reinterpret_cast<uintptr_t>(host);
+  g_mapped.erase(std::remove_if(g_mapped.begin(), g_mapped.end(), [h](const auto& b) { return b.host == h; }), g_mapped.end());
+  g_mapped_generation.fetch_add(1, std::memory_order_release);
+}
+}  // namespace
+
+const void* mapped_host_address(MappedView* view, const void* dev, size_t bytes) {
+  if (view->generation != g_mapped_generation.load(std::memory_order_acquire)) {
+    std::lock_guard<std::mutex> lock(g_mapped_mu);
+    view->blocks = g_mapped;
+    view->generation = g_mapped_generation.load(std::memory_order_relaxed);
+  }
+  const uintptr_t at = reinterpret_cast<uintptr_t>(dev);
+  auto b = std::upper_bound(view->blocks.begin(), view->blocks.end(), at, [](uintptr_t a, const auto& x) { return a < x.dev; });
+  if (b == view->blocks.begin()) return nullptr;
+  --b;
+  if (bytes > b->bytes || at - b->dev > b->bytes - bytes) return nullptr;
+  return reinterpret_cast<const void*>(b->host + (at - b->dev));
+}
+
 }  // namespace tcpxu
 
 using namespace tcpxu;
@@ -229,11 +262,13 @@ int tcpxuMappedAlloc(int device, size_t bytes, void** host_ptr, void** dev_ptr) 
   TCPXU_HIP(hipHostMalloc(host_ptr, bytes, hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable));
   memset(*host_ptr, 0, bytes);
   TCPXU_HIP(hipHostGetDevicePointer(dev_ptr, *host_ptr, 0));
+  mapped_block_added(*host_ptr, *dev_ptr, bytes);
   return TCPXU_SUCCESS;
 }
 
 int tcpxuMappedFree(int device, void* host_ptr) {
   TCPXU_TRY(use_device(device));
+  mapped_block_removed(host_ptr);
   TCPXU_HIP(hipHostFree(host_ptr));
   return TCPXU_SUCCESS;
 }

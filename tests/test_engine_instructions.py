@@ -47,3 +47,13 @@ def test_engine_kernel_uses_no_scratch(engine_asm):
     if meta is None:  # the metadata lists the size before the name in some releases
         meta = re.search(r"\.private_segment_fixed_size:\s+(\d+)(?:(?!\.name:).)*?\.name:\s+\S*unpack_engine_kernel", engine_asm, re.S)
     assert meta and int(meta.group(1)) == 0
+
+
+def test_looks_at_the_ring_have_m0_and_the_order_of_completion_to_themselves(engine_asm):
+    """A look names its place in LDS in m0, and is waited for by counting as well: nothing else in the kernel writes m0, and
+    the leader (all that comes behind the first look, and what goes through an entry) has no flat_ instruction."""
+    body = function_body(engine_asm, "unpack_engine_kernel")
+    looks = [x.start() for x in re.finditer(r"global_load_lds_dword", body)]
+    assert len(looks) == 3 and len(re.findall(r"\bm0\b", body)) == 3
+    assert re.search(r"s_waitcnt vmcnt\(3\)", body[looks[-1] :])
+    assert "flat_" not in body[looks[0] :]
