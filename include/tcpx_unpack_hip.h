@@ -120,9 +120,9 @@ typedef struct tcpxuEngineConfig {
                                tells of short fragments 32, 48 or 64; a submission of at most 32 descriptors stays
                                whole once 8 or more are in flight (tcpxuEngineTicketPlan gives the same answers) */
   uint32_t spin_limit;      /* the kernel leaves by itself after this many consecutive empty polls of the ring
-                               (about 1.2 us each) and is launched again by the next submission, so that a
-                               device-wide synchronize never waits on an idle engine; 0 = default (400, about
-                               half a millisecond), 0xFFFFFFFF = never leave */
+                               (1.75 us each) and is launched again by the next submission, so that a
+                               device-wide synchronize never waits on an idle engine; 0 = default (400, 0.7
+                               milliseconds), 0xFFFFFFFF = never leave */
 } tcpxuEngineConfig;
 
 int tcpxuEngineCreate(int device, const tcpxuEngineConfig* config, tcpxuEngine** engine);

@@ -107,8 +107,23 @@ __host__ __device__ __forceinline__ uint32_t full_ticket_size(uint32_t bytes, ui
   // average, 64 slots in flight: 59.6 % of the roofline in tickets of 32, 60.6 % in 40, 61.1 % in 48, 61.3 % in 64).
   return bytes == 0 || b >= 2731ull * n ? 16u : b >= 2048ull * n ? 32u : b >= 1366ull * n ? 48u : 64u;
 }
+// Ticket size for a call's submissions of whole pages where it hands over kManyInFlight or more, between 12 and 50
+// descriptors per worker workgroup in all.  A burst does not go on as a stream does: the tickets of 14 that keep a
+// stream's workgroups from running dry leave it a last round that is nearly empty, and so do those of 16 (2.2 tickets a
+// workgroup at 35 descriptors a workgroup, 1.4 of 24).  Sixteen requests of 4 MiB in wire fragments in tickets of 14 / 16 /
+// 18 / 20 / 24 / 28 / 32: 33.9 / 32.4 / 31.6 / 30.8 / 30.5 / 31.4 / 31.6 us; 64 of 1 MiB, 16 / 20 / 24 / 28: 31.4 / 30.0 /
+// 29.3 / 30.6; eight of 4 MiB (17 descriptors a workgroup), by backlog / 24: 22.0 / 21.0.  Below that the sizes by backlog
+// are better, which begin at 8 and reach all the workgroups sooner (eight of 2 MiB: 17.0 us, in tickets of 24 17.8).
+// Above (64 requests of 4 MiB: 100.7 us in tickets of 16, 101.9 of 24) the last round is a small part of the whole.
+constexpr uint32_t kBurstTicket = 24;
+inline bool burst_of_pages(uint32_t submissions, uint32_t n, uint32_t bytes, uint32_t workers) {
+  const uint64_t all = static_cast<uint64_t>(submissions) * n;
+  return submissions >= kManyInFlight && n > kSmallSubmission && full_ticket_size(bytes, n) == kFullTicket &&
+         all >= 12ull * workers && all < 50ull * workers;
+}
 __host__ __device__ __forceinline__ uint32_t ticket_size_for_submission(uint32_t in_flight, uint32_t n,
                                                                         uint32_t bytes, uint32_t workers, bool burst) {
+  if (burst) return kBurstTicket;
   if (n <= kCarriedDescs) return kCarriedDescs;
   if (in_flight >= kManyInFlight && n <= kSmallSubmission) return kSmallSubmission;
   const uint64_t all = static_cast<uint64_t>(in_flight) * n;
@@ -121,7 +136,7 @@ __host__ __device__ __forceinline__ uint32_t ticket_size_for_submission(uint32_t
   // workgroup: every workgroup holds a ticket and has the next one staged, and hardly any wait unclaimed): tickets
   // of 14 make a seventh more of them, and the workgroups run dry less often -- one comm 71.1 -> 72.2 % of the
   // roofline, two to four comms the same as with 16 (72.4-72.5 %).
-  return backlog < kDeepBacklog * workers && !burst ? 14u : kFullTicket;
+  return backlog < kDeepBacklog * workers ? 14u : kFullTicket;
 }
 constexpr uint32_t kMaxDescsPerSubmission = 1u << 20;
 constexpr uint32_t kSmallestAdaptiveTicket = 8;  // the least ticket_size_for_submission returns
@@ -142,7 +157,7 @@ constexpr uint32_t kStormBacklog = 128;  // entries published beyond a poll's 64
 constexpr uint32_t kAuxProbe = 35;  // lane of an auxiliary load that reads the stamp of an entry ahead
 constexpr uint32_t kAuxTicketsDone = 32, kAuxHostStop = 33, kAuxJobsCompleted = 34;  // lanes of the auxiliary load
 constexpr uint32_t kNeverIdleOut = 0xFFFFFFFFu;
-constexpr uint32_t kDefaultIdlePolls = 400;  // empty polls (about 1.2 us each) before the kernel leaves by itself
+constexpr uint32_t kDefaultIdlePolls = 400;  // empty polls (of 1.75 us) before the kernel leaves by itself
 constexpr int kTcpxuInProgress = TCPXU_IN_PROGRESS;
 
 // 64-byte record: four 16-byte sectors of three payload words and one stamp word.
@@ -172,12 +187,12 @@ constexpr uint32_t kMoreAfter = 1u << 30, kMoreBefore = 1u << 29;
 // of a call, and only while the leader keeps up, because only the first four entries of a look bring theirs and the copy
 // costs the host 50 ns each (2048 requests in one call: 1 us in 67).
 constexpr uint32_t kCarriedEntry = 1u << 31;   // in a submission's payload word 10, beside the count
-// There too: how many more submissions the same call hands over.  The leader looks at the ring faster than the host
-// writes it, so the first submissions of a burst would be cut up as if each came alone (eleven requests of 2000 short
-// fragments in one call: 28.4 -> 26.2 us).
-// And whether that call handed over kManyInFlight or more: a burst does not go on as a stream does, so the tickets of 14
-// that keep a stream's workgroups from running dry only leave it an uneven last round (sixteen requests of 4 MiB: 33.9 us
-// in tickets of 14, 32.1 in tickets of 16).
+// There too, of a submission of short fragments: how many more the same call hands over.  The leader looks at the ring
+// faster than the host writes it, so the first submissions of a burst would be cut up as if each came alone (eleven
+// requests of 2000 short fragments in one call: 28.4 -> 26.2 us).  Whole pages are not sized so: there
+// small tickets reach all the workgroups sooner (32 requests of 2 MiB: 32.5 us, and 36.5 with every one sized for all).
+// And of whole pages: whether it is of a burst that burst_of_pages names.  The host works that out, since every
+// instruction that the leader spends on an entry is waited for by all that follow it.
 constexpr uint32_t kBurstEntry = 1u << 30;
 constexpr uint32_t kFollowShift = 21, kMostFollow = 0x1FF;
 constexpr uint32_t kCountMask = (1u << kFollowShift) - 1u;  // 1 .. 2^20 descriptors
@@ -574,7 +589,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
   uint64_t idle = 0;
   uint32_t reason = 0;
   uint32_t polls = 0, entries = 0, deep_polls = 0;  // of this launch; added to the running totals at the end
-  uint32_t wide = 0;       // the last entry taken was one of several tickets and the last of its call
+  uint32_t wide = 0;       // the last entry taken was one of several tickets, with none on its way that count for the size
   uint32_t direct = 0;     // the next poll brings its entries into registers (flags in scalar registers, like the positions)
   uint32_t deep = 0;       // and so many as 64 of them (a ring of fewer never has them)
   uint32_t under_way = 0;  // looks asked for and not gone through
@@ -990,8 +1005,8 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
       if (lane == 0) sys_store(&ctl->completed, mirrored);
       lanes_together();
     }
-    // (kLooks of them go into the round trip that spin_limit counts)
-    if (spin_limit != kNeverIdleOut && nothing_there && ++idle > static_cast<uint64_t>(spin_limit) * kLooks) {
+    // (spin_limit counts polls that ask when the last is done, one in 1.75 us; looks are gone through every 0.97)
+    if (spin_limit != kNeverIdleOut && nothing_there && 5 * ++idle > 9 * static_cast<uint64_t>(spin_limit)) {
       // Idle for long enough: leave, so that a device-wide synchronize by anybody returns.  The host relaunches
       // the kernel with its next submission.  A submission must not fall between "the leader stopped looking"
       // and "the host thinks the kernel is running": the leader announces that it is leaving, then looks once
@@ -1724,8 +1739,9 @@ int tcpxuEngineSubmitMany(tcpxuEngine* e, const tcpxuSubmission* subs, uint32_t 
       p[2 * i] = static_cast<uint32_t>(v[i]);
       p[2 * i + 1] = static_cast<uint32_t>(v[i] >> 32);
     }
-    p[10] = sub.n_descs | std::min(take - 1 - k, kMostFollow) << kFollowShift | (take >= kManyInFlight ? kBurstEntry : 0u);
-
+    const bool pages = full_ticket_size(sub.payload_bytes, sub.n_descs) == kFullTicket;
+    p[10] = sub.n_descs | (pages ? 0u : std::min(take - 1 - k, kMostFollow) << kFollowShift) |
+            (burst_of_pages(take, sub.n_descs, sub.payload_bytes, e->workgroups - 1) ? kBurstEntry : 0u);
     p[11] = sub.payload_bytes;
     if (k < kCarriedEntries && sub.n_descs != 0 && sub.n_descs <= kCarriedDescs && stamp != 0 && e->tail - head < kCarryBehind &&
         carry_descriptors(e, sub, stamp))

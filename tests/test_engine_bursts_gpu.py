@@ -1,0 +1,50 @@
+"""Bursts: several submissions handed over in one call, on both sides of the lines where the size of their tickets changes
+(an engine of 32 workers: 12 x 32 and 50 x 32 descriptors in all, eight submissions, more than 32 descriptors each), with a
+payload hint that says whole pages, one that says short fragments, and none."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from conftest import GpuBuffers, first_difference, oracle_expected
+from test_engine_gpu import Engine, Mapped
+
+pytestmark = pytest.mark.gpu
+
+PAGES = 512
+WORKERS = 32
+
+
+@pytest.mark.parametrize("hint", [4096, 1000, 0])
+@pytest.mark.parametrize("subs_n", [(8, 47), (8, 48), (8, 199), (8, 200), (7, 90), (12, 32), (12, 33), (40, 40), (3, 500)])
+def test_burst(pkg, hip, oracle, subs_n, hint):
+    count, per = subs_n
+    rng = np.random.default_rng(count * per)
+    n = count * per
+    lens = rng.integers(0, 700, n)
+    descs = np.zeros(n, dtype=np.dtype([("src_off", "<u4"), ("len", "<u4"), ("dst_off", "<u8")]))
+    descs["len"] = lens
+    descs["src_off"] = rng.integers(0, (PAGES - 1) * 4096, n)
+    descs["dst_off"] = np.cumsum(lens) - lens
+    total = int(lens.sum())
+    pool = rng.integers(0, 256, PAGES * 4096, dtype=np.uint8)
+    expect = oracle_expected(oracle, pool, descs, total, 0)
+    g = GpuBuffers(pool, descs, total)
+    m = Mapped(pkg, hip, descs, count)
+    e = Engine(pkg, hip, workgroups=WORKERS + 1)
+    subs = (pkg.Submission * count)()
+    print("burst: %d of %d descriptors, hint %d" % (count, per, hint), flush=True)
+    e.start()
+    accepted = ctypes.c_uint32()
+    for turn in (1, 2, 3):  # the first finds the engine idle, the others just emptied
+        for i in range(count):
+            subs[i] = pkg.Submission(g.pool.data_ptr(), g.dst_base, m.desc_dev(i * per), m.flag_dev(i), turn, per, hint * per)
+        assert hip.tcpxuEngineSubmitMany(e.h, subs, count, ctypes.byref(accepted)) == pkg.SUCCESS, hip.tcpxuLastError()
+        assert accepted.value == count
+        for i in range(count):
+            m.wait(i, turn)
+    e.stop()
+    got = g.result()
+    e.destroy()
+    m.free()
+    assert first_difference(got, expect) is None, repr(first_difference(got, expect))
