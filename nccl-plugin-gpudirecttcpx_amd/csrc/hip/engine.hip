@@ -95,7 +95,11 @@ __host__ __device__ __forceinline__ uint32_t tickets_for(uint32_t n, uint32_t pe
 constexpr uint32_t kManyInFlight = 8, kSmallSubmission = 32;
 constexpr uint32_t kCarriedDescs = 16;  // descriptors that travel with a submission, and then with its one ticket (see below)
 constexpr uint32_t kLaneTickets = 32;  // tickets of one submission that the lanes holding its entry still write themselves
-constexpr uint32_t kLeaderBehind = 8;  // entries waiting in one poll from which the leader counts as the bottleneck
+// Entries waiting in one poll from which the leader counts as the bottleneck.  A look comes round twice as often as a poll
+// that asks when the last is done, and shows half as many.  (Four requests of 4 MiB in one call, 8.7 descriptors a workgroup:
+// 20.8 us with 8, where the tickets of 8 that the backlog asks for are a few more than there are workgroups, 16.8 with 4 or
+// 3; 64 of 1 MiB 29.0 and 28.8, streams of 1 MiB requests and storms the same.)
+constexpr uint32_t kLeaderBehind = 4;
 constexpr uint32_t kFullTicket = 16;
 constexpr uint32_t kDeepBacklog = 100;  // descriptors per worker workgroup from which whole pages go in tickets of 16
 __host__ __device__ __forceinline__ uint32_t full_ticket_size(uint32_t bytes, uint32_t n) {
@@ -707,7 +711,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     const uint32_t expect = static_cast<uint32_t>(s + k_of_lane + 1);
     const uint64_t ok_mask = __ballot(sect.w == expect);
     // Entries of this poll that are there, counted from the first: lane 4k tells whether all four sectors of entry
-    // k are.  Eight or more mean that submissions queue up at the leader itself.
+    // k are.  kLeaderBehind or more mean that submissions queue up at the leader itself.
     const uint64_t whole = ok_mask & (ok_mask >> 1) & (ok_mask >> 2) & (ok_mask >> 3) & 0x1111111111111111ull;
     const uint64_t missing = ~whole & 0x1111111111111111ull;
     const uint32_t ready = missing != 0 ? static_cast<uint32_t>(__builtin_ctzll(missing)) >> 2 : kPollEntries;

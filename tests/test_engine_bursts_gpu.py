@@ -16,7 +16,7 @@ WORKERS = 32
 
 
 @pytest.mark.parametrize("hint", [4096, 1000, 0])
-@pytest.mark.parametrize("subs_n", [(8, 47), (8, 48), (8, 199), (8, 200), (7, 90), (12, 32), (12, 33), (40, 40), (3, 500)])
+@pytest.mark.parametrize("subs_n", [(8, 47), (8, 48), (8, 199), (8, 200), (7, 90), (12, 32), (12, 33), (40, 40), (4, 70), (3, 500)])
 def test_burst(pkg, hip, oracle, subs_n, hint):
     count, per = subs_n
     rng = np.random.default_rng(count * per)
