@@ -229,10 +229,10 @@ int tcpxuEngineRunning(tcpxuEngine* engine, int* running);
  * (a hipStream_t, NULL = the default stream): one kernel, whose last workgroup to finish stores `done_value` to
  * `*done_flag_dev` (device-visible 8-byte word, e.g. the alias of mapped host memory; may be NULL when stream order is
  * all the caller needs: the call is then tcpxuUnpackBatch).  Asynchronous.  It calls no hipMalloc, hipFree or other
- * allocating routine: what counts the workgroups lives in a fixed array of device memory inside the library (72 KiB,
- * held by every GPU the library runs on until the process ends), a set of counters for each of 64 calls in turn, which
+ * allocating routine: what counts the workgroups lives in a fixed array of device memory inside the library (1.1 MiB,
+ * held by every GPU the library runs on until the process ends), a set of counters for each of 1024 calls in turn, which
  * a call leaves as it found it.  Calls may overlap on a GPU (two streams, two threads, a replayed graph beside an
- * ordinary call) as long as fewer than 64 calls after a call are made while it is under way.
+ * ordinary call) unless two whose kernels run at the same time were made, or captured, a multiple of 1024 calls apart.
  * Under HIP graph capture: make one ordinary call on the device first -- it looks up the array's address and loads
  * the kernels' code, which do not belong under capture -- then capture; a replay launches the same kernel with the
  * same arguments. */

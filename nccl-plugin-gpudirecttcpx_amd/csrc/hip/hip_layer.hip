@@ -105,9 +105,11 @@ __global__ void complete_empty_slot_kernel(uint64_t* done_flag, uint64_t done_va
 }
 
 // The counters, in a fixed array of device memory: a set for each of kSlotCalls calls in turn, so that calls may overlap
-// on a GPU (two streams, a call beside a replayed graph) as long as fewer than that many are under way.  In host code
-// the name is only a handle for hipGetSymbolAddress; kernels get the address it returns.
-constexpr uint32_t kSlotCalls = 64;
+// on a GPU (two streams, a call beside a replayed graph) unless two whose kernels run at the same time were made a multiple
+// of that many apart.  1024, so that a stream which falls behind, or a graph, meets that by no ordinary chance; 64 measured
+// the same (a 4 MiB slot 6.15 us a call).  In host code the name is only a handle for hipGetSymbolAddress; kernels get the
+// address it returns.
+constexpr uint32_t kSlotCalls = 1024;
 static __device__ SlotCounters slot_counters[kSlotCalls];
 
 struct DeviceProps {

@@ -74,3 +74,23 @@ def test_calls_on_two_streams_at_once(pkg, hip, oracle):
     assert first_difference(buf.result(), expect) is None
     assert first_difference(second.cpu().numpy(), expect) is None
     mapped.free()
+
+
+def test_every_set_of_counters_is_used_again(pkg, hip, oracle):
+    """2100 calls in a row, every one with a completion word of its own: the 1024 sets come round twice, each after lists of
+    another length on either side of the line between one counter and nine."""
+    import torch
+
+    descs, total = ragged_list(300, 4)
+    pool = np.random.default_rng(5).integers(0, 256, PAGES * 4096, dtype=np.uint8)
+    expect = oracle_expected(oracle, pool, descs, total)
+    buf = GpuBuffers(pool, descs, total)
+    calls = 2100
+    mapped = Mapped(pkg, hip, descs, calls)
+    for call in range(calls):
+        n = (300, 3, 257)[call % 3] if call != calls - 1 else 300
+        pkg.check(hip.tcpxuUnpackSlotNoAlloc(0, buf.pool.data_ptr(), buf.dst_base, mapped.desc_dev(0), n, mapped.flag_dev(call), 1 + call, None), "tcpxuUnpackSlotNoAlloc")
+    torch.cuda.synchronize()
+    assert (np.asarray(mapped.flags[:calls]) == np.arange(1, calls + 1)).all()
+    assert first_difference(buf.result(), expect) is None
+    mapped.free()
