@@ -32,6 +32,10 @@ void DevmemSocket::push_locked(const tcpxSynthFrag* frags, size_t n) {
 bool PageLedger::open(size_t arena_pages) {
   pages = static_cast<Page*>(calloc(arena_pages, sizeof(Page)));
   n_pages = pages ? arena_pages : 0;
+  // One store to each page of it, through volatile so that it is not taken for what calloc has done already.
+  constexpr size_t kEntriesPerHostPage = 4096 / sizeof(Page);
+  for (size_t i = 0; i < n_pages; i += kEntriesPerHostPage) *static_cast<volatile uint16_t*>(&pages[i].given) = 0;
+  if (n_pages != 0) *static_cast<volatile uint16_t*>(&pages[n_pages - 1].given) = 0;  // (the block need not start on a page)
   return pages != nullptr;
 }
 
