@@ -222,8 +222,9 @@ ssize_t process_recv_cmsg(struct msghdr* msg, DataPipe* p, int offset, uint64_t 
     d.len = v.frag_size;
     d.dst_off = static_cast<uint64_t>(dst_offset) + dst_base;
     cnt++;
-    if (cnt >= static_cast<uint64_t>(kSlotPages)) {  // src/sock/tcpx.h:183-187
-      WARN("received %lu/%d segs, failstop", static_cast<unsigned long>(cnt), kSlotPages);
+    // src/sock/tcpx.h:183-187, per chunk however it arrived: what receive_chunk put into the slot counts too.
+    if (cnt + p->cnt_before >= static_cast<uint64_t>(kSlotPages)) {
+      WARN("received %lu/%d segs, failstop", static_cast<unsigned long>(cnt + p->cnt_before), kSlotPages);
       *p->pgtok_cnt = n_toks;
       *result = fail_stop("too many fragments in one task");
       return -1;

@@ -227,6 +227,7 @@ ncclResult_t flow_progress(Comm* comm, int flow) {
         // socket, where the reference has the thread that enqueues do it: the pipe then never leaves this thread.)
         t->started = true;
         t->pipe->cnt_cache = 0;
+        t->pipe->cnt_before = t->cnt;
         t->pipe->bytes_cnt = t->offset;
         t->pipe->pgtoks = t->pgtoks;
         t->pipe->pgtok_cnt = t->pgtok_cnt;
@@ -353,8 +354,9 @@ ncclResult_t receive_chunk(Comm* comm, Request* r, int* got) {
   return ncclSuccess;
 }
 
-// enqueueTask, src/net_tcpx.cc:1037-1097 (receive part); the first `received` bytes of the chunk have been received.
-void enqueue_task(Comm* comm, Request* r, int received) {
+// enqueueTask, src/net_tcpx.cc:1037-1097 (receive part); the first `received` bytes of the chunk have been received,
+// in `descs` descriptors.
+void enqueue_task(Comm* comm, Request* r, int received, uint32_t descs) {
   const int flow = r->next_flow;
   const int sz = r->next_size;
   TaskRing* tasks = &comm->flows[flow].tasks;
@@ -368,7 +370,7 @@ void enqueue_task(Comm* comm, Request* r, int received) {
   t->request_offset = r->offset;
   t->size = sz;
   t->flow = static_cast<uint16_t>(flow);
-  t->cnt = 0;
+  t->cnt = descs;
   t->watch.configure(static_cast<uint64_t>(g.timeout_threshold_ns), static_cast<uint64_t>(g.timeout_frequency_ns));
   t->pgtoks = nullptr;
   t->pgtok_cnt = nullptr;
@@ -555,6 +557,7 @@ ncclResult_t take_control_messages(Comm* comm, bool* progress) {
     TaskRing* tasks = &comm->flows[ar->next_flow].tasks;
     if (!tasks->has_free()) break;  // "No free space for recv task": retried at the next poll
     int received = 0;
+    uint32_t descs = 0;
     if (comm->receive_at_once && tasks->empty() && ar->next_size > 0) {
       TCPXCHECK(receive_chunk(comm, ar, &received));
       if (received == ar->next_size) {
@@ -563,9 +566,10 @@ ncclResult_t take_control_messages(Comm* comm, bool* progress) {
         *progress = true;
         continue;
       }
+      descs = static_cast<uint32_t>(comm->direct.cnt_cache);
     }
     comm->end_flow_idx = ar->next_flow;
-    enqueue_task(comm, ar, received);
+    enqueue_task(comm, ar, received, descs);
     *progress = true;
   } while (ar->offset < ar->size);
   return ncclSuccess;

@@ -172,6 +172,7 @@ struct DataPipe {  // struct tcpxDataPipe, src/sock/datapipe.h:25-46
   union loadMeta* list;                      // where descriptors go: scatter_list
   uint64_t list_room;                        // how many fit there
   uint64_t cnt_cache = 0;
+  uint64_t cnt_before = 0;  // descriptors of the same chunk that went into the slot before this pipe took over
   int bytes_cnt = 0;
   size_t* pgtok_cnt = nullptr;
   PageToken* pgtoks = nullptr;
@@ -267,7 +268,8 @@ struct alignas(64) Task {  // struct tcpxTask, src/work_queue.h:38-59 (receive-s
   void* data = nullptr;
   Request* r = nullptr;
   ncclResult_t result = ncclSuccess;
-  uint32_t cnt = 0;                // descriptors the task produced (the pipe's cnt_cache when its last byte arrived)
+  uint32_t cnt = 0;                // on the way out, descriptors of the chunk that are in the slot already; on the way
+                                   // back, those the task produced (the pipe's cnt_cache when its last byte arrived)
   DataPipe* pipe = nullptr;        // the slot's own, for the life of the ring
   PageToken* pgtoks = nullptr;     // passive side: where the task's page tokens go (the request's slot, per flow)
   size_t* pgtok_cnt = nullptr;

@@ -96,6 +96,38 @@ def test_a_slot_that_is_just_full_and_one_descriptor_more(env, comm, fragments):
     comm.dereg(mh)
 
 
+@pytest.mark.parametrize("there", [0, 1, 1000, 2046, "all"])
+@pytest.mark.parametrize("fragments", [2047, 2048])
+def test_the_most_fragments_of_one_chunk(env, comm, fragments, there):  # noqa: F811
+    """A chunk of 2048 fragments is refused (src/sock/tcpx.h:183-187) and one of 2047 is not, however much of it is there
+    when its control message is read."""
+    comm.emu = env.emu
+    frags = np.zeros(fragments, dtype=env.pkg.Workload(1, shrink=6).frag_dtype)
+    frags["frag_offset"] = np.arange(fragments) * 4096
+    frags["frag_size"] = 2
+    frags["frag_token"] = np.arange(fragments)
+    there = fragments if there == "all" else there
+    buf, ptr = host_buffer(2 * fragments)
+    mh = comm.reg(ptr, 2 * fragments)
+    rc, req = comm.irecv(ptr, 2 * fragments, mh)
+    comm.ctrl(0, 2 * fragments, 0, 2 * fragments)
+    if there:
+        comm.deliver(0, frags[:there])
+    if there < fragments:
+        assert comm.test(req)[:2] == (0, 0)
+        comm.deliver(0, frags[there:])
+    for _ in range(20):
+        rc, done, _ = comm.test(req)
+        if rc or done:
+            break
+    if fragments == 2048:
+        assert rc == INTERNAL_ERROR
+        return
+    assert (rc, done) == (0, 1) and comm.consumed(req) == 0
+    assert np.array_equal(buf, env.arena_np[: 4096 * fragments].reshape(fragments, 4096)[:, :2].reshape(-1))
+    comm.dereg(mh)
+
+
 def test_pages_are_given_back_by_the_comm_that_received_them(env, comm):  # noqa: F811
     """Two comms receive from the same pages; each gives back its own references."""
     other = env.driver.RecvComm(0)
