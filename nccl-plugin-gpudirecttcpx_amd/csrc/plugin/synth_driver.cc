@@ -89,10 +89,7 @@ extern "C" ncclResult_t tcpxSynthRunRequests(void* recvComm, const tcpxSynthFrag
   uint32_t next = 0, oldest = 0;
   ncclResult_t rc = ncclSuccess;
   const double t0 = now_s();
-  // The clock is looked at once in kPollsPerLook polls that find nothing; a look costs as much as a poll.
-  constexpr uint32_t kPollsPerLook = 64;
-  uint32_t polls = 0;
-  double waiting_since = 0;
+  QuietTimeout quiet;
   while (rc == ncclSuccess && oldest < n_requests) {
     while (rc == ncclSuccess && next < n_requests && next - oldest < window) {
       const tcpxSynthRequest& r = requests[next];
@@ -125,15 +122,10 @@ extern "C" ncclResult_t tcpxSynthRunRequests(void* recvComm, const tcpxSynthFrag
       }
       if ((rc = tcpxIrecvConsumed(comm, 1, request)) != ncclSuccess) break;
       ++oldest;
-      polls = 0;
-    } else if (++polls % kPollsPerLook == 0) {
-      const double now = now_s();
-      if (polls == kPollsPerLook) {
-        waiting_since = now;
-      } else if (now > waiting_since + 1e-3 * timeout_ms) {
-        WARN("request %u did not complete within %u ms", oldest, timeout_ms);
-        rc = ncclInternalError;
-      }
+      quiet.reset();
+    } else if (quiet.expired(1e-3 * timeout_ms, now_s)) {
+      WARN("request %u did not complete within %u ms", oldest, timeout_ms);
+      rc = ncclInternalError;
     }
   }
   if (seconds) *seconds = now_s() - t0;

@@ -47,6 +47,33 @@ struct SlownessWatch {
   bool should_warn(ClockFn now, uint64_t* nanos);  // tcpxTimeoutDetectionShouldWarn
 };
 
+// The time-out of a loop of polls: how long no poll has found anything, with the clock (seconds) looked at only once in
+// kPollsPerLook polls, since a look costs as much as a poll.
+struct QuietTimeout {
+  static constexpr uint32_t kPollsPerLook = 64;
+  uint32_t polls = 0;  // since the last look
+  bool waiting = false;
+  double since = 0;    // the first look of this wait
+
+  void reset() {
+    polls = 0;
+    waiting = false;
+  }
+  // Counts a poll that has found nothing; true if the wait has lasted longer than `seconds`.
+  template <typename Now>
+  bool expired(double seconds, Now now) {
+    if (++polls != kPollsPerLook) return false;
+    polls = 0;
+    const double t = now();
+    if (!waiting) {
+      waiting = true;
+      since = t;
+      return false;
+    }
+    return t > since + seconds;
+  }
+};
+
 // The waits that can be watched.  The first three keep the reference's positions (src/flags.h:64-69); TX_COMP is
 // a wait of the sending side, accepted in the flags and never armed here.
 enum SlownessKind { kSlowTxComp = 0, kSlowSendRecv = 1, kSlowRxCtrl = 2, kSlowUnpack = 3, kSlowKinds = 4 };
