@@ -118,7 +118,7 @@ ssize_t DevmemSocket::recvmsg(struct msghdr* msg, size_t max_bytes) {
       ledger->give(f->frag_token);
       ++refs;
     }
-    if (end - f > static_cast<ptrdiff_t>(kPrefetchFrags)) __builtin_prefetch(&ledger->pages[f[kPrefetchFrags].frag_token], 1);
+    if (end - f > static_cast<ptrdiff_t>(kPrefetchFrags)) ledger->prefetch(f[kPrefetchFrags].frag_token);
     if (take != f->frag_size) {  // byte budget ended inside the fragment: the rest stays queued
       f->frag_offset += take;
       f->frag_size -= take;
@@ -135,7 +135,7 @@ int DevmemSocket::dontneed(const PageToken* tokens, size_t n) {
   uint64_t given_back = 0;
   int rc = 0;
   for (size_t i = 0; i < n && rc == 0; ++i) {
-    if (i + kPrefetchFrags < n) __builtin_prefetch(&ledger->pages[tokens[i + kPrefetchFrags].token_start], 1);
+    if (i + kPrefetchFrags < n) ledger->prefetch(tokens[i + kPrefetchFrags].token_start);
     for (uint32_t k = 0; k < tokens[i].token_count; ++k) {
       const uint32_t page = tokens[i].token_start + k;
       if (page >= ledger->n_pages || !ledger->take_back(page)) {

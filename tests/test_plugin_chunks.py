@@ -149,3 +149,25 @@ def test_pages_are_given_back_by_the_comm_that_received_them(env, comm):  # noqa
         assert comm.outstanding_pages() == before + 4 - 2 * i
     other.close()
     assert comm.outstanding_pages() == before
+
+
+@pytest.mark.parametrize("token", [ARENA_BYTES // 4096, 2**32 - 1])
+def test_a_token_that_names_no_page(env, comm, token):  # noqa: F811
+    """It is received like any other (the bytes are where the fragment's offset says) and refused when it is given back;
+    its entry, which does not exist, is neither read nor asked for ahead."""
+    frags = np.zeros(16, dtype=env.pkg.Workload(1, shrink=6).frag_dtype)
+    frags["frag_offset"] = np.arange(16) * 4096
+    frags["frag_size"] = 4096
+    frags["frag_token"] = np.arange(16) * 3
+    frags["frag_token"][12] = token  # (far enough from the first to be asked for ahead)
+    before = comm.outstanding_pages()
+    buf, ptr = host_buffer(16 * 4096)
+    mh = comm.reg(ptr, 16 * 4096)
+    rc, req = comm.irecv(ptr, 16 * 4096, mh)
+    comm.ctrl(0, 16 * 4096, 0, 16 * 4096)
+    comm.deliver(0, frags)
+    while not comm.test(req)[1]:
+        pass
+    assert np.array_equal(buf, env.arena_np[: 16 * 4096])
+    assert comm.outstanding_pages() == before + 15
+    assert comm.consumed(req) == INTERNAL_ERROR and comm.outstanding_pages() == before + 3
