@@ -176,7 +176,8 @@ ncclResult_t tcpxSetFailStopForTesting(int enabled);
 typedef struct tcpxFlowStats {
   uint64_t flow_id;
   uint64_t rx_ctrl_done_cnt; /* control messages that named this flow */
-  uint64_t rx_cnt;           /* recvmsg calls, counted while task-level stats are on (src/stats/tracepoint.cc:72-82) */
+  uint64_t rx_cnt;           /* recvmsg calls, counted while task-level stats are on (src/stats/tracepoint.cc:72-82);
+                                the look that finds nothing when a chunk's control message is read is not one of them */
   uint64_t rx_slow_cnt;      /* slowness reports of recvmsg (src/stats/tracepoint.cc:22-52) */
 } tcpxFlowStats;
 

@@ -361,6 +361,45 @@ def test_tracepoints_follow_the_ring_transitions(pkg):
         assert s.drain() == []
 
 
+@pytest.mark.parametrize("stats", ["0", "1"])
+@pytest.mark.parametrize("late", [0, 3])
+def test_task_level_statistics_describe_the_path_that_runs_without_them(pkg, stats, late):
+    """Forty chunks of one fragment on one flow, the last `late` of them still on their way when the control messages are
+    read.  What is there goes into the slot in one call, with the statistics on as without them (as tasks it would take
+    two calls, six to a pass), and the statistics see forty tasks and every recvmsg that brought something."""
+    n = 40
+    with session(pkg, TELEMETRY_ENABLE_TASK_LEVEL_STATS=stats) as s:
+        s.emu.emu_set_hold(1)
+        buf, ptr = host_buffer(n * 4096)
+        mh = s.comm.reg(ptr, n * 4096)
+        rc, req = s.comm.irecv(ptr, n * 4096, mh)
+        frags = s.frags(n * 4096, flow=1)
+        for i in range(n):
+            s.comm.ctrl(1, 4096, i * 4096, n * 4096)
+        s.comm.deliver(1, frags[: n - late])
+        assert s.comm.test(req)[:2] == (0, 0)
+        if late:
+            assert s.emu.emu_pending() == 0
+            assert s.flow_stats(1).rx_cnt >= (n - late if stats == "1" else 0)
+            s.comm.deliver(1, frags[n - late :])
+            before = s.flow_stats(1).rx_cnt
+            assert s.comm.test(req)[:2] == (0, 0)
+            assert s.flow_stats(1).rx_cnt - before == (late if stats == "1" else 0)
+        elif stats == "1":
+            assert s.flow_stats(1).rx_cnt == n
+        assert s.emu.emu_pending() == 1
+        s.emu.emu_release(1)
+        assert s.comm.test(req)[:2] == (0, 1)
+        assert s.comm.consumed(req) == 0
+        per_task = {}
+        for e in s.drain():
+            per_task.setdefault(e.object, []).append(e.state)
+        cycle = host_logic.TASK_TRACE_SEQUENCE
+        assert all(tuple(v) == cycle * (len(v) // len(cycle)) for v in per_task.values())
+        assert sum(len(v) for v in per_task.values()) == (len(cycle) * n if stats == "1" else 0)
+        s.comm.dereg(mh)
+
+
 def test_levels_and_sampling_select_the_events(pkg):
     with session(pkg) as s:  # both levels off: nothing is recorded
         run_small_workload(s)
