@@ -171,6 +171,8 @@ ssize_t process_recv_cmsg(struct msghdr* msg, DataPipe* p, int offset, uint64_t 
   union loadMeta* const list = p->list;
   uint64_t cnt = p->cnt_cache;
   const uint64_t cnt_end = p->list_room;
+  // src/sock/tcpx.h:183-187, per chunk however it arrived: what receive_chunk put into the slot counts too.
+  const uint64_t cnt_most = static_cast<uint64_t>(kSlotPages) - p->cnt_before;
   PageToken* const toks = p->pgtoks;
   size_t n_toks = *p->pgtok_cnt;
   uint32_t next_token = 0;  // the page that would continue the last run
@@ -222,8 +224,7 @@ ssize_t process_recv_cmsg(struct msghdr* msg, DataPipe* p, int offset, uint64_t 
     d.len = v.frag_size;
     d.dst_off = static_cast<uint64_t>(dst_offset) + dst_base;
     cnt++;
-    // src/sock/tcpx.h:183-187, per chunk however it arrived: what receive_chunk put into the slot counts too.
-    if (cnt + p->cnt_before >= static_cast<uint64_t>(kSlotPages)) {
+    if (cnt >= cnt_most) {
       WARN("received %lu/%d segs, failstop", static_cast<unsigned long>(cnt + p->cnt_before), kSlotPages);
       *p->pgtok_cnt = n_toks;
       *result = fail_stop("too many fragments in one task");

@@ -322,13 +322,22 @@ void chunk_taken(Comm* comm, Request* r) {
   }
 }
 
+// Task-level statistics of a chunk that receive_chunk took `calls` recvmsg calls for, from `since` on: if that was all of
+// it, of the task that it would have been, the flow's next free one.
+__attribute__((noinline, cold)) void count_received_chunk(Comm* comm, FlowData* fd, int calls, bool whole, int64_t since) {
+  for (; calls != 0; --calls) FlowData::bump(fd->rx_cnt);
+  if (!whole || !comm->trace) return;
+  const Task* t = fd->tasks.next_free();
+  comm->trace->enqueue('T', t, comm->passive, kTaskActiveTs, since, g.sampling_factor);
+  for (int state : {kTaskCompletingTs, kTaskInactiveTs, kTaskFreeTs}) tp_task(comm, t, state);
+}
+
 // A chunk whose control message has been read and whose bytes are there already: received at once, its descriptors
 // written where the GPU will read them, without a task, its ring and a copy from a task's list in between (8 MiB of
 // fragments that are a chunk each: 88 -> 55 us of host time, with the driver's feeding in one pass).  For a flow on which nothing is queued -- a socket
 // delivers in order -- and where the proxy thread serves the sockets itself.  *got receives the bytes that were there:
-// fewer than the chunk has mean that a task waits for the rest.  Task-level statistics see a chunk received here as the
-// task that it would have been (the flow's next free one), and count the calls that found bytes; a call that finds none is
-// the waiting task's to count, which makes it again.
+// fewer than the chunk has mean that a task waits for the rest.  Task-level statistics see a chunk received here as a task
+// and count the calls that found bytes; a call that finds none is the waiting task's to count, which makes it again.
 ncclResult_t receive_chunk(Comm* comm, Request* r, int* got) {
   const int flow = r->next_flow;
   FlowData* fd = &comm->flows[flow];
@@ -341,19 +350,17 @@ ncclResult_t receive_chunk(Comm* comm, Request* r, int* got) {
   p->bytes_cnt = 0;
   p->pgtoks = &u->pgtoks[static_cast<size_t>(flow) * kSlotPages];
   p->pgtok_cnt = &u->pgtok_cnts[flow];
-  if (comm->task_stats) tp_task(comm, fd->tasks.next_free(), kTaskActiveTs);
-  int at = 0;
+  const int64_t since = __builtin_expect(comm->task_stats, 0) ? trace_timestamp() : 0;
+  int at = 0, calls = 0;
   while (at < r->next_size) {
     ncclResult_t res = ncclSuccess;
     const ssize_t bytes = devmem_recv(&fd->sock, r->next_size, at, p, static_cast<uint64_t>(r->offset), &res);
     if (res != ncclSuccess) return res;
     if (bytes <= 0) break;
-    if (comm->task_stats) FlowData::bump(fd->rx_cnt);
+    ++calls;
     at += static_cast<int>(bytes);
   }
-  if (comm->task_stats && at == r->next_size) {
-    for (int ts : {kTaskCompletingTs, kTaskInactiveTs, kTaskFreeTs}) tp_task(comm, fd->tasks.next_free(), ts);
-  }
+  if (__builtin_expect(comm->task_stats, 0)) count_received_chunk(comm, fd, calls, at == r->next_size, since);
   u->cnt_cache += p->cnt_cache;
   fd->bytes += static_cast<uint64_t>(at);
   *got = at;
@@ -361,8 +368,8 @@ ncclResult_t receive_chunk(Comm* comm, Request* r, int* got) {
 }
 
 // enqueueTask, src/net_tcpx.cc:1037-1097 (receive part); the first `received` bytes of the chunk have been received,
-// in `descs` descriptors.  `announced`: receive_chunk has recorded the task as active.
-void enqueue_task(Comm* comm, Request* r, int received, uint32_t descs, bool announced) {
+// in `descs` descriptors.
+void enqueue_task(Comm* comm, Request* r, int received, uint32_t descs) {
   const int flow = r->next_flow;
   const int sz = r->next_size;
   TaskRing* tasks = &comm->flows[flow].tasks;
@@ -388,7 +395,7 @@ void enqueue_task(Comm* comm, Request* r, int received, uint32_t descs, bool ann
     // Unlike the reference, the count is not zeroed here: a request may put several chunks on the same flow, and
     // every chunk's pages must be given back when the request is consumed.  It is zeroed when the slot is taken.
   }
-  if (!announced) tp_task(comm, t, kTaskActiveTs);
+  tp_task(comm, t, kTaskActiveTs);
   tasks->enqueue();  // FREE -> ACTIVE
   ++comm->tasks_live;
   chunk_taken(comm, r);
@@ -564,8 +571,7 @@ ncclResult_t take_control_messages(Comm* comm, bool* progress) {
     if (!tasks->has_free()) break;  // "No free space for recv task": retried at the next poll
     int received = 0;
     uint32_t descs = 0;
-    const bool at_once = comm->receive_at_once && tasks->empty() && ar->next_size > 0;
-    if (at_once) {
+    if (comm->receive_at_once && tasks->empty() && ar->next_size > 0) {
       TCPXCHECK(receive_chunk(comm, ar, &received));
       if (received == ar->next_size) {
         ar->size_pending -= received;
@@ -576,7 +582,7 @@ ncclResult_t take_control_messages(Comm* comm, bool* progress) {
       descs = static_cast<uint32_t>(comm->direct.cnt_cache);
     }
     comm->end_flow_idx = ar->next_flow;
-    enqueue_task(comm, ar, received, descs, at_once);
+    enqueue_task(comm, ar, received, descs);
     *progress = true;
   } while (ar->offset < ar->size);
   return ncclSuccess;

@@ -356,9 +356,9 @@ struct Comm {  // struct tcpxComm, src/common.h:159-216
   uint32_t tasks_live = 0;    // tasks enqueued and not yet reaped, all flows
   uint32_t to_submit = 0;     // transmitting requests that the engine has not been given
   uint32_t submit_from = 0;   // ring position: every transmitting request before it has been given to the engine
+  bool task_stats = false;       // task-level statistics are on
   bool receive_at_once = false;  // chunks whose bytes are there go straight into the slot (see receive_chunk)
   DataPipe direct{false};        // the pipe for that
-  bool task_stats = false;       // task-level statistics are on
   UnpackQueue* queue = nullptr;
   DeviceState* device = nullptr;
   uint64_t done_seq = 0;
