@@ -20,6 +20,17 @@ COUNTS = [1, 2, 15, 16, 17, 0, 3, 16, 40, 5, 8, 16, 1]
 @pytest.mark.parametrize("kind", ["mapped", "device", "offsets beyond 4 GiB"])
 @pytest.mark.parametrize("ring", [16, 0])
 def test_small_lists(pkg, hip, oracle, ring, kind, per_call):
+    small_lists(pkg, hip, oracle, kind, per_call, ring_entries=ring)
+
+
+@pytest.mark.parametrize("workers", [1, 3])
+def test_lists_of_tickets_that_are_there_at_the_first_look(pkg, hip, oracle, workers):
+    """More tickets than workers, in bursts with a wait after each: a fetcher's first looks, which do not ask for the list
+    that travels, find most of them, and its later looks, which do, the first of a burst."""
+    small_lists(pkg, hip, oracle, "mapped", 40, workgroups=workers + 1)
+
+
+def small_lists(pkg, hip, oracle, kind, per_call, **config):
     rng = np.random.default_rng(per_call)
     counts = np.array([COUNTS[i % len(COUNTS)] for i in range(160)])
     first = np.cumsum(counts) - counts
@@ -36,12 +47,12 @@ def test_small_lists(pkg, hip, oracle, ring, kind, per_call):
     descs["dst_off"] += far
     g = GpuBuffers(pool, descs, total)
     m = Mapped(pkg, hip, descs, len(counts))
-    e = Engine(pkg, hip, ring_entries=ring)
+    e = Engine(pkg, hip, **config)
     subs = (pkg.Submission * len(counts))()
     for i in range(len(counts)):
         at = g.descs.data_ptr() + 16 * int(first[i]) if kind == "device" else m.desc_dev(int(first[i]))
         subs[i] = pkg.Submission(g.pool.data_ptr(), g.dst_base - far, at, m.flag_dev(i), i + 1, int(counts[i]), 0)
-    print("small lists: ring %d, %s, %d a call" % (ring, kind, per_call), flush=True)
+    print("small lists: %r, %s, %d a call" % (config, kind, per_call), flush=True)
     e.start()
     accepted = ctypes.c_uint32()
     at, deadline = 0, time.time() + 20
