@@ -95,12 +95,15 @@ __host__ __device__ __forceinline__ uint32_t tickets_for(uint32_t n, uint32_t pe
 constexpr uint32_t kManyInFlight = 8, kSmallSubmission = 32;
 constexpr uint32_t kCarriedDescs = 16;  // descriptors that travel with a submission, and then with its one ticket (see below)
 constexpr uint32_t kLaneTickets = 32;  // tickets of one submission that the lanes holding its entry still write themselves
-// Entries waiting in one poll from which the leader counts as the bottleneck.  A look comes round twice as often as a poll
-// that asks when the last is done, and shows half as many.  (Four requests of 4 MiB in one call, 8.7 descriptors a workgroup:
-// 20.8 us with 8, where the tickets of 8 that the backlog asks for are a few more than there are workgroups, 16.8 with 4 or
-// 3; 64 of 1 MiB 29.0 and 28.8, streams of 1 MiB requests and storms the same.)
-constexpr uint32_t kLeaderBehind = 4;
-constexpr uint32_t kFullTicket = 16;
+// Entries waiting in one poll from which the leader counts as the bottleneck and makes no tickets of fewer than 16: eight,
+// or four for entries whose backlog asks for fewer than 14.  A look comes round twice as often as a poll that asks when the
+// last is done, and shows half as many.  (Four requests of 4 MiB in one call, 8.7 descriptors a workgroup: 20.8 us with 8
+// throughout, where the tickets of 8 that the backlog asks for are a few more than there are workgroups, 16.8 with 4 or 3;
+// 64 of 1 MiB 29.0 and 28.8, streams of 1 MiB requests and storms the same.  Tickets of 14 are a stream's, which four
+// entries in one look say nothing about: one comm's sixteen slots 70.9 % of the roofline with 4 throughout, 71.8 with 8 for
+// those; raised to 14 only, five requests of 4 MiB take 18.2 us instead of 17.3.)
+constexpr uint32_t kLeaderBehind = 8, kLeaderBehindShallow = 4;
+constexpr uint32_t kFullTicket = 16, kStreamTicket = 14;
 constexpr uint32_t kDeepBacklog = 100;  // descriptors per worker workgroup from which whole pages go in tickets of 16
 __host__ __device__ __forceinline__ uint32_t full_ticket_size(uint32_t bytes, uint32_t n) {
   static_assert(kFullTicket == 16 && kMaxDescsPerTicket == 64, "the steps below");
@@ -140,7 +143,7 @@ __host__ __device__ __forceinline__ uint32_t ticket_size_for_submission(uint32_t
   // workgroup: every workgroup holds a ticket and has the next one staged, and hardly any wait unclaimed): tickets
   // of 14 make a seventh more of them, and the workgroups run dry less often -- one comm 71.1 -> 72.2 % of the
   // roofline, two to four comms the same as with 16 (72.4-72.5 %).
-  return backlog < kDeepBacklog * workers ? 14u : kFullTicket;
+  return backlog < kDeepBacklog * workers ? kStreamTicket : kFullTicket;
 }
 constexpr uint32_t kMaxDescsPerSubmission = 1u << 20;
 constexpr uint32_t kSmallestAdaptiveTicket = 8;  // the least ticket_size_for_submission returns
@@ -717,11 +720,12 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     const uint32_t expect = static_cast<uint32_t>(s + k_of_lane + 1);
     const uint64_t ok_mask = __ballot(sect.w == expect);
     // Entries of this poll that are there, counted from the first: lane 4k tells whether all four sectors of entry
-    // k are.  kLeaderBehind or more mean that submissions queue up at the leader itself.
+    // k are.
     const uint64_t whole = ok_mask & (ok_mask >> 1) & (ok_mask >> 2) & (ok_mask >> 3) & 0x1111111111111111ull;
     const uint64_t missing = ~whole & 0x1111111111111111ull;
     const uint32_t ready = missing != 0 ? static_cast<uint32_t>(__builtin_ctzll(missing)) >> 2 : kPollEntries;
-    const bool leader_behind = ready >= kLeaderBehind;
+    // The ticket size below which tickets are made 16 instead (see kLeaderBehind; 0: none are).
+    const uint32_t too_small = ready >= kLeaderBehind ? kFullTicket : ready >= kLeaderBehindShallow ? kStreamTicket : 0u;
     const uint32_t tickets_done = lane_value(aux, kAuxTicketsDone);
     const uint32_t jobs_completed = lane_value(aux, kAuxJobsCompleted);
     // Payload word i of entry k: component i % 3 of sector i / 3, held by lane 4k + i / 3.
@@ -757,7 +761,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
       v.target_prev = bcast(ax, kPollEntries + k_of_lane);
       v.in_flight = static_cast<uint32_t>(s0 + k_of_lane) - jobs_completed + 1u + follow;
       v.per_ticket = fixed_per_ticket != 0 ? fixed_per_ticket : ticket_size_for_submission(v.in_flight, v.n, v.bytes, workers, burst);
-      if (fixed_per_ticket == 0 && leader_behind && v.per_ticket < kFullTicket) v.per_ticket = kFullTicket;  // see below
+      if (fixed_per_ticket == 0 && v.per_ticket < too_small) v.per_ticket = kFullTicket;  // see below
       v.sane = all_sectors && v.n - 1u < kMaxDescsPerSubmission;  // 1 .. 2^20 descriptors
       v.slot_free = done_now == v.target_prev;  // every ticket ever issued for the job slot has been counted
       v.slot = static_cast<uint32_t>(s0 + k_of_lane) & ring_mask;
@@ -920,7 +924,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
         // a stream of 1 MiB requests of 256 whole pages, 64 in flight, is served at 1.44 M/s in tickets of 8 (which
         // the backlog alone asks for: the workers empty it as fast as it comes), at 1.96 M/s in tickets of 16, and at
         // 1.64 M/s with this rule, which holds for part of the time.
-        if (fixed_per_ticket == 0 && leader_behind && per_ticket < kFullTicket) per_ticket = kFullTicket;
+        if (fixed_per_ticket == 0 && per_ticket < too_small) per_ticket = kFullTicket;
         const uint32_t nt = tickets_for(n, per_ticket);
         const uint32_t slot = static_cast<uint32_t>(s + k) & ring_mask;
         const uint32_t done_now = lane_value(aux, k);
