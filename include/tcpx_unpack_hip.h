@@ -225,17 +225,16 @@ int tcpxuEngineRunning(tcpxuEngine* engine, int* running);
 /* tcpxuEngineSubmit for callers that cannot allocate and cannot keep a persistent kernel: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the reference.
  * Unpacks one slot -- `n_descs` descriptors (at most TCPXU_SLOT_PAGES = 2048; more is TCPXU_INVALID_ARGUMENT and
- * nothing is launched) at `descs_dev`, from `bounce_base` into `dst_base` -- with an ordinary launch on `stream`
- * (a hipStream_t, NULL = the default stream): one kernel, whose last workgroup to finish stores `done_value` to
- * `*done_flag_dev` (device-visible 8-byte word, e.g. the alias of mapped host memory; may be NULL when stream order is
- * all the caller needs: the call is then tcpxuUnpackBatch).  Asynchronous.  It calls no hipMalloc, hipFree or other
- * allocating routine: what counts the workgroups lives in a fixed array of device memory inside the library (1.1 MiB,
- * held by every GPU the library runs on until the process ends), a set of counters for each of 1024 calls in turn, which
- * a call leaves as it found it.  Calls may overlap on a GPU (two streams, two threads, a replayed graph beside an
- * ordinary call) unless two whose kernels run at the same time were made, or captured, a multiple of 1024 calls apart.
- * Under HIP graph capture: make one ordinary call on the device first -- it looks up the array's address and loads
- * the kernels' code, which do not belong under capture -- then capture; a replay launches the same kernel with the
- * same arguments. */
+ * nothing is launched) at `descs_dev`, from `bounce_base` into `dst_base` -- with ordinary launches on `stream`
+ * (a hipStream_t, NULL = the default stream) and then stores `done_value` to `*done_flag_dev` (device-visible 8-byte
+ * word, e.g. the alias of mapped host memory; may be NULL when stream order is all the caller needs: the call is then
+ * tcpxuUnpackBatch).  Up to 16 descriptors are one kernel, more are two, the second of which writes the word.
+ * Asynchronous.  It calls no hipMalloc, hipFree or other allocating routine and keeps nothing in device memory, so calls
+ * may overlap on a GPU without limit: two streams, two threads, a replayed graph beside an ordinary call, two
+ * executables of one captured graph (as far as their destinations and words allow it).
+ * Under HIP graph capture: make one ordinary call on the device first -- it reads the device's properties and loads the
+ * kernels' code, which do not belong under capture -- then capture; a replay launches the same kernels with the same
+ * arguments. */
 int tcpxuUnpackSlotNoAlloc(int device, const void* bounce_base, void* dst_base, const void* descs_dev,
                            uint32_t n_descs, void* done_flag_dev, uint64_t done_value, void* stream);
 

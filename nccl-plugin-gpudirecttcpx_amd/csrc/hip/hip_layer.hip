@@ -56,61 +56,28 @@ __global__ __launch_bounds__(kBatchThreads) __attribute__((amdgpu_waves_per_eu(8
   if (i < n_descs) copy_descriptor(bounce, dst, descs, n_descs, i, lane);
 }
 
-// One slot with a completion word (tcpxuUnpackSlotNoAlloc): the same, and the workgroup that finishes last writes the
-// word.  Counting is two more trips to memory at the end of the chain; they are kept short by counting per workgroup in
-// LDS first and, where many workgroups would queue up at one counter, in eight counters before the last (270 workgroups
-// of a 4 MiB slot: 7.9 us a call with one counter, 6.4 with eight and one; 16 fragments: 4.5 and 4.9).  The last one at
-// a counter sets it back to zero, so that the next call finds it as this one did.
-constexpr uint32_t kSlotSubCounters = 8;
-constexpr uint32_t kSlotOneCounterGroups = 64;  // workgroups up to which one counter is the faster way (69: even)
-struct SlotCounters {
-  struct alignas(128) Line {
-    uint32_t count;
-  };
-  Line sub[kSlotSubCounters];
-  Line top;
-};
-__global__ __launch_bounds__(kBatchThreads) __attribute__((amdgpu_waves_per_eu(8))) void unpack_slot_kernel(
-    const uint8_t* __restrict__ bounce, uint8_t* __restrict__ dst, const tcpxuLoadMeta* __restrict__ descs,
-    uint32_t n_descs, uint32_t n_groups, uint64_t* done_flag, uint64_t done_value, SlotCounters* counters) {
-  __shared__ uint32_t waves_done;
+// One slot with a completion word (tcpxuUnpackSlotNoAlloc).  The word may be written once every wavefront's stores are
+// acknowledged, and nothing that a kernel could count that in is its own: a fixed array of counters is shared by whatever
+// runs at the same time (two executables of one captured graph pass the same arguments), and then the word comes early or
+// never.  So up to kSmallSlot descriptors are one workgroup, which knows by its barrier, and a longer list is the kernel
+// above followed by one of one thread that writes the word: the order of the stream says the rest.  (Us a call, with counters
+// that overlapping launches shared -> so: 1 whole page 3.95 -> 3.5, 4 pages 4.15 -> 3.7, 16 pages 4.3 -> 4.7, 17 to 128 pages
+// 4.4-4.6 -> 5.1-5.5, a 4 MiB slot of wire fragments 6.25 -> 6.4.  One workgroup for 24 descriptors 5.5, for 32 7.0.)
+constexpr uint32_t kSmallSlot = 16;  // a wavefront each, the most that a workgroup can have
+__global__ __launch_bounds__(kSmallSlot* kWaveLanes) void unpack_small_slot_kernel(const uint8_t* __restrict__ bounce, uint8_t* __restrict__ dst,
+                                                                                  const tcpxuLoadMeta* __restrict__ descs, uint32_t n_descs,
+                                                                                  uint64_t* done_flag, uint64_t done_value) {
   const uint32_t lane = threadIdx.x & (kWaveLanes - 1);
   const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWaveLanes)));
-  if (threadIdx.x == 0) waves_done = 0;
-  __syncthreads();
-  const uint32_t group = static_cast<uint32_t>(xcd_contiguous_index(blockIdx.x, n_groups));
-  const uint32_t i = group * kBatchWaves + wave;
-  if (group < n_groups && i < n_descs) copy_descriptor(bounce, dst, descs, n_descs, i, lane);
+  copy_descriptor(bounce, dst, descs, n_descs, wave, lane);
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // this wavefront's write-through stores are acknowledged
-  if (lane != 0) return;
-  // Every count is a read-modify-write at agent scope that follows the acknowledgement of the stores it stands for.
-  auto last_at = [](uint32_t* counter, uint32_t of) {
-    if (__hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u != of) return false;
-    __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return true;
-  };
-  if (__hip_atomic_fetch_add(&waves_done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) + 1u != kBatchWaves) return;
-  uint32_t at_top = gridDim.x;
-  if (n_groups > kSlotOneCounterGroups) {
-    // The grid is a multiple of eight workgroups, so each of the eight counters has an eighth of them.
-    static_assert(kSlotSubCounters == 8, "the grid is rounded up to a multiple of eight");
-    if (!last_at(&counters->sub[blockIdx.x % kSlotSubCounters].count, gridDim.x / kSlotSubCounters)) return;
-    at_top = kSlotSubCounters;
-  }
-  if (last_at(&counters->top.count, at_top)) __hip_atomic_store(done_flag, done_value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(done_flag, done_value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-// An empty slot: nothing to copy, only the word.
-__global__ void complete_empty_slot_kernel(uint64_t* done_flag, uint64_t done_value) {
+// The word of a longer slot, in stream order after its bytes, or of an empty one.
+__global__ void complete_slot_kernel(uint64_t* done_flag, uint64_t done_value) {
   __hip_atomic_store(done_flag, done_value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-
-// The counters, in a fixed array of device memory: a set for each of kSlotCalls calls in turn, so that calls may overlap
-// on a GPU (two streams, a call beside a replayed graph) unless two whose kernels run at the same time were made a multiple
-// of that many apart.  1024, so that a stream which falls behind, or a graph, meets that by no ordinary chance; 64 measured
-// the same (a 4 MiB slot 6.15 us a call).  In host code the name is only a handle for hipGetSymbolAddress; kernels get the
-// address it returns.
-constexpr uint32_t kSlotCalls = 1024;
-static __device__ SlotCounters slot_counters[kSlotCalls];
 
 struct DeviceProps {
   bool valid = false;
@@ -366,26 +333,6 @@ int tcpxuUnpackBatch(int device, const void* bounce_base, void* dst_base, const 
   return launch_batch(bounce_base, dst_base, descs, n_descs, static_cast<hipStream_t>(stream));
 }
 
-// The address of the counters on each device, asked for once per device with that device current.
-static std::atomic<SlotCounters*> g_slot_counters[kMaxDevices];
-static std::atomic<uint32_t> g_slot_calls[kMaxDevices];
-
-static int next_slot_counters(int device, SlotCounters** out) {
-  SlotCounters* all = g_slot_counters[device].load(std::memory_order_acquire);
-  if (!all) {  // (two threads may both ask; they get the same answer)
-    void* p = nullptr;
-    TCPXU_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(slot_counters)));
-    if (!p) {
-      set_error("the slot counters have no address on device %d", device);
-      return TCPXU_INTERNAL_ERROR;
-    }
-    all = static_cast<SlotCounters*>(p);
-    g_slot_counters[device].store(all, std::memory_order_release);
-  }
-  *out = all + g_slot_calls[device].fetch_add(1, std::memory_order_relaxed) % kSlotCalls;
-  return TCPXU_SUCCESS;
-}
-
 int tcpxuUnpackSlotNoAlloc(int device, const void* bounce_base, void* dst_base, const void* descs_dev,
                            uint32_t n_descs, void* done_flag_dev, uint64_t done_value, void* stream) {
   if (n_descs > TCPXU_SLOT_PAGES) {
@@ -405,16 +352,14 @@ int tcpxuUnpackSlotNoAlloc(int device, const void* bounce_base, void* dst_base, 
   hipStream_t s = static_cast<hipStream_t>(stream);
   // Without a completion word the end of the launch says everything.
   if (!done_flag_dev) return launch_batch(bounce_base, dst_base, static_cast<const tcpxuLoadMeta*>(descs_dev), n_descs, s);
-  if (n_descs == 0) {
-    void* args[] = {&done_flag_dev, &done_value};
-    TCPXU_HIP(hipLaunchKernel(reinterpret_cast<const void*>(complete_empty_slot_kernel), dim3(1), dim3(1), args, 0, s));
+  if (n_descs != 0 && n_descs <= kSmallSlot) {
+    void* args[] = {&bounce_base, &dst_base, &descs_dev, &n_descs, &done_flag_dev, &done_value};
+    TCPXU_HIP(hipLaunchKernel(reinterpret_cast<const void*>(unpack_small_slot_kernel), dim3(1), dim3(n_descs * kWaveLanes), args, 0, s));
     return TCPXU_SUCCESS;
   }
-  SlotCounters* counters = nullptr;
-  TCPXU_TRY(next_slot_counters(device, &counters));
-  uint32_t groups = (n_descs + kBatchWaves - 1) / kBatchWaves;
-  void* args[] = {&bounce_base, &dst_base, &descs_dev, &n_descs, &groups, &done_flag_dev, &done_value, &counters};
-  TCPXU_HIP(hipLaunchKernel(reinterpret_cast<const void*>(unpack_slot_kernel), dim3((groups + 7) / 8 * 8), dim3(kBatchThreads), args, 0, s));
+  TCPXU_TRY(launch_batch(bounce_base, dst_base, static_cast<const tcpxuLoadMeta*>(descs_dev), n_descs, s));
+  void* args[] = {&done_flag_dev, &done_value};
+  TCPXU_HIP(hipLaunchKernel(reinterpret_cast<const void*>(complete_slot_kernel), dim3(1), dim3(1), args, 0, s));
   return TCPXU_SUCCESS;
 }
 

@@ -57,3 +57,16 @@ def test_looks_at_the_ring_have_m0_and_the_order_of_completion_to_themselves(eng
     assert len(looks) == 3 and len(re.findall(r"\bm0\b", body)) == 3
     assert re.search(r"s_waitcnt vmcnt\(3\)", body[looks[-1] :])
     assert "flat_" not in body[looks[0] :]
+
+
+def test_kernels_launched_per_list_keep_nothing_between_launches(tmp_path):
+    """Two launches with the same arguments may run at the same time (executables of one captured graph): nothing in device
+    memory may be counted in or kept for the next."""
+    flags = subprocess.check_output(["make", "-s", "-C", CSRC, "print-hipflags"], text=True).split()
+    out = tmp_path / "hip_layer.s"
+    subprocess.run(["hipcc", *flags, "-S", "--cuda-device-only", "-o", str(out), "hip/hip_layer.hip"], cwd=CSRC, check=True,
+                   stdout=subprocess.PIPE, stderr=subprocess.PIPE)  # fmt: skip
+    asm = out.read_text()
+    assert re.search(r"unpack_batch_kernel", asm)
+    assert not re.search(r"\b(global|flat|buffer)_atomic", asm)
+    assert not re.search(r"^\s*\.(l?comm|zero\s+\d{3,})", asm, re.M)

@@ -1,6 +1,8 @@
-"""The kernels that are launched per list, at the list lengths where their grids and counters change: whole and partial
-workgroups of four descriptors, grids rounded up to eight workgroups, one counter up to 64 workgroups of a slot and eight
-beyond (tcpxuUnpackBatch, tcpxuUnpackSlotNoAlloc; byte-exact against the CPU oracle)."""
+"""The kernels that are launched per list, at the list lengths where their grids change: whole and partial workgroups of
+four descriptors, grids rounded up to eight workgroups, a slot of one workgroup and of two launches (tcpxuUnpackBatch,
+tcpxuUnpackSlotNoAlloc; byte-exact against the CPU oracle)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -26,7 +28,7 @@ def ragged_list(n, seed):
     return descs, int(lens.sum())
 
 
-@pytest.mark.parametrize("n", [1, 3, 4, 5, 32, 33, 255, 256, 257, 1023, 2047, 2048])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 16, 17, 32, 33, 255, 256, 257, 1023, 2047, 2048])
 @pytest.mark.parametrize("misalign", [0, 5])
 def test_list_lengths(pkg, hip, oracle, n, misalign):
     import torch
@@ -40,7 +42,7 @@ def test_list_lengths(pkg, hip, oracle, n, misalign):
     pkg.check(hip.tcpxuUnpackBatch(0, buf.pool.data_ptr(), buf.dst_base, buf.descs.data_ptr(), n, None), "tcpxuUnpackBatch")
     torch.cuda.synchronize()
     assert first_difference(buf.result(), expect) is None
-    for call in range(3):  # each finds the counters as the one before left them
+    for call in range(3):
         buf.reset()
         pkg.check(hip.tcpxuUnpackSlotNoAlloc(0, buf.pool.data_ptr(), buf.dst_base, mapped.desc_dev(0), n, mapped.flag_dev(call), 70 + call, None), "tcpxuUnpackSlotNoAlloc")
         torch.cuda.synchronize()
@@ -50,7 +52,7 @@ def test_list_lengths(pkg, hip, oracle, n, misalign):
 
 
 def test_calls_on_two_streams_at_once(pkg, hip, oracle):
-    """Every call has counters of its own: slots on two streams complete in whatever order they run."""
+    """Calls share nothing: slots on two streams complete in whatever order they run."""
     import torch
 
     descs, total = ragged_list(700, 9)
@@ -77,8 +79,8 @@ def test_calls_on_two_streams_at_once(pkg, hip, oracle):
 
 
 def test_every_set_of_counters_is_used_again(pkg, hip, oracle):
-    """2100 calls in a row, every one with a completion word of its own: the 1024 sets come round twice, each after lists of
-    another length on either side of the line between one counter and nine."""
+    """2100 calls in a row, every one with a completion word of its own, lists on either side of the line between one launch
+    and two in turn: no call depends on how many came before."""
     import torch
 
     descs, total = ragged_list(300, 4)
@@ -93,4 +95,44 @@ def test_every_set_of_counters_is_used_again(pkg, hip, oracle):
     torch.cuda.synchronize()
     assert (np.asarray(mapped.flags[:calls]) == np.arange(1, calls + 1)).all()
     assert first_difference(buf.result(), expect) is None
+    mapped.free()
+
+
+@pytest.mark.parametrize("n", [16, 700])
+def test_replays_of_the_same_call_at_the_same_time(pkg, hip, oracle, n):
+    """One call captured into two graphs, arguments and completion word the same, the two replayed on two streams at once
+    and an ordinary call after them: every round ends with the bytes and the word."""
+    import torch
+
+    descs, total = ragged_list(n, 12)
+    pool = np.random.default_rng(13).integers(0, 256, PAGES * 4096, dtype=np.uint8)
+    expect = oracle_expected(oracle, pool, descs, total)
+    buf = GpuBuffers(pool, descs, total)
+    mapped = Mapped(pkg, hip, descs, 2)
+
+    def call(flag, stream):
+        rc = hip.tcpxuUnpackSlotNoAlloc(0, buf.pool.data_ptr(), buf.dst_base, mapped.desc_dev(0), n, mapped.flag_dev(flag), 77, ctypes.c_void_p(stream))
+        pkg.check(rc, "tcpxuUnpackSlotNoAlloc")
+
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    call(0, streams[0].cuda_stream)  # the ordinary call that loads the kernels
+    torch.cuda.synchronize()
+    graphs = [torch.cuda.CUDAGraph() for _ in range(2)]
+    for g, s in zip(graphs, streams):
+        with torch.cuda.graph(g, stream=s):
+            call(1, torch.cuda.current_stream().cuda_stream)
+    for replay in range(20):
+        print("replays of the same call: %d descriptors, round %d" % (n, replay), flush=True)
+        buf.reset()
+        mapped.flags[0] = mapped.flags[1] = 0
+        for _ in range(5):
+            for g, s in zip(graphs, streams):
+                with torch.cuda.stream(s):
+                    g.replay()
+        torch.cuda.synchronize()
+        assert int(mapped.flags[1]) == 77 and first_difference(buf.result(), expect) is None
+        buf.reset()
+        call(0, streams[0].cuda_stream)
+        torch.cuda.synchronize()
+        assert int(mapped.flags[0]) == 77 and first_difference(buf.result(), expect) is None
     mapped.free()

@@ -1,9 +1,8 @@
 """tcpxuUnpackSlotNoAlloc, the entry point that allocates nothing, against tcpxuEngineSubmit on the same slots,
 through the C-ABI (GPU).
 
-Two calls in a row share the library's fixed scratch memory, the second with a smaller slot than the first, so
-what the first call left there (ticket records with the same stamps, counters at their final values) must not
-leak into the second.  Output = the destination bytes with their guard bands and the completion word; the bar is
+Two calls in a row, the second with a smaller slot than the first: a call keeps nothing, so nothing of the first may
+show in the second.  Output = the destination bytes with their guard bands and the completion word; the bar is
 byte-exact, against the engine's output and against the CPU oracle.
 """
 import ctypes
@@ -56,8 +55,7 @@ def test_two_calls_in_a_row_match_the_engine(pkg, hip, oracle, config, seed, shr
     wl, pool = slots_of(pkg, config, seed, shrink)
     info = wl.info
     reqs = [(int(r["first_desc"]), int(r["n_descs"])) for r in wl.requests]
-    # first the largest slot, then a smaller one: a quarter of another request, so the second call writes fewer
-    # tickets than the first left behind
+    # first the largest slot, then a smaller one: a quarter of another request
     big = max(reqs, key=lambda r: r[1])
     other = next(r for r in reqs if r != big) if len(reqs) > 1 else big
     small = (other[0], max(1, other[1] // 4))
@@ -84,7 +82,7 @@ def test_two_calls_in_a_row_match_the_engine(pkg, hip, oracle, config, seed, shr
 
 
 def test_two_calls_captured_into_a_hip_graph_and_replayed(pkg, hip, oracle):
-    """What the entry point is for: after one ordinary call (which looks up the scratch memory's address and loads the
+    """What the entry point is for: after one ordinary call (which reads the device's properties and loads the
     kernels' code, neither of which belongs under capture), two calls in a row -- a large slot, then a smaller one --
     are captured into a HIP graph on a caller's stream and replayed; every replay, with the pool refilled, the
     destination reset and the completion words cleared by ordinary eager work in between, must give the oracle's
@@ -129,7 +127,7 @@ def test_two_calls_captured_into_a_hip_graph_and_replayed(pkg, hip, oracle):
 
 
 def test_no_completion_word_and_the_default_stream(pkg, hip, oracle):
-    """Without a completion word stream order is the only signal; the scratch memory then takes the store."""
+    """Without a completion word stream order is the only signal, and no word is written."""
     wl, pool = slots_of(pkg, 1, 0xA110E, shrink=2)
     info = wl.info
     expect = oracle_expected(oracle, pool, wl.descs, info.dst_bytes, info.dst_misalign)
