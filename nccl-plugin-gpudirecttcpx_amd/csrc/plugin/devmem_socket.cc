@@ -13,7 +13,7 @@ namespace tcpx {
 DataPipe::DataPipe(bool own_list)
     // 2048 control messages of CMSG_SPACE(sizeof(struct iovec)) bytes (src/devcomm/unpack_defs1.h:32-36).
     : ctrl_data(static_cast<size_t>(kSlotPages) * CMSG_SPACE(sizeof(struct iovec))), scatter_list(own_list ? kSlotPages : 0),
-      list(scatter_list.data()), list_room(scatter_list.size()) {}
+      list(scatter_list.data()) {}
 
 void DevmemSocket::push(const tcpxSynthFrag* frags, size_t n) {
   std::lock_guard<std::mutex> lock(mu);
@@ -171,8 +171,6 @@ ssize_t process_recv_cmsg(struct msghdr* msg, DataPipe* p, int offset, uint64_t 
   union loadMeta* const list = p->list;
   uint64_t cnt = p->cnt_cache;
   const uint64_t cnt_end = p->list_room;
-  // src/sock/tcpx.h:183-187, per chunk however it arrived: what receive_chunk put into the slot counts too.
-  const uint64_t cnt_most = static_cast<uint64_t>(kSlotPages) - p->cnt_before;
   PageToken* const toks = p->pgtoks;
   size_t n_toks = *p->pgtok_cnt;
   uint32_t next_token = 0;  // the page that would continue the last run
@@ -210,10 +208,16 @@ ssize_t process_recv_cmsg(struct msghdr* msg, DataPipe* p, int offset, uint64_t 
       return -1;
     }
     next_token = v.frag_token + 1u;
-    if (cnt == cnt_end) {  // (a list that does not start at the slot's first descriptor; src/net_tcpx.cc:1350-1353)
-      WARN("request too many pages, %lu more than its slot had room for, failstop", static_cast<unsigned long>(cnt + 1 - cnt_end));
+    if (cnt == cnt_end) {
       *p->pgtok_cnt = n_toks;
-      *result = fail_stop("request needs more descriptors than a slot holds");
+      const uint64_t of_chunk = cnt + 1 + p->cnt_before;
+      if (of_chunk >= static_cast<uint64_t>(kSlotPages)) {  // src/sock/tcpx.h:183-187
+        WARN("received %lu/%d segs, failstop", static_cast<unsigned long>(of_chunk), kSlotPages);
+        *result = fail_stop("too many fragments in one task");
+      } else {  // src/net_tcpx.cc:1350-1353
+        WARN("request too many pages, one more than its slot had room for, failstop");
+        *result = fail_stop("request needs more descriptors than a slot holds");
+      }
       return -1;
     }
     // src/sock/tcpx.h:178-181: where the fragment lies in the bounce buffer, how long it is, and where in the
@@ -224,12 +228,6 @@ ssize_t process_recv_cmsg(struct msghdr* msg, DataPipe* p, int offset, uint64_t 
     d.len = v.frag_size;
     d.dst_off = static_cast<uint64_t>(dst_offset) + dst_base;
     cnt++;
-    if (cnt >= cnt_most) {
-      WARN("received %lu/%d segs, failstop", static_cast<unsigned long>(cnt + p->cnt_before), kSlotPages);
-      *p->pgtok_cnt = n_toks;
-      *result = fail_stop("too many fragments in one task");
-      return -1;
-    }
     dst_offset += v.frag_size;
   }
   p->cnt_cache = cnt;

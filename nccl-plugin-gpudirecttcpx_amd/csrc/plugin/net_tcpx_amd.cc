@@ -228,6 +228,7 @@ ncclResult_t flow_progress(Comm* comm, int flow) {
         t->started = true;
         t->pipe->cnt_cache = 0;
         t->pipe->cnt_before = t->cnt;
+        t->pipe->list_room = static_cast<uint64_t>(kSlotPages) - 1 - t->cnt;
         t->pipe->bytes_cnt = t->offset;
         t->pipe->pgtoks = t->pgtoks;
         t->pipe->pgtok_cnt = t->pgtok_cnt;
@@ -345,7 +346,7 @@ ncclResult_t receive_chunk(Comm* comm, Request* r, int* got) {
   DataPipe* p = &comm->direct;
   u->flows[flow] = flow;
   p->list = u->mem + u->cnt_cache;
-  p->list_room = static_cast<uint64_t>(kSlotPages) - u->cnt_cache;
+  p->list_room = static_cast<uint64_t>(kSlotPages) - std::max<uint64_t>(u->cnt_cache, 1);
   p->cnt_cache = 0;
   p->bytes_cnt = 0;
   p->pgtoks = &u->pgtoks[static_cast<size_t>(flow) * kSlotPages];

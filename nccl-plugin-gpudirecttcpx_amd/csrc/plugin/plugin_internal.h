@@ -170,7 +170,7 @@ struct DataPipe {  // struct tcpxDataPipe, src/sock/datapipe.h:25-46
   std::vector<char> ctrl_data;           // control-message buffer handed to recvmsg
   std::vector<union loadMeta> scatter_list;  // [kSlotPages]
   union loadMeta* list;                      // where descriptors go: scatter_list
-  uint64_t list_room;                        // how many fit there
+  uint64_t list_room = 0;                    // how many may go there: what fits, and fewer than kSlotPages of one chunk
   uint64_t cnt_cache = 0;
   uint64_t cnt_before = 0;  // descriptors of the same chunk that went into the slot before this pipe took over
   int bytes_cnt = 0;
