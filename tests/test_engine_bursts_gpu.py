@@ -1,6 +1,6 @@
-"""Bursts: several submissions handed over in one call, on both sides of the lines where the size of their tickets changes
-(an engine of 32 workers: 12 x 32 and 50 x 32 descriptors in all, eight submissions, more than 32 descriptors each), with a
-payload hint that says whole pages, one that says short fragments, and none."""
+"""Bursts: several submissions handed over in one call to an engine of 32 workers, on both sides of the lines where the size
+of their tickets changes (three, four and eight submissions, 32 descriptors each, the backlog per worker), with a payload hint
+that says whole pages, one that says short fragments -- those submissions say how many more of their call follow -- and none."""
 import ctypes
 
 import numpy as np
