@@ -117,8 +117,9 @@ typedef struct tcpxuEngineConfig {
                                the backlog of descriptors not yet unpacked: 8 when the engine is idle (lowest
                                latency), 12, then 14 while the backlog is there but shallow (below 100 descriptors
                                per workgroup), 16 when it is deep (highest throughput), and with a payload hint that
-                               tells of short fragments 32, 48 or 64; a submission of at most 32 descriptors stays
-                               whole once 8 or more are in flight (tcpxuEngineTicketPlan gives the same answers) */
+                               tells of short fragments 32, 48 or 64; a submission of at most 16 descriptors is one
+                               ticket, and so is one of at most 32 once 8 or more are in flight (tcpxuEngineTicketPlan
+                               gives the same answers for one submission, and says what it does not know) */
   uint32_t spin_limit;      /* the kernel leaves by itself after this many consecutive empty polls of the ring
                                (1.75 us each) and is launched again by the next submission, so that a
                                device-wide synchronize never waits on an idle engine; 0 = default (400, 0.7
@@ -176,8 +177,9 @@ int tcpxuEngineSubmitMany(tcpxuEngine* engine, const tcpxuSubmission* submission
  * the given descs_per_ticket (0 = by backlog), a submission of n_descs descriptors and payload_bytes (0 = unknown)
  * with `in_flight` submissions not yet completed (itself included) is handed out in *n_tickets tickets of
  * *per_ticket descriptors; *max_descs is the most descriptors a submission may carry.  Outputs may be NULL.
- * (One more rule lives in the kernel alone, because it depends on what the leader finds at run time: while eight or
- * more submissions wait in one of its polls, tickets sized by backlog are at least 16 descriptors.)
+ * (What it does not know: how many more submissions a call hands over, which count as in flight for one of short
+ * fragments; and what the leader finds at run time: while eight or more submissions wait in one of its polls, tickets sized
+ * by backlog are at least 16 descriptors, and while four or more do, those that would be of fewer than 14 are 16.)
  * TCPXU_INVALID_ARGUMENT for an n_descs beyond that limit. */
 int tcpxuEngineTicketPlan(uint32_t workgroups, uint32_t descs_per_ticket, uint32_t in_flight, uint32_t n_descs,
                           uint64_t payload_bytes, uint32_t* per_ticket, uint32_t* n_tickets, uint32_t* max_descs);
