@@ -114,8 +114,24 @@ __host__ __device__ __forceinline__ uint32_t full_ticket_size(uint32_t bytes, ui
   // average, 64 slots in flight: 59.6 % of the roofline in tickets of 32, 60.6 % in 40, 61.1 % in 48, 61.3 % in 64).
   return bytes == 0 || b >= 2731ull * n ? 16u : b >= 2048ull * n ? 32u : b >= 1366ull * n ? 48u : 64u;
 }
+// Ticket size for a call's submissions of whole pages where it hands over kManyInFlight or more, between 12 and 40
+// descriptors per worker workgroup in all.  A burst does not go on as a stream does: by backlog, its submissions are cut as
+// small as what the leader has seen of it so far asks for, and the last round is nearly empty.  Microseconds a call, with
+// other buffers from pass to pass, by backlog / in tickets of 18 / 20 / 22 / 24: eight requests of 4 MiB 24.9 / 24.2 / 24.4 /
+// 25.1 / 25.4, sixteen 35.5 / 35.6 / 36.1 / 36.5 / 36.6, 16 of 2 MiB 26.1 / 24.3 / 24.2 / 24.2 / 24.3, 32 of 2 MiB 38.5 / 36.1 /
+// 36.6 / 36.9 / 37.0, 40 of 1 MiB 28.9 / 28.9 / 29.7 / 29.9 / 29.9, 64 of 1 MiB 35.8 / 35.7 / 35.8 / 36.1 / 35.5.  Where a part of
+// the buffers is still in the caches, sixteen of 4 MiB take 33.5 by backlog and 32.6 with 18 to 24 (on some boxes 31.8 and
+// 32.5).  Above the range the last round is a small part of the whole (24 requests of 4 MiB, 48 a workgroup: 46.5 by backlog,
+// 47.3 in tickets of 18); below it the sizes by backlog, which begin at 8, reach all the workgroups sooner.
+constexpr uint32_t kBurstTicket = 18;
+inline bool burst_of_pages(uint32_t submissions, uint32_t n, uint32_t bytes, uint32_t workers) {
+  const uint64_t all = static_cast<uint64_t>(submissions) * n;
+  return submissions >= kManyInFlight && n > kSmallSubmission && full_ticket_size(bytes, n) == kFullTicket &&
+         all >= 12ull * workers && all < 40ull * workers;
+}
 __host__ __device__ __forceinline__ uint32_t ticket_size_for_submission(uint32_t in_flight, uint32_t n,
-                                                                        uint32_t bytes, uint32_t workers) {
+                                                                        uint32_t bytes, uint32_t workers, bool burst) {
+  if (burst) return kBurstTicket;
   if (n <= kCarriedDescs) return kCarriedDescs;
   if (in_flight >= kManyInFlight && n <= kSmallSubmission) return kSmallSubmission;
   const uint64_t all = static_cast<uint64_t>(in_flight) * n;
@@ -182,7 +198,10 @@ constexpr uint32_t kCarriedEntry = 1u << 31;   // in a submission's payload word
 // There too, of a submission of short fragments: how many more the same call hands over.  The leader looks at the ring
 // faster than the host writes it, so the first submissions of a burst would be cut up as if each came alone (eleven
 // requests of 2000 short fragments in one call: 28.4 -> 26.2 us).  Whole pages are not sized so: there
-// small tickets reach all the workgroups sooner (32 requests of 2 MiB: 35.1 us, and 36.5 with every one sized for all).
+// small tickets reach all the workgroups sooner (32 requests of 2 MiB by what has been seen 35.1 us, and 36.5 with every one sized for all).
+// And of whole pages: whether it is of a burst that burst_of_pages names.  The host works that out, since every
+// instruction that the leader spends on an entry is waited for by all that follow it.
+constexpr uint32_t kBurstEntry = 1u << 30;
 constexpr uint32_t kFollowShift = 21, kMostFollow = 0x1FF;
 constexpr uint32_t kCountMask = (1u << kFollowShift) - 1u;  // 1 .. 2^20 descriptors
 __device__ __forceinline__ uint32_t following(uint32_t count_word) { return (count_word >> kFollowShift) & kMostFollow; }
@@ -735,13 +754,14 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
       v.n = bcast(sc.y, lane | 3u);      // payload word 10 sits in .y of sector 3
       v.ticket_bits = v.n & kCarriedEntry;  // (made a ticket's below, or cleared)
       const uint32_t follow = following(v.n);
+      const bool burst = (v.n & kBurstEntry) != 0;
       v.n &= kCountMask;
       v.bytes = bcast(sc.z, lane | 3u);  // payload word 11 sits in .z of sector 3
       const bool all_sectors = ((okm >> (4 * k_of_lane)) & 0xFull) == 0xFull;
       const uint32_t done_now = bcast(ax, k_of_lane);
       v.target_prev = bcast(ax, kPollEntries + k_of_lane);
       v.in_flight = static_cast<uint32_t>(s0 + k_of_lane) - jobs_completed + 1u + follow;
-      v.per_ticket = fixed_per_ticket != 0 ? fixed_per_ticket : ticket_size_for_submission(v.in_flight, v.n, v.bytes, workers);
+      v.per_ticket = fixed_per_ticket != 0 ? fixed_per_ticket : ticket_size_for_submission(v.in_flight, v.n, v.bytes, workers, burst);
       if (fixed_per_ticket == 0 && v.per_ticket < too_small) v.per_ticket = kFullTicket;  // see below
       v.sane = all_sectors && v.n - 1u < kMaxDescsPerSubmission;  // 1 .. 2^20 descriptors
       v.slot_free = done_now == v.target_prev;  // every ticket ever issued for the job slot has been counted
@@ -899,7 +919,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
         const uint32_t in_flight = static_cast<uint32_t>(s + k) - jobs_completed + 1u + following(count_word);
         uint32_t per_ticket = fixed_per_ticket != 0
                                   ? fixed_per_ticket
-                                  : ticket_size_for_submission(in_flight, n, payload_of(fl, 11), workers);
+                                  : ticket_size_for_submission(in_flight, n, payload_of(fl, 11), workers, (count_word & kBurstEntry) != 0);
         // Small tickets spread a small backlog over many workgroups, at the price of more tickets to write.  When
         // submissions queue up at the leader, its time per submission is what limits the engine, not the spread:
         // a stream of 1 MiB requests of 256 whole pages, 64 in flight, is served at 1.44 M/s in tickets of 8 (which
@@ -1735,7 +1755,8 @@ int tcpxuEngineSubmitMany(tcpxuEngine* e, const tcpxuSubmission* subs, uint32_t 
       p[2 * i + 1] = static_cast<uint32_t>(v[i] >> 32);
     }
     const bool pages = full_ticket_size(sub.payload_bytes, sub.n_descs) == kFullTicket;
-    p[10] = sub.n_descs | (pages ? 0u : std::min(take - 1 - k, kMostFollow) << kFollowShift);
+    p[10] = sub.n_descs | (pages ? 0u : std::min(take - 1 - k, kMostFollow) << kFollowShift) |
+            (burst_of_pages(take, sub.n_descs, sub.payload_bytes, e->workgroups - 1) ? kBurstEntry : 0u);
     p[11] = sub.payload_bytes;
     if (k < kCarriedEntries && sub.n_descs != 0 && sub.n_descs <= kCarriedDescs && stamp != 0 && e->tail - head < kCarryBehind &&
         carry_descriptors(e, sub, stamp))
@@ -1867,7 +1888,7 @@ int tcpxuEngineTicketPlan(uint32_t workgroups, uint32_t descs_per_ticket, uint32
   }
   const uint32_t bytes = payload_bytes > 0xFFFFFFFFull ? 0xFFFFFFFFu : static_cast<uint32_t>(payload_bytes);
   const uint32_t per = descs_per_ticket != 0 ? descs_per_ticket
-                                             : ticket_size_for_submission(in_flight, n_descs, bytes, workgroups - 1);
+                                             : ticket_size_for_submission(in_flight, n_descs, bytes, workgroups - 1, false);
   if (per_ticket) *per_ticket = per;
   if (n_tickets) *n_tickets = (n_descs + per - 1) / per;
   return TCPXU_SUCCESS;

@@ -1,6 +1,7 @@
 """Bursts: several submissions handed over in one call to an engine of 32 workers, on both sides of the lines where the size
-of their tickets changes (three, four and eight submissions, 32 descriptors each, the backlog per worker), with a payload hint
-that says whole pages, one that says short fragments -- those submissions say how many more of their call follow -- and none."""
+of their tickets changes (three, four and eight submissions, 32 descriptors each, 12 x 32 and 40 x 32 descriptors in all), with
+a payload hint that says whole pages, one that says short fragments -- those submissions say how many more of their call
+follow -- and none."""
 import ctypes
 
 import numpy as np
@@ -16,7 +17,7 @@ WORKERS = 32
 
 
 @pytest.mark.parametrize("hint", [4096, 1000, 0])
-@pytest.mark.parametrize("subs_n", [(8, 47), (8, 48), (8, 199), (8, 200), (7, 90), (12, 32), (12, 33), (40, 40), (4, 70), (3, 500)])
+@pytest.mark.parametrize("subs_n", [(8, 47), (8, 48), (8, 159), (8, 160), (8, 199), (8, 200), (7, 90), (12, 32), (12, 33), (40, 40), (4, 70), (3, 500)])
 def test_burst(pkg, hip, oracle, subs_n, hint):
     count, per = subs_n
     rng = np.random.default_rng(count * per)
