@@ -177,8 +177,9 @@ int tcpxuEngineSubmitMany(tcpxuEngine* engine, const tcpxuSubmission* submission
  * the given descs_per_ticket (0 = by backlog), a submission of n_descs descriptors and payload_bytes (0 = unknown)
  * with `in_flight` submissions not yet completed (itself included) is handed out in *n_tickets tickets of
  * *per_ticket descriptors; *max_descs is the most descriptors a submission may carry.  Outputs may be NULL.
- * (What it does not know: how many more submissions a call hands over, which count as in flight for one of short
- * fragments; and what the leader finds at run time: while eight or more submissions wait in one of its polls, tickets sized
+ * (What it does not know: how many submissions a call hands over together -- the ones still to come count as in flight for
+ * one of short fragments, and eight or more of whole pages, of more than 32 descriptors each and 12 to 40 per worker
+ * workgroup in all, go in tickets of 18 -- and what the leader finds at run time: while eight or more submissions wait in one of its polls, tickets sized
  * by backlog are at least 16 descriptors, and while four or more do, those that would be of fewer than 14 are 16.)
  * TCPXU_INVALID_ARGUMENT for an n_descs beyond that limit. */
 int tcpxuEngineTicketPlan(uint32_t workgroups, uint32_t descs_per_ticket, uint32_t in_flight, uint32_t n_descs,
