@@ -120,7 +120,7 @@ __host__ __device__ __forceinline__ uint32_t full_ticket_size(uint32_t bytes, ui
 // other buffers from pass to pass, by backlog / in tickets of 18 / 20 / 22 / 24: eight requests of 4 MiB 24.9 / 24.2 / 24.4 /
 // 25.1 / 25.4, sixteen 35.5 / 35.6 / 36.1 / 36.5 / 36.6, 16 of 2 MiB 26.1 / 24.3 / 24.2 / 24.2 / 24.3, 32 of 2 MiB 38.5 / 36.1 /
 // 36.6 / 36.9 / 37.0, 40 of 1 MiB 28.9 / 28.9 / 29.7 / 29.9 / 29.9, 64 of 1 MiB 35.8 / 35.7 / 35.8 / 36.1 / 35.5.  Where a part of
-// the buffers is still in the caches, sixteen of 4 MiB take 33.5 by backlog and 32.6 with 18 to 24 (on some boxes 31.8 and
+// the buffers is still in the caches, sixteen of 4 MiB take 33.5 by backlog and 32.6 with 18 to 24 (on some machines 31.8 and
 // 32.5).  Above the range the last round is a small part of the whole (24 requests of 4 MiB, 48 a workgroup: 46.5 by backlog,
 // 47.3 in tickets of 18); below it the sizes by backlog, which begin at 8, reach all the workgroups sooner.
 constexpr uint32_t kBurstTicket = 18;
