@@ -1270,8 +1270,8 @@ __device__ __forceinline__ void copy_ticket(const LdsStage* stage, uint32_t wave
   auto produce = [&](CopyRound& out, const CopyRound& prev) -> bool {
     if (nvec_left != 0) {
       out = prev;
-      out.has_edge = false;  // the first round has copied the edge bytes and the shared line
-      out.share_next = false;
+      out.edges = 0;  // the first round has copied the edge bytes and the shared line
+      out.share_next = 0;
       out.src_vec = prev.src_vec + (static_cast<size_t>(prev.nvec) << 4);
       out.dst_vec = prev.dst_vec + (static_cast<size_t>(prev.nvec) << 4);
       out.nvec = nvec_left < kVecPerRound ? nvec_left : kVecPerRound;

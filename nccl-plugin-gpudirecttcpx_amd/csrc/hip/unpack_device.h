@@ -24,7 +24,6 @@ constexpr int kVecPerLane = 4;
 constexpr uint32_t kVecPerRound = kVecPerLane * kWaveLanes;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef u32x4 u32x4_any __attribute__((aligned(1)));  // 16-byte vector at any byte alignment
 
 // Payload always lives in global memory (the arena and the caller's receive buffer), so every payload access
 // is cast to the global address space: the compiler then emits global_* instead of flat_* instructions even
@@ -78,8 +77,8 @@ __device__ __forceinline__ void store_byte_sys(uint8_t* p, uint8_t v) {
 // Both owners decide with the same inputs whether the rule applies to a boundary:
 constexpr uint32_t kLineBytes = 128;
 // The line must hold nothing but the end of A and the beginning of B -- A reaches back to the line's first byte, B
-// on to its last -- and each of the two must be long enough for a 16-byte load of its own bytes and not be one of
-// the tiny fragments that are copied bytewise.
+// on to its last -- and each of the two must be at least 16 bytes and not be one of the tiny fragments that are copied
+// bytewise.
 __device__ __forceinline__ bool fragment_is_tiny(const uint8_t* dst, uint32_t len);
 __device__ __forceinline__ bool shares_line(uint64_t dst_a, uint32_t len_a, uint64_t dst_b, uint32_t len_b) {
   const uint32_t in_line = static_cast<uint32_t>(dst_a + len_a) & (kLineBytes - 1);  // bytes of A in the line
@@ -88,31 +87,29 @@ __device__ __forceinline__ bool shares_line(uint64_t dst_a, uint32_t len_a, uint
          !fragment_is_tiny(reinterpret_cast<const uint8_t*>(dst_b), len_b);
 }
 
-// 16 bytes starting at byte `shift` (0..16) of the 32 bytes a:b.
-__device__ __forceinline__ u32x4 extract16(u32x4 a, u32x4 b, uint32_t shift) {
-  const uint32_t q = shift >> 2, r = shift & 3u;
-  const uint32_t w[9] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3], 0u};
-  uint32_t sel[5];
-#pragma unroll
-  for (int k = 0; k < 5; ++k)
-    sel[k] = q == 0 ? w[k] : q == 1 ? w[k + 1] : q == 2 ? w[k + 2] : q == 3 ? w[k + 3] : w[k + 4];
-  u32x4 out;
-#pragma unroll
-  for (int d = 0; d < 4; ++d) out[d] = __builtin_amdgcn_alignbyte(sel[d + 1], sel[d], r);
-  return out;
+// A window on memory: a buffer resource, whose accesses the hardware checks against its length, dword by dword.  A lane
+// whose offset lies beyond it reads zeros without a trip to memory, and stores nothing: which lanes take part in an
+// access costs no instruction.
+typedef __amdgpu_buffer_rsrc_t Window;
+__device__ __forceinline__ Window window(const uint8_t* p, uint32_t bytes) {
+  constexpr int kRaw32 = 0x00020000;  // word 3: no swizzling, 32-bit data
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p), 0, static_cast<int>(bytes), kRaw32);
 }
+constexpr uint32_t kOutside = 0x80000000u;       // an offset outside any window of a round's vectors or of a line
+constexpr int kSystem = 17, kSystemStream = 19;  // scopes of a window's accesses: sc0 sc1; sc0 sc1 nt (see above)
 
 // One round of a wavefront's copy work: up to 4 KiB of 16-byte vectors with a 16-byte aligned destination, the
 // edge bytes of the fragment (a head and a tail of fewer than 16 bytes where the fragment keeps its own partial
-// lines), and the shared last line (eight vectors, each assembled from up to two sources).
+// lines), and the shared last line (32 dwords, each from one of two sources, and one of them from both).
 // Loading and storing are separate steps, with an explicit wait for everything in flight between them.
 //
-// Only the lanes that have something to move take part in a memory instruction, and a part of the round that
-// has nothing to move is skipped by the whole wavefront: the edge bytes where the fragment shares its first and
-// last line with its neighbours, the shared line where it does not, the extra dword where the source needs no
-// shifting.  (An earlier form issued the same eight loads and six stores in every round, with idle lanes
-// repeating a neighbour's access; at an 8 MiB chunk of 4 KiB fragments the four main vectors alone ran 5 % faster
-// than that.)
+// Between them lie the instructions that bound rounds of short fragments (16 wavefronts a compute unit, each waiting for
+// its own): so the vectors go through windows, with one offset per lane and no comparison, mask, branch or 64-bit address
+// per vector, the line goes by dwords, where the boundary cuts one (by vectors, it took a shift by a number of dwords that
+// the compiler made thirty branches of), and the edge bytes are not waited for ahead of the vectors.  A part of the round
+// that has nothing to move is skipped by the whole wavefront.  (Against masked accesses and a line of eight vectors: 4 MiB
+// of wire fragments in one launch 4.9 -> 4.4 us, 64 KiB of fragments of any length 4.2 -> 3.6, 256 MiB of them 99.6 -> 95.8,
+// through the engine 113.7 -> 109.1; whole pages by the half GiB, which the memory system bounds, 0.3 % slower.)
 constexpr uint32_t kNoEdge = 0xFFFFFFFFu;
 struct CopyRound {
   // Wave-uniform (scalar registers):
@@ -124,43 +121,25 @@ struct CopyRound {
   uint32_t nvec;            // vectors in this round, 0..kVecPerRound (0: nothing but a shared line or edge bytes)
   uint32_t frag_len;
   uint32_t line_off;        // offset of the shared last line from dst_frag
-  bool share_next;          // this round completes the fragment's last line out of the next fragment
-  bool has_edge;            // this round copies edge bytes (some lane has one)
-  // Per lane:
-  uint32_t edge_off;        // offset of this lane's edge byte in the fragment, kNoEdge if it has none
+  uint32_t share_next;      // this round completes the fragment's last line out of the next fragment
+  uint32_t edges;           // edge bytes that this round copies: head | tail << 8
 };
 constexpr int kDppWaveShiftLeft1 = 0x130;  // lane i receives lane i+1's value; lane 63 keeps the first operand
 struct CopyRegs {
   u32x4 r[kVecPerLane];
-  u32x4 line;  // lanes 0..7: the shared line's vectors as loaded; lane 8: the first 16 bytes of the next fragment
-  uint32_t tail_dword;
+  uint32_t line, line_next;  // the shared line's dwords from this fragment and from the next, zero where the other's are
+  uint32_t tail_dword;       // the dword behind a round of kVecPerRound vectors, the same in every lane
   uint32_t edge_byte;
 };
-constexpr uint32_t kLineVecs = kLineBytes / 16;  // lanes that take part in the shared line
 
-// The shared last line, lanes 0..7, one 16-byte vector each.  The fragment (A) has `rem` = frag_len - line_off bytes
-// in the line (1..127), the next fragment (B) the rest.  Where the boundary falls is the same for the whole
-// wavefront, so nothing here is worked out per lane beyond an address:
-//   vectors before the boundary are 16 bytes of A, vectors after it 16 bytes of B, each loaded where it lies
-//   (any alignment) and stored as loaded;
-//   the one vector the boundary cuts (none if rem is a multiple of 16) is the last `cut` bytes of A followed by
-//   the first 16 - cut bytes of B: its lane loads A's last 16 bytes, lane 8 of the same instruction loads B's first
-//   16 for it, and it takes bytes [16 - cut, 32 - cut) of the two, a shift by a wave-uniform amount.
-// shares_line has seen to it that every one of these loads stays inside its fragment.
-// (An earlier form gave every lane two loads and a shift of its own, by a per-lane amount: some sixty vector
-// instructions a line instead of some twenty, a sixth of the time of a round of a 2 KiB fragment.)
-struct LinePlan {
-  uint32_t rem;       // bytes of this fragment in the line
-  uint32_t cut_lane;  // the vector the boundary falls in
-  uint32_t cut;       // bytes of this fragment in that vector, 0 = the boundary falls between two vectors
-};
-__device__ __forceinline__ LinePlan line_plan(const CopyRound& c) {
-  LinePlan p;
-  p.rem = c.frag_len - c.line_off;
-  p.cut_lane = p.rem >> 4;
-  p.cut = p.rem & 15u;
-  return p;
-}
+// The shared last line, lanes 0..31, a dword each.  The fragment (A) has `rem` = frag_len - line_off bytes in the line
+// (1..127), the next fragment (B) the rest.  Dwords before the boundary are 4 bytes of A, dwords after it 4 bytes of B,
+// loaded where they lie (any alignment) and stored as loaded.  The one dword that the boundary cuts (none if rem is a
+// multiple of 4) is the last bytes of A followed by the first of B: its lane loads A's last 4 bytes, lane 32 loads B's first
+// 4, and a shift of the two by the same amount for the whole wavefront makes it.  A load for each side, since a window has
+// one base; a lane of the other side is outside and reads zero.  shares_line has seen to it that every one of these loads
+// stays inside its fragment.
+constexpr uint32_t kLineDwords = kLineBytes / 4;
 
 // Source realignment.  A 16-byte load whose address is not a multiple of 4 is split by the memory pipeline and
 // runs at roughly two thirds of the rate of one that is (a multiple of 4 that is not a multiple of 16 costs
@@ -169,43 +148,45 @@ __device__ __forceinline__ LinePlan line_plan(const CopyRound& c) {
 // round therefore loads from the 4-byte aligned address just below (`skew` = 0..3 bytes below, the same for
 // every vector of the round) and shifts the bytes into place in registers: a vector is bytes [skew, skew+16)
 // of its own four dwords plus one more dword, and that fifth dword is the first dword of the next vector --
-// which the neighbouring lane holds.  Only the round's last vector has no neighbour; its fifth dword comes
-// from one extra 4-byte load by lane 0 (with skew > 0 that dword starts inside the fragment, and an aligned dword
-// never leaves the 4 KiB page it starts in; with skew 0 nothing of it is used and it is not loaded).
-__device__ __forceinline__ uint32_t load_dword_sys(const uint8_t* p) {
-  return __hip_atomic_load((const TCPXU_GLOBAL uint32_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+// which the neighbouring lane holds.  For the round's last vector the window ends one dword further, so that the lane
+// after it loads that dword and nothing else (with skew > 0 it starts inside the fragment, and an aligned dword never
+// leaves the 4 KiB page it starts in; with skew 0 nothing of it is used and the window ends with the last vector).  A round
+// of kVecPerRound vectors has no lane left for it and takes one load more.
+
+// Lanes [0,head) carry the head, lanes [16,16+tail) the tail (both < 16 bytes); the other lanes have none.
+__device__ __forceinline__ uint32_t edge_offset(const CopyRound& c, uint32_t lane) {
+  const uint32_t in_tail = lane - 16u;
+  uint32_t off = in_tail < (c.edges >> 8) ? c.line_off + in_tail : kNoEdge;
+  if (lane < (c.edges & 0xFFu)) off = lane;
+  return off;
 }
 
 __device__ __forceinline__ void round_load(const CopyRound& c, CopyRegs& x, uint32_t lane) {
   const uint32_t skew = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(c.src_vec)) & 3u;
   const uint8_t* base4 = c.src_vec - skew;
-  // No register of the round is cleared first: a lane that loads nothing stores nothing (the same conditions guard
-  // the stores), and what the shifts read from such a lane never reaches a stored byte.  The empty statement only
-  // tells the compiler that the registers have a value (clearing them was a tenth of a short round's instructions).
-  asm volatile("" : "=v"(x.r[0]), "=v"(x.r[1]), "=v"(x.r[2]), "=v"(x.r[3]), "=v"(x.line), "=v"(x.tail_dword), "=v"(x.edge_byte));
-  if (c.has_edge) {
-    if (c.edge_off != kNoEdge) x.edge_byte = load_byte_sys(c.src_frag + c.edge_off);
+  const uint32_t at = lane << 4;
+  // No register of the round is cleared first: what the shifts read from one that was not loaded never reaches a stored
+  // byte.  The empty statement only tells the compiler that the registers have a value.
+  asm volatile("" : "=v"(x.r[0]), "=v"(x.r[1]), "=v"(x.r[2]), "=v"(x.r[3]), "=v"(x.line), "=v"(x.line_next), "=v"(x.tail_dword),
+               "=v"(x.edge_byte));
+  if (c.share_next != 0) {  // (first: two source pages are asked for before the bulk of one of them)
+    const uint32_t rem = c.frag_len - c.line_off, at4 = lane << 2;
+    const bool in_next = at4 >= rem;
+    const uint32_t own = in_next ? kOutside : min(at4 + 4u, rem);
+    const uint32_t next = lane == kLineDwords ? 0u : in_next ? at4 - rem : kOutside;
+    x.line = __builtin_amdgcn_raw_buffer_load_b32(window(c.src_frag + c.line_off - 4, rem + 4), own, 0, kSystem);
+    x.line_next = __builtin_amdgcn_raw_buffer_load_b32(window(c.src_next, kLineBytes - rem > 4 ? kLineBytes - rem : 4), next, 0, kSystem);
   }
+  const uint32_t bytes = ((c.nvec << 4) + skew + 3u) & ~3u;
+  const Window from = window(base4, bytes);
 #pragma unroll
   for (int k = 0; k < kVecPerLane; ++k) {
-    const uint32_t v = static_cast<uint32_t>(k) * kWaveLanes + lane;
-    if (v < c.nvec) x.r[k] = load_vec_sys(base4 + (v << 4));
+    constexpr uint32_t kStep = 16 * kWaveLanes;
+    if (k == 0 || bytes > k * kStep) x.r[k] = __builtin_amdgcn_raw_buffer_load_b128(from, at + k * kStep, 0, kSystem);
   }
-  if (skew != 0 && c.nvec != 0) {
-    if (lane == 0) x.tail_dword = load_dword_sys(base4 + (c.nvec << 4));
-  }
-  if (c.share_next) {
-    const LinePlan p = line_plan(c);
-    // One load instruction: the line's eight vectors in lanes 0..7 and, where the boundary cuts a vector, the next
-    // fragment's first 16 bytes in lane 8 (a load of its own for that one lane was a fifth of a ragged round's loads).
-    if (lane < kLineVecs + (p.cut != 0 ? 1u : 0u)) {
-      const uint32_t off = lane << 4;
-      const uint8_t* from = lane < p.cut_lane ? c.src_frag + c.line_off + off : c.src_next + (off - p.rem);
-      if (p.cut != 0 && lane == p.cut_lane) from = c.src_frag + c.frag_len - 16u;
-      if (lane == kLineVecs) from = c.src_next;
-      x.line = load_vec_sys(from);
-    }
-  }
+  if (bytes > 16 * kVecPerRound) x.tail_dword = __builtin_amdgcn_raw_buffer_load_b32(from, 16 * kVecPerRound, 0, kSystem);
+  if (c.edges != 0)
+    x.edge_byte = __builtin_amdgcn_raw_buffer_load_b8(window(c.src_frag, c.frag_len), edge_offset(c, lane), 0, kSystem);
 }
 
 // Waits for every load of the round (and for whatever else the wavefront has in flight) rather than let each
@@ -214,7 +195,7 @@ __device__ __forceinline__ void round_load(const CopyRound& c, CopyRegs& x, uint
 // use of them can be scheduled before it.
 __device__ __forceinline__ void round_wait(CopyRegs& x) {
   asm volatile("s_waitcnt vmcnt(0)"
-               : "+v"(x.r[0]), "+v"(x.r[1]), "+v"(x.r[2]), "+v"(x.r[3]), "+v"(x.line),
+               : "+v"(x.r[0]), "+v"(x.r[1]), "+v"(x.r[2]), "+v"(x.r[3]), "+v"(x.line), "+v"(x.line_next),
                  "+v"(x.tail_dword), "+v"(x.edge_byte)
                :
                : "memory");
@@ -224,44 +205,36 @@ __device__ __forceinline__ void round_wait(CopyRegs& x) {
 // Shifts the loaded bytes into place and stores them; the round's loads must have landed (round_wait).
 __device__ __forceinline__ void round_store_loaded(const CopyRound& c, CopyRegs& x, uint32_t lane) {
   const uint32_t skew = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(c.src_vec)) & 3u;
-  const uint32_t last = c.nvec - 1;
-  const uint32_t tail_dword = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x.tail_dword), 0));
+  const uint32_t at = lane << 4;
+  const uint32_t bytes = c.nvec << 4;
+  const Window to = window(c.dst_vec, bytes);
 #pragma unroll
   for (int k = 0; k < kVecPerLane; ++k) {
+    constexpr uint32_t kStep = 16 * kWaveLanes;
+    if (k != 0 && bytes <= k * kStep) continue;
     // First dword of the next vector: lane+1 of this register, or lane 0 of the next register for lane 63.
-    // (a DPP wavefront shift: one vector instruction, no trip through the LDS crossbar)
-    uint32_t next0 = static_cast<uint32_t>(
-        __builtin_amdgcn_update_dpp(0, static_cast<int>(x.r[k][0]), kDppWaveShiftLeft1, 0xF, 0xF, false));
-    if (k + 1 < kVecPerLane) {
-      const uint32_t wrap = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x.r[k + 1 < kVecPerLane ? k + 1 : k][0]), 0));
-      if (lane == 63u) next0 = wrap;
-    }
-    const uint32_t v = static_cast<uint32_t>(k) * kWaveLanes + lane;
-    const uint32_t w4 = v < last ? next0 : tail_dword;  // the last vector uses the extra dword
+    // (a DPP wavefront shift, which leaves lane 63 what it is given: no trip through the LDS crossbar)
+    const int wrap = k + 1 < kVecPerLane ? __builtin_amdgcn_readlane(static_cast<int>(x.r[k + 1 < kVecPerLane ? k + 1 : k][0]), 0)
+                                         : static_cast<int>(x.tail_dword);
+    const uint32_t next0 = static_cast<uint32_t>(
+        __builtin_amdgcn_update_dpp(wrap, static_cast<int>(x.r[k][0]), kDppWaveShiftLeft1, 0xF, 0xF, false));
     u32x4 out;
     out[0] = __builtin_amdgcn_alignbyte(x.r[k][1], x.r[k][0], skew);
     out[1] = __builtin_amdgcn_alignbyte(x.r[k][2], x.r[k][1], skew);
     out[2] = __builtin_amdgcn_alignbyte(x.r[k][3], x.r[k][2], skew);
-    out[3] = __builtin_amdgcn_alignbyte(w4, x.r[k][3], skew);
-    if (v < c.nvec) store_vec_stream(c.dst_vec + (v << 4), out);
+    out[3] = __builtin_amdgcn_alignbyte(next0, x.r[k][3], skew);
+    __builtin_amdgcn_raw_buffer_store_b128(out, to, at + k * kStep, 0, kSystemStream);
   }
-  if (c.share_next) {
-    const LinePlan p = line_plan(c);
-    u32x4 line = x.line;
-    if (p.cut != 0) {
-      // (lane 8's vector, the same for every lane: scalar registers)
-      u32x4 next16;
-#pragma unroll
-      for (int d = 0; d < 4; ++d)
-        next16[d] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x.line[d]), static_cast<int>(kLineVecs)));
-      const u32x4 cut_vector = extract16(x.line, next16, 16u - p.cut);
-      if (lane == p.cut_lane) line = cut_vector;
-    }
-    if (lane < kLineVecs) store_vec_stream(c.dst_frag + c.line_off + (lane << 4), line);
+  if (c.share_next != 0) {
+    const uint32_t rem = c.frag_len - c.line_off;
+    x.line |= x.line_next;
+    const uint32_t next4 = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x.line), kLineDwords));
+    const uint32_t cut = __builtin_amdgcn_alignbyte(next4, x.line, (0u - rem) & 3u);
+    const uint32_t out = lane == rem >> 2 ? cut : x.line;
+    __builtin_amdgcn_raw_buffer_store_b32(out, window(c.dst_frag + c.line_off, kLineBytes), lane << 2, 0, kSystemStream);
   }
-  if (c.has_edge) {
-    if (c.edge_off != kNoEdge) store_byte_sys(c.dst_frag + c.edge_off, static_cast<uint8_t>(x.edge_byte));
-  }
+  if (c.edges != 0)
+    __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(x.edge_byte), window(c.dst_frag, c.frag_len), edge_offset(c, lane), 0, kSystem);
 }
 
 __device__ __forceinline__ void round_store(const CopyRound& c, CopyRegs& x, uint32_t lane) {
@@ -321,11 +294,7 @@ __device__ __forceinline__ CopyRound first_round_of(const uint8_t* src, uint8_t*
   c.frag_len = len;
   c.line_off = end_off;
   c.share_next = share_next;
-  // Lanes [0,head) carry the head, lanes [16,16+tail) the tail (both < 16 bytes); the other lanes have none.
-  c.has_edge = (head | tail) != 0;
-  c.edge_off = kNoEdge;
-  if (lane < head) c.edge_off = lane;
-  else if (lane >= 16u && lane - 16u < tail) c.edge_off = end_off + (lane - 16u);
+  c.edges = head | (tail << 8);
   c.nvec = nvec < kVecPerRound ? nvec : kVecPerRound;
   *nvec_left = nvec - c.nvec;
   return c;
@@ -364,8 +333,8 @@ __device__ __forceinline__ void copy_descriptor(const uint8_t* bounce, uint8_t* 
     round_load(r, x, lane);
     round_store(r, x, lane);
     if (left == 0) return;
-    r.has_edge = false;
-    r.share_next = false;
+    r.edges = 0;
+    r.share_next = 0;
     r.src_vec += static_cast<size_t>(r.nvec) << 4;
     r.dst_vec += static_cast<size_t>(r.nvec) << 4;
     r.nvec = left < kVecPerRound ? left : kVecPerRound;
