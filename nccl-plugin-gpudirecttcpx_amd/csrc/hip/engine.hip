@@ -1248,7 +1248,7 @@ __device__ void retire_ticket(DevState* st, uint32_t* jobs_done, const LdsStage*
 }
 
 // Copy wavefront `wave` of kCopyWaves: its run of consecutive fragments of the staged ticket (an eighth of the
-// ticket, rounded up), one round (at most 4 KiB) in flight at a time.  A wavefront that writes one contiguous
+// ticket, rounded up), one round (at most 4 KiB) in flight at a time, or two.  A wavefront that writes one contiguous
 // stretch of the destination after another measured about 1 % faster end to end than fragments dealt out in turn
 // (wave, wave + kCopyWaves, ...).
 __device__ __forceinline__ void copy_ticket(const LdsStage* stage, uint32_t wave, uint32_t lane, lds_u32* waves_on_last) {
@@ -1300,22 +1300,30 @@ __device__ __forceinline__ void copy_ticket(const LdsStage* stage, uint32_t wave
     }
     return false;
   };
-  // In a ticket of short fragments (one of more than kFullTicket descriptors: the leader makes those for
-  // submissions whose payload says so) the next round is worked out -- its record read from LDS, its scalars set
-  // up -- while the loads of the round in flight are on their way, not after its stores: that work is a seventh of
-  // a short round's time (fragments of 1.8 KiB on average: 62.5 % -> 63.6 % of the roofline).  In a ticket of whole
-  // pages it stays where it was: they move up to 1 % faster with that pause between a round's stores and the next
-  // round's loads.
-  const bool ahead = n > kFullTicket;
+  // Two rounds under way at a time -- the second is worked out and asked for while the first one's loads are on their way,
+  // and both are waited for together -- in a ticket of more than kFullTicket descriptors (the leader makes those of short
+  // fragments, whose rounds leave half of a wavefront's registers empty) and in a request's only ticket, which is waited
+  // for.  The other tickets are of whole pages in a stream, where sixteen wavefronts a compute unit with a page each are
+  // all that the memory system takes.  (All one at a time / all in pairs: 2048 requests of 64 KiB through the plugin, 16
+  // posted at a time, 1045 / 1000 us, 256 MiB of ragged fragments 109.3 / 108.4, of whole pages 103.9 / 105.7.)
+  const bool pairs = n > kFullTicket || (uniform(stage->payload[10]) & kOnlyTicket) != 0;
   CopyRound r, next;
-  CopyRegs x;
+  CopyRegs x, y;
   bool more = produce(r, r);
   while (more) {
     round_load(r, x, lane);
-    if (ahead) more = produce(next, r);
-    round_store(r, x, lane);
-    if (!ahead) more = produce(next, r);
-    r = next;
+    if (pairs) {
+      const bool second = produce(next, r);
+      if (second) round_load(next, y, lane);
+      rounds_wait(x, y);
+      round_store_loaded(r, x, lane);
+      if (second) round_store_loaded(next, y, lane);
+      more = second && produce(r, next);
+    } else {
+      round_store(r, x, lane);
+      more = produce(next, r);
+      r = next;
+    }
   }
 }
 

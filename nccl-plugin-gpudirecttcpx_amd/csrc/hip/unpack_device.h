@@ -201,6 +201,11 @@ __device__ __forceinline__ void round_wait(CopyRegs& x) {
                : "memory");
   static_assert(kVecPerLane == 4, "the statement above names the four vectors of a round");
 }
+// The same for two rounds whose loads are under way together.
+__device__ __forceinline__ void rounds_wait(CopyRegs& x, CopyRegs& y) {
+  round_wait(x);
+  round_wait(y);
+}
 
 // Shifts the loaded bytes into place and stores them; the round's loads must have landed (round_wait).
 __device__ __forceinline__ void round_store_loaded(const CopyRound& c, CopyRegs& x, uint32_t lane) {

@@ -74,3 +74,27 @@ def test_fragment_beyond_2_gib(pkg, hip, kernel):
     for src, length, dst in zip(srcs, lens, dsts):
         assert torch.equal(out[GUARD + int(dst) :][:length], pool[src : src + length])
     assert bool((out[: GUARD + 3] == SENTINEL).all()) and bool((out[-GUARD:] == SENTINEL).all())
+
+
+@pytest.mark.parametrize("per_ticket", [0, 8, 16, 17, 24, 33, 64])
+def test_rounds_in_pairs(pkg, hip, oracle, per_ticket):
+    """Shares of one to eight fragments a wavefront, odd and even, with tiny, empty and several-round fragments first, second
+    and last in a pair: requests of one ticket (pairs), of several small ones (one at a time), of several large ones (pairs)."""
+    engine = Engine(pkg, hip, descs_per_ticket=per_ticket)
+    engine.start()
+    for n in (1, 2, 8, 9, 15, 16, 17, 31, 64, 65, 130):
+        rng = np.random.default_rng(100 * per_ticket + n)
+        lens = rng.choice([0, 1, 29, 31, 700, 2048, 4095, 4096, 4097, 9000], size=n, p=[0.1, 0.05, 0.05, 0.05, 0.2, 0.2, 0.1, 0.1, 0.05, 0.1])
+        descs = np.zeros(n, dtype=np.dtype([("src_off", "<u4"), ("len", "<u4"), ("dst_off", "<u8")]))
+        descs["len"], descs["dst_off"] = lens, np.cumsum(lens) - lens
+        descs["src_off"] = rng.integers(0, (1 << 20) - 9000, n)
+        pool = rng.integers(0, 256, 1 << 20, dtype=np.uint8)
+        total = int(lens.sum())
+        expect = oracle_expected(oracle, pool, descs, total, 5)
+        buf, mapped = GpuBuffers(pool, descs, total, 5), Mapped(pkg, hip, descs, 1)
+        print("tickets of %d, %d descriptors, %d bytes" % (per_ticket, n, total), flush=True)
+        engine.submit(buf.pool.data_ptr(), buf.dst_base, mapped.desc_dev(0), n, mapped.flag_dev(0), 9)
+        mapped.wait(0, 9)
+        assert first_difference(buf.result(), expect) is None
+        mapped.free()
+    engine.destroy()
