@@ -1092,3 +1092,32 @@ def test_engine_stamps_order_the_stages_of_a_submission(pkg, hip, oracle):
     e.destroy()
     m.free()
     assert first_difference(got, expect) is None, repr(first_difference(got, expect))
+
+
+@pytest.mark.parametrize("workgroups", [2, 3, 9, 257, 258, 513, 640])
+def test_grids_of_any_size_serve_every_ticket(pkg, hip, oracle, workgroups):
+    """A worker on the leader's compute unit leaves if enough others have started elsewhere, and only then: two workers,
+    one more or less than that many, the default grid and a grid with workgroups that find no place while it runs; each
+    through several launches, every request served."""
+    rng = np.random.default_rng(workgroups)
+    lens = rng.choice([0, 100, 2000, 4096], size=3000)
+    descs = np.zeros(3000, dtype=np.dtype([("src_off", "<u4"), ("len", "<u4"), ("dst_off", "<u8")]))
+    descs["len"], descs["dst_off"] = lens, np.cumsum(lens) - lens
+    descs["src_off"] = rng.integers(0, (4 << 20) - 4096, 3000)
+    pool = rng.integers(0, 256, 4 << 20, dtype=np.uint8)
+    expect = oracle_expected(oracle, pool, descs, int(lens.sum()))
+    g, m = GpuBuffers(pool, descs, int(lens.sum())), Mapped(pkg, hip, descs, 60)
+    e = Engine(pkg, hip, workgroups=workgroups)
+    print("grid of %d workgroups" % workgroups, flush=True)
+    for launch in range(4):
+        g.reset()
+        e.start()
+        for i in range(60):
+            e.submit(g.pool.data_ptr(), g.dst_base, m.desc_dev(50 * i), 50, m.flag_dev(i), launch + 1)
+        for i in range(60):
+            m.wait(i, launch + 1)
+        assert first_difference(g.result(), expect) is None
+        e.stop()
+    assert e.completed() == 240
+    e.destroy()
+    m.free()
