@@ -306,15 +306,21 @@ __device__ __forceinline__ CopyRound first_round_of(const uint8_t* src, uint8_t*
 }
 
 // Copies descriptor i of a list of n with the calling wavefront (all arguments wave-uniform but `lane`): what the
-// kernels that are launched per list do.  Lanes 0 to 2 read the descriptor before it, its own and the one after it,
-// one load for the three, and hand them over through scalar registers: nothing is staged, nobody waits at a barrier.
+// kernels that are launched per list do.  The descriptor before it, its own and the one after it are read into scalar
+// registers: nothing is staged, nobody waits at a barrier.  They come through the scalar cache, which two compute units
+// share and which is empty when a kernel begins (the list stays as it is until the kernel has ended, so that what it keeps
+// is what is there): neighbouring wavefronts need the same lines, and with lists in the host's memory each request for one
+// is a read over PCIe.  (By vector loads, two or three requests a wavefront -> so: 4 MiB of wire fragments, list in the
+// host's memory, 4.20 -> 4.00 us, 1 MiB 3.53 -> 3.43; 512 MiB, list in the GPU's, 177.9 -> 176.7.  One load for a workgroup
+// of 4, 8 or 16 wavefronts, handed over in LDS: 4 MiB 4.31, 4.31 and 4.97.)
 // A fragment that is longer than a round takes several, the first with its edges and its shared line.
 __device__ __forceinline__ void copy_descriptor(const uint8_t* bounce, uint8_t* dst, const tcpxuLoadMeta* descs, uint64_t n,
                                                 uint64_t i, uint32_t lane) {
-  u32x4 d = {0u, 0u, 0u, 0u};
-  const uint64_t at = i + lane - 1u;  // (wraps around before the first: not below n either)
-  if (lane < 3 && at < n) d = *reinterpret_cast<const u32x4*>(descs + at);
-  auto word = [&](int of, int k) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(d[k]), of)); };
+  typedef const __attribute__((address_space(4))) u32x4* constant_ptr;
+  const constant_ptr list = (constant_ptr)(descs + i);
+  const u32x4 none = {0u, 0u, 0u, 0u};
+  const u32x4 d[3] = {i != 0 ? list[-1] : none, list[0], i + 1 < n ? list[1] : none};
+  auto word = [&](int of, int k) { return d[of][k]; };
   auto place = [&](int of) { return reinterpret_cast<uint64_t>(dst) + ((static_cast<uint64_t>(word(of, 3)) << 32) | word(of, 2)); };
   constexpr int kPrev = 0, kOwn = 1, kNext = 2;
   const uint32_t len = word(kOwn, 1);

@@ -136,3 +136,46 @@ def test_replays_of_the_same_call_at_the_same_time(pkg, hip, oracle, n):
         torch.cuda.synchronize()
         assert int(mapped.flags[0]) == 77 and first_difference(buf.result(), expect) is None
     mapped.free()
+
+
+@pytest.mark.parametrize("n", [1, 5, 16, 40])
+@pytest.mark.parametrize("captured", [False, True])
+def test_a_list_rewritten_between_calls_is_read_afresh(pkg, hip, oracle, n, captured):
+    """The same slot of mapped memory and the same completion word, another list each time, written as soon as the word
+    says that the last one has been copied: the descriptors come through a cache, which must not keep the last list's."""
+    import torch
+
+    pool = np.random.default_rng(n).integers(0, 256, PAGES * 4096, dtype=np.uint8)
+    room = n * 5000 + 3 * 4096
+    lists = [ragged_list(n, 1000 * n + k)[0] for k in range(60)]
+    expect = [oracle_expected(oracle, pool, d, room) for d in lists]
+    buf = GpuBuffers(pool, lists[0], room)
+    mapped = Mapped(pkg, hip, lists[0], 1)
+    stream = torch.cuda.Stream()
+
+    def call():
+        pkg.check(
+            hip.tcpxuUnpackSlotNoAlloc(0, buf.pool.data_ptr(), buf.dst_base, mapped.desc_dev(0), n, mapped.flag_dev(0), 5, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)),
+            "tcpxuUnpackSlotNoAlloc",
+        )
+
+    with torch.cuda.stream(stream):
+        call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    if captured:
+        with torch.cuda.graph(graph, stream=stream):
+            call()
+    print("lists of %d rewritten, captured: %s" % (n, captured), flush=True)
+    for k, d in enumerate(lists):
+        buf.reset()
+        mapped.flags[0] = 0
+        ctypes.memmove(mapped.host.value + mapped.flag_bytes, d.ctypes.data, d.nbytes)
+        for _ in range(2):  # the second right behind the first, with the list that the first one has seen
+            with torch.cuda.stream(stream):
+                graph.replay() if captured else call()
+            mapped.wait(0, 5)
+            mapped.flags[0] = 0
+        assert first_difference(buf.result(), expect[k]) is None, "list %d" % k
+    torch.cuda.synchronize()
+    mapped.free()
