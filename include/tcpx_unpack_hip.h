@@ -232,7 +232,7 @@ int tcpxuEngineRunning(tcpxuEngine* engine, int* running);
  * nothing is launched) at `descs_dev`, from `bounce_base` into `dst_base` -- with ordinary launches on `stream`
  * (a hipStream_t, NULL = the default stream) and then stores `done_value` to `*done_flag_dev` (device-visible 8-byte
  * word, e.g. the alias of mapped host memory; may be NULL when stream order is all the caller needs: the call is then
- * tcpxuUnpackBatch).  Up to 16 descriptors are one kernel, more are two, the second of which writes the word.
+ * tcpxuUnpackBatch).  Up to 24 descriptors are one kernel, more are two, the second of which writes the word.
  * Asynchronous.  It calls no hipMalloc, hipFree or other allocating routine and keeps nothing in device memory, so calls
  * may overlap on a GPU without limit: two streams, two threads, a replayed graph beside an ordinary call, two
  * executables of one captured graph (as far as their destinations and words allow it).

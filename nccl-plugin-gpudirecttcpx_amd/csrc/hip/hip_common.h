@@ -16,6 +16,7 @@ constexpr int kMaxDevices = 64;
 void set_error(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
 int use_device(int device);            // hipSetDevice + cache properties
 int device_compute_units(int device);  // valid after use_device
+bool device_known(int device);         // use_device has been there
 
 // The blocks that tcpxuMappedAlloc has given out, as one caller last saw them: it looks an address up in its own copy
 // and takes a new one only when blocks have come or gone since.
@@ -36,7 +37,7 @@ class DeviceScope {
  public:
   explicit DeviceScope(int device) {
     if (hipGetDevice(&saved_) != hipSuccess) saved_ = -1;
-    rc_ = use_device(device);
+    if (saved_ != device || !device_known(device)) rc_ = use_device(device);
     if (saved_ == device) saved_ = -1;  // nothing to put back
   }
   ~DeviceScope() {

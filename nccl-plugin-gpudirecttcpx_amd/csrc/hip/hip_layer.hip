@@ -60,16 +60,18 @@ __global__ __launch_bounds__(kBatchThreads) __attribute__((amdgpu_waves_per_eu(8
 // acknowledged, and nothing that a kernel could count that in is its own: a fixed array of counters is shared by whatever
 // runs at the same time (two executables of one captured graph pass the same arguments), and then the word comes early or
 // never.  So up to kSmallSlot descriptors are one workgroup, which knows by its barrier, and a longer list is the kernel
-// above followed by one of one thread that writes the word: the order of the stream says the rest.  (Us a call, with counters
-// that overlapping launches shared -> so: 1 whole page 3.95 -> 3.5, 4 pages 4.15 -> 3.7, 16 pages 4.3 -> 4.7, 17 to 128 pages
-// 4.4-4.6 -> 5.1-5.5, a 4 MiB slot of wire fragments 6.25 -> 6.4.  One workgroup for 24 descriptors 5.5, for 32 7.0.)
-constexpr uint32_t kSmallSlot = 16;  // a wavefront each, the most that a workgroup can have
-__global__ __launch_bounds__(kSmallSlot* kWaveLanes) void unpack_small_slot_kernel(const uint8_t* __restrict__ bounce, uint8_t* __restrict__ dst,
+// above followed by one of one thread that writes the word: the order of the stream says the rest.  A workgroup has sixteen
+// wavefronts at the most, so beyond 16 descriptors some of them take two, one after the other, while a second launch costs
+// the host 2.8 us.  (Us a call, one workgroup / two launches: 18 whole pages 4.2 / 6.3, 20 4.35 / 6.3, 24 4.9 / 6.3, 32 5.9 / 6.3,
+// 40 7.1 / 6.3; a call that is waited for: 24 pages 15.4 / 15.9, 32 16.6 / 15.8.)
+constexpr uint32_t kSmallSlot = 24;
+constexpr uint32_t kSmallSlotWaves = 16;
+__global__ __launch_bounds__(kSmallSlotWaves* kWaveLanes) void unpack_small_slot_kernel(const uint8_t* __restrict__ bounce, uint8_t* __restrict__ dst,
                                                                                   const tcpxuLoadMeta* __restrict__ descs, uint32_t n_descs,
                                                                                   uint64_t* done_flag, uint64_t done_value) {
   const uint32_t lane = threadIdx.x & (kWaveLanes - 1);
   const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWaveLanes)));
-  copy_descriptor(bounce, dst, descs, n_descs, wave, lane);
+  for (uint32_t i = wave; i < n_descs; i += kSmallSlotWaves) copy_descriptor(bounce, dst, descs, n_descs, i, lane);
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // this wavefront's write-through stores are acknowledged
   __syncthreads();
   if (threadIdx.x == 0) __hip_atomic_store(done_flag, done_value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -80,7 +82,7 @@ __global__ void complete_slot_kernel(uint64_t* done_flag, uint64_t done_value) {
 }
 
 struct DeviceProps {
-  bool valid = false;
+  std::atomic<bool> valid{false};
   int compute_units = 0;
   char name[256] = "";
 };
@@ -88,18 +90,20 @@ DeviceProps g_props[kMaxDevices];
 
 }  // namespace
 
+bool device_known(int device) { return device >= 0 && device < kMaxDevices && g_props[device].valid.load(std::memory_order_acquire); }
+
 int use_device(int device) {
   if (device < 0 || device >= kMaxDevices) {
     set_error("device index %d out of range", device);
     return TCPXU_INVALID_ARGUMENT;
   }
   TCPXU_HIP(hipSetDevice(device));
-  if (!g_props[device].valid) {
+  if (!device_known(device)) {
     hipDeviceProp_t p;
     TCPXU_HIP(hipGetDeviceProperties(&p, device));
     g_props[device].compute_units = p.multiProcessorCount;
     snprintf(g_props[device].name, sizeof g_props[device].name, "%s (%s)", p.name, p.gcnArchName);
-    g_props[device].valid = true;
+    g_props[device].valid.store(true, std::memory_order_release);
   }
   return TCPXU_SUCCESS;
 }
@@ -354,7 +358,7 @@ int tcpxuUnpackSlotNoAlloc(int device, const void* bounce_base, void* dst_base, 
   if (!done_flag_dev) return launch_batch(bounce_base, dst_base, static_cast<const tcpxuLoadMeta*>(descs_dev), n_descs, s);
   if (n_descs != 0 && n_descs <= kSmallSlot) {
     void* args[] = {&bounce_base, &dst_base, &descs_dev, &n_descs, &done_flag_dev, &done_value};
-    TCPXU_HIP(hipLaunchKernel(reinterpret_cast<const void*>(unpack_small_slot_kernel), dim3(1), dim3(n_descs * kWaveLanes), args, 0, s));
+    TCPXU_HIP(hipLaunchKernel(reinterpret_cast<const void*>(unpack_small_slot_kernel), dim3(1), dim3(std::min(n_descs, kSmallSlotWaves) * kWaveLanes), args, 0, s));
     return TCPXU_SUCCESS;
   }
   TCPXU_TRY(launch_batch(bounce_base, dst_base, static_cast<const tcpxuLoadMeta*>(descs_dev), n_descs, s));

@@ -51,6 +51,13 @@ def test_list_lengths(pkg, hip, oracle, n, misalign):
     mapped.free()
 
 
+@pytest.mark.parametrize("n", [15, 18, 23, 24, 25])
+@pytest.mark.parametrize("misalign", [0, 5])
+def test_list_lengths_around_one_workgroup(pkg, hip, oracle, n, misalign):
+    """A slot whose workgroup has a wavefront for every descriptor, two descriptors for some, and two launches."""
+    test_list_lengths(pkg, hip, oracle, n, misalign)
+
+
 def test_calls_on_two_streams_at_once(pkg, hip, oracle):
     """Calls share nothing: slots on two streams complete in whatever order they run."""
     import torch
