@@ -101,6 +101,20 @@ ssize_t DevmemSocket::recvmsg(struct msghdr* msg, size_t max_bytes) {
   uint64_t refs = 0;
   tcpxSynthFrag* f = rx.data() + head;
   tcpxSynthFrag* const end = rx.data() + rx.size();
+  const size_t n_pages = ledger->n_pages;
+  if (limit == 0) {
+    // Fragments that fit whole, without what only the last one needs to be asked.  (This loop, the one over messages in
+    // process_recv_cmsg and the first case of dontneed: a fragment of a bulk message 6.4 -> 4.6 ns of host time.)
+    for (const tcpxSynthFrag* const stop = f + std::min(end - f, out_end - out); f != stop && f->frag_size <= max_bytes - bytes; ++f) {
+      *out++ = WireCmsg{CMSG_LEN(sizeof(DevmemVec)), SOL_SOCKET, kScmDevmemOffset, {f->frag_offset, f->frag_size, f->frag_token}, 0};
+      bytes += f->frag_size;
+      if (f->frag_token < n_pages) {
+        ledger->give(f->frag_token);
+        ++refs;
+      }
+      if (end - f > static_cast<ptrdiff_t>(kPrefetchFrags)) ledger->prefetch(f[kPrefetchFrags].frag_token);
+    }
+  }
   for (; f != end; ++f) {
     if (f->frag_size != 0) {
       if (bytes >= max_bytes || payload_left == 0) break;
@@ -136,6 +150,10 @@ int DevmemSocket::dontneed(const PageToken* tokens, size_t n) {
   int rc = 0;
   for (size_t i = 0; i < n && rc == 0; ++i) {
     if (i + kPrefetchFrags < n) ledger->prefetch(tokens[i + kPrefetchFrags].token_start);
+    if (tokens[i].token_count == 1 && tokens[i].token_start < ledger->n_pages && ledger->take_back(tokens[i].token_start)) {
+      ++given_back;
+      continue;
+    }
     for (uint32_t k = 0; k < tokens[i].token_count; ++k) {
       const uint32_t page = tokens[i].token_start + k;
       if (page >= ledger->n_pages || !ledger->take_back(page)) {
@@ -176,7 +194,29 @@ ssize_t process_recv_cmsg(struct msghdr* msg, DataPipe* p, int offset, uint64_t 
   uint32_t next_token = 0;  // the page that would continue the last run
   if (n_toks > 0) next_token = toks[n_toks - 1].token_start + toks[n_toks - 1].token_count;
   const uint64_t dst_base = static_cast<uint64_t>(offset) + dst_base_offset;
+  const char* const control_end = static_cast<const char*>(msg->msg_control) + msg->msg_controllen;
   for (struct cmsghdr* cm = CMSG_FIRSTHDR(msg); cm; cm = next_cmsg(msg, cm)) {
+    // A run of devmem fragments as the kernel writes them, as many as there is room for: one comparison of the header each.
+    const WireCmsg* w = reinterpret_cast<const WireCmsg*>(cm);
+    const size_t room = std::min<size_t>({static_cast<size_t>(control_end - reinterpret_cast<const char*>(cm)) / sizeof(WireCmsg),
+                                          static_cast<size_t>(cnt_end - cnt), static_cast<size_t>(kSlotPages) - n_toks});
+    const WireCmsg* const w_end = w + room;
+    for (; w != w_end && w->len == CMSG_LEN(sizeof(DevmemVec)) && w->level == SOL_SOCKET && w->type == kScmDevmemOffset; ++w) {
+      const DevmemVec v = w->v;
+      if (n_toks > 0 && next_token == v.frag_token) toks[n_toks - 1].token_count++;
+      else toks[n_toks++] = PageToken{v.frag_token, 1};
+      next_token = v.frag_token + 1u;
+      union loadMeta& d = list[cnt++];
+      d.src_off = v.frag_offset;
+      d.len = v.frag_size;
+      d.dst_off = static_cast<uint64_t>(dst_offset) + dst_base;
+      dst_offset += v.frag_size;
+    }
+    if (const ptrdiff_t taken = w - reinterpret_cast<const WireCmsg*>(cm); taken != 0) {
+      num_cm += static_cast<int>(taken);
+      cm = next_cmsg(msg, reinterpret_cast<struct cmsghdr*>(const_cast<WireCmsg*>(w - 1)));
+      if (!cm) break;
+    }
     if (cm->cmsg_level != SOL_SOCKET || (cm->cmsg_type != kScmDevmemOffset && cm->cmsg_type != kScmDevmemHeader)) {
       INFO(NCCL_NET, "cmsg: unknown %u.%u", cm->cmsg_level, cm->cmsg_type);
       continue;
