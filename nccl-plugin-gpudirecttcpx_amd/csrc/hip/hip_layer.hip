@@ -38,19 +38,20 @@ namespace {
 // out new ones as they finish.  (Against workgroups of twelve wavefronts that staged their batch's descriptors in LDS,
 // where a list of up to 8192 kept four of the twelve busy: 16 fragments 2.9 -> 2.4 us a launch (what the host needs for
 // one), 4 MiB of wire fragments 5.1 -> 4.3 us, 8 MiB 6.6 -> 5.0, 16 MiB 10.0 -> 7.0, 64 MiB 23.6 -> 22.4; 256 MiB of
-// 1.8 KiB fragments 126-140 -> 99 us = 5.4 TB/s r+w, which wants all 32 wavefronts: with 16 resident it takes 136 us.
-// Whole pages by the half GiB move 2 % faster with 16 resident, 190 against 194 us; the list does not say which they
-// are.  Half a fragment per wavefront, or two wavefronts to a workgroup, measured no better for short lists.)
+// 1.8 KiB fragments 126-140 -> 99 us; since then, with the round of unpack_device.h, descriptors by scalar loads and XCDs in
+// turn: 4 MiB 3.8, 64 MiB 24.2, 256 MiB of 1.8 KiB fragments 90.8 = 5.9 TB/s r+w.  Those want all 32 wavefronts -- with 24 / 16
+// resident 98.7 / 116.5 us where 32 took 95.5 -- while long fragments want fewer, 512 MiB of wire fragments 176.2 / 172.9 where
+// 32 took 178.3, and the list does not say which they are.  Two descriptors per wavefront with 16 resident: 180.4 and 102.
+// Half a fragment per wavefront, or two wavefronts to a workgroup, measured no better for short lists.)
 constexpr uint32_t kBatchWaves = 4;
 constexpr uint32_t kBatchThreads = kBatchWaves * kWaveLanes;
+constexpr uint32_t kContiguousDescs = 4096;  // see xcd_near_index
 __global__ __launch_bounds__(kBatchThreads) __attribute__((amdgpu_waves_per_eu(8))) void unpack_batch_kernel(
     const uint8_t* __restrict__ bounce, uint8_t* __restrict__ dst, const tcpxuLoadMeta* __restrict__ descs,
     uint64_t n_descs, uint64_t first_group, uint32_t n_groups) {
   const uint32_t lane = threadIdx.x & (kWaveLanes - 1);
   const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWaveLanes)));
-  // Neighbouring groups go to the same XCD: they share a destination line and, in mapped memory, the line that their
-  // descriptors come in.
-  const uint64_t group = xcd_contiguous_index(blockIdx.x, n_groups);
+  const uint32_t group = xcd_near_index(blockIdx.x, n_groups, kContiguousDescs / kBatchWaves);
   if (group >= n_groups) return;
   const uint64_t i = (first_group + group) * kBatchWaves + wave;
   if (i < n_descs) copy_descriptor(bounce, dst, descs, n_descs, i, lane);

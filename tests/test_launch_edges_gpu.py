@@ -58,6 +58,25 @@ def test_list_lengths_around_one_workgroup(pkg, hip, oracle, n, misalign):
     test_list_lengths(pkg, hip, oracle, n, misalign)
 
 
+@pytest.mark.parametrize("n", [2049, 4095, 4096, 4097, 4604, 4607, 4608, 4609, 4613, 6144, 6145, 7001])
+def test_lists_around_whole_turns_of_the_xcds(pkg, hip, oracle, n):
+    """Beyond 4096 descriptors the XCDs take runs of 24 groups of four descriptors in turn, 768 descriptors a turn: lists of
+    whole turns, of one group or descriptor more or less, and of some left over."""
+    rng = np.random.default_rng(n)
+    lens = rng.choice([0, 20, 100, 300, 1500], size=n)
+    descs = np.zeros(n, dtype=np.dtype([("src_off", "<u4"), ("len", "<u4"), ("dst_off", "<u8")]))
+    descs["len"], descs["dst_off"] = lens, np.cumsum(lens) - lens
+    descs["src_off"] = rng.integers(0, (1 << 20) - 1500, n)
+    total = int(lens.sum())
+    pool = rng.integers(0, 256, 1 << 20, dtype=np.uint8)
+    expect = oracle_expected(oracle, pool, descs, total, 9)
+    buf = GpuBuffers(pool, descs, total, 9)
+    print("list of %d descriptors" % n, flush=True)
+    pkg.check(hip.tcpxuUnpackBatch(0, buf.pool.data_ptr(), buf.dst_base, buf.descs.data_ptr(), n, None), "tcpxuUnpackBatch")
+    pkg.check(hip.tcpxuDeviceSynchronize(0), "sync")
+    assert first_difference(buf.result(), expect) is None
+
+
 def test_calls_on_two_streams_at_once(pkg, hip, oracle):
     """Calls share nothing: slots on two streams complete in whatever order they run."""
     import torch
