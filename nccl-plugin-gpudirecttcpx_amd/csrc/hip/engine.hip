@@ -124,6 +124,24 @@ __host__ __device__ __forceinline__ uint32_t full_ticket_size(uint32_t bytes, ui
 // 32.5).  Above the range the last round is a small part of the whole (24 requests of 4 MiB, 48 a workgroup: 46.5 by backlog,
 // 47.3 in tickets of 18); below it the sizes by backlog, which begin at 8, reach all the workgroups sooner.
 constexpr uint32_t kBurstTicket = 18;
+// Ticket size for submissions of fragments of a third to half a page (the step of 48) where a call hands over kManyInFlight or
+// more, or while the backlog is shallow: 32.  What is being written at a time is then a narrower stretch of the destination,
+// which the memory takes faster, and the last round is shorter.  Only where the leader writes tickets of 32 in the same way as
+// tickets of 48 -- from the entry's lanes, or one entry after the other -- since it is the leader that a stream waits for where
+// that changes.  (48 / 32, us a call of ragged fragments, with other buffers from pass to pass: 256 MiB in requests of 3 MiB
+// 110.4 / 107.9, 64 MiB 36.6 / 36.1, 24 MiB 21.9 / 20.4, 64 MiB in requests of 1 MiB 38.7 / 38.3; a stream of 1 MiB requests, 64
+// in flight, 4.86 / 5.22 TB/s r+w.  Where the way changes, requests of 1400 fragments of 1.5 KiB, 64 in flight: 5.36 / 4.54; and
+// requests of 3 MiB, one entry after the other either way, 64 in flight: 5.34 in tickets of 48, 5.20 if a backlog that looks
+// shallow for a moment makes some of them 32.)
+constexpr uint32_t kShortBurstTicket = 32, kShortTicket = 48;
+__host__ __device__ __forceinline__ uint32_t short_ticket_size(uint32_t full, uint32_t n, bool burst, bool shallow) {
+  const bool in_lanes = n <= kLaneTickets * kShortBurstTicket, never_in_lanes = n > kLaneTickets * kShortTicket;
+  return full == kShortTicket && ((burst && (in_lanes || never_in_lanes)) || (shallow && in_lanes)) ? kShortBurstTicket : full;
+}
+inline bool burst_of_short_fragments(uint32_t submissions, uint32_t n, uint32_t bytes, uint32_t workers) {
+  return submissions >= kManyInFlight && n > kSmallSubmission && full_ticket_size(bytes, n) == kShortTicket &&
+         static_cast<uint64_t>(submissions) * n >= 18ull * workers;
+}
 inline bool burst_of_pages(uint32_t submissions, uint32_t n, uint32_t bytes, uint32_t workers) {
   const uint64_t all = static_cast<uint64_t>(submissions) * n;
   return submissions >= kManyInFlight && n > kSmallSubmission && full_ticket_size(bytes, n) == kFullTicket &&
@@ -131,7 +149,10 @@ inline bool burst_of_pages(uint32_t submissions, uint32_t n, uint32_t bytes, uin
 }
 __host__ __device__ __forceinline__ uint32_t ticket_size_for_submission(uint32_t in_flight, uint32_t n,
                                                                         uint32_t bytes, uint32_t workers, bool burst) {
-  if (burst) return kBurstTicket;
+  if (burst) {
+    const uint32_t full = full_ticket_size(bytes, n);
+    return full == kFullTicket ? kBurstTicket : short_ticket_size(full, n, true, false);
+  }
   if (n <= kCarriedDescs) return kCarriedDescs;
   if (in_flight >= kManyInFlight && n <= kSmallSubmission) return kSmallSubmission;
   const uint64_t all = static_cast<uint64_t>(in_flight) * n;
@@ -139,7 +160,7 @@ __host__ __device__ __forceinline__ uint32_t ticket_size_for_submission(uint32_t
   const uint32_t size = ticket_size_for(backlog, workers);
   if (size < kFullTicket) return size;
   const uint32_t full = full_ticket_size(bytes, n);
-  if (full > kFullTicket) return full;
+  if (full > kFullTicket) return short_ticket_size(full, n, false, backlog < kDeepBacklog * workers);
   // Whole pages and a backlog that is there but not deep (one comm's sixteen slots of 4 MiB are 34 descriptors per
   // workgroup: every workgroup holds a ticket and has the next one staged, and hardly any wait unclaimed): tickets
   // of 14 make a seventh more of them, and the workgroups run dry less often -- one comm 71.1 -> 72.2 % of the
@@ -199,7 +220,7 @@ constexpr uint32_t kCarriedEntry = 1u << 31;   // in a submission's payload word
 // faster than the host writes it, so the first submissions of a burst would be cut up as if each came alone (eleven
 // requests of 2000 short fragments in one call: 28.4 -> 26.2 us).  Whole pages are not sized so: there
 // small tickets reach all the workgroups sooner (32 requests of 2 MiB by what has been seen 35.1 us, and 36.5 with every one sized for all).
-// And of whole pages: whether it is of a burst that burst_of_pages names.  The host works that out, since every
+// And whether it is of a burst that burst_of_pages or burst_of_short_fragments names.  The host works that out, since every
 // instruction that the leader spends on an entry is waited for by all that follow it.
 constexpr uint32_t kBurstEntry = 1u << 30;
 constexpr uint32_t kFollowShift = 21, kMostFollow = 0x1FF;
@@ -1796,7 +1817,10 @@ int tcpxuEngineSubmitMany(tcpxuEngine* e, const tcpxuSubmission* subs, uint32_t 
     }
     const bool pages = full_ticket_size(sub.payload_bytes, sub.n_descs) == kFullTicket;
     p[10] = sub.n_descs | (pages ? 0u : std::min(take - 1 - k, kMostFollow) << kFollowShift) |
-            (burst_of_pages(take, sub.n_descs, sub.payload_bytes, e->workgroups - 1) ? kBurstEntry : 0u);
+            (burst_of_pages(take, sub.n_descs, sub.payload_bytes, e->workgroups - 1) ||
+                     burst_of_short_fragments(take, sub.n_descs, sub.payload_bytes, e->workgroups - 1)
+                 ? kBurstEntry
+                 : 0u);
     p[11] = sub.payload_bytes;
     if (k < kCarriedEntries && sub.n_descs != 0 && sub.n_descs <= kCarriedDescs && stamp != 0 && e->tail - head < kCarryBehind &&
         carry_descriptors(e, sub, stamp))

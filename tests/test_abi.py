@@ -99,6 +99,21 @@ def test_ticket_plan_arithmetic(pkg):
     assert plan(1, 0, 1, 8)[0] == pkg.INVALID_ARGUMENT and plan(769, 65, 1, 8)[0] == pkg.INVALID_ARGUMENT
 
 
+@pytest.mark.parametrize("n,shallow,deep", [(1, 16, 16), (600, 32, 48), (1024, 32, 48), (1025, 48, 48), (1537, 48, 48)])
+def test_ticket_plan_of_short_fragments_by_backlog(pkg, n, shallow, deep):
+    """Fragments of 1800 bytes: tickets of 32 below a hundred descriptors per worker if the leader writes them as it does
+    tickets of 48; 512 workers."""
+    per, nt, lim = ctypes.c_uint32(), ctypes.c_uint32(), ctypes.c_uint32()
+
+    def size(in_flight):
+        rc = pkg.hip_layer().tcpxuEngineTicketPlan(513, 0, in_flight, n, 1800 * n, ctypes.byref(per), ctypes.byref(nt), ctypes.byref(lim))
+        assert rc == 0
+        return per.value
+
+    last_shallow = (100 * 512 - 1) // n
+    assert size(last_shallow) == shallow and size(last_shallow + 1) == deep
+
+
 def test_struct_sizes_match_the_headers(pkg):
     assert ctypes.sizeof(pkg.LoadMeta) == 16 and ctypes.sizeof(pkg.SynthFrag) == 16
     assert ctypes.sizeof(pkg.SynthRequest) == 32 and ctypes.sizeof(pkg.SynthInfo) == 48

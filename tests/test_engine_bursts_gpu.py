@@ -49,3 +49,9 @@ def test_burst(pkg, hip, oracle, subs_n, hint):
     e.destroy()
     m.free()
     assert first_difference(got, expect) is None, repr(first_difference(got, expect))
+
+
+@pytest.mark.parametrize("subs_n", [(8, 71), (8, 72), (8, 1024), (8, 1025), (8, 1536), (8, 1537), (9, 2048)])
+def test_burst_of_fragments_of_half_a_page(pkg, hip, oracle, subs_n):
+    """The sizes where such submissions change between tickets of 12, 32 and 48, and the leader's way of writing them."""
+    test_burst(pkg, hip, oracle, subs_n, 1800)
