@@ -272,10 +272,21 @@ struct alignas(256) StopWord {
   uint32_t value;
 };
 
+// The three words that every workgroup counts in, and two of which every look of the leader reads, lie 4 KiB apart: an atomic
+// takes its memory channel 12 ns, and in one line they waited for each other and the looks for them.  (64 / 4096 bytes apart, us
+// a call with other buffers from pass to pass: a request of 64 KiB 8.53 / 8.33, 256 of them 21.9 / 21.3, 64 MiB of ragged
+// fragments 36.6 / 35.9, of wire fragments 32.7 / 32.3; a stream of 64 KiB requests, 256 in flight, 2.47 / 2.56 TB/s r+w; 256
+// bytes apart measures the same but for that stream, 2.49.)
+constexpr size_t kCountersApart = 4096;
+struct alignas(256) Counter {
+  uint64_t value;
+  uint8_t apart[kCountersApart - sizeof(uint64_t)];
+};
+static_assert(sizeof(Counter) == kCountersApart, "no further apart than that");
 struct DevState {  // device memory
-  alignas(64) uint64_t ticket_head;     // next ticket number to claim
-  alignas(64) uint64_t tickets_done;    // tickets whose payload is written
-  alignas(64) uint64_t jobs_completed;  // submissions completed since creation
+  Counter ticket_head;     // next ticket number to claim
+  Counter tickets_done;    // tickets whose payload is written
+  Counter jobs_completed;  // submissions completed since creation
   alignas(64) uint64_t sub_head;        // leader-private: next submission index
   uint64_t tickets_out;                 // leader-private: tickets written so far
   uint64_t leader_polls, leader_entries, leader_deep_polls;  // leader-private: running totals (see HostCtl)
@@ -521,7 +532,7 @@ __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevS
     feeding = kGroups;
 #pragma unroll
     for (uint32_t g = 0; g < kGroups; ++g) fetch_group_untracked(sc[g], ax[g], s + g * kPollEntries);
-    asm volatile("global_load_dword %0, %1, off sc0 sc1" : "=v"(tickets_done) : "v"(reinterpret_cast<const uint32_t*>(&st->tickets_done)) : "memory");
+    asm volatile("global_load_dword %0, %1, off sc0 sc1" : "=v"(tickets_done) : "v"(reinterpret_cast<const uint32_t*>(&st->tickets_done.value)) : "memory");
     asm volatile("s_waitcnt vmcnt(0)" : "+v"(tickets_done) : : "memory");
 #pragma unroll
     for (uint32_t g = 0; g < kGroups; ++g) asm volatile("" : "+v"(sc[g]), "+v"(ax[g]) : : "memory");
@@ -620,7 +631,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
   };
   uint64_t s = same_in_all_lanes(sys_load(&st->sub_head));
   uint64_t tickets_out = same_in_all_lanes(sys_load(&st->tickets_out));
-  uint64_t mirrored = same_in_all_lanes(sys_load(&st->jobs_completed));  // completed submissions, as the host was last told
+  uint64_t mirrored = same_in_all_lanes(sys_load(&st->jobs_completed.value));  // completed submissions, as the host was last told
   // Read once: the grid's size comes from the dispatch packet, a scalar load with a wait behind it wherever it is asked.
   const uint32_t workers = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(gridDim.x - 1)));
   uint64_t idle = 0;
@@ -640,9 +651,9 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
   //   lanes 0-15  jobs_done of the job slots of entries s..s+15    lanes 16-31  job_target of the same slots
   //   lane 32     low word of tickets_done                         lane 33      low word of the host stop word
   //   lane 34     low word of jobs_completed                       other lanes repeat lane 33.
-  const uint32_t* const tickets_done_lo = reinterpret_cast<const uint32_t*>(&st->tickets_done);
+  const uint32_t* const tickets_done_lo = reinterpret_cast<const uint32_t*>(&st->tickets_done.value);
   const uint32_t* const host_stop_lo = reinterpret_cast<const uint32_t*>(&ctl->stop);
-  const uint32_t* const jobs_completed_lo = reinterpret_cast<const uint32_t*>(&st->jobs_completed);
+  const uint32_t* const jobs_completed_lo = reinterpret_cast<const uint32_t*>(&st->jobs_completed.value);
 
   for (;;) {
     // (Every 64 entries it takes count as one deep poll in this launch's figures.)
@@ -934,7 +945,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
         if (lane == 0) {
           sys_store_global(reinterpret_cast<uint64_t*>((static_cast<uint64_t>(flag_hi) << 32) | flag_lo),
                     (static_cast<uint64_t>(val_hi) << 32) | val_lo);
-          __hip_atomic_fetch_add(&st->jobs_completed, 1ull, __ATOMIC_RELAXED, SYS);
+          __hip_atomic_fetch_add(&st->jobs_completed.value, 1ull, __ATOMIC_RELAXED, SYS);
         }
         lanes_together();
       } else {
@@ -1255,17 +1266,17 @@ __device__ void retire_ticket(DevState* st, uint32_t* jobs_done, const LdsStage*
       if (stamps) sys_store(&stamps[kStampsPerJob * job + 3], clock_now());
       sys_store(reinterpret_cast<uint64_t*>(done_flag), done_value);
       __hip_atomic_fetch_add(&jobs_done[job], 1u, __ATOMIC_RELAXED, SYS);
-      __hip_atomic_fetch_add(&st->tickets_done, 1ull, __ATOMIC_RELAXED, SYS);
-      __hip_atomic_fetch_add(&st->jobs_completed, 1ull, __ATOMIC_RELAXED, SYS);
+      __hip_atomic_fetch_add(&st->tickets_done.value, 1ull, __ATOMIC_RELAXED, SYS);
+      __hip_atomic_fetch_add(&st->jobs_completed.value, 1ull, __ATOMIC_RELAXED, SYS);
       return;
     }
     const uint32_t count = __hip_atomic_fetch_add(&jobs_done[job], 1u, __ATOMIC_RELAXED, SYS) + 1u;
-    __hip_atomic_fetch_add(&st->tickets_done, 1ull, __ATOMIC_RELAXED, SYS);
+    __hip_atomic_fetch_add(&st->tickets_done.value, 1ull, __ATOMIC_RELAXED, SYS);
     if (count == target) {
       // Every other ticket's payload was in memory before it was counted, and so is this one's.
       if (stamps) sys_store(&stamps[kStampsPerJob * job + 3], clock_now());
       sys_store(reinterpret_cast<uint64_t*>(done_flag), done_value);
-      __hip_atomic_fetch_add(&st->jobs_completed, 1ull, __ATOMIC_RELAXED, SYS);
+      __hip_atomic_fetch_add(&st->jobs_completed.value, 1ull, __ATOMIC_RELAXED, SYS);
     }
   }
 }
@@ -1418,7 +1429,7 @@ __device__ void worker_loop(DevState* st, uint32_t* jobs_done, uint32_t flags, u
         break;
       }
       uint64_t t = 0;
-      if (lane == 0) t = __hip_atomic_fetch_add(&st->ticket_head, 1ull, __ATOMIC_RELAXED, SYS);
+      if (lane == 0) t = __hip_atomic_fetch_add(&st->ticket_head.value, 1ull, __ATOMIC_RELAXED, SYS);
       const uint64_t ticket = bcast64(t, 0);
       bool give_up = false, stop_before = false, first_look = true;
       uint32_t backoff = 1, looks = 0;
@@ -1486,8 +1497,8 @@ __global__ __launch_bounds__(kEngineThreads) __attribute__((amdgpu_waves_per_eu(
     if (before + 1 == gridDim.x) {
       // Last workgroup out: every ticket that was written has been counted.  Ticket numbers claimed beyond the
       // last written one are given back, so the next launch starts where this one ended.
-      sys_store(&st->ticket_head, sys_load(&st->tickets_out));
-      sys_store(&ctl->completed, sys_load(&st->jobs_completed));
+      sys_store(&st->ticket_head.value, sys_load(&st->tickets_out));
+      sys_store(&ctl->completed, sys_load(&st->jobs_completed.value));
       drain_memory_ops();
       sys_store(&ctl->exited, static_cast<uint64_t>(sys_load(&st->exit_reason)));
     }
@@ -1626,7 +1637,7 @@ int tcpxuEngineCreate(int device, const tcpxuEngineConfig* config, tcpxuEngine**
         rc = TCPXU_INVALID_ARGUMENT;
         break;
       }
-      uint64_t* const counts[] = {&e->st->ticket_head, &e->st->tickets_done, &e->st->jobs_completed, &e->st->sub_head,
+      uint64_t* const counts[] = {&e->st->ticket_head.value, &e->st->tickets_done.value, &e->st->jobs_completed.value, &e->st->sub_head,
                                   &e->st->tickets_out};  // device addresses: only computed here, never read
       for (uint64_t* c : counts) {
         if (hipMemcpy(c, &from, sizeof from, hipMemcpyHostToDevice) != hipSuccess) {
