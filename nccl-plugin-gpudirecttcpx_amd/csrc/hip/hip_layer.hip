@@ -29,7 +29,7 @@ void set_error(const char* fmt, ...) {
 
 namespace {
 
-// Launch-per-batch unpack: one wavefront per descriptor, four to a workgroup, as many workgroups as it takes.
+// Launch-per-batch unpack: one wavefront per descriptor, in workgroups of kWaves, as many workgroups as it takes.
 //
 // What bounds a short list is the chain launch -> descriptor -> payload -> store, each link a trip to memory; what
 // bounds a long one is the memory system, and for short fragments how many wavefronts keep loads in flight.  Hence no
@@ -43,17 +43,27 @@ namespace {
 // resident 98.7 / 116.5 us where 32 took 95.5 -- while long fragments want fewer, 512 MiB of wire fragments 176.2 / 172.9 where
 // 32 took 178.3, and the list does not say which they are.  Two descriptors per wavefront with 16 resident: 180.4 and 102.
 // Half a fragment per wavefront, or two wavefronts to a workgroup, measured no better for short lists.)
-constexpr uint32_t kBatchWaves = 4;
-constexpr uint32_t kBatchThreads = kBatchWaves * kWaveLanes;
+//
+// A wavefront is a workgroup of its own in lists of up to kShortList descriptors: nobody waits for three others to be placed
+// or to finish.  In longer ones four begin together, and what is written at a time is a little more compact.  (Workgroups of
+// one / two / four wavefronts, us a launch with other buffers from pass to pass: 4 MiB of wire fragments, list in the host's
+// memory, 3.53 / 3.60 / 3.79, 3 MiB of ragged ones 4.07 / 4.09 / 4.15; list in the GPU's memory, 8 MiB of wire fragments 3.42 /
+// 3.45 / 3.52, 16 MiB 6.26 / 6.29 / 6.38, 16 MiB of ragged ones, 9100 descriptors, 7.35 / 7.34 / 7.30, 256 MiB of them 92.9 / 92.4 /
+// 92.5, 512 MiB of wire fragments 170.4 / 170.8 / 171.1, of whole pages 191.3 / 191.6 / 191.4.  Of eight and sixteen, 4 MiB 3.70
+// and 4.45.)
+constexpr uint64_t kShortList = 8192;
+constexpr uint32_t kLongListWaves = 4;
 constexpr uint32_t kContiguousDescs = 4096;  // see xcd_near_index
-__global__ __launch_bounds__(kBatchThreads) __attribute__((amdgpu_waves_per_eu(8))) void unpack_batch_kernel(
+template <uint32_t kWaves>
+__global__ __launch_bounds__(kWaves* kWaveLanes) __attribute__((amdgpu_waves_per_eu(8))) void unpack_batch_kernel(
     const uint8_t* __restrict__ bounce, uint8_t* __restrict__ dst, const tcpxuLoadMeta* __restrict__ descs,
     uint64_t n_descs, uint64_t first_group, uint32_t n_groups) {
+  static_assert(kXcdRunDescs % kWaves == 0 && kContiguousDescs % kWaves == 0, "whole workgroups");
   const uint32_t lane = threadIdx.x & (kWaveLanes - 1);
   const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWaveLanes)));
-  const uint32_t group = xcd_near_index(blockIdx.x, n_groups, kContiguousDescs / kBatchWaves);
+  const uint32_t group = xcd_near_index(blockIdx.x, n_groups, kContiguousDescs / kWaves, kXcdRunDescs / kWaves);
   if (group >= n_groups) return;
-  const uint64_t i = (first_group + group) * kBatchWaves + wave;
+  const uint64_t i = (first_group + group) * kWaves + wave;
   if (i < n_descs) copy_descriptor(bounce, dst, descs, n_descs, i, lane);
 }
 
@@ -321,13 +331,16 @@ static int launch_batch(const void* bounce_base, void* dst_base, const tcpxuLoad
     set_error("descriptor array must be 16-byte aligned");
     return TCPXU_INVALID_ARGUMENT;
   }
-  uint64_t groups = (n_descs + kBatchWaves - 1) / kBatchWaves;
+  const bool short_list = n_descs <= kShortList;
+  const uint32_t waves = short_list ? 1 : kLongListWaves;
+  const void* kernel = short_list ? reinterpret_cast<const void*>(unpack_batch_kernel<1>) : reinterpret_cast<const void*>(unpack_batch_kernel<kLongListWaves>);
+  uint64_t groups = (n_descs + waves - 1) / waves;
   // (A launch holds fewer than 2^32 threads: a list of more than 32 Mi descriptors takes several.)
   constexpr uint64_t kGroupsPerLaunch = 1ull << 23;
   for (uint64_t first = 0; first < groups; first += kGroupsPerLaunch) {
     uint32_t here = static_cast<uint32_t>(std::min(groups - first, kGroupsPerLaunch));
     void* args[] = {&bounce_base, &dst_base, &descs, &n_descs, &first, &here};
-    TCPXU_HIP(hipLaunchKernel(reinterpret_cast<const void*>(unpack_batch_kernel), dim3((here + 7) / 8 * 8), dim3(kBatchThreads), args, 0, stream));
+    TCPXU_HIP(hipLaunchKernel(kernel, dim3((here + 7) / 8 * 8), dim3(waves * kWaveLanes), args, 0, stream));
   }
   return TCPXU_SUCCESS;
 }

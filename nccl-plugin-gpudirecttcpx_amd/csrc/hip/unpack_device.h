@@ -358,7 +358,7 @@ __device__ __forceinline__ void copy_descriptor(const uint8_t* bounce, uint8_t* 
 // lines that their descriptors come in in common.
 //
 // In a short list every XCD takes one contiguous eighth: its descriptors arrive a line at a time, over PCIe perhaps.  In a
-// longer one it takes runs of kXcdRun in turn, so that what is being written at a time is one stretch of the destination
+// longer one it takes runs of kXcdRunDescs in turn, so that what is being written at a time is one stretch of the destination
 // and not eight of them, each an eighth of the message away from the next.  (Groups of four descriptors, contiguous eighths
 // / runs of 1 / 8 / 24 / 32 / 64, us: 512 MiB of wire fragments 177.3 / 172.8 / 172.0 / 172.3 / 174.5 / 174.1, of whole pages
 // 194.3 / 191.0 / 191.1 / 190.7 / 189.7 / 189.5, 256 MiB of whole pages 98.0 / 95.7 / 96.6 / 95.7 / 95.4 / 95.9, of ragged
@@ -366,15 +366,15 @@ __device__ __forceinline__ void copy_descriptor(const uint8_t* bounce, uint8_t* 
 // worse for whole pages, 203.8 and 198.6.  A slot of 4 MiB whose list is in the host's memory 3.95 / 4.53 / 4.02 / - / 4.04 / -;
 // 8 MiB, 2155 descriptors, 4.75 and 4.79 in runs of 24, 16 MiB 8.67 and 8.65.)
 constexpr uint32_t kXcds = 8;
-constexpr uint32_t kXcdRun = 24;
-__device__ __forceinline__ uint32_t xcd_near_index(uint32_t wg, uint32_t items, uint32_t contiguous_up_to) {
+constexpr uint32_t kXcdRunDescs = 96;
+__device__ __forceinline__ uint32_t xcd_near_index(uint32_t wg, uint32_t items, uint32_t contiguous_up_to, uint32_t run) {
   if (items <= contiguous_up_to) {
     const uint32_t per_xcd = (items + kXcds - 1) / kXcds;
     return (wg % kXcds) * per_xcd + wg / kXcds;  // may be >= items: caller skips
   }
-  const uint32_t turn = wg / (kXcds * kXcdRun) * (kXcds * kXcdRun);  // the first item of this turn, and its first workgroup
-  if (turn + kXcds * kXcdRun > items) return wg;                     // (what is left beyond whole turns; caller skips as above)
-  return turn + (wg % kXcds) * kXcdRun + (wg - turn) / kXcds;
+  const uint32_t turn = wg / (kXcds * run) * (kXcds * run);  // the first item of this turn, and its first workgroup
+  if (turn + kXcds * run > items) return wg;                 // (what is left beyond whole turns; caller skips as above)
+  return turn + (wg % kXcds) * run + (wg - turn) / kXcds;
 }
 
 }  // namespace tcpxu

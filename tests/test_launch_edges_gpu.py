@@ -77,6 +77,12 @@ def test_lists_around_whole_turns_of_the_xcds(pkg, hip, oracle, n):
     assert first_difference(buf.result(), expect) is None
 
 
+@pytest.mark.parametrize("n", [7679, 7680, 7681, 8191, 8192, 8193, 8196, 8197, 8447, 8448, 8449, 9217])
+def test_lists_around_workgroups_of_one_wavefront_and_of_four(pkg, hip, oracle, n):
+    """Up to 8192 descriptors a workgroup is one wavefront, beyond that four; turns of 768 descriptors either way."""
+    test_lists_around_whole_turns_of_the_xcds(pkg, hip, oracle, n)
+
+
 def test_calls_on_two_streams_at_once(pkg, hip, oracle):
     """Calls share nothing: slots on two streams complete in whatever order they run."""
     import torch
