@@ -18,7 +18,6 @@ namespace tcpxu {
 
 constexpr int kWaveLanes = 64;
 constexpr int kWgThreads = 256;
-constexpr int kWavesPerWg = kWgThreads / kWaveLanes;
 // Vectors a lane keeps in flight per round: 4 x 16 B x 64 lanes = one 4 KiB page per wavefront per round.
 constexpr int kVecPerLane = 4;
 constexpr uint32_t kVecPerRound = kVecPerLane * kWaveLanes;
@@ -48,18 +47,12 @@ __device__ __forceinline__ void store_vec_sys(uint8_t* p, u32x4 v) {
 // The bulk of the payload is stored with the non-temporal hint on top of the system scope (sc0 sc1 nt): the
 // destination is written once and not read again by this kernel, and telling the caches so keeps it from
 // displacing other data (at an 8 MiB chunk of 4 KiB fragments, all from HBM: 2.80 against 2.58 TB/s of payload).
-// The hint on the loads as well measured no faster.  No builtin combines the hint with a scope, so the store is
-// written as an instruction; the s_nop covers the wait state the hardware wants between a store of more than
+// The hint on the loads as well measured no faster.  A round's stores go through windows (below), which take scope and hint
+// as a number; the one here, for kernels that copy a single stretch, is written as an instruction, since no builtin
+// combines the two on a plain address.  The s_nop covers the wait state the hardware wants between a store of more than
 // 8 bytes and a write to its data registers, which the compiler cannot insert for an instruction it does not see.
-#ifndef TCPXU_STORE_NT
-#define TCPXU_STORE_NT 1
-#endif
 __device__ __forceinline__ void store_vec_stream(uint8_t* p, u32x4 v) {
-#if TCPXU_STORE_NT
   asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt\n\ts_nop 1" : : "v"((gvec_ptr)p), "v"(v) : "memory");
-#else
-  store_vec_sys(p, v);
-#endif
 }
 __device__ __forceinline__ uint32_t load_byte_sys(const uint8_t* p) {
   return __hip_atomic_load((const TCPXU_GLOBAL uint8_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
