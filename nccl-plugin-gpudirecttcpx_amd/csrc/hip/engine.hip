@@ -1127,6 +1127,9 @@ struct alignas(16) RoundRec {
 };
 static_assert(sizeof(RoundRec) == 48, "three 16-byte LDS reads");
 
+// In a staged ticket's word 10 (see copy_ticket), where the descriptors of a ticket of more than kFullTicket never travel.
+constexpr uint32_t kRoundsAlone = kCarriedTicket;
+static_assert(kCarriedDescs <= kFullTicket, "the bit has another meaning in tickets that bring their descriptors");
 struct Stage {
   uint32_t payload[kPayloadWords];
   uint32_t go;
@@ -1205,7 +1208,10 @@ __device__ uint32_t try_fetch_ticket(DevState* st, const uint32_t* stop_word, ui
   // the line before taken from what the neighbour found about the line after, one round of lane exchanges less but more
   // branches, 200 requests of 256 KiB in one call took 47.4 us instead of 46.9, 32 of 2 MiB 32.8 instead of 32.4.
   const uint32_t off_line = (static_cast<uint32_t>(fdst) | len) & (kLineBytes - 1);
-  if (__any(lane < n && (off_line != 0 || len == 0))) {
+  const bool off_lines = __any(lane < n && (off_line != 0 || len == 0));
+  if (lane == 0 && !off_lines && n > kBurstTicket && n <= kShortBurstTicket && (ticket_bits & kOnlyTicket) == 0)
+    stage->payload[10] = ticket_bits | kRoundsAlone;
+  if (off_lines) {
     // The neighbours' descriptors decide which destination lines are shared with them.  A fragment's neighbours are
     // the nearest descriptors of the ticket that are not empty: an empty descriptor between two fragments (a
     // zero-length control message's, a fragment cut to nothing) leaves them back to back in the destination.
@@ -1338,21 +1344,29 @@ __device__ __forceinline__ void copy_ticket(const LdsStage* stage, uint32_t wave
   // and both are waited for together -- in a ticket of more than kFullTicket descriptors (the leader makes those of short
   // fragments, whose rounds leave half of a wavefront's registers empty) and in a request's only ticket, which is waited
   // for.  The other tickets are of whole pages in a stream, where sixteen wavefronts a compute unit with a page each are
-  // all that the memory system takes.  (All one at a time / all in pairs: 2048 requests of 64 KiB through the plugin, 16
-  // posted at a time, 1045 / 1000 us, 256 MiB of ragged fragments 109.3 / 108.4, of whole pages 103.9 / 105.7.)
+  // all that the memory system takes; so are, in tickets of kShortBurstTicket, those of fragments that lie on destination
+  // lines, which have next to nothing between their loads and their stores.  (All one at a time / all in pairs: 2048 requests
+  // of 64 KiB through the plugin, 16 posted at a time, 1045 / 1000 us, 256 MiB of ragged fragments 114.2 / 107.6, of whole pages
+  // 103.9 / 105.7; streams of fragments on lines, 2 KiB in tickets of 32, 5.67 / 5.38 TB/s r+w, 1 KiB in tickets of 64, 5.29 / 5.35;
+  // 64 MiB of pages in tickets of 18 31.2 / 30.9 us.)
   const bool pairs = n > kFullTicket || (uniform(stage->payload[10]) & kOnlyTicket) != 0;
+  const bool alone = n > kFullTicket && (uniform(stage->payload[10]) & kRoundsAlone) != 0;
   CopyRound r, next;
   CopyRegs x, y;
   bool more = produce(r, r);
   while (more) {
     round_load(r, x, lane);
     if (pairs) {
-      const bool second = produce(next, r);
+      const bool second = !alone && produce(next, r);
       if (second) round_load(next, y, lane);
       rounds_wait(x, y);
       round_store_loaded(r, x, lane);
-      if (second) round_store_loaded(next, y, lane);
-      more = second && produce(r, next);
+      if (second) {
+        round_store_loaded(next, y, lane);
+        r = next;
+      }
+      more = (second || alone) && produce(next, r);
+      r = next;
     } else {
       round_store(r, x, lane);
       more = produce(next, r);

@@ -98,3 +98,30 @@ def test_rounds_in_pairs(pkg, hip, oracle, per_ticket):
         assert first_difference(buf.result(), expect) is None
         mapped.free()
     engine.destroy()
+
+
+@pytest.mark.parametrize("per_ticket", [18, 19, 24, 32, 33])
+def test_rounds_of_fragments_on_lines(pkg, hip, oracle, per_ticket):
+    """Fragments of whole destination lines, some of several rounds: in tickets of 19 to 32 one round at a time, in smaller and
+    larger ones and in a request's only ticket in pairs; with one fragment off the lines, in pairs as well."""
+    engine = Engine(pkg, hip, descs_per_ticket=per_ticket)
+    engine.start()
+    for n in (per_ticket - 1, per_ticket, per_ticket + 1, 3 * per_ticket + 5):
+        for odd in (0, 1):
+            rng = np.random.default_rng(100 * per_ticket + 2 * n + odd)
+            lens = rng.choice([128, 1024, 2048, 4096, 4096 + 128, 9 * 1024], size=n)
+            lens[-1] += 4 * odd
+            descs = np.zeros(n, dtype=np.dtype([("src_off", "<u4"), ("len", "<u4"), ("dst_off", "<u8")]))
+            descs["len"], descs["dst_off"] = lens, np.cumsum(lens) - lens
+            descs["src_off"] = rng.integers(0, (1 << 20) - 9500, n)
+            pool = rng.integers(0, 256, 1 << 20, dtype=np.uint8)
+            total = int(lens.sum())
+            expect = oracle_expected(oracle, pool, descs, total, 0)
+            buf, mapped = GpuBuffers(pool, descs, total, 0), Mapped(pkg, hip, descs, 1)
+            assert buf.dst_base % 128 == 0
+            print("tickets of %d, %d descriptors, %d bytes" % (per_ticket, n, total), flush=True)
+            engine.submit(buf.pool.data_ptr(), buf.dst_base, mapped.desc_dev(0), n, mapped.flag_dev(0), 9)
+            mapped.wait(0, 9)
+            assert first_difference(buf.result(), expect) is None
+            mapped.free()
+    engine.destroy()
