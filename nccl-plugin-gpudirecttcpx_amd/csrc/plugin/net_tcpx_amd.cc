@@ -621,6 +621,25 @@ ncclResult_t ensure_engine(DeviceState* ds) {
 }
 
 
+// The descriptors the engine reads: the mapped slot, or a second copy in the GPU's own memory, written through the BAR
+// ahead of the submission, which saves the GPU a PCIe round trip before it can start copying.  For a small request, of
+// which a comm has at most 16 in flight; and for a longer one if the comm has no other, posted or at the GPU, so that this
+// one's way is all that anybody waits for.  (The one place for those is free again: everything that was submitted before
+// has been reported done.)  With others the host's time for the copy costs more than it gives.  (Us, mapped slot / copy: a
+// lone request of 18 descriptors 8.7 / 8.0, of 32 whole pages 8.6 / 7.7, of 128 8.9 / 8.0, of 256 9.7 / 9.0, of 512 11.0 / 10.2; of
+// 1078 the copy takes as long as it saves.  16 posted at a time: 8 MiB in requests of 18 84.5 / 100, four requests of 64
+// whole pages 11.6 / 11.9 with a copy of the first.)
+__attribute__((noinline)) const void* descriptors_for_engine(Comm* comm, const Request* r) {
+  UnpackQueue* q = comm->queue;
+  const bool small = r->slot.cnt_cache <= kStagedDescs;
+  const bool alone = comm->slots_at_gpu == 0 && comm->to_submit == 1 && !comm->rq.has(kReqActive) && !comm->rq.has(kReqPosted);
+  if (!q->stage || (!small && (!alone || r->slot.cnt_cache > kAloneDescs))) return q->meta_dev->nccl.mem[r->slot.idx];
+  const size_t at = small ? r->slot.idx * kStagedDescs : static_cast<size_t>(kStagedDescs) * kQueueDepth;
+  memcpy(q->stage + at, r->slot.mem, sizeof(union loadMeta) * r->slot.cnt_cache);
+  g.ops->visible_flush();
+  return q->stage_dev + at;
+}
+
 // Publishes a completed receive request's descriptor count and hands its slot to the engine (device type "host").
 // The count and the release are the reference's publish (src/net_tcpx.cc:1350-1357); the submission is this
 // build's doorbell.  *submitted stays false when the engine's submission ring is full: the caller tries again at
@@ -636,16 +655,7 @@ ncclResult_t publish_to_engine(Comm* comm, Request* r, bool* submitted) {
   std::atomic_thread_fence(std::memory_order_release);
   q->meta->done[r->slot.idx].value = 0;
   r->done_value = ++comm->done_seq;
-  // The descriptors the engine reads: the mapped slot, or -- for a small request, of which a comm has at
-  // most 16 in flight -- a second copy in the GPU's own memory, written through the BAR ahead of the
-  // submission, which saves the GPU a PCIe round trip before it can start copying.
-  const void* descs_dev = q->meta_dev->nccl.mem[r->slot.idx];
-  if (q->stage && r->slot.cnt_cache <= kStagedDescs) {
-    union loadMeta* copy = q->stage + r->slot.idx * kStagedDescs;
-    memcpy(copy, r->slot.mem, sizeof(union loadMeta) * r->slot.cnt_cache);
-    g.ops->visible_flush();
-    descs_dev = q->stage_dev + r->slot.idx * kStagedDescs;
-  }
+  const void* descs_dev = descriptors_for_engine(comm, r);
   // The request's size goes along as a hint (it sizes the engine's tickets for fragments shorter than a page).
   const uint32_t n_descs = static_cast<uint32_t>(r->slot.cnt_cache);
   void* done_flag = &q->meta_dev->done[r->slot.idx].value;

@@ -396,12 +396,14 @@ struct QueueBlock {  // mapped metadata + device handle, recycled between comms 
   QueueMeta* meta;
   QueueMeta* meta_dev;
   struct unpackNetDeviceHandle* dev_handle;
-  // Device memory the host can write, kQueueDepth x kStagedDescs descriptors, or null: where the descriptors of a
-  // small request are copied to as well, so that the GPU need not fetch them over PCIe.
+  // Device memory the host can write, kStageDescs descriptors, or null: where the descriptors of a small request, or of one
+  // that is alone, are copied to as well, so that the GPU need not fetch them over PCIe (see publish_to_engine).
   union loadMeta* stage;
   union loadMeta* stage_dev;
 };
-constexpr uint32_t kStagedDescs = 16;
+constexpr uint32_t kStagedDescs = 16;   // a small request's, of which each slot has its own
+constexpr uint32_t kAloneDescs = 512;   // of a request that is alone at the GPU, behind the slots' own
+constexpr uint32_t kStageDescs = kStagedDescs * kQueueDepth + kAloneDescs;
 
 struct DeviceState {
   int dev = 0;

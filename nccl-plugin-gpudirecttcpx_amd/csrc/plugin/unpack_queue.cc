@@ -30,7 +30,7 @@ ncclResult_t unpack_queue_new(int dev, bool passive, UnpackQueue** queue) {
     }
     void *sh = nullptr, *sd = nullptr;
     if (!g.ops->visible_alloc || !g.ops->visible_flush ||
-        g.ops->visible_alloc(dev, sizeof(union loadMeta) * kStagedDescs * kQueueDepth, &sh, &sd) != TCPXU_SUCCESS) {
+        g.ops->visible_alloc(dev, sizeof(union loadMeta) * kStageDescs, &sh, &sd) != TCPXU_SUCCESS) {
       sh = sd = nullptr;  // optional: every request's descriptors are then read from the mapped slot
     }
     blk = QueueBlock{static_cast<QueueMeta*>(h), static_cast<QueueMeta*>(d),

@@ -166,6 +166,52 @@ def test_small_requests_hand_over_a_second_copy_of_their_descriptors(env, comm):
         env.emu.emu_set_visible_off(0)
 
 
+@pytest.mark.parametrize("n,staged", [(16, 1), (17, 1), (512, 1), (513, 0)])
+def test_a_request_that_is_alone_at_the_gpu_hands_over_a_second_copy(env, comm, n, staged):
+    """Of up to 512 descriptors, and again once it has been reported done; while it is there, the next one that is not small
+    goes by its mapped slot, and leaves the first one's copy alone."""
+    rng = np.random.default_rng(n)
+    frags = np.zeros(3 * n, dtype=env.pkg.Workload(1, shrink=6).frag_dtype)
+    frags["frag_size"] = 100
+    frags["frag_token"] = rng.permutation(3 * n) % (ARENA_BYTES // 4096)
+    frags["frag_offset"] = frags["frag_token"] * 4096 + rng.integers(0, 3996, 3 * n)
+    env.arena_np[:] = rng.integers(0, 256, len(env.arena_np), dtype=np.uint8)
+    buf, ptr = host_buffer(300 * n)
+    mh = comm.reg(ptr, 300 * n)
+    env.emu.emu_set_hold(1)
+    start = env.emu.emu_counter(0), env.emu.emu_counter(6)
+
+    def counted():
+        return env.emu.emu_counter(0) - start[0], env.emu.emu_counter(6) - start[1]
+
+    def post(i, oldest=None):
+        rc, req = comm.irecv(ptr + i * 100 * n, 100 * n, mh)
+        assert rc == 0
+        comm.ctrl(0, 100 * n, 0, 100 * n)
+        comm.deliver(0, frags[i * n : (i + 1) * n])
+        submitted = env.emu.emu_counter(0)
+        for _ in range(100000):
+            assert comm.test(oldest or req)[:2] == (0, 0)  # (only the oldest may be asked for)
+            if env.emu.emu_counter(0) == submitted + 1:
+                return req
+        raise AssertionError("request never reached the engine")
+
+    first = post(0)
+    second = post(1, first)
+    small = int(n <= 16)
+    assert counted() == (2, staged + small)
+    assert env.emu.emu_release(2) == 2
+    for req in (first, second):
+        assert comm.test(req)[:2] == (0, 1) and comm.consumed(req) == 0
+    third = post(2)
+    assert counted() == (3, 2 * staged + small)
+    assert env.emu.emu_release(1) == 1
+    assert comm.test(third)[:2] == (0, 1) and comm.consumed(third) == 0
+    comm.dereg(mh)
+    want = b"".join(env.arena_np[int(f["frag_offset"]) : int(f["frag_offset"]) + 100].tobytes() for f in frags)
+    assert buf.tobytes() == want
+
+
 def test_the_request_size_goes_along_with_the_submission(env, comm):
     """The slot is handed to the engine with the request's byte count as a hint (the sum of its descriptors'
     lengths); one request at a time, so that the last submission seen is the request just completed."""
