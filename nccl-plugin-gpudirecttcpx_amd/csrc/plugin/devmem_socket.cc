@@ -41,19 +41,6 @@ bool PageLedger::open(size_t arena_pages) {
 
 namespace {
 
-// One control message as it lies in the buffer: the fields of struct cmsghdr, the vector, and the padding that the
-// kernel zeroes too.
-struct WireCmsg {
-  size_t len;
-  int level, type;
-  DevmemVec v;
-  uint32_t pad;
-};
-static_assert(sizeof(WireCmsg) == CMSG_SPACE(sizeof(DevmemVec)) && offsetof(WireCmsg, v) == CMSG_LEN(0) &&
-                  offsetof(WireCmsg, level) == offsetof(struct cmsghdr, cmsg_level) &&
-                  offsetof(WireCmsg, type) == offsetof(struct cmsghdr, cmsg_type),
-              "one control message: header, 12 bytes, 4 of padding");
-
 constexpr size_t kPrefetchFrags = 8;  // page entries asked for ahead: the pages of a message lie anywhere in the arena
 
 }  // namespace
@@ -169,14 +156,14 @@ int DevmemSocket::dontneed(const PageToken* tokens, size_t n) {
 
 // The control message after `cm`, or null: the bounds of CMSG_NXTHDR, without the call into the C library that the
 // macro makes for every message.
-static inline struct cmsghdr* next_cmsg(const struct msghdr* msg, struct cmsghdr* cm) {
+static inline CmsgHeader* next_cmsg(const struct msghdr* msg, CmsgHeader* cm) {
   const size_t at = static_cast<size_t>(reinterpret_cast<char*>(cm) - static_cast<char*>(msg->msg_control));
   const size_t left = msg->msg_controllen - at;
-  if (cm->cmsg_len < sizeof(struct cmsghdr) || CMSG_ALIGN(cm->cmsg_len) > left ||
-      left - CMSG_ALIGN(cm->cmsg_len) < sizeof(struct cmsghdr))
+  if (cm->len < sizeof(CmsgHeader) || CMSG_ALIGN(cm->len) > left ||
+      left - CMSG_ALIGN(cm->len) < sizeof(CmsgHeader))
     return nullptr;
-  struct cmsghdr* next = reinterpret_cast<struct cmsghdr*>(reinterpret_cast<char*>(cm) + CMSG_ALIGN(cm->cmsg_len));
-  if (CMSG_ALIGN(next->cmsg_len) > left - CMSG_ALIGN(cm->cmsg_len)) return nullptr;  // runs past the end of the buffer
+  CmsgHeader* next = reinterpret_cast<CmsgHeader*>(reinterpret_cast<char*>(cm) + CMSG_ALIGN(cm->len));
+  if (CMSG_ALIGN(next->len) > left - CMSG_ALIGN(cm->len)) return nullptr;  // runs past the end of the buffer
   return next;
 }
 
@@ -195,7 +182,7 @@ ssize_t process_recv_cmsg(struct msghdr* msg, DataPipe* p, int offset, uint64_t 
   if (n_toks > 0) next_token = toks[n_toks - 1].token_start + toks[n_toks - 1].token_count;
   const uint64_t dst_base = static_cast<uint64_t>(offset) + dst_base_offset;
   const char* const control_end = static_cast<const char*>(msg->msg_control) + msg->msg_controllen;
-  for (struct cmsghdr* cm = CMSG_FIRSTHDR(msg); cm; cm = next_cmsg(msg, cm)) {
+  for (CmsgHeader* cm = reinterpret_cast<CmsgHeader*>(CMSG_FIRSTHDR(msg)); cm; cm = next_cmsg(msg, cm)) {
     // A run of devmem fragments as the kernel writes them, as many as there is room for: one comparison of the header each.
     const WireCmsg* w = reinterpret_cast<const WireCmsg*>(cm);
     const size_t room = std::min<size_t>({static_cast<size_t>(control_end - reinterpret_cast<const char*>(cm)) / sizeof(WireCmsg),
@@ -214,17 +201,17 @@ ssize_t process_recv_cmsg(struct msghdr* msg, DataPipe* p, int offset, uint64_t 
     }
     if (const ptrdiff_t taken = w - reinterpret_cast<const WireCmsg*>(cm); taken != 0) {
       num_cm += static_cast<int>(taken);
-      cm = next_cmsg(msg, reinterpret_cast<struct cmsghdr*>(const_cast<WireCmsg*>(w - 1)));
+      cm = next_cmsg(msg, reinterpret_cast<CmsgHeader*>(const_cast<WireCmsg*>(w - 1)));
       if (!cm) break;
     }
-    if (cm->cmsg_level != SOL_SOCKET || (cm->cmsg_type != kScmDevmemOffset && cm->cmsg_type != kScmDevmemHeader)) {
-      INFO(NCCL_NET, "cmsg: unknown %u.%u", cm->cmsg_level, cm->cmsg_type);
+    if (cm->level != SOL_SOCKET || (cm->type != kScmDevmemOffset && cm->type != kScmDevmemHeader)) {
+      INFO(NCCL_NET, "cmsg: unknown %u.%u", cm->level, cm->type);
       continue;
     }
     ++num_cm;
     DevmemVec v;
-    memcpy(&v, CMSG_DATA(cm), sizeof v);
-    if (cm->cmsg_type == kScmDevmemHeader) {
+    memcpy(&v, reinterpret_cast<const char*>(cm) + CMSG_LEN(0), sizeof v);
+    if (cm->type == kScmDevmemHeader) {
       // Payload that landed in host memory instead of a bounce page.  The reference has no working copy for it
       // (its gpu_inline_memcpy is a no-op, src/devcomm/nccl/inline.cu:48-60) and stops; so does this build.
       if (v.frag_size > 0) {

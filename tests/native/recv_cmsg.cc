@@ -158,8 +158,29 @@ static bool socket_case(int at) {
   return true;
 }
 
+// The walk reads the caller's buffer as headers and as WireCmsg in turn, and recvmsg writes it as the latter: what goes in one
+// way must come out the other, whatever the compiler has inlined.
+__attribute__((noipa)) static size_t written_as_wire(CmsgHeader* h, WireCmsg* w) {
+  h->len = 1;
+  w->len = 2;
+  return h->len;
+}
+__attribute__((noipa)) static size_t written_as_header(CmsgHeader* h, WireCmsg* w) {
+  w->len = 1;
+  h->len = 2;
+  return w->len;
+}
+static bool both_views_are_one_memory() {
+  const int at = 0;
+  alignas(16) static char control[sizeof(WireCmsg)];
+  CHECK(written_as_wire(reinterpret_cast<CmsgHeader*>(control), reinterpret_cast<WireCmsg*>(control)) == 2);
+  CHECK(written_as_header(reinterpret_cast<CmsgHeader*>(control), reinterpret_cast<WireCmsg*>(control)) == 2);
+  return true;
+}
+
 int main() {
   tcpxSetFailStopForTesting(0);
+  if (!both_views_are_one_memory()) return 1;
   for (int at = 0; at < 20000; ++at)
     if (!walk_case(at)) return 1;
   for (int at = 0; at < 3000; ++at)
