@@ -42,10 +42,10 @@
 #include <thread>
 #include <vector>
 
+#include "engine_rules.h"
 #include "hip_common.h"
 #include "tcpx_unpack_hip.h"
 #include "unpack_device.h"
-
 
 namespace tcpxu {
 namespace {
@@ -292,7 +292,7 @@ struct DevState {  // device memory
   uint64_t leader_polls, leader_entries, leader_deep_polls;  // leader-private: running totals (see HostCtl)
   alignas(64) uint32_t exited_wgs;      // reset at every start, as are the stop words
   uint32_t exit_reason;
-  alignas(64) uint32_t leader_place;    // likewise: the leader's compute unit (see worker_loop)
+  alignas(64) uint32_t leader_place;    // likewise: the leader's compute unit (see kEnoughElsewhere)
   uint32_t workers_elsewhere;           // worker workgroups that have started on other ones
   alignas(256) StopWord stop[kStopReplicas];
   alignas(64) Record tickets[kTicketRing];
@@ -1382,14 +1382,6 @@ __device__ __forceinline__ uint32_t compute_unit_here() {
   asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
   return (hw & 0xFF00u) | ((xcc & 0xFu) << 16) | 1u;  // compute unit, array and engine of one of the eight XCDs
 }
-// The leader has its compute unit to itself.  Loads seem to return to a compute unit in the order in which it issued them,
-// so the looks at the host's ring and the copy's loads wait for each other where both are under way.  A worker workgroup
-// that finds itself there claims no ticket and leaves (its place then goes to the one workgroup of the grid that found
-// none, which does the same) -- provided that this many others have started elsewhere: a small grid, or one that is placed
-// while other kernels hold most of the GPU, keeps all of its workers.  (Requests of 64 KiB: 2048 in one call 67.5 -> 63.5 us,
-// 1024 41.4 -> 39.3, 16 to 256 within 2 % either way; a stream with 1024 in flight 40.5 -> 48.5 M/s, one comm's sixteen slots
-// of 4 MiB 71.9 -> 72.5 % of the roofline; large requests the same, so two workers of 512 are not missed.)
-constexpr uint32_t kEnoughElsewhere = 256;
 
 __device__ void worker_loop(DevState* st, uint32_t* jobs_done, uint32_t flags, uint64_t* stamps) {
   __shared__ Stage stages[2];
@@ -1417,11 +1409,14 @@ __device__ void worker_loop(DevState* st, uint32_t* jobs_done, uint32_t flags, u
     // clear: claim only when the copy has finished; bit 0 set: claim right away while tickets are queueing up,
     // i.e. the previous ticket was already there at the first look.)
     const uint32_t* stop_word = &st->stop[blockIdx.x % kStopReplicas].value;
-    // (Workgroup 0 is the first to be started, and this is the first thing that it does.)
-    uint32_t leader_place;
-    while ((leader_place = same_in_all_lanes32(sys_load(&st->leader_place))) == 0) __builtin_amdgcn_s_sleep(1);
-    const bool beside_leader = leader_place == same_in_all_lanes32(compute_unit_here());
-    if (!beside_leader && lane == 0) __hip_atomic_fetch_add(&st->workers_elsewhere, 1u, __ATOMIC_RELAXED, SYS);
+    bool beside_leader = false;
+    if (enough_can_be_elsewhere(gridDim.x)) {
+      // (Workgroup 0 is the first to be started, and this is the first thing that it does.)
+      uint32_t leader_place;
+      while ((leader_place = same_in_all_lanes32(sys_load(&st->leader_place))) == 0) __builtin_amdgcn_s_sleep(1);
+      beside_leader = leader_place == same_in_all_lanes32(compute_unit_here());
+      if (!beside_leader && lane == 0) __hip_atomic_fetch_add(&st->workers_elsewhere, 1u, __ATOMIC_RELAXED, SYS);
+    }
     auto not_needed = [&] { return beside_leader && same_in_all_lanes32(sys_load(&st->workers_elsewhere)) >= kEnoughElsewhere; };
     // (The others may be just starting: a few tens of microseconds for them, before a number is claimed that has to be served.)
     for (uint32_t looks = 0; beside_leader && looks < 32 && !not_needed(); ++looks) __builtin_amdgcn_s_sleep(16);
