@@ -178,10 +178,12 @@ int tcpxuEngineSubmitMany(tcpxuEngine* engine, const tcpxuSubmission* submission
  * with `in_flight` submissions not yet completed (itself included) is handed out in *n_tickets tickets of
  * *per_ticket descriptors; *max_descs is the most descriptors a submission may carry.  Outputs may be NULL.
  * (What it does not know: how many submissions a call hands over together -- the ones still to come count as in flight for
- * one of short fragments, and eight or more of whole pages, of more than 32 descriptors each and 12 to 40 per worker
- * workgroup in all, go in tickets of 18 -- and what the leader finds at run time: while eight or more submissions wait in
- * one of its polls, tickets sized by backlog are at least 16 descriptors, and while four or more do, those that would be of
- * fewer than 14 are 16.)
+ * one of short fragments; eight or more of whole pages, of more than 32 descriptors each and 12 to 40 per worker
+ * workgroup in all, go in tickets of 18; and eight or more of fragments of a third to half a page, 18 to 1000 per worker
+ * workgroup in all, go in tickets of 32 (not those of 1025 to 1536 descriptors, nor a call that finds 40 per worker
+ * workgroup queued) -- and what the leader finds at run time: while eight or more submissions wait in one of its polls,
+ * tickets sized by backlog are at least 16 descriptors, and while four or more do, those that would be of fewer than 14
+ * are 16.)
  * TCPXU_INVALID_ARGUMENT for an n_descs beyond that limit. */
 int tcpxuEngineTicketPlan(uint32_t workgroups, uint32_t descs_per_ticket, uint32_t in_flight, uint32_t n_descs,
                           uint64_t payload_bytes, uint32_t* per_ticket, uint32_t* n_tickets, uint32_t* max_descs);

@@ -1,5 +1,9 @@
-// The engine's decisions by numbers, at the numbers where they change (no GPU).
+// The engine's decisions by numbers, at the numbers where they change and against plain restatements (no GPU).
 #include "engine_rules.h"
+
+#include <algorithm>
+#include <cstdio>
+#include <random>
 
 using namespace tcpxu;
 
@@ -9,4 +13,53 @@ static_assert(!enough_can_be_elsewhere(2) && !enough_can_be_elsewhere(64), "smal
 static_assert(!enough_can_be_elsewhere(257) && enough_can_be_elsewhere(258) && 258 - 2 == kEnoughElsewhere, "the line");
 static_assert(enough_can_be_elsewhere(513), "two workers on each of 256 compute units");
 
-int main() { return 0; }
+#define CHECK(c)                                                  \
+  do {                                                            \
+    if (!(c)) {                                                   \
+      std::printf("line %d: %s does not hold\n", __LINE__, #c);   \
+      return 1;                                                   \
+    }                                                             \
+  } while (0)
+
+// A submission's ticket size, said with divisions; `burst` as the host marks it.
+static uint32_t size_of(uint64_t in_flight, uint64_t n, uint64_t bytes, uint64_t workers, bool burst) {
+  const double mean = bytes == 0 ? 4096.0 : static_cast<double>(bytes) / n;
+  const uint32_t full = mean >= 2731 ? 16 : mean >= 2048 ? 32 : mean >= 1366 ? 48 : 64;
+  if (burst) return full == 16 ? 18 : n > 1024 && n <= 1536 ? 48 : 32;
+  if (n <= 16) return 16;
+  if (in_flight >= 8 && n <= 32) return 32;
+  const double per_worker = static_cast<double>(std::min<uint64_t>(in_flight * n, 1u << 20)) / workers;
+  if (per_worker < 13) return 8;
+  if (per_worker < 18) return 12;
+  if (full == 16) return per_worker < 100 ? 14 : 16;
+  return full == 48 && n <= 1024 && per_worker < 100 ? 32 : full;
+}
+
+int main() {
+  std::mt19937_64 rng(1);
+  for (int i = 0; i < 2000000; ++i) {
+    const uint32_t n = 1 + static_cast<uint32_t>(rng() % (rng() % 2 ? 3000 : 1u << 20)), in_flight = 1 + static_cast<uint32_t>(rng() % 300);
+    const uint32_t workers = 1 + static_cast<uint32_t>(rng() % 1000);
+    const uint64_t mean = rng() % 4200;  // (0: the caller did not say)
+    const uint32_t bytes = static_cast<uint32_t>(std::min<uint64_t>(n * mean, 0xFFFFFFFFu));
+    const bool marked = burst_of_pages(8, n, bytes, workers) || burst_of_short_fragments(8, n, bytes, workers);
+    for (bool burst : {false, true})
+      if (!burst || marked) CHECK(ticket_size_for_submission(in_flight, n, bytes, workers, burst) == size_of(in_flight, n, bytes, workers, burst));
+    const uint32_t per = 1 + static_cast<uint32_t>(rng() % 64);
+    CHECK(tickets_for(n, per) == (n + per - 1) / per);
+  }
+  // Bursts of short fragments (1800 bytes) on 512 workers: eight submissions or more, from 18 to fewer than 1000 descriptors per
+  // worker in all, where fewer than 40 per worker are queued already.
+  auto burst = [](uint32_t submissions, uint32_t n, uint32_t mean) { return burst_of_short_fragments(submissions, n, n * mean, 512); };
+  CHECK(!burst(7, 1600, 1800) && burst(8, 1600, 1800));
+  for (const uint32_t n : {1024u, 1025u, 1536u, 1537u})  // lengths between, of which the leader would write such tickets in another way
+    CHECK(ticket_size_for_submission(16, n, n * 1800, 512, true) == (n == 1024 || n == 1537 ? 32u : 48u));
+  CHECK(!burst(16, 575, 1800) && burst(16, 576, 1800));          // 18 x 512
+  CHECK(burst(500, 1023, 1800) && !burst(500, 1024, 1800));      // 1000 x 512
+  CHECK(burst(319, 1605, 1800) && !burst(320, 1600, 1800));
+  CHECK(!burst(16, 1600, 1365) && burst(16, 1600, 1366) && burst(16, 1600, 2047) && !burst(16, 1600, 2048) && !burst(16, 1600, 0));
+  CHECK(few_ahead_of_burst(0, 1u << 20, 1) && few_ahead_of_burst(12, 1706, 512) && !few_ahead_of_burst(12, 1707, 512));
+  CHECK(!few_ahead_of_burst(UINT64_MAX / (1u << 20), 1u << 20, 512));
+  std::puts("engine rules ok");
+  return 0;
+}
