@@ -235,6 +235,11 @@ int tcpxuEngineRunning(tcpxuEngine* engine, int* running);
  * (a hipStream_t, NULL = the default stream) and then stores `done_value` to `*done_flag_dev` (device-visible 8-byte
  * word, e.g. the alias of mapped host memory; may be NULL when stream order is all the caller needs: the call is then
  * tcpxuUnpackBatch).  Up to 24 descriptors are one kernel, more are two, the second of which writes the word.
+ * That one kernel is one workgroup, chosen for fragments of up to a page, which is what a bounce page holds: the call does
+ * not know the lengths, and on longer ones it is slower than two kernels would be, since one compute unit moves all of it
+ * (microseconds a call, one kernel / two, of 8 / 16 / 24 descriptors: of 4 KiB 3.4 / 5.9, 4.1 / 5.9, 5.0 / 5.9, of 8 KiB
+ * 4.1 / 5.9, 5.5 / 5.9, 7.0 / 6.0, of 64 KiB 12.9 / 11.0, 25.3 / 11.0, 35.7 / 11.0).  A caller with lists of 128 KiB and
+ * more in so few descriptors adds empty ones up to 25, or passes no word and lets the stream's order tell.
  * Asynchronous.  It calls no hipMalloc, hipFree or other allocating routine and keeps nothing in device memory, so calls
  * may overlap on a GPU without limit: two streams, two threads, a replayed graph beside an ordinary call, two
  * executables of one captured graph (as far as their destinations and words allow it).

@@ -75,6 +75,12 @@ __global__ __launch_bounds__(kWaves* kWaveLanes) __attribute__((amdgpu_waves_per
 // wavefronts at the most, so beyond 16 descriptors some of them take two, one after the other, while a second launch costs
 // the host 2.8 us.  (Us a call, one workgroup / two launches: 18 whole pages 4.2 / 6.3, 20 4.35 / 6.3, 24 4.9 / 6.3, 32 5.9 / 6.3,
 // 40 7.1 / 6.3; a call that is waited for: 24 pages 15.4 / 15.9, 32 16.6 / 15.8.)
+//
+// The line lies where it does for fragments of up to a page.  What one workgroup does not do well is bytes, 128 KiB in and out
+// of one compute unit for 3 us; of longer fragments it takes fewer to reach that (24 of 4 KiB 5.0 / 5.9, of 6 KiB 6.4 / 5.9, of 64 KiB
+// 35.7 / 11.0; 17 of 6 KiB 5.2 / 5.9, of 9000 bytes 6.7 / 6.0; 16 of 8 KiB 5.5 / 5.9, of 16 KiB 8.2 / 5.9; 8 of 16 KiB 5.3 / 6.0, of
+// 64 KiB 12.9 / 11.0; 4 of 64 KiB 11.0 / 10.9).  The host does not know the lengths -- a call may be captured or queued before
+// its list is written -- so the entry point's description says what that costs and how a caller of such lists avoids it.
 constexpr uint32_t kSmallSlot = 24;
 constexpr uint32_t kSmallSlotWaves = 16;
 __global__ __launch_bounds__(kSmallSlotWaves* kWaveLanes) void unpack_small_slot_kernel(const uint8_t* __restrict__ bounce, uint8_t* __restrict__ dst,

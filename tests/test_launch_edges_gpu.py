@@ -58,6 +58,27 @@ def test_list_lengths_around_one_workgroup(pkg, hip, oracle, n, misalign):
     test_list_lengths(pkg, hip, oracle, n, misalign)
 
 
+@pytest.mark.parametrize("n", [2, 16, 17, 24, 25])
+@pytest.mark.parametrize("length", [9000, 70001])
+def test_few_descriptors_of_many_rounds_each(pkg, hip, oracle, n, length):
+    """Fragments of several pages through one workgroup, a wavefront's second one behind its first, and through two launches."""
+    import torch
+
+    rng = np.random.default_rng(n)
+    descs = np.zeros(n, dtype=np.dtype([("src_off", "<u4"), ("len", "<u4"), ("dst_off", "<u8")]))
+    descs["len"], descs["dst_off"] = length, np.arange(n) * length
+    descs["src_off"] = rng.integers(0, PAGES * 4096 - length, n)
+    pool = rng.integers(0, 256, PAGES * 4096, dtype=np.uint8)
+    expect = oracle_expected(oracle, pool, descs, n * length, 5)
+    buf = GpuBuffers(pool, descs, n * length, 5)
+    mapped = Mapped(pkg, hip, descs, 1)
+    print("slot of %d descriptors of %d bytes" % (n, length), flush=True)
+    pkg.check(hip.tcpxuUnpackSlotNoAlloc(0, buf.pool.data_ptr(), buf.dst_base, mapped.desc_dev(0), n, mapped.flag_dev(0), 7, None), "tcpxuUnpackSlotNoAlloc")
+    torch.cuda.synchronize()
+    assert int(mapped.flags[0]) == 7 and first_difference(buf.result(), expect) is None
+    mapped.free()
+
+
 @pytest.mark.parametrize("n", [2049, 4095, 4096, 4097, 4604, 4607, 4608, 4609, 4613, 6144, 6145, 7001])
 def test_lists_around_whole_turns_of_the_xcds(pkg, hip, oracle, n):
     """Beyond 4096 descriptors the XCDs take runs of 24 groups of four descriptors in turn, 768 descriptors a turn: lists of
