@@ -141,7 +141,7 @@ struct HostCtl {  // mapped host memory
   alignas(64) uint64_t tail;       // host -> GPU: submissions published so far
   alignas(64) uint64_t stop;       // host -> GPU: drain and exit
   alignas(64) uint64_t head;       // GPU -> host: submissions the leader has consumed
-  alignas(64) uint64_t completed;  // GPU -> host: submissions fully unpacked (mirrored when idle and at exit)
+  alignas(64) uint64_t completed;  // GPU -> host: submissions fully unpacked (told with a look that finds nothing, if it has changed, and at exit)
   alignas(64) uint64_t exited;     // GPU -> host: 0 running, 1 stopped on request, 2 left after being idle
   alignas(64) uint64_t exiting;    // GPU -> host: the leader is about to leave for idleness (see leader_loop)
   // GPU -> host, written by the leader when it leaves: its polls of the ring, the entries they consumed and the
