@@ -1259,7 +1259,8 @@ __device__ __forceinline__ void copy_ticket(const LdsStage* stage, uint32_t wave
   }
 }
 
-// The compute unit that the calling wavefront runs on, as a number that is never zero.
+// The compute unit that the calling wavefront runs on, as an odd number; kNoPlace is none's.
+constexpr uint32_t kNoPlace = 2;
 __device__ __forceinline__ uint32_t compute_unit_here() {
   uint32_t hw, xcc;
   asm volatile("s_getreg_b32 %0, hwreg(HW_REG_HW_ID)" : "=s"(hw));
@@ -1293,14 +1294,11 @@ __device__ void worker_loop(DevState* st, uint32_t* jobs_done, uint32_t flags, u
     // clear: claim only when the copy has finished; bit 0 set: claim right away while tickets are queueing up,
     // i.e. the previous ticket was already there at the first look.)
     const uint32_t* stop_word = &st->stop[blockIdx.x % kStopReplicas].value;
-    bool beside_leader = false;
-    if (enough_can_be_elsewhere(gridDim.x)) {
-      // (Workgroup 0 is the first to be started, and this is the first thing that it does.)
-      uint32_t leader_place;
-      while ((leader_place = same_in_all_lanes32(sys_load(&st->leader_place))) == 0) __builtin_amdgcn_s_sleep(1);
-      beside_leader = leader_place == same_in_all_lanes32(compute_unit_here());
-      if (!beside_leader && lane == 0) __hip_atomic_fetch_add(&st->workers_elsewhere, 1u, __ATOMIC_RELAXED, SYS);
-    }
+    // (Workgroup 0 is the first to be started, and this is the first thing that it does.)
+    uint32_t leader_place;
+    while ((leader_place = same_in_all_lanes32(sys_load(&st->leader_place))) == 0) __builtin_amdgcn_s_sleep(1);
+    const bool beside_leader = leader_place == same_in_all_lanes32(compute_unit_here());
+    if (!beside_leader && lane == 0) __hip_atomic_fetch_add(&st->workers_elsewhere, 1u, __ATOMIC_RELAXED, SYS);
     auto not_needed = [&] { return beside_leader && same_in_all_lanes32(sys_load(&st->workers_elsewhere)) >= kEnoughElsewhere; };
     // (The others may be just starting: a few tens of microseconds for them, before a number is claimed that has to be served.)
     for (uint32_t looks = 0; beside_leader && looks < 32 && !not_needed(); ++looks) __builtin_amdgcn_s_sleep(16);
@@ -1377,7 +1375,7 @@ __global__ __launch_bounds__(kEngineThreads) __attribute__((amdgpu_waves_per_eu(
                                                                    uint32_t flags, uint64_t* stamps) {
   if (blockIdx.x == 0) {
     __shared__ Look looks[kLooks];
-    if (threadIdx.x == 0) sys_store_global(&st->leader_place, compute_unit_here());
+    if (threadIdx.x == 0) sys_store_global(&st->leader_place, enough_can_be_elsewhere(gridDim.x) ? compute_unit_here() : kNoPlace);
     if (threadIdx.x < kWaveLanes)
       leader_loop(ctl, st, jobs_done, job_target, ring_mask, per_ticket, spin_limit, stamps, (LdsLook*)&looks[0]);
   } else {
