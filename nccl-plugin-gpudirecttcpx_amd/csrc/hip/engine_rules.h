@@ -102,9 +102,11 @@ constexpr uint32_t kBurstTicket = 18;
 // * Calls of kLongBurst descriptors per worker and more, whose last round is nothing beside the rest: 250 of 1000 fragments
 //   162.9 us / 163.2, 512 310.3 / 312.9, 1000 584.5 / 592.3 (300 of 1700, below the line, 329.8 / 328.8).
 // * Calls that find kAheadOfBurst descriptors per worker queued already: a stream, which larger tickets move faster once it
-//   is deep, and which has no last round.  Calls of 16 requests, other calls under way 1 / 3 / 7: of 1700 fragments 6.31 / 6.20 /
-//   5.96 TB/s in tickets of 48, 6.60 / 6.10 / 5.95 in tickets of 32, 6.72 / 6.20 / 5.96 by this line; of 1000 fragments 4.36 /
-//   6.98 / 5.56 in tickets of 48, 4.31 / 6.99 / 5.47 in tickets of 32, 4.32 / 6.92 / 5.56 by this line.
+//   is deep, and which has no last round.  Calls of 16 requests, other calls under way 1 / 2 / 3 / 7, TB/s r+w: of 1700 fragments
+//   6.30 / 7.27 / 6.20 / 5.96 in tickets of 48, 6.55 / 7.16 / 6.08 / 5.94 in tickets of 32, 6.79 / 7.05 / 6.22 / 5.96 by this line;
+//   of 1000 fragments, 1 / 3 / 7, 4.36 / 6.98 / 5.56 in tickets of 48, 4.15 / 6.94 / 5.46 in tickets of 32, 4.15 / 6.80 / 5.56 by this line.
+//   (With two and three calls in the caches it is the leader that a stream waits for, and working out a size by backlog takes it
+//   longer than reading the mark.)
 // * Streams of more than 1024 fragments a request, whose leader would have that microsecond to spend on each.
 constexpr uint32_t kShortBurstTicket = 32, kShortTicket = 48;
 constexpr uint32_t kLongBurst = 1000, kAheadOfBurst = 40;
@@ -134,12 +136,8 @@ TCPXU_RULE uint32_t ticket_size_for_submission(uint32_t in_flight, uint32_t n, u
   const uint32_t size = ticket_size_for(backlog, workers);
   if (size < kFullTicket) return size;
   const uint32_t full = full_ticket_size(bytes, n);
-  if (full > kFullTicket) {
-    // (Asked one after the other: as one condition the leader works out all of it for every entry, 0.02 us that calls of 16
-    // requests of 1700 fragments wait for, two others under way, 7.11 -> 7.23 TB/s r+w.)
-    if (full != kShortTicket || n > kLaneTickets * kShortBurstTicket) return full;
-    return backlog < kDeepBacklog * workers ? kShortBurstTicket : full;
-  }
+  if (full > kFullTicket)
+    return full == kShortTicket && n <= kLaneTickets * kShortBurstTicket && backlog < kDeepBacklog * workers ? kShortBurstTicket : full;
   // Whole pages and a backlog that is there but not deep (one comm's sixteen slots of 4 MiB are 34 descriptors per
   // workgroup: every workgroup holds a ticket and has the next one staged, and hardly any wait unclaimed): tickets
   // of 14 make a seventh more of them, and the workgroups run dry less often -- one comm 71.1 -> 72.2 % of the
