@@ -67,8 +67,8 @@ constexpr uint32_t kPollEntries = 16;  // submission entries fetched per load in
 // is what capped a storm of one-ticket requests near 9 M/s.
 constexpr uint32_t kDeepGroups = 3;    // groups of kPollEntries beyond the first in a deep poll
 constexpr uint32_t kStormBacklog = 128;  // entries published beyond a poll's 64 from which the leader takes them in a rolling loop
-constexpr uint32_t kAuxProbe = 35;  // lane of an auxiliary load that reads the stamp of an entry ahead
-constexpr uint32_t kAuxTicketsDone = 32, kAuxHostStop = 33, kAuxJobsCompleted = 34;  // lanes of the auxiliary load
+constexpr uint32_t kAuxHostStop = 33, kAuxJobsCompleted = 34;  // lanes of the auxiliary load
+constexpr uint32_t kAuxProbe = 35;  // and in a deep poll, the stamp of an entry ahead
 constexpr uint32_t kNeverIdleOut = 0xFFFFFFFFu;
 constexpr uint32_t kDefaultIdlePolls = 400;  // empty polls (of 1.75 us) before the kernel leaves by itself
 constexpr int kTcpxuInProgress = TCPXU_IN_PROGRESS;
@@ -156,7 +156,7 @@ struct alignas(256) StopWord {
   uint32_t value;
 };
 
-// The three words that every workgroup counts in, and two of which every look of the leader reads, lie 4 KiB apart: an atomic
+// The three words that every workgroup counts in, and one of which every look of the leader reads, lie 4 KiB apart: an atomic
 // takes its memory channel 12 ns, and in one line they waited for each other and the looks for them.  (64 / 4096 bytes apart, us
 // a call with other buffers from pass to pass: a request of 64 KiB 8.53 / 8.33, 256 of them 21.9 / 21.3, 64 MiB of ragged
 // fragments 36.6 / 35.9, of wire fragments 32.7 / 32.3; a stream of 64 KiB requests, 256 in flight, 2.47 / 2.56 TB/s r+w; 256
@@ -181,7 +181,9 @@ struct DevState {  // device memory
   alignas(256) StopWord stop[kStopReplicas];
   alignas(64) Record tickets[kTicketRing];
   CarriedList carried[kTicketRing];  // of the tickets that say so
-  // uint32_t jobs_done[ring_entries], then uint32_t job_target[ring_entries] follow
+  // uint32_t jobs_done[ring_entries], then uint32_t job_target[ring_entries] follow: per job slot, the tickets counted and the
+  // tickets ever issued of the submissions of several tickets that it has had.  (A submission's only ticket completes it
+  // and is not counted there.)
 };
 
 // ---- scoped memory operations -------------------------------------------------------------------------------------
@@ -214,10 +216,21 @@ __device__ __forceinline__ uint64_t bcast64(uint64_t v, uint32_t src_lane) {
 // ---- looks at the ring ----------------------------------------------------------------------------------------------
 // A look brings sixteen entries, the descriptors that travel with the first four, and what is known of the entries' job
 // slots, straight into LDS.  kLooks of them are under way at a time, so that an entry waits half the round trip to the
-// host's memory (1.2 us) less for the look that sees it, and going through one look hides behind the next; in LDS because a
-// look that is still under way when the leader leaves this way of polling would otherwise land in registers that have found
-// another use.  A lone request of 16 pages, submit -> done: 9.3 us with one, 8.6 with two, 9.4 with three (going through a
-// look takes 0.4 us, so more than two under way only grow old before their turn comes), and 10.5 with four.
+// host's memory (1.25 us, whatever it brings) less for the look that sees it, and going through one look hides behind the next;
+// in LDS because a look that is still under way when the leader leaves this way of polling would otherwise land in registers that
+// have found another use.
+// What bounds a lone request here is how soon a look shows it and how soon it is a ticket then, and both are instructions of a
+// single wavefront: a pass of the leader's whole loop takes 0.95 us, and while every look cost one, looks came round no sooner
+// than that, however many were under way.  Hence a loop of their own that does the least: a look that shows nothing costs it
+// 0.25 us, entries of one ticket each, wherever their descriptors lie, and an entry of several by itself are written there and
+// then, and anything else leaves it.  Nor does a look read what the workgroups count in, beyond the count of completed
+// submissions: their counting waits for it (see nothing_under_way).  (Us, before / now, buffers in turn: a request of 64 KiB of
+// pages 8.30 / 7.70, through the plugin 7.35 / 6.88, 2048 of them through the plugin, 16 posted at a time, 1030 / 930; sixteen
+// requests of 4 MiB 32.4 / 30.9; a hundred of 200 KB through the plugin, 4 posted at a time, 227 / 209.  A request alone at random
+// times, publish -> done as the host sees it, 1 / 16 / 32 / 256 / 1024 pages: 5.45 / 6.5 / 7.5 / 7.65 / 8.85 before, 4.95 / 6.1 / 7.0 /
+// 7.35 / 8.6 now.)
+// Four under way, one each 0.38 us, are no faster for one request (6.20 and 6.25 over those sizes), and the 2048 take 990, since
+// the host writes entries whose lines are being read.
 // (A look asked for before an earlier one was gone through shows the job slots' counters as they were then.  That is safe:
 // a ring has sixteen entries or more, so none of a look's entries shares its slot with another of them, and what was
 // issued for the slot's last tenant was written before the look was asked for.)
@@ -226,8 +239,10 @@ struct alignas(16) Look {
   uint32_t sect[kWaveLanes][4];     // lane 4k+j: sector j of entry base+k
   uint32_t carried[kWaveLanes][4];  // lane 16k+j: descriptor j of entry base+k
   uint32_t aux[kWaveLanes];         // see leader_loop
-  uint32_t base, pad[3];            // low word of the first entry's number
 };
+constexpr uint32_t kAskedBits = 16, kAskedMask = (1u << kAskedBits) - 1u;
+static_assert(kLooks * kAskedBits <= 64, "leader_loop keeps them in one register");
+static_assert(kCarriedEntries * kCarriedDescs == kWaveLanes, "a lane to a descriptor");
 constexpr int kLookSleep = 2;  // in 64 clocks; 0 to 4 measured alike
 constexpr uint32_t kLookLoads = 3;  // vector memory instructions of a look
 constexpr uint32_t kManyAtOnce = 3, kManySmall = 6;  // see where they are used
@@ -266,35 +281,31 @@ __device__ __forceinline__ uint64_t clock_now() { return wall_clock64(); }
 // What the four lanes of an entry know about it, for the sixteen entries of one group at once.
 struct EntryView {
   uint32_t n, bytes, per_ticket, target_prev, in_flight, slot;
-  uint32_t ticket_bits;  // kCarriedTicket where the entry's descriptors go along, else 0
   bool sane, slot_free;
 };
 
 // How many of a group's entries, from the first, can become tickets now, one each; `room` is what the ticket ring still
 // takes.
 __device__ __forceinline__ uint32_t single_tickets_run(const EntryView& v, uint32_t room) {
-  const uint64_t not_now = ~__ballot(v.sane && v.slot_free);
+  const uint64_t not_now = ~__ballot(v.sane);
   const uint32_t run = not_now == 0 ? kPollEntries : static_cast<uint32_t>(__builtin_ctzll(not_now)) >> 2;
   return std::min(run, room);
 }
 
 // Every entry of a group fits one ticket (a storm of small requests): the leading run of them becomes tickets in
 // one store instruction.  Returns the length of the run.
-__device__ __forceinline__ uint32_t write_single_tickets_of_group(DevState* st, uint32_t* job_target, uint64_t* stamps,
-                                                                  uint64_t& tickets_out, uint32_t lane, const EntryView& v,
-                                                                  const u32x4& sc, uint32_t room) {
+__device__ __forceinline__ uint32_t write_single_tickets_of_group(DevState* st, uint64_t* stamps, uint64_t& tickets_out,
+                                                                  uint32_t lane, const EntryView& v, const u32x4& sc,
+                                                                  uint32_t room) {
   const uint32_t k_of_lane = lane >> 2;
   const uint32_t run = single_tickets_run(v, room);
   if (run != 0) {
     if (k_of_lane < run) {
       const uint64_t t = tickets_out + k_of_lane;
       const uint32_t stamp = static_cast<uint32_t>(t + 1);
-      const uint32_t target = v.target_prev + 1u;
       u32x4 out{sc.x, sc.y, sc.z, stamp};
       if ((lane & 3u) == 3) {
-        out.y = v.n | (v.slot << 8) | kOnlyTicket | v.ticket_bits;
-        out.z = target;
-        sys_store_global(&job_target[v.slot], target);
+        out.y = v.n | (v.slot << 8) | kOnlyTicket;
         if (stamps) sys_store_global(&stamps[kStampsPerJob * v.slot], clock_now());
       }
       store_vec_sys(reinterpret_cast<uint8_t*>(&st->tickets[t & (kTicketRing - 1)]) + 16 * (lane & 3u), out);
@@ -345,7 +356,7 @@ __device__ __forceinline__ T* same_in_all_lanes_ptr(T* p) {
 // The compiler would wait for everything in flight at the top of such a loop.  So the loop's loads are written as
 // instructions, which it does not track, and each step waits for its own group by count: the memory instructions of
 // a wavefront complete in the order issued, and between a group's loads and its turn the other kGroups - 1 groups
-// have had theirs, each with two stores (the tickets, their job slots' targets) and, while the loop feeds, two loads:
+// have had theirs, each with two stores (the tickets, how far it has got) and, while the loop feeds, two loads:
 // 4 x (kGroups - 1) instructions at the least, so "at most that many outstanding" means that the group's own loads
 // have landed.  (More are issued when stamps are on, and the head word once a round: counting too few only waits for
 // a little more than is needed; fewer would let a group be read before it has landed, so this function must not
@@ -361,17 +372,13 @@ struct StormEnd {
   uint64_t s, tickets_out;
   uint32_t entries;  // taken off the ring
 };
-__device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevState* st_in, uint32_t* jobs_done_in,
-                                                          uint64_t* stamps_in, uint32_t ring_mask_in,
+__device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevState* st_in, uint64_t* stamps_in, uint32_t ring_mask_in,
                                                           uint32_t fixed_per_ticket_in, uint64_t s_in, uint64_t tickets_out_in) {
-  // Arguments arrive in vector registers.  These are the same in every lane and go back to scalar registers.  (The job
-  // slots' targets follow their counts in memory: one pointer for both.)
+  // Arguments arrive in vector registers.  These are the same in every lane and go back to scalar registers.
   HostCtl* ctl = same_in_all_lanes_ptr(ctl_in);
   DevState* st = same_in_all_lanes_ptr(st_in);
-  uint32_t* jobs_done = same_in_all_lanes_ptr(jobs_done_in);
   uint64_t* stamps = same_in_all_lanes_ptr(stamps_in);
   const uint32_t ring_mask = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(ring_mask_in)));
-  uint32_t* job_target = jobs_done + ring_mask + 1u;
   const uint32_t fixed_per_ticket = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(fixed_per_ticket_in)));
   uint64_t s = same_in_all_lanes64(s_in);
   uint64_t tickets_out = same_in_all_lanes64(tickets_out_in);
@@ -382,26 +389,17 @@ __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevS
   // and one more.  (1024 requests of 64 KiB in flight: 40.3 M/s with four, 44.6 with five -- where the copy itself is
   // the bound -- and 45.5 with six, which spills registers; 384 in flight: 29.4, 27.2, 26.4.)
   constexpr uint32_t kGroups = 5;
-  // The four lanes that hold an entry's sectors also fetch what is known of its job slot -- tickets counted as done
-  // (first lane), tickets ever issued (second) -- so that both reach all four with a move inside the quad; the other two
-  // lanes read the stamp of the last entry of the group that would be asked for next (the probe).  What of a lane's two
-  // addresses does not change from group to group is worked out once (and hidden from the compiler, which would work
-  // it out again with a branch per kind of lane in every step): address = base + (((s_g + add) & ring_mask) << shift).
-  const uint32_t kind = lane & 3;
-  uint64_t entry_base = reinterpret_cast<uint64_t>(&ctl->ring[0]) + 16 * kind;
-  uint64_t aux_base = kind == 0   ? reinterpret_cast<uint64_t>(jobs_done)
-                      : kind == 1 ? reinterpret_cast<uint64_t>(job_target)
-                                  : reinterpret_cast<uint64_t>(&ctl->ring[0].w[15]);
-  uint32_t aux_add = kind < 2 ? k_of_lane : (kGroups + 1) * kPollEntries - 1;
-  uint32_t aux_shift = kind < 2 ? 2 : 6;
-  static_assert(sizeof(Record) == 64 && sizeof(uint32_t) == 4, "the shifts above");
-  asm volatile("" : "+v"(entry_base), "+v"(aux_base), "+v"(aux_add), "+v"(aux_shift));
+  // Every lane also reads the stamp of the last entry of the group that would be asked for next (the probe).  What of a
+  // lane's address does not change from group to group is worked out once (and hidden from the compiler, which would work it
+  // out again in every step).
+  uint64_t entry_base = reinterpret_cast<uint64_t>(&ctl->ring[0]) + 16 * (lane & 3);
+  asm volatile("" : "+v"(entry_base));
+  const uint64_t probe_base = reinterpret_cast<uint64_t>(&ctl->ring[0].w[15]);
+  static_assert(sizeof(Record) == 64, "the shifts below");
   auto fetch_group_untracked = [&](u32x4& sc, uint32_t& ax, uint64_t s_g) {
     const uint32_t at_s = static_cast<uint32_t>(s_g);  // (the mask keeps low bits only)
     const uint64_t entry = entry_base + (static_cast<uint64_t>((at_s + k_of_lane) & ring_mask) << 6);
-    const uint64_t at = aux_base + (static_cast<uint64_t>((at_s + aux_add) & ring_mask) << aux_shift);
-    // (The job slots' words first: loads return in the order issued, so entries that are there whole -- every sector
-    // carries its stamp -- vouch for the words that were asked for before them.)
+    const uint64_t at = probe_base + (static_cast<uint64_t>((at_s + (kGroups + 1) * kPollEntries - 1) & ring_mask) << 6);
     asm volatile("global_load_dword %0, %1, off sc0 sc1" : "=v"(ax) : "v"(at) : "memory");
     asm volatile("global_load_dwordx4 %0, %1, off sc0 sc1" : "=v"(sc) : "v"(entry) : "memory");
   };
@@ -445,16 +443,15 @@ __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevS
       // ordinary way.
       EntryView more;
       more.n = quad_value<3>(sc.y) & kCountMask;  // payload word 10 sits in .y of sector 3
-      more.ticket_bits = 0;  // (whoever takes the ticket fetches the descriptors: they are nobody's wait with a deep queue)
       more.bytes = 0, more.per_ticket = 0, more.in_flight = 0;  // (not looked at by write_single_tickets_of_group)
-      more.target_prev = quad_value<1>(ax);
+      more.target_prev = 0, more.slot_free = true;
       more.sane = ((okm >> (4 * k_of_lane)) & 0xFull) == 0xFull && more.n - 1u < kMaxDescsPerSubmission;
-      more.slot_free = quad_value<0>(ax) == more.target_prev;
       more.slot = static_cast<uint32_t>(s_g + k_of_lane) & ring_mask;
       const uint32_t one_ticket = fixed_per_ticket != 0 ? fixed_per_ticket : queue_deep ? kMaxDescsPerTicket : kSmallSubmission;
-      if (__ballot(more.sane && more.n > one_ticket) == 0) run = write_single_tickets_of_group(st, job_target, stamps, tickets_out, lane, more, sc, left);
+      if (__ballot(more.sane && more.n > one_ticket) == 0) run = write_single_tickets_of_group(st, stamps, tickets_out, lane, more, sc, left);
     }
     consumed += run;
+    if (run != 0 && lane == 0) sys_store_global(&st->sub_head, s_g + run);  // (one of the two stores counted above)
     if (run != kPollEntries) return false;
     if (feeding == kGroups) {
       const uint64_t next = s_g + kGroups * kPollEntries;
@@ -518,7 +515,9 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
   uint64_t mirrored = same_in_all_lanes(sys_load(&st->jobs_completed.value));  // completed submissions, as the host was last told
   // Read once: the grid's size comes from the dispatch packet, a scalar load with a wait behind it wherever it is asked.
   const uint32_t workers = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(gridDim.x - 1)));
-  uint64_t idle = 0;
+  uint32_t idle = 0;
+  // spin_limit counts polls that ask when the last is done, one in 1.75 us; looks are gone through every 0.75.
+  const uint32_t idle_limit = spin_limit == kNeverIdleOut ? kNeverIdleOut : static_cast<uint32_t>(std::min<uint64_t>(7ull * spin_limit / 3, kNeverIdleOut - 1u));
   uint32_t reason = 0;
   uint32_t polls = 0, entries = 0, deep_polls = 0;  // of this launch; added to the running totals at the end
   uint32_t wide = 0;       // the last entry taken was one of several tickets, with none on its way that count for the size
@@ -526,6 +525,89 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
   uint32_t deep = 0;       // and so many as 64 of them (a ring of fewer never has them)
   uint32_t under_way = 0;  // looks asked for and not gone through
   uint32_t look = 0;       // the next to ask for, modulo kLooks
+  uint64_t asked_at = 0;   // the low bits of the first entry's number of each, the youngest's lowest
+  // A word that workgroups count in is not one to look at all the time: reading it makes their counting wait (sixteen requests of
+  // 4 MiB, looks every 0.75 us: 32.8 us with looks that read the finished tickets' count and the job slots', which share their
+  // lines with those being counted in, 31.3 without; looks every 0.38 us 51 and 30.7).  So two facts are kept instead.
+  // The low word of the tickets known to be done: all of them when nothing is under way, otherwise asked for when the ticket
+  // ring may be half full.
+  uint32_t tickets_done = static_cast<uint32_t>(tickets_out);
+  // Entries below this one have job slots known to be free: what is counted there is then what has been issued.
+  uint64_t free_until = s + ring_mask + 1u;
+  auto nothing_under_way = [&]() {  // every submission before entry s is completed, and its tickets counted
+    tickets_done = static_cast<uint32_t>(tickets_out);
+    free_until = s + ring_mask + 1u;
+  };
+  auto too_many_out = [&]() { return static_cast<uint32_t>(tickets_out) - tickets_done > kTicketRing / 2; };
+  // The tickets of one submission of at least one descriptor, entry s_k, sixteen of them to a store instruction; false if they
+  // cannot be written now.  `too_small`: see kLeaderBehind.
+  auto write_tickets = [&](uint64_t s_k, u32x4 v, uint32_t count_word, uint32_t bytes, uint32_t dst_lo, uint32_t done_now, uint32_t target_prev,
+                           uint32_t completed, uint32_t too_small, uint32_t lane) {
+    const uint32_t n = count_word & kCountMask;
+    // Submissions not yet completed, this one and those on their way included, taken to be as long as this one.
+    const uint32_t in_flight = static_cast<uint32_t>(s_k) - completed + 1u + following(count_word);
+    uint32_t per_ticket = fixed_per_ticket != 0
+                              ? fixed_per_ticket
+                              : ticket_size_for_submission(in_flight, n, bytes, workers, (count_word & kBurstEntry) != 0);
+    // Small tickets spread a small backlog over many workgroups, at the price of more tickets to write.  When
+    // submissions queue up at the leader, its time per submission is what limits the engine, not the spread:
+    // a stream of 1 MiB requests of 256 whole pages, 64 in flight, is served at 1.44 M/s in tickets of 8 (which
+    // the backlog alone asks for: the workers empty it as fast as it comes), at 1.96 M/s in tickets of 16, and at
+    // 1.64 M/s with this rule, which holds for part of the time.
+    if (fixed_per_ticket == 0 && per_ticket < too_small) per_ticket = kFullTicket;
+    const uint32_t nt = tickets_for(n, per_ticket);
+    const uint32_t slot = static_cast<uint32_t>(s_k) & ring_mask;
+    // The job slot is free once every ticket ever issued for it has been counted; the ticket ring has room
+    // while fewer than its size are outstanding (32-bit wrapping arithmetic).  Otherwise leave this entry
+    // for a later poll.
+    if (done_now != target_prev && nt != 1) return false;
+    if (static_cast<uint32_t>(tickets_out) + nt - tickets_done > kTicketRing) return false;
+    const uint32_t target = nt == 1 ? target_prev : target_prev + nt;
+    if (lane == 0) {
+      sys_store_global(&job_target[slot], target);
+      if (stamps) sys_store_global(&stamps[kStampsPerJob * slot], clock_now());
+    }
+    // Four neighbouring lanes write the four sectors of one ticket, so that one store instruction of the
+    // wavefront fills 16 consecutive tickets (1 KiB of whole lines).  A ticket's sector differs from the entry's
+    // in two places only: `v` is the entry's sector of the lane's own kind.
+    // What changes from one pass to the next is kept running, per lane, instead of being worked out from the
+    // ticket's index each time (the leader spends three quarters of its time on a stream of 4 MiB requests in
+    // this loop and the lines before it).
+    const uint32_t sector = lane & 3u;
+    const uint32_t first = lane >> 2;
+    constexpr uint32_t kPerPass = kWaveLanes / 4;
+    // (asked in this order: a request that is alone pays for nothing but the first comparison)
+    const bool across = in_flight >= kManyInFlight && shares_across_tickets(in_flight, n, bytes, dst_lo);
+    const uint64_t descs = (static_cast<uint64_t>(v.z) << 32) | v.y;  // in the lanes of sector 1: dst_hi, descs
+    if (sector == 3) v.z = target;                                     // in the lanes of sector 3: val_hi, n, bytes
+    uint64_t d = descs + static_cast<uint64_t>(first) * per_ticket * sizeof(tcpxuLoadMeta);
+    const uint64_t d_step = static_cast<uint64_t>(kPerPass) * per_ticket * sizeof(tcpxuLoadMeta);
+    uint32_t left = n - first * per_ticket;  // descriptors from this lane's ticket on (meaningless beyond nt)
+    uint32_t at = static_cast<uint32_t>(tickets_out) + first;  // low word of the ticket number
+    uint8_t* const ring = reinterpret_cast<uint8_t*>(st->tickets) + 16 * sector;
+    // The ticket's own word: count | job slot | whether the submission has tickets before and after this one
+    // (the last ticket is the one that takes all that is left).
+    const uint32_t across_bits = across ? kMoreBefore | kMoreAfter : 0u;
+    const uint32_t fixed_bits = (slot << 8) | (nt == 1 ? kOnlyTicket : 0u), after_bit = across_bits & kMoreAfter;
+    uint32_t before_bit = first != 0 ? across_bits & kMoreBefore : 0u;
+    for (uint32_t i = first; i < nt; i += kPerPass) {
+      v.w = at + 1u;  // the stamp
+      if (sector == 1) {
+        v.y = static_cast<uint32_t>(d);
+        v.z = static_cast<uint32_t>(d >> 32);
+      }
+      if (sector == 3) v.y = std::min(per_ticket, left) | fixed_bits | (left > per_ticket ? after_bit : 0u) | before_bit;
+      before_bit = across_bits & kMoreBefore;  // every ticket but the submission's first
+      store_vec_sys(ring + static_cast<size_t>(at & (kTicketRing - 1)) * sizeof(Record), v);
+      d += d_step;
+      left -= kPerPass * per_ticket;
+      at += kPerPass;
+    }
+    lanes_together();
+    tickets_out += nt;
+    wide = nt > 1 && following(count_word) == 0 ? 1u : 0u;
+    return true;
+  };
   bool storm_next = false;
   uint32_t storm_backoff = 0, storm_backoff_len = 4;  // polls until the rolling loop is next tried from the several-tickets way
   const bool ring_allows_deep = ring_mask + 1u >= (kDeepGroups + 1) * kPollEntries;
@@ -533,17 +615,17 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
   // Fixed per-lane roles in the auxiliary load (second load of every poll), so that both loads of a poll are
   // issued back to back by all lanes and waited for once:
   //   lanes 0-15  jobs_done of the job slots of entries s..s+15    lanes 16-31  job_target of the same slots
-  //   lane 32     low word of tickets_done                         lane 33      low word of the host stop word
-  //   lane 34     low word of jobs_completed                       other lanes repeat lane 33.
-  const uint32_t* const tickets_done_lo = reinterpret_cast<const uint32_t*>(&st->tickets_done.value);
+  //   lane 33     low word of the host stop word                   lane 34      low word of jobs_completed
+  //   other lanes repeat lane 33 (in a deep poll lane 35 reads the stamp of an entry ahead).
   const uint32_t* const host_stop_lo = reinterpret_cast<const uint32_t*>(&ctl->stop);
   const uint32_t* const jobs_completed_lo = reinterpret_cast<const uint32_t*>(&st->jobs_completed.value);
 
   for (;;) {
+    if (too_many_out()) tickets_done = same_in_all_lanes32(static_cast<uint32_t>(sys_load(&st->tickets_done.value)));
     // (Every 64 entries it takes count as one deep poll in this launch's figures.)
     if (storm_next) {
       storm_next = false;
-      const StormEnd end = leader_storm(ctl, st, jobs_done, stamps, ring_mask, fixed_per_ticket, s, tickets_out);
+      const StormEnd end = leader_storm(ctl, st, stamps, ring_mask, fixed_per_ticket, s, tickets_out);
       s = same_in_all_lanes(end.s);
       tickets_out = same_in_all_lanes(end.tickets_out);
       const uint32_t taken = same_in_all_lanes32(end.entries);
@@ -568,26 +650,22 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     // One round trip fetches entries s .. s+15: lane 4k+j reads sector j (three payload words and the stamp) of
     // entry s+k.
     const uint32_t k_of_lane = lane >> 2;
-    const uint8_t* const sect_of_lane = reinterpret_cast<const uint8_t*>(&ctl->ring[(s + k_of_lane) & ring_mask]) + 16 * (lane & 3);
+    const uint8_t* sect_of_lane = reinterpret_cast<const uint8_t*>(&ctl->ring[(s + k_of_lane) & ring_mask]) + 16 * (lane & 3);
     const uint32_t* aux_addr = host_stop_lo;
-    if (lane < kPollEntries) aux_addr = &jobs_done[(s + lane) & ring_mask];
+    if (lane < kPollEntries) aux_addr = (s + kPollEntries <= free_until ? job_target : jobs_done) + ((s + lane) & ring_mask);
     else if (lane < 2 * kPollEntries) aux_addr = &job_target[(s + lane - kPollEntries) & ring_mask];
-    else if (lane == kAuxTicketsDone) aux_addr = tickets_done_lo;
     else if (lane == kAuxJobsCompleted) aux_addr = jobs_completed_lo;
     u32x4 sect;
     uint32_t aux;
     uint32_t gone = 0;  // entries of this look's sixteen that an earlier look has brought
     // A deep poll: entries s+16 .. s+63 and their job slots' counters ride along in the same round trip.
     u32x4 sect_more[kDeepGroups];
-    uint32_t aux_more[kDeepGroups];
 #pragma unroll
-    for (uint32_t g = 0; g < kDeepGroups; ++g) {
-      sect_more[g] = u32x4{0u, 0u, 0u, 0u};
-      aux_more[g] = 0;
-    }
+    for (uint32_t g = 0; g < kDeepGroups; ++g) sect_more[g] = u32x4{0u, 0u, 0u, 0u};
     if (direct != 0) {
       under_way = 0;  // (what has been asked for lands in LDS and is not looked at)
       sect = load_vec_sys(sect_of_lane);
+      if (deep != 0 && lane == kAuxProbe) aux_addr = &ctl->ring[(s + (kDeepGroups + 1) * kPollEntries + kStormBacklog - 1) & ring_mask].w[15];
       aux = sys_load(aux_addr);
       if (deep != 0) {
         ++deep_polls;
@@ -595,40 +673,126 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
         for (uint32_t g = 0; g < kDeepGroups; ++g) {
           const uint64_t s_g = s + (g + 1) * kPollEntries;
           sect_more[g] = load_vec_sys(reinterpret_cast<const uint8_t*>(&ctl->ring[(s_g + k_of_lane) & ring_mask]) + 16 * (lane & 3));
-          // (The upper lanes of the last group's load read the stamp of the entry kStormBacklog beyond the poll's 64.)
-          if (lane < 2 * kPollEntries || g == kDeepGroups - 1)
-            aux_more[g] = sys_load(lane < kPollEntries       ? &jobs_done[(s_g + lane) & ring_mask]
-                                   : lane < 2 * kPollEntries ? &job_target[(s_g + lane - kPollEntries) & ring_mask]
-                                                             : &ctl->ring[(s_g + kPollEntries + kStormBacklog - 1) & ring_mask].w[15]);
         }
       }
       // All of it waited for here: left to the places where it is used, which looks reach as well, the compiler would
       // wait there for what looks have under way.
       asm volatile("" : "+v"(sect), "+v"(aux));
 #pragma unroll
-      for (uint32_t g = 0; g < kDeepGroups; ++g) asm volatile("" : "+v"(sect_more[g]), "+v"(aux_more[g]));
+      for (uint32_t g = 0; g < kDeepGroups; ++g) asm volatile("" : "+v"(sect_more[g]));
     } else {
       // Ask for looks from s on until kLooks are under way, then wait for the oldest: a wavefront's vector memory
       // instructions complete in the order issued, and at least kLookLoads for each of the others (stores on top of them)
       // have been issued since its own.
-      const uint8_t* const carried_of_lane = reinterpret_cast<const uint8_t*>(&ctl->ring[ring_mask + 1u]) +
-                                             ((s + lane / kCarriedDescs) & ring_mask) * sizeof(CarriedList) + 16 * (lane % kCarriedDescs);
+      // Stays here for as long as looks show nothing or entries of one ticket each, few enough for looks.
+      const uint32_t list_of = lane / kCarriedDescs, list_at = lane % kCarriedDescs;  // the four lists, a descriptor to a lane
+      const uint8_t* const lists = reinterpret_cast<const uint8_t*>(&ctl->ring[ring_mask + 1u]) + 16 * list_at;
+      LdsLook* l;
+      bool all_taken;
 #pragma unroll 1
-      for (; under_way != kLooks; under_way = same_in_all_lanes32(under_way + 1u)) {
-        LdsLook* l = &looks[look];
-        if (lane == 0) l->base = static_cast<uint32_t>(s);
-        ask_for_look(l, aux_addr, carried_of_lane, sect_of_lane);
-        look = same_in_all_lanes32((look + 1u) % kLooks);
+      for (;;) {
+#pragma unroll 1
+        while (under_way != kLooks) {
+          ask_for_look(&looks[look], aux_addr, lists + ((s + list_of) & ring_mask) * sizeof(CarriedList), sect_of_lane);
+          look = same_in_all_lanes32((look + 1u) % kLooks);
+          asked_at = same_in_all_lanes64((asked_at << kAskedBits) | (s & kAskedMask));
+          under_way = same_in_all_lanes32(under_way + 1u);
+        }
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"((kLooks - 1) * kLookLoads) : "memory");
+        l = &looks[(look - under_way) % kLooks];
+        under_way = same_in_all_lanes32(under_way - 1u);
+        gone = same_in_all_lanes32(static_cast<uint32_t>(s - (asked_at >> (kAskedBits * under_way))) & kAskedMask);
+        // Entry s sits `gone` places from the front; what lies beyond the sixteen is not in this look.
+        u32x4 sc = *reinterpret_cast<lds_u32x4*>(l->sect[(lane + 4 * gone) % kWaveLanes]);
+        const uint32_t word = l->aux[lane];
+        u32x4 travels = *reinterpret_cast<lds_u32x4*>(l->carried[(lane + kCarriedDescs * gone) % kWaveLanes]);
+        const uint32_t list_count = l->sect[(4 * (list_of + gone) + 3) % kWaveLanes][1];
+        const uint32_t completed = lane_value(word, kAuxJobsCompleted);
+        const uint64_t there = __ballot(sc.w == static_cast<uint32_t>(s + k_of_lane + 1) && k_of_lane + gone < kPollEntries);
+        all_taken = false;
+        if ((there & 0xFull) != 0xFull) {  // entry s is not there
+          if (lane_value(word, kAuxHostStop) != 0) break;
+          if (completed == static_cast<uint32_t>(s)) nothing_under_way();
+          if (completed != static_cast<uint32_t>(mirrored)) {
+            mirrored = same_in_all_lanes64(mirrored + (completed - static_cast<uint32_t>(mirrored)));
+            if (lane == 0) sys_store_global(&ctl->completed, mirrored);
+            lanes_together();
+          }
+          idle = same_in_all_lanes32(idle + 1u);
+          if (idle >= idle_limit) break;
+          ++polls;
+          __builtin_amdgcn_s_sleep(kLookSleep);
+          continue;
+        }
+        // The leading entries of one ticket each (sized as ticket_size_for_submission does).
+        const uint32_t count = quad_value<3>(sc.y), n = count & kCountMask;
+        const uint32_t in_flight = static_cast<uint32_t>(s + k_of_lane + 1) - completed + following(count);
+        const uint32_t one_ticket = fixed_per_ticket != 0 ? fixed_per_ticket : in_flight >= kManyInFlight ? kSmallSubmission : kCarriedDescs;
+        const uint64_t singles = __ballot(n - 1u < one_ticket) & there;
+        auto leading = [](uint64_t m) {
+          const uint64_t not_whole = ~(m & (m >> 1) & (m >> 2) & (m >> 3)) & 0x1111111111111111ull;
+          return not_whole == 0 ? kPollEntries : static_cast<uint32_t>(__builtin_ctzll(not_whole)) >> 2;
+        };
+        const uint32_t ready = leading(there);
+        uint32_t run = same_in_all_lanes32(std::min(leading(singles), kTicketRing - (static_cast<uint32_t>(tickets_out) - tickets_done)));
+        if (run == 0) {
+          // One of several tickets, by itself, is handed out here too.
+          const uint32_t count_word = lane_value(sc.y, 3);
+          if (ready != 1 || (count_word & kCountMask) == 0) break;
+          const u32x4 own = *reinterpret_cast<lds_u32x4*>(l->sect[4 * gone + (lane & 3u)]);
+          if (!write_tickets(s, own, count_word, lane_value(sc.z, 3), lane_value(sc.z, 0), lane_value(word, gone), lane_value(word, kPollEntries + gone), completed, 0u, lane)) break;
+          run = 1;
+        } else {
+          // The lists that have arrived whole go beside the tickets; the others are fetched by their workgroups.  (A list left beside
+          // a ticket's place without the ticket would be taken for that of the one that comes there later.)
+          uint32_t bits = 0;
+          const uint64_t says_so = __ballot((count & kCarriedEntry) != 0);
+          if ((says_so & 0xFFFFull) != 0) {
+            const uint32_t list_n = list_count & kCountMask;
+            const uint64_t t = tickets_out + list_of;
+            const bool list_there = list_at >= list_n || travels.w == static_cast<uint32_t>(s + list_of + 1);
+            const bool goes = list_of < run && list_of + gone < kCarriedEntries && (list_count & kCarriedEntry) != 0 && list_n <= kCarriedDescs && static_cast<uint32_t>(t + 1) != 0;
+            const uint64_t arrived = __ballot(list_there && goes);
+            if (goes && list_at < list_n && ((arrived >> (kCarriedDescs * list_of)) & 0xFFFFull) == 0xFFFFull) {
+              travels.w = static_cast<uint32_t>(t + 1);
+              store_vec_sys(reinterpret_cast<uint8_t*>(&st->carried[t & (kTicketRing - 1)]) + 16 * list_at, travels);
+            }
+            lanes_together();
+            if (k_of_lane < kCarriedEntries && ((arrived >> (kCarriedDescs * k_of_lane)) & 0xFFFFull) == 0xFFFFull) bits = kCarriedTicket;
+          }
+          if (k_of_lane < run) {
+            const uint64_t t = tickets_out + k_of_lane;
+            sc.w = static_cast<uint32_t>(t + 1);
+            if ((lane & 3u) == 3) {
+              const uint32_t slot = static_cast<uint32_t>(s + k_of_lane) & ring_mask;
+              sc.y = n | (slot << 8) | kOnlyTicket | bits;
+              if (stamps) sys_store_global(&stamps[kStampsPerJob * slot], clock_now());
+            }
+            store_vec_sys(reinterpret_cast<uint8_t*>(&st->tickets[t & (kTicketRing - 1)]) + 16 * (lane & 3u), sc);
+          }
+          lanes_together();
+          tickets_out += run;
+          wide = 0;
+        }
+        all_taken = run == ready;
+        s = same_in_all_lanes64(s + run);
+        tickets_out = same_in_all_lanes64(tickets_out);
+        if (lane == 0) sys_store_global(&ctl->head, s);
+        lanes_together();
+        entries += run;
+        idle = 0;
+        ++polls;
+        gone += run;
+        deep = same_in_all_lanes32(ring_allows_deep && gone >= kPollEntries ? 1u : 0u);
+        direct = same_in_all_lanes32(deep != 0 || run >= kManySmall ? 1u : 0u);
+        if (!all_taken || direct != 0 || too_many_out()) break;
+        sect_of_lane = reinterpret_cast<const uint8_t*>(&ctl->ring[(s + k_of_lane) & ring_mask]) + 16 * (lane & 3);
+        if (lane < kPollEntries) aux_addr = (s + kPollEntries <= free_until ? job_target : jobs_done) + ((s + lane) & ring_mask);
+        else if (lane < 2 * kPollEntries) aux_addr = &job_target[(s + lane - kPollEntries) & ring_mask];
       }
-      asm volatile("s_waitcnt vmcnt(%0)" : : "n"((kLooks - 1) * kLookLoads) : "memory");
-      LdsLook* l = &looks[(look - under_way) % kLooks];
-      under_way = same_in_all_lanes32(under_way - 1u);
-      gone = static_cast<uint32_t>(s) - static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(l->base)));
-      // Entry s sits `gone` places from the front.  What lies beyond the sixteen is not in this look: its stamp is made
-      // one that it cannot have, below.
-      const uint32_t from = (lane + 4 * gone) & (kWaveLanes - 1), from_list = (lane + kCarriedDescs * gone) & (kWaveLanes - 1);
-      sect = *reinterpret_cast<lds_u32x4*>(l->sect[from]);
-      sect_more[0] = *reinterpret_cast<lds_u32x4*>(l->carried[from_list]);
+      if (all_taken) continue;  // (a poll into registers is next)
+      // What stopped the loop is for the rest of this pass, from entry s on.
+      sect = *reinterpret_cast<lds_u32x4*>(l->sect[(lane + 4 * gone) & (kWaveLanes - 1)]);
       aux = l->aux[lane < 2 * kPollEntries ? (lane & kPollEntries) | ((lane + gone) & (kPollEntries - 1)) : lane];
     }
     // (After the two ways have met: a choice per lane at the end of one of them would make the compiler take everything
@@ -645,7 +809,6 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     const uint32_t ready = missing != 0 ? static_cast<uint32_t>(__builtin_ctzll(missing)) >> 2 : kPollEntries;
     // The ticket size below which tickets are made 16 instead (see kLeaderBehind; 0: none are).
     const uint32_t too_small = ready >= kLeaderBehind ? kFullTicket : ready >= kLeaderBehindShallow ? kStreamTicket : 0u;
-    const uint32_t tickets_done = lane_value(aux, kAuxTicketsDone);
     const uint32_t jobs_completed = lane_value(aux, kAuxJobsCompleted);
     // Payload word i of entry k: component i % 3 of sector i / 3, held by lane 4k + i / 3.
     auto payload_of = [&](uint32_t first_lane, int i) {
@@ -660,9 +823,10 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     // each (it fetches an entry's words from their lanes into scalars first: about half a microsecond) capped a
     // stream of 1 MiB requests at 2 M/s and a storm of 64 KiB requests at 1.6 M/s.  Taken when the run has some
     // width: a lone entry of many tickets is written faster by the loop below, sixteen tickets to the instruction.
-    // (Not for a lone entry of more descriptors than a ticket holds, nor for a first entry of more than 32 tickets of
-    // the size its payload asks for -- 512 whole pages, up to 2048 short fragments: nothing here would apply to
-    // them, and what is worked out per lane first would only add to their latency.)
+    // (Not for a lone entry that a look shows, which its loop could not write either, nor for one of more descriptors than
+    // a ticket holds, nor for a first entry of more than 32 tickets of the size its payload asks for
+    // -- 512 whole pages, up to 2048 short fragments: nothing here would apply to them, and what is worked out per lane
+    // first would only add to their latency.)
     uint32_t consumed = 0;
     bool deep_next = false;
     const uint32_t n_first = lane_value(sect.y, 3) & kCountMask;
@@ -670,7 +834,6 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     auto view_entries = [&](const u32x4& sc, uint32_t ax, uint64_t s0, uint64_t okm) {
       EntryView v;
       v.n = bcast(sc.y, lane | 3u);      // payload word 10 sits in .y of sector 3
-      v.ticket_bits = v.n & kCarriedEntry;  // (made a ticket's below, or cleared)
       const uint32_t follow = following(v.n);
       const bool burst = (v.n & kBurstEntry) != 0;
       v.n &= kCountMask;
@@ -687,10 +850,10 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
       return v;
     };
     auto write_single_tickets = [&](const EntryView& v, const u32x4& sc, uint32_t room) {
-      return write_single_tickets_of_group(st, job_target, stamps, tickets_out, lane, v, sc, room);
+      return write_single_tickets_of_group(st, stamps, tickets_out, lane, v, sc, room);
     };
     if ((ok_mask & 0xFull) == 0xFull &&  // entry s is there
-        (n_first <= kMaxDescsPerTicket || (ready >= 2 && n_first <= lane_tickets_hold))) {
+        ((n_first <= kMaxDescsPerTicket && direct != 0) || (ready >= 2 && n_first <= lane_tickets_hold))) {
       EntryView ev = view_entries(sect, aux, s, ok_mask);
       const uint32_t n = ev.n, bytes = ev.bytes, per_ticket = ev.per_ticket, target_prev = ev.target_prev;
       const uint32_t in_flight = ev.in_flight, slot = ev.slot;
@@ -699,30 +862,6 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
       const uint32_t room = kTicketRing - (static_cast<uint32_t>(tickets_out) - tickets_done);
       const uint32_t sector = lane & 3u;
       if (__ballot(sane && n > per_ticket) == 0) {
-        const uint64_t says_so = __ballot(ev.ticket_bits != 0);
-        ev.ticket_bits = 0;
-        if (direct == 0 && (says_so & ((1ull << (4 * kCarriedEntries)) - 1ull)) != 0) {
-          // Of the entries that carry descriptors, those whose sectors have all arrived (the others' are fetched by
-          // their workgroups) and which become tickets now (a list left beside a ticket's place without the ticket
-          // would be taken for that of the one that comes there later).
-          static_assert(kCarriedEntries * kCarriedDescs == kWaveLanes, "a lane to a descriptor");
-          const uint32_t of = lane / kCarriedDescs, at = lane % kCarriedDescs;
-          const uint32_t count = bcast(n, 4 * of);
-          const uint64_t t = tickets_out + of;
-          const uint32_t stamp = static_cast<uint32_t>(t + 1);
-          const bool mine = at < count;
-          const uint32_t run = single_tickets_run(ev, room);  // (all lanes ask)
-          u32x4 carried = sect_more[0];
-          const uint64_t there = __ballot(!mine || carried.w == static_cast<uint32_t>(s + of + 1));
-          const bool whole_list = of + gone < kCarriedEntries && ((there >> (kCarriedDescs * of)) & 0xFFFFull) == 0xFFFFull && ((says_so >> (4 * of)) & 1u) != 0 &&
-                                  count <= kCarriedDescs && stamp != 0 && of < run;
-          if (whole_list && mine) {
-            carried.w = stamp;
-            store_vec_sys(reinterpret_cast<uint8_t*>(&st->carried[t & (kTicketRing - 1)]) + 16 * at, carried);
-          }
-          const uint64_t lists = __ballot(whole_list);
-          if (k_of_lane < kCarriedEntries && ((lists >> (kCarriedDescs * k_of_lane)) & 1u) != 0) ev.ticket_bits = kCarriedTicket;
-        }
         consumed = write_single_tickets(ev, sect, room);
         wide = 0;
         if (deep != 0 && consumed == kPollEntries) {
@@ -732,7 +871,6 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
           // compute unit.
           uint32_t left = room - consumed;
           u32x4 sc0 = sect_more[0], sc1 = sect_more[1], sc2 = sect_more[2];
-          uint32_t ax0 = aux_more[0], ax1 = aux_more[1], ax2 = aux_more[2];
           static_assert(kDeepGroups == 3, "the rotation below");
 #pragma unroll 1
           for (uint32_t g = 0; g < kDeepGroups; ++g) {
@@ -740,15 +878,13 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
             const uint64_t okm = __ballot(sc0.w == static_cast<uint32_t>(s_g + k_of_lane + 1));
             uint32_t run = 0;
             if ((okm & 0xFull) == 0xFull) {
-              EntryView more = view_entries(sc0, ax0, s_g, okm);
-              more.ticket_bits = 0;
+              const EntryView more = view_entries(sc0, aux, s_g, okm);  // (whose job slots single tickets do not ask about)
               if (__ballot(more.sane && more.n > more.per_ticket) == 0) run = write_single_tickets(more, sc0, left);
             }
             consumed += run;
             left -= run;
             if (run != kPollEntries) break;
             sc0 = sc1, sc1 = sc2;
-            ax0 = ax1, ax1 = ax2;
           }
         }
         deep_next = ring_allows_deep && consumed + gone >= kPollEntries;  // everything that the look could show was there
@@ -757,7 +893,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
         // far the host has got is read off the ring itself: the host's tail word is a line that the host writes with
         // every publish, and a poll that reads it as well waits half a microsecond longer for it.
         storm_next = ring_allows_storm && consumed == (kDeepGroups + 1) * kPollEntries &&
-                     lane_value(aux_more[kDeepGroups - 1], kAuxProbe) == static_cast<uint32_t>(s + (kDeepGroups + 1) * kPollEntries + kStormBacklog);
+                     lane_value(aux, kAuxProbe) == static_cast<uint32_t>(s + (kDeepGroups + 1) * kPollEntries + kStormBacklog);
       } else if (ready >= 2 && n_first <= kLaneTickets * lane_value(per_ticket, 0)) {
         // Several entries, some of more than one ticket, the first of them not too many.  (The empty statement keeps
         // the compiler from working this block's division and lane exchanges out ahead of the branch, where every
@@ -765,7 +901,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
         uint32_t n_here = n, per_here = per_ticket;
         asm volatile("" : "+v"(n_here), "+v"(per_here));
         const uint32_t nt = sane ? tickets_for(n_here, per_here) : 0u;
-        const bool regular = sane && nt <= kLaneTickets && slot_free;
+        const bool regular = sane && nt <= kLaneTickets && (slot_free || nt == 1);
         const uint64_t irregular = ~__ballot(regular);
         const uint32_t run_regular = irregular == 0 ? kPollEntries : static_cast<uint32_t>(__builtin_ctzll(irregular)) >> 2;
         // Tickets of the entries before this one and up to this one (the four lanes of an entry hold the same values).
@@ -783,7 +919,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
         // Taken when the run has some width (`most` is over the regular run, which the room may have cut: an upper
         // bound, good enough for the choice): a lone entry of many tickets is written faster by the loop below.
         if (run != 0 && total >= 2 * same_in_all_lanes32(most)) {
-          const uint32_t target = target_prev + nt;
+          const uint32_t target = nt == 1 ? target_prev : target_prev + nt;
           const bool across = shares_across_tickets(in_flight, n, bytes, bcast(sect.z, lane & ~3u));  // dst_lo: .z of sector 0
           const uint64_t first_ticket = tickets_out + (upto - mine);
           const bool takes_part = k_of_lane < run;
@@ -833,73 +969,9 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
         }
         lanes_together();
       } else {
-        // Submissions not yet completed, this one and those on their way included, taken to be as long as this one.
-        const uint32_t in_flight = static_cast<uint32_t>(s + k) - jobs_completed + 1u + following(count_word);
-        uint32_t per_ticket = fixed_per_ticket != 0
-                                  ? fixed_per_ticket
-                                  : ticket_size_for_submission(in_flight, n, payload_of(fl, 11), workers, (count_word & kBurstEntry) != 0);
-        // Small tickets spread a small backlog over many workgroups, at the price of more tickets to write.  When
-        // submissions queue up at the leader, its time per submission is what limits the engine, not the spread:
-        // a stream of 1 MiB requests of 256 whole pages, 64 in flight, is served at 1.44 M/s in tickets of 8 (which
-        // the backlog alone asks for: the workers empty it as fast as it comes), at 1.96 M/s in tickets of 16, and at
-        // 1.64 M/s with this rule, which holds for part of the time.
-        if (fixed_per_ticket == 0 && per_ticket < too_small) per_ticket = kFullTicket;
-        const uint32_t nt = tickets_for(n, per_ticket);
-        const uint32_t slot = static_cast<uint32_t>(s + k) & ring_mask;
-        const uint32_t done_now = lane_value(aux, k);
-        const uint32_t target_prev = lane_value(aux, kPollEntries + k);
-        // The job slot is free once every ticket ever issued for it has been counted; the ticket ring has room
-        // while fewer than its size are outstanding (32-bit wrapping arithmetic).  Otherwise leave this entry
-        // for a later poll.
-        if (done_now != target_prev) break;
-        if (static_cast<uint32_t>(tickets_out) + nt - tickets_done > kTicketRing) break;
-        const uint32_t target = target_prev + nt;
-        if (lane == 0) {
-          sys_store(&job_target[slot], target);
-          if (stamps) sys_store(&stamps[kStampsPerJob * slot], clock_now());
-        }
-        // Four neighbouring lanes write the four sectors of one ticket, so that one store instruction of the
-        // wavefront fills 16 consecutive tickets (1 KiB of whole lines).  A ticket's sector differs from the entry's
-        // in two places only, so every lane fetches the entry's sector of its own kind from the lane that holds it
-        // (three lane exchanges, where fetching the twelve words one by one into scalars took twelve).
-        // What changes from one pass to the next is kept running, per lane, instead of being worked out from the
-        // ticket's index each time (the leader spends three quarters of its time on a stream of 4 MiB requests in
-        // this loop and the lines before it).
-        const uint32_t sector = lane & 3u;
-        const uint32_t first = lane >> 2;
-        constexpr uint32_t kPerPass = kWaveLanes / 4;
-        // (asked in this order: a request that is alone pays for nothing but the first comparison)
-        const bool across = in_flight >= kManyInFlight && shares_across_tickets(in_flight, n, payload_of(fl, 11), payload_of(fl, 2));
-        const uint32_t holder = fl + sector;
-        u32x4 v{bcast(sect.x, holder), bcast(sect.y, holder), bcast(sect.z, holder), 0u};
-        const uint64_t descs = (static_cast<uint64_t>(v.z) << 32) | v.y;  // in the lanes of sector 1: dst_hi, descs
-        if (sector == 3) v.z = target;                                     // in the lanes of sector 3: val_hi, n, bytes
-        uint64_t d = descs + static_cast<uint64_t>(first) * per_ticket * sizeof(tcpxuLoadMeta);
-        const uint64_t d_step = static_cast<uint64_t>(kPerPass) * per_ticket * sizeof(tcpxuLoadMeta);
-        uint32_t left = n - first * per_ticket;  // descriptors from this lane's ticket on (meaningless beyond nt)
-        uint32_t at = static_cast<uint32_t>(tickets_out) + first;  // low word of the ticket number
-        uint8_t* const ring = reinterpret_cast<uint8_t*>(st->tickets) + 16 * sector;
-        // The ticket's own word: count | job slot | whether the submission has tickets before and after this one
-        // (the last ticket is the one that takes all that is left).
-        const uint32_t across_bits = across ? kMoreBefore | kMoreAfter : 0u;
-        const uint32_t fixed_bits = (slot << 8) | (nt == 1 ? kOnlyTicket : 0u), after_bit = across_bits & kMoreAfter;
-        uint32_t before_bit = first != 0 ? across_bits & kMoreBefore : 0u;
-        for (uint32_t i = first; i < nt; i += kPerPass) {
-          v.w = at + 1u;  // the stamp
-          if (sector == 1) {
-            v.y = static_cast<uint32_t>(d);
-            v.z = static_cast<uint32_t>(d >> 32);
-          }
-          if (sector == 3) v.y = std::min(per_ticket, left) | fixed_bits | (left > per_ticket ? after_bit : 0u) | before_bit;
-          before_bit = across_bits & kMoreBefore;  // every ticket but the submission's first
-          store_vec_sys(ring + static_cast<size_t>(at & (kTicketRing - 1)) * sizeof(Record), v);
-          d += d_step;
-          left -= kPerPass * per_ticket;
-          at += kPerPass;
-        }
-        lanes_together();
-        tickets_out += nt;
-        wide = nt > 1 && following(count_word) == 0 ? 1u : 0u;
+        const uint32_t holder = fl + (lane & 3u);
+        const u32x4 v{bcast(sect.x, holder), bcast(sect.y, holder), bcast(sect.z, holder), 0u};
+        if (!write_tickets(s + k, v, count_word, payload_of(fl, 11), payload_of(fl, 2), lane_value(aux, k), lane_value(aux, kPollEntries + k), jobs_completed, too_small, lane)) break;
       }
       ++consumed;
     }
@@ -941,8 +1013,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
       if (lane == 0) sys_store(&ctl->completed, mirrored);
       lanes_together();
     }
-    // (spin_limit counts polls that ask when the last is done, one in 1.75 us; looks are gone through every 0.97)
-    if (spin_limit != kNeverIdleOut && nothing_there && 5 * ++idle > 9 * static_cast<uint64_t>(spin_limit)) {
+    if (spin_limit != kNeverIdleOut && nothing_there && ++idle > idle_limit) {
       // Idle for long enough: leave, so that a device-wide synchronize by anybody returns.  The host relaunches
       // the kernel with its next submission.  A submission must not fall between "the leader stopped looking"
       // and "the host thinks the kernel is running": the leader announces that it is leaving, then looks once
@@ -1152,10 +1223,9 @@ __device__ void retire_ticket(DevState* st, uint32_t* jobs_done, const LdsStage*
     const uint64_t done_value = (static_cast<uint64_t>(stage->payload[9]) << 32) | stage->payload[8];
     if ((stage->payload[10] & kOnlyTicket) != 0) {
       // The submission's only ticket completes it: tell the caller first, count afterwards (nobody waits for the
-      // counts' round trips; the leader reads them when it wants the job slot again).
+      // counts' round trips).  Its job slot has nothing to count.
       if (stamps) sys_store(&stamps[kStampsPerJob * job + 3], clock_now());
       sys_store(reinterpret_cast<uint64_t*>(done_flag), done_value);
-      __hip_atomic_fetch_add(&jobs_done[job], 1u, __ATOMIC_RELAXED, SYS);
       __hip_atomic_fetch_add(&st->tickets_done.value, 1ull, __ATOMIC_RELAXED, SYS);
       __hip_atomic_fetch_add(&st->jobs_completed.value, 1ull, __ATOMIC_RELAXED, SYS);
       return;
