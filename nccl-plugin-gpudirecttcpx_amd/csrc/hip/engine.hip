@@ -1486,6 +1486,7 @@ struct tcpxuEngine {
   uint32_t* jobs_done = nullptr;   // [ring_entries], device memory
   uint32_t* job_target = nullptr;  // [ring_entries], device memory, leader-private
   uint64_t tail = 0;  // host copy
+  uint64_t head_seen = 0;  // the leader's position as last read
   bool launched = false;  // between a launch and the Stop that reaps it (the kernel may have left by itself)
   bool failed = false;    // the kernel stopped answering (see tcpxuEngineSubmitSized); nothing more is accepted
   uint64_t launches = 0;
@@ -1607,7 +1608,7 @@ int tcpxuEngineCreate(int device, const tcpxuEngineConfig* config, tcpxuEngine**
           break;
         }
       }
-      e->tail = from;
+      e->tail = e->head_seen = from;
       e->ctl->tail = e->ctl->head = e->ctl->completed = from;
     }
   } while (false);
@@ -1768,7 +1769,12 @@ int tcpxuEngineSubmitMany(tcpxuEngine* e, const tcpxuSubmission* subs, uint32_t 
     set_error("the engine stopped answering earlier and accepts nothing more");
     return TCPXU_INTERNAL_ERROR;
   }
-  const uint64_t head = reinterpret_cast<std::atomic<uint64_t>*>(&e->ctl->head)->load(std::memory_order_acquire);
+  // (The leader writes its position into the host's memory with all that it takes, and a line that the GPU has written costs a
+  // call a trip to DRAM.  What fits between the last position read and kCarryBehind entries on fits the smallest ring, and the
+  // leader is no further behind than that.  Requests of 1 / 4 / 8 / 16 pages through the plugin, 16 posted at a time, us a
+  // request: 0.413 / 0.59 / 0.428 / 0.468 with a look in every call, 0.394 / 0.53 / 0.404 / 0.444 with one in sixteen.)
+  uint64_t head = e->head_seen;
+  if (e->tail + n - head > kCarryBehind) head = e->head_seen = host_load(&e->ctl->head);
   const uint64_t room = e->ring_entries - (e->tail - head);
   const uint32_t take = static_cast<uint32_t>(std::min<uint64_t>(room, n));
   if (take == 0) return kTcpxuInProgress;
