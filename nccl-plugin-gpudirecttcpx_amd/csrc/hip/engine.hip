@@ -67,8 +67,8 @@ constexpr uint32_t kPollEntries = 16;  // submission entries fetched per load in
 // is what capped a storm of one-ticket requests near 9 M/s.
 constexpr uint32_t kDeepGroups = 3;    // groups of kPollEntries beyond the first in a deep poll
 constexpr uint32_t kStormBacklog = 128;  // entries published beyond a poll's 64 from which the leader takes them in a rolling loop
-constexpr uint32_t kAuxHostStop = 33, kAuxJobsCompleted = 34;  // lanes of the auxiliary load
-constexpr uint32_t kAuxProbe = 35;  // and in a deep poll, the stamp of an entry ahead
+// Lanes of the auxiliary load, among those that read nothing of an entry's own (see leader_loop).
+constexpr uint32_t kAuxHostStop = 2, kAuxJobsCompleted = 6, kAuxProbe = 10;
 constexpr uint32_t kNeverIdleOut = 0xFFFFFFFFu;
 constexpr uint32_t kDefaultIdlePolls = 400;  // empty polls (of 1.75 us) before the kernel leaves by itself
 constexpr int kTcpxuInProgress = TCPXU_IN_PROGRESS;
@@ -324,6 +324,13 @@ template <int q>
 __device__ __forceinline__ uint32_t quad_value(uint32_t v) {
   static_assert(q >= 0 && q < 4, "a lane of the quad");
   return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), q * 0x55, 0xF, 0xF, false));
+}
+
+// The value `lanes` lanes below in the same row of sixteen, 0 where there is none.
+template <int lanes>
+__device__ __forceinline__ uint32_t row_shift(uint32_t v) {
+  static_assert(lanes > 0 && lanes < 16, "within a row");
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x110 + lanes, 0xF, 0xF, true));
 }
 
 __device__ __forceinline__ uint32_t same_in_all_lanes32(uint32_t v) {
@@ -613,10 +620,11 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
   const bool ring_allows_deep = ring_mask + 1u >= (kDeepGroups + 1) * kPollEntries;
   const bool ring_allows_storm = ring_mask + 1u >= 2 * ((kDeepGroups + 1) * kPollEntries + kStormBacklog);
   // Fixed per-lane roles in the auxiliary load (second load of every poll), so that both loads of a poll are
-  // issued back to back by all lanes and waited for once:
-  //   lanes 0-15  jobs_done of the job slots of entries s..s+15    lanes 16-31  job_target of the same slots
-  //   lane 33     low word of the host stop word                   lane 34      low word of jobs_completed
-  //   other lanes repeat lane 33 (in a deep poll lane 35 reads the stamp of an entry ahead).
+  // issued back to back by all lanes and waited for once.  What is known of an entry's job slot is in two of the four lanes that
+  // hold its sectors, where the other two get at it with one move:
+  //   lane 4k     jobs_done of the job slot of entry s+k           lane 4k+1    job_target of the same slot
+  //   lane 2      low word of the host stop word                   lane 6       low word of jobs_completed
+  //   lane 10     in a deep poll, the stamp of an entry ahead      other lanes repeat lane 2.
   const uint32_t* const host_stop_lo = reinterpret_cast<const uint32_t*>(&ctl->stop);
   const uint32_t* const jobs_completed_lo = reinterpret_cast<const uint32_t*>(&st->jobs_completed.value);
 
@@ -652,8 +660,12 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     const uint32_t k_of_lane = lane >> 2;
     const uint8_t* sect_of_lane = reinterpret_cast<const uint8_t*>(&ctl->ring[(s + k_of_lane) & ring_mask]) + 16 * (lane & 3);
     const uint32_t* aux_addr = host_stop_lo;
-    if (lane < kPollEntries) aux_addr = (s + kPollEntries <= free_until ? job_target : jobs_done) + ((s + lane) & ring_mask);
-    else if (lane < 2 * kPollEntries) aux_addr = &job_target[(s + lane - kPollEntries) & ring_mask];
+    const uint32_t kind = lane & 3u;
+    auto job_slot_word = [&](uint64_t s0) {  // of the lanes that read one, for the sixteen entries from s0 on
+      // (the slots' targets follow their counts in memory)
+      return jobs_done + (((static_cast<uint32_t>(s0) + k_of_lane) & ring_mask) + (kind == 1 || s0 + kPollEntries <= free_until ? ring_mask + 1u : 0u));
+    };
+    if (kind < 2) aux_addr = job_slot_word(s);
     else if (lane == kAuxJobsCompleted) aux_addr = jobs_completed_lo;
     u32x4 sect;
     uint32_t aux;
@@ -662,6 +674,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     u32x4 sect_more[kDeepGroups];
 #pragma unroll
     for (uint32_t g = 0; g < kDeepGroups; ++g) sect_more[g] = u32x4{0u, 0u, 0u, 0u};
+    uint32_t aux_more[kDeepGroups] = {};
     if (direct != 0) {
       under_way = 0;  // (what has been asked for lands in LDS and is not looked at)
       sect = load_vec_sys(sect_of_lane);
@@ -673,13 +686,14 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
         for (uint32_t g = 0; g < kDeepGroups; ++g) {
           const uint64_t s_g = s + (g + 1) * kPollEntries;
           sect_more[g] = load_vec_sys(reinterpret_cast<const uint8_t*>(&ctl->ring[(s_g + k_of_lane) & ring_mask]) + 16 * (lane & 3));
+          aux_more[g] = sys_load(job_slot_word(s_g));
         }
       }
       // All of it waited for here: left to the places where it is used, which looks reach as well, the compiler would
       // wait there for what looks have under way.
       asm volatile("" : "+v"(sect), "+v"(aux));
 #pragma unroll
-      for (uint32_t g = 0; g < kDeepGroups; ++g) asm volatile("" : "+v"(sect_more[g]));
+      for (uint32_t g = 0; g < kDeepGroups; ++g) asm volatile("" : "+v"(sect_more[g]), "+v"(aux_more[g]));
     } else {
       // Ask for looks from s on until kLooks are under way, then wait for the oldest: a wavefront's vector memory
       // instructions complete in the order issued, and at least kLookLoads for each of the others (stores on top of them)
@@ -740,7 +754,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
           const uint32_t count_word = lane_value(sc.y, 3);
           if (ready != 1 || (count_word & kCountMask) == 0) break;
           const u32x4 own = *reinterpret_cast<lds_u32x4*>(l->sect[4 * gone + (lane & 3u)]);
-          if (!write_tickets(s, own, count_word, lane_value(sc.z, 3), lane_value(sc.z, 0), lane_value(word, gone), lane_value(word, kPollEntries + gone), completed, 0u, lane)) break;
+          if (!write_tickets(s, own, count_word, lane_value(sc.z, 3), lane_value(sc.z, 0), lane_value(word, 4 * gone), lane_value(word, 4 * gone + 1), completed, 0u, lane)) break;
           run = 1;
         } else {
           // The lists that have arrived whole go beside the tickets; the others are fetched by their workgroups.  (A list left beside
@@ -787,13 +801,12 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
         direct = same_in_all_lanes32(deep != 0 || run >= kManySmall ? 1u : 0u);
         if (!all_taken || direct != 0 || too_many_out()) break;
         sect_of_lane = reinterpret_cast<const uint8_t*>(&ctl->ring[(s + k_of_lane) & ring_mask]) + 16 * (lane & 3);
-        if (lane < kPollEntries) aux_addr = (s + kPollEntries <= free_until ? job_target : jobs_done) + ((s + lane) & ring_mask);
-        else if (lane < 2 * kPollEntries) aux_addr = &job_target[(s + lane - kPollEntries) & ring_mask];
+        if (kind < 2) aux_addr = job_slot_word(s);
       }
       if (all_taken) continue;  // (a poll into registers is next)
       // What stopped the loop is for the rest of this pass, from entry s on.
       sect = *reinterpret_cast<lds_u32x4*>(l->sect[(lane + 4 * gone) & (kWaveLanes - 1)]);
-      aux = l->aux[lane < 2 * kPollEntries ? (lane & kPollEntries) | ((lane + gone) & (kPollEntries - 1)) : lane];
+      aux = l->aux[kind < 2 ? (lane + 4 * gone) & (kWaveLanes - 1) : lane];
     }
     // (After the two ways have met: a choice per lane at the end of one of them would make the compiler take everything
     // that differs between them for different from lane to lane.)
@@ -833,19 +846,18 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     const uint32_t lane_tickets_hold = kLaneTickets * (fixed_per_ticket != 0 ? fixed_per_ticket : full_ticket_size(lane_value(sect.z, 3), n_first));
     auto view_entries = [&](const u32x4& sc, uint32_t ax, uint64_t s0, uint64_t okm) {
       EntryView v;
-      v.n = bcast(sc.y, lane | 3u);      // payload word 10 sits in .y of sector 3
+      v.n = quad_value<3>(sc.y);      // payload word 10 sits in .y of sector 3
       const uint32_t follow = following(v.n);
       const bool burst = (v.n & kBurstEntry) != 0;
       v.n &= kCountMask;
-      v.bytes = bcast(sc.z, lane | 3u);  // payload word 11 sits in .z of sector 3
+      v.bytes = quad_value<3>(sc.z);  // payload word 11 sits in .z of sector 3
       const bool all_sectors = ((okm >> (4 * k_of_lane)) & 0xFull) == 0xFull;
-      const uint32_t done_now = bcast(ax, k_of_lane);
-      v.target_prev = bcast(ax, kPollEntries + k_of_lane);
+      v.target_prev = quad_value<1>(ax);
       v.in_flight = static_cast<uint32_t>(s0 + k_of_lane) - jobs_completed + 1u + follow;
       v.per_ticket = fixed_per_ticket != 0 ? fixed_per_ticket : ticket_size_for_submission(v.in_flight, v.n, v.bytes, workers, burst);
       if (fixed_per_ticket == 0 && v.per_ticket < too_small) v.per_ticket = kFullTicket;  // see below
       v.sane = all_sectors && v.n - 1u < kMaxDescsPerSubmission;  // 1 .. 2^20 descriptors
-      v.slot_free = done_now == v.target_prev;  // every ticket ever issued for the job slot has been counted
+      v.slot_free = quad_value<0>(ax) == v.target_prev;  // every ticket ever issued for the job slot has been counted
       v.slot = static_cast<uint32_t>(s0 + k_of_lane) & ring_mask;
       return v;
     };
@@ -854,105 +866,110 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     };
     if ((ok_mask & 0xFull) == 0xFull &&  // entry s is there
         ((n_first <= kMaxDescsPerTicket && direct != 0) || (ready >= 2 && n_first <= lane_tickets_hold))) {
-      EntryView ev = view_entries(sect, aux, s, ok_mask);
-      const uint32_t n = ev.n, bytes = ev.bytes, per_ticket = ev.per_ticket, target_prev = ev.target_prev;
-      const uint32_t in_flight = ev.in_flight, slot = ev.slot;
-      const bool sane = ev.sane, slot_free = ev.slot_free;
-      // The ticket ring has room while fewer than its size are outstanding (32-bit wrapping arithmetic).
-      const uint32_t room = kTicketRing - (static_cast<uint32_t>(tickets_out) - tickets_done);
-      const uint32_t sector = lane & 3u;
-      if (__ballot(sane && n > per_ticket) == 0) {
-        consumed = write_single_tickets(ev, sect, room);
-        wide = 0;
-        if (deep != 0 && consumed == kPollEntries) {
-          // The groups that rode along, in order, each as long as the one before it went through whole.  One loop
-          // body that the groups pass through in turn (the registers rotate), so that the three are not worked out
-          // side by side in three times the registers: the kernel must stay within 80 for two workgroups per
-          // compute unit.
-          uint32_t left = room - consumed;
-          u32x4 sc0 = sect_more[0], sc1 = sect_more[1], sc2 = sect_more[2];
-          static_assert(kDeepGroups == 3, "the rotation below");
+      // The groups of sixteen in order (one, or the four of a deep poll), each as long as the one before it went through whole.
+      // One loop body that the groups pass through in turn (the registers rotate), so that they are not worked out side by side
+      // in as many times the registers: the kernel must stay within 80 for two workgroups per compute unit.
+      // (Entries of several tickets go by 64 a round trip as well as those of one, and what an entry's four lanes need of each
+      // other and of the entries before theirs they get with moves, not by trips through the LDS.  Calls of many requests of a
+      // few tickets each wait for nothing but this, us before / now: 96 MiB of ragged fragments in requests of 200 KiB 109 / 72, 256 MiB
+      // in 512 KiB 139 / 113, 128 MiB of pages in 300 KiB 96 / 64.5, 100 in 260 87.5 / 58.5, 16 in 260 21.8 / 18.5; with the moves and
+      // sixteen a round trip 103, 134, 91.)
+      u32x4 sc = sect, sc1 = sect_more[0], sc2 = sect_more[1], sc3 = sect_more[2];
+      uint32_t ax = aux, ax1 = aux_more[0], ax2 = aux_more[1], ax3 = aux_more[2];
+      static_assert(kDeepGroups == 3, "the rotation below");
+      uint32_t groups = deep != 0 ? kDeepGroups + 1 : 1, several = 0;
+      // The first of no more descriptors than one ticket holds: if hundreds more wait, the rolling loop makes one ticket of each
+      // such entry (asked once in a while, after sixteen of several tickets).
+      const bool may_be_one_each = n_first <= kMaxDescsPerTicket && ring_allows_storm && storm_backoff == 0;
 #pragma unroll 1
-          for (uint32_t g = 0; g < kDeepGroups; ++g) {
-            const uint64_t s_g = s + consumed;
-            const uint64_t okm = __ballot(sc0.w == static_cast<uint32_t>(s_g + k_of_lane + 1));
-            uint32_t run = 0;
-            if ((okm & 0xFull) == 0xFull) {
-              const EntryView more = view_entries(sc0, aux, s_g, okm);  // (whose job slots single tickets do not ask about)
-              if (__ballot(more.sane && more.n > more.per_ticket) == 0) run = write_single_tickets(more, sc0, left);
+      for (;;) {
+        const uint64_t s_g = s + consumed;
+        const uint64_t okm = __ballot(sc.w == static_cast<uint32_t>(s_g + k_of_lane + 1));
+        if ((okm & 0xFull) != 0xFull) break;
+        const EntryView ev = view_entries(sc, ax, s_g, okm);
+        uint32_t run = 0;
+        const uint32_t n = ev.n, bytes = ev.bytes, per_ticket = ev.per_ticket, target_prev = ev.target_prev;
+        const uint32_t in_flight = ev.in_flight, slot = ev.slot;
+        const bool sane = ev.sane, slot_free = ev.slot_free;
+        // The ticket ring has room while fewer than its size are outstanding (32-bit wrapping arithmetic).
+        const uint32_t room = kTicketRing - (static_cast<uint32_t>(tickets_out) - tickets_done);
+        const uint32_t sector = lane & 3u;
+        if (__ballot(sane && n > per_ticket) == 0) {
+          run = write_single_tickets(ev, sc, room);
+          wide = 0;
+        } else if (ready >= 2 && lane_value(n, 0) <= kLaneTickets * lane_value(per_ticket, 0)) {
+          // Several entries, some of more than one ticket, the first of them not too many.  (The empty statement keeps
+          // the compiler from working this block's division and lane exchanges out ahead of the branch, where every
+          // poll would pay for them.)
+          uint32_t n_here = n, per_here = per_ticket;
+          asm volatile("" : "+v"(n_here), "+v"(per_here));
+          const uint32_t nt = sane ? tickets_for(n_here, per_here) : 0u;
+          const bool regular = sane && nt <= kLaneTickets && (slot_free || nt == 1);
+          const uint64_t irregular = ~__ballot(regular);
+          const uint32_t run_regular = irregular == 0 ? kPollEntries : static_cast<uint32_t>(__builtin_ctzll(irregular)) >> 2;
+          // Tickets of the entries before this one and up to this one (the four lanes of an entry hold the same values).
+          const uint32_t mine = k_of_lane < run_regular ? nt : 0u;
+          uint32_t upto = mine, most = mine;  // (moves along a row of sixteen lanes, then what the rows before add)
+          upto += row_shift<4>(upto);
+          upto += row_shift<8>(upto);
+          most = std::max(most, row_shift<4>(most));
+          most = std::max(most, row_shift<8>(most));
+          const uint32_t rows[3] = {lane_value(upto, 15), lane_value(upto, 31), lane_value(upto, 47)};
+          upto += (lane >= 16 ? rows[0] : 0u) + (lane >= 32 ? rows[1] : 0u) + (lane >= 48 ? rows[2] : 0u);
+          most = std::max(std::max(lane_value(most, 15), lane_value(most, 31)), std::max(lane_value(most, 47), lane_value(most, 63)));
+          const uint64_t no_room = ~__ballot(k_of_lane < run_regular && upto <= room);
+          const uint32_t fit = no_room == 0 ? kPollEntries : static_cast<uint32_t>(__builtin_ctzll(no_room)) >> 2;
+          const uint32_t total = fit != 0 ? lane_value(upto, 4 * fit - 4) : 0u;
+          // Taken when the run has some width (`most` is over the regular run, which the room may have cut: an upper
+          // bound, good enough for the choice): a lone entry of many tickets is written faster by the loop below.
+          if (fit != 0 && total >= 2 * most) {
+            const uint32_t target = nt == 1 ? target_prev : target_prev + nt;
+            const bool across = shares_across_tickets(in_flight, n, bytes, quad_value<0>(sc.z));  // dst_lo: .z of sector 0
+            const uint64_t first_ticket = tickets_out + (upto - mine);
+            const bool takes_part = k_of_lane < fit;
+            for (uint32_t i = 0; __ballot(takes_part && i < nt) != 0; ++i) {
+              if (takes_part && i < nt) {
+                const uint64_t t = first_ticket + i;
+                const uint32_t stamp = static_cast<uint32_t>(t + 1);
+                u32x4 v{sc.x, sc.y, sc.z, stamp};
+                if (sector == 1) {  // dst_hi, then where this ticket's descriptors start
+                  const uint64_t d = ((static_cast<uint64_t>(sc.z) << 32) | sc.y) +
+                                     static_cast<uint64_t>(i) * per_ticket * sizeof(tcpxuLoadMeta);
+                  v.y = static_cast<uint32_t>(d);
+                  v.z = static_cast<uint32_t>(d >> 32);
+                }
+                if (sector == 3) {  // val_hi, then the ticket's own words
+                  v.y = std::min(per_ticket, n - i * per_ticket) | (slot << 8) | neighbour_bits(i, nt, across);
+                  v.z = target;
+                }
+                store_vec_sys(reinterpret_cast<uint8_t*>(&st->tickets[t & (kTicketRing - 1)]) + 16 * sector, v);
+              }
             }
-            consumed += run;
-            left -= run;
-            if (run != kPollEntries) break;
-            sc0 = sc1, sc1 = sc2;
+            if (takes_part && sector == 3) {
+              sys_store(&job_target[slot], target);
+              if (stamps) sys_store(&stamps[kStampsPerJob * slot], clock_now());
+            }
+            tickets_out += static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(total)));
+            run = same_in_all_lanes32(fit);
+            several = 1;
+            wide = following(lane_value(sc.y, 4 * run - 1)) == 0 ? 1u : 0u;
           }
         }
-        deep_next = ring_allows_deep && consumed + gone >= kPollEntries;  // everything that the look could show was there
-        // All 64 entries of a deep poll became tickets and the entry kStormBacklog beyond them is published (entries
-        // are published in order, so everything up to it is there): a storm, taken from the top of the next pass.  How
-        // far the host has got is read off the ring itself: the host's tail word is a line that the host writes with
-        // every publish, and a poll that reads it as well waits half a microsecond longer for it.
+        consumed = same_in_all_lanes32(consumed + run);
+        if (several != 0 && may_be_one_each) break;
+        if (run != kPollEntries || --groups == 0) break;
+        sc = sc1, sc1 = sc2, sc2 = sc3;
+        ax = ax1, ax1 = ax2, ax2 = ax3;
+      }
+      deep_next = ring_allows_deep && consumed + gone >= kPollEntries;  // everything that the look could show was there
+      // All 64 entries of a deep poll became tickets and the entry kStormBacklog beyond them is published (entries
+      // are published in order, so everything up to it is there): a storm, taken from the top of the next pass.  How
+      // far the host has got is read off the ring itself: the host's tail word is a line that the host writes with
+      // every publish, and a poll that reads it as well waits half a microsecond longer for it.
+      if (several != 0) storm_next = may_be_one_each && consumed >= kPollEntries;
+      else
         storm_next = ring_allows_storm && consumed == (kDeepGroups + 1) * kPollEntries &&
                      lane_value(aux, kAuxProbe) == static_cast<uint32_t>(s + (kDeepGroups + 1) * kPollEntries + kStormBacklog);
-      } else if (ready >= 2 && n_first <= kLaneTickets * lane_value(per_ticket, 0)) {
-        // Several entries, some of more than one ticket, the first of them not too many.  (The empty statement keeps
-        // the compiler from working this block's division and lane exchanges out ahead of the branch, where every
-        // poll would pay for them.)
-        uint32_t n_here = n, per_here = per_ticket;
-        asm volatile("" : "+v"(n_here), "+v"(per_here));
-        const uint32_t nt = sane ? tickets_for(n_here, per_here) : 0u;
-        const bool regular = sane && nt <= kLaneTickets && (slot_free || nt == 1);
-        const uint64_t irregular = ~__ballot(regular);
-        const uint32_t run_regular = irregular == 0 ? kPollEntries : static_cast<uint32_t>(__builtin_ctzll(irregular)) >> 2;
-        // Tickets of the entries before this one and up to this one (the four lanes of an entry hold the same values).
-        const uint32_t mine = k_of_lane < run_regular ? nt : 0u;
-        uint32_t upto = mine, most = mine;
-#pragma unroll
-        for (uint32_t d = 4; d < kWaveLanes; d <<= 1) {
-          const uint32_t below = static_cast<uint32_t>(__shfl_up(static_cast<int>(upto), d, kWaveLanes));
-          if (lane >= d) upto += below;
-          most = std::max(most, static_cast<uint32_t>(__shfl_xor(static_cast<int>(most), static_cast<int>(d), kWaveLanes)));
-        }
-        const uint64_t no_room = ~__ballot(k_of_lane < run_regular && upto <= room);
-        const uint32_t run = no_room == 0 ? kPollEntries : static_cast<uint32_t>(__builtin_ctzll(no_room)) >> 2;
-        const uint32_t total = run != 0 ? lane_value(upto, 4 * run - 4) : 0u;
-        // Taken when the run has some width (`most` is over the regular run, which the room may have cut: an upper
-        // bound, good enough for the choice): a lone entry of many tickets is written faster by the loop below.
-        if (run != 0 && total >= 2 * same_in_all_lanes32(most)) {
-          const uint32_t target = nt == 1 ? target_prev : target_prev + nt;
-          const bool across = shares_across_tickets(in_flight, n, bytes, bcast(sect.z, lane & ~3u));  // dst_lo: .z of sector 0
-          const uint64_t first_ticket = tickets_out + (upto - mine);
-          const bool takes_part = k_of_lane < run;
-          for (uint32_t i = 0; __ballot(takes_part && i < nt) != 0; ++i) {
-            if (takes_part && i < nt) {
-              const uint64_t t = first_ticket + i;
-              const uint32_t stamp = static_cast<uint32_t>(t + 1);
-              u32x4 v{sect.x, sect.y, sect.z, stamp};
-              if (sector == 1) {  // dst_hi, then where this ticket's descriptors start
-                const uint64_t d = ((static_cast<uint64_t>(sect.z) << 32) | sect.y) +
-                                   static_cast<uint64_t>(i) * per_ticket * sizeof(tcpxuLoadMeta);
-                v.y = static_cast<uint32_t>(d);
-                v.z = static_cast<uint32_t>(d >> 32);
-              }
-              if (sector == 3) {  // val_hi, then the ticket's own words
-                v.y = std::min(per_ticket, n - i * per_ticket) | (slot << 8) | neighbour_bits(i, nt, across);
-                v.z = target;
-              }
-              store_vec_sys(reinterpret_cast<uint8_t*>(&st->tickets[t & (kTicketRing - 1)]) + 16 * sector, v);
-            }
-          }
-          if (takes_part && sector == 3) {
-            sys_store(&job_target[slot], target);
-            if (stamps) sys_store(&stamps[kStampsPerJob * slot], clock_now());
-          }
-          tickets_out += static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(total)));
-          consumed = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(run)));
-          wide = following(lane_value(sect.y, 4 * consumed - 1)) == 0 ? 1u : 0u;
-          // Sixteen entries of a few tickets each, the first of them of no more descriptors than one ticket holds: if
-          // hundreds more wait, the rolling loop makes one ticket of each such entry (asked once in a while).
-          storm_next = consumed == kPollEntries && n_first <= kMaxDescsPerTicket && ring_allows_storm && storm_backoff == 0;
-        }
-      }
     }
 #pragma unroll 1
     for (uint32_t k = consumed; k < kPollEntries; ++k) {
@@ -971,7 +988,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
       } else {
         const uint32_t holder = fl + (lane & 3u);
         const u32x4 v{bcast(sect.x, holder), bcast(sect.y, holder), bcast(sect.z, holder), 0u};
-        if (!write_tickets(s + k, v, count_word, payload_of(fl, 11), payload_of(fl, 2), lane_value(aux, k), lane_value(aux, kPollEntries + k), jobs_completed, too_small, lane)) break;
+        if (!write_tickets(s + k, v, count_word, payload_of(fl, 11), payload_of(fl, 2), lane_value(aux, 4 * k), lane_value(aux, 4 * k + 1), jobs_completed, too_small, lane)) break;
       }
       ++consumed;
     }
