@@ -222,7 +222,7 @@ __device__ __forceinline__ uint64_t bcast64(uint64_t v, uint32_t src_lane) {
 // What bounds a lone request here is how soon a look shows it and how soon it is a ticket then, and both are instructions of a
 // single wavefront: a pass of the leader's whole loop takes 0.95 us, and while every look cost one, looks came round no sooner
 // than that, however many were under way.  Hence a loop of their own that does the least: a look that shows nothing costs it
-// 0.25 us, entries of one ticket each, wherever their descriptors lie, and an entry of several by itself are written there and
+// 0.25 us, entries of one ticket each, wherever their descriptors lie, and entries of several, if few wait, are written there and
 // then, and anything else leaves it.  Nor does a look read what the workgroups count in, beyond the count of completed
 // submissions: their counting waits for it (see nothing_under_way).  (Us, before / now, buffers in turn: a request of 64 KiB of
 // pages 8.30 / 7.70, through the plugin 7.35 / 6.88, 2048 of them through the plugin, 16 posted at a time, 1030 / 930; sixteen
@@ -245,6 +245,11 @@ static_assert(kLooks * kAskedBits <= 64, "leader_loop keeps them in one register
 static_assert(kCarriedEntries * kCarriedDescs == kWaveLanes, "a lane to a descriptor");
 constexpr int kLookSleep = 2;  // in 64 clocks; 0 to 4 measured alike
 constexpr uint32_t kLookLoads = 3;  // vector memory instructions of a look
+// Entries in a look up to which those of several tickets are handed out one after the other where they are looked at.  From
+// kLeaderBehindShallow on the leader counts as behind, and that is for its ordinary way.  (With 1 / 2 / 3 / 5 here: two ragged requests
+// of 1 and 0.7 MB in one call 12.3 / 11.7 / 11.7 / 11.6 us, 12.1 before looks had a loop; a hundred of 200 KB through the plugin,
+// 4 posted at a time, 209 / 207 / 205 / 205; six of 280 KB 12.0 / 12.2 / 12.2 / 12.4.)
+constexpr uint32_t kFewReady = kLeaderBehindShallow - 1;
 constexpr uint32_t kManyAtOnce = 3, kManySmall = 6;  // see where they are used
 #define TCPXU_LDS __attribute__((address_space(3)))
 typedef TCPXU_LDS Look LdsLook;
@@ -698,24 +703,27 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
       // Ask for looks from s on until kLooks are under way, then wait for the oldest: a wavefront's vector memory
       // instructions complete in the order issued, and at least kLookLoads for each of the others (stores on top of them)
       // have been issued since its own.
-      // Stays here for as long as looks show nothing or entries of one ticket each, few enough for looks.
+      // Stays here for as long as looks show nothing, entries of one ticket each, few enough for looks, or few of any kind.
       const uint32_t list_of = lane / kCarriedDescs, list_at = lane % kCarriedDescs;  // the four lists, a descriptor to a lane
       const uint8_t* const lists = reinterpret_cast<const uint8_t*>(&ctl->ring[ring_mask + 1u]) + 16 * list_at;
-      LdsLook* l;
+      LdsLook* l = nullptr;
       bool all_taken;
+      uint32_t again = 0;  // the look that was gone through last has more to show
 #pragma unroll 1
       for (;;) {
+        if (again == 0) {
 #pragma unroll 1
-        while (under_way != kLooks) {
-          ask_for_look(&looks[look], aux_addr, lists + ((s + list_of) & ring_mask) * sizeof(CarriedList), sect_of_lane);
-          look = same_in_all_lanes32((look + 1u) % kLooks);
-          asked_at = same_in_all_lanes64((asked_at << kAskedBits) | (s & kAskedMask));
-          under_way = same_in_all_lanes32(under_way + 1u);
+          while (under_way != kLooks) {
+            ask_for_look(&looks[look], aux_addr, lists + ((s + list_of) & ring_mask) * sizeof(CarriedList), sect_of_lane);
+            look = same_in_all_lanes32((look + 1u) % kLooks);
+            asked_at = same_in_all_lanes64((asked_at << kAskedBits) | (s & kAskedMask));
+            under_way = same_in_all_lanes32(under_way + 1u);
+          }
+          asm volatile("s_waitcnt vmcnt(%0)" : : "n"((kLooks - 1) * kLookLoads) : "memory");
+          l = &looks[(look - under_way) % kLooks];
+          under_way = same_in_all_lanes32(under_way - 1u);
+          gone = same_in_all_lanes32(static_cast<uint32_t>(s - (asked_at >> (kAskedBits * under_way))) & kAskedMask);
         }
-        asm volatile("s_waitcnt vmcnt(%0)" : : "n"((kLooks - 1) * kLookLoads) : "memory");
-        l = &looks[(look - under_way) % kLooks];
-        under_way = same_in_all_lanes32(under_way - 1u);
-        gone = same_in_all_lanes32(static_cast<uint32_t>(s - (asked_at >> (kAskedBits * under_way))) & kAskedMask);
         // Entry s sits `gone` places from the front; what lies beyond the sixteen is not in this look.
         u32x4 sc = *reinterpret_cast<lds_u32x4*>(l->sect[(lane + 4 * gone) % kWaveLanes]);
         const uint32_t word = l->aux[lane];
@@ -750,9 +758,9 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
         const uint32_t ready = leading(there);
         uint32_t run = same_in_all_lanes32(std::min(leading(singles), kTicketRing - (static_cast<uint32_t>(tickets_out) - tickets_done)));
         if (run == 0) {
-          // One of several tickets, by itself, is handed out here too.
+          // One of several tickets, by itself or among few, is handed out here too.
           const uint32_t count_word = lane_value(sc.y, 3);
-          if (ready != 1 || (count_word & kCountMask) == 0) break;
+          if (ready > kFewReady || (count_word & kCountMask) == 0) break;
           const u32x4 own = *reinterpret_cast<lds_u32x4*>(l->sect[4 * gone + (lane & 3u)]);
           if (!write_tickets(s, own, count_word, lane_value(sc.z, 3), lane_value(sc.z, 0), lane_value(word, 4 * gone), lane_value(word, 4 * gone + 1), completed, 0u, lane)) break;
           run = 1;
@@ -799,7 +807,8 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
         gone += run;
         deep = same_in_all_lanes32(ring_allows_deep && gone >= kPollEntries ? 1u : 0u);
         direct = same_in_all_lanes32(deep != 0 || run >= kManySmall ? 1u : 0u);
-        if (!all_taken || direct != 0 || too_many_out()) break;
+        if ((!all_taken && ready > kFewReady) || direct != 0 || too_many_out()) break;
+        again = all_taken ? 0u : 1u;
         sect_of_lane = reinterpret_cast<const uint8_t*>(&ctl->ring[(s + k_of_lane) & ring_mask]) + 16 * (lane & 3);
         if (kind < 2) aux_addr = job_slot_word(s);
       }
