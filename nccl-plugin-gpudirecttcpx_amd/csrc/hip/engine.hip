@@ -122,9 +122,6 @@ constexpr uint32_t kAskAfter = 4;
 struct alignas(64) CarriedList {
   uint32_t w[kCarriedDescs][4];
 };
-__host__ __device__ __forceinline__ uint32_t neighbour_bits(uint32_t i, uint32_t nt, bool across) {
-  return (nt == 1 ? kOnlyTicket : 0u) | (across && i != 0 ? kMoreBefore : 0u) | (across && i + 1 < nt ? kMoreAfter : 0u);
-}
 // Whether a submission's tickets share destination lines across their ends.  It saves two partial writes of a line
 // per ticket boundary and costs every ticket's pick-up two more descriptors to read and look at: worth it when the
 // engine is busy (8 MiB workload +0.3 points of the roofline, fragments of 1.8 KiB +0.4), not for a request that is
@@ -878,11 +875,11 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
       // The groups of sixteen in order (one, or the four of a deep poll), each as long as the one before it went through whole.
       // One loop body that the groups pass through in turn (the registers rotate), so that they are not worked out side by side
       // in as many times the registers: the kernel must stay within 80 for two workgroups per compute unit.
-      // (Entries of several tickets go by 64 a round trip as well as those of one, and what an entry's four lanes need of each
-      // other and of the entries before theirs they get with moves, not by trips through the LDS.  Calls of many requests of a
-      // few tickets each wait for nothing but this, us before / now: 96 MiB of ragged fragments in requests of 200 KiB 109 / 72, 256 MiB
-      // in 512 KiB 139 / 113, 128 MiB of pages in 300 KiB 96 / 64.5, 100 in 260 87.5 / 58.5, 16 in 260 21.8 / 18.5; with the moves and
-      // sixteen a round trip 103, 134, 91.)
+      // (Entries of several tickets go by 64 a round trip as well as those of one, what an entry's four lanes need of each other
+      // and of the entries before theirs they get with moves, not by trips through the LDS, and what changes from one ticket to
+      // the next is kept running.  Calls of many requests of a few tickets each wait for nothing but this, us before / now: 96 MiB
+      // of ragged fragments in requests of 200 KiB 109 / 66, 128 MiB of pages in 300 KiB 96 / 60.6, 100 in 260 87.5 / 53.8, 16 in 260
+      // 21.8 / 17.7; with the moves alone 103 and 91, with them and 64 a round trip 71.3, 64.1, 58.0 and 18.4.)
       u32x4 sc = sect, sc1 = sect_more[0], sc2 = sect_more[1], sc3 = sect_more[2];
       uint32_t ax = aux, ax1 = aux_more[0], ax2 = aux_more[1], ax3 = aux_more[2];
       static_assert(kDeepGroups == 3, "the rotation below");
@@ -934,25 +931,27 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
           if (fit != 0 && total >= 2 * most) {
             const uint32_t target = nt == 1 ? target_prev : target_prev + nt;
             const bool across = shares_across_tickets(in_flight, n, bytes, quad_value<0>(sc.z));  // dst_lo: .z of sector 0
-            const uint64_t first_ticket = tickets_out + (upto - mine);
             const bool takes_part = k_of_lane < fit;
-            for (uint32_t i = 0; __ballot(takes_part && i < nt) != 0; ++i) {
-              if (takes_part && i < nt) {
-                const uint64_t t = first_ticket + i;
-                const uint32_t stamp = static_cast<uint32_t>(t + 1);
-                u32x4 v{sc.x, sc.y, sc.z, stamp};
-                if (sector == 1) {  // dst_hi, then where this ticket's descriptors start
-                  const uint64_t d = ((static_cast<uint64_t>(sc.z) << 32) | sc.y) +
-                                     static_cast<uint64_t>(i) * per_ticket * sizeof(tcpxuLoadMeta);
+            const uint32_t nt_here = takes_part ? nt : 0u;
+            // What changes from one ticket to the next is kept running here too (see write_tickets).
+            u32x4 v{sc.x, sc.y, sector == 3 ? target : sc.z, 0u};  // in the lanes of sector 1: dst_hi, descs; of sector 3: val_hi, n, bytes
+            uint64_t d = (static_cast<uint64_t>(sc.z) << 32) | sc.y;
+            uint32_t left = n, at = static_cast<uint32_t>(tickets_out) + (upto - mine), before_bit = 0;
+            const uint32_t own_bits = (slot << 8) | (nt == 1 ? kOnlyTicket : 0u);
+            for (uint32_t i = 0; i < most; ++i) {
+              if (i < nt_here) {
+                v.w = at + 1u;  // the stamp
+                if (sector == 1) {
                   v.y = static_cast<uint32_t>(d);
                   v.z = static_cast<uint32_t>(d >> 32);
                 }
-                if (sector == 3) {  // val_hi, then the ticket's own words
-                  v.y = std::min(per_ticket, n - i * per_ticket) | (slot << 8) | neighbour_bits(i, nt, across);
-                  v.z = target;
-                }
-                store_vec_sys(reinterpret_cast<uint8_t*>(&st->tickets[t & (kTicketRing - 1)]) + 16 * sector, v);
+                if (sector == 3) v.y = std::min(per_ticket, left) | own_bits | (across && left > per_ticket ? kMoreAfter : 0u) | before_bit;
+                store_vec_sys(reinterpret_cast<uint8_t*>(&st->tickets[at & (kTicketRing - 1)]) + 16 * sector, v);
               }
+              before_bit = across ? kMoreBefore : 0u;
+              d += per_ticket * sizeof(tcpxuLoadMeta);
+              left -= per_ticket;
+              ++at;
             }
             if (takes_part && sector == 3) {
               sys_store(&job_target[slot], target);
