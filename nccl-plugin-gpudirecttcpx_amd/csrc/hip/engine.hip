@@ -28,7 +28,7 @@
 //
 // Liveness: no workgroup ever waits for another worker.  Workers wait only for the leader (their ticket) and
 // watch the stop word while they do; the leader waits for nothing (a full ticket ring or job table just defers
-// a submission to the next poll).  The host stop word, or the optional spin limit, ends the leader; the leader
+// a submission to a later poll, and the leader asks for what is done before that one).  The host stop word, or the optional spin limit, ends the leader; the leader
 // drains its stores, then sets the stop words; a worker that sees one looks at its ticket a last time and leaves.
 #include <hip/hip_runtime.h>
 
@@ -50,7 +50,6 @@
 namespace tcpxu {
 namespace {
 
-constexpr uint32_t kTicketRing = 1u << 16;  // tickets in flight at most
 constexpr uint32_t kMaxDescsPerSubmission = 1u << 20;
 constexpr uint32_t kSmallestAdaptiveTicket = 8;  // the least ticket_size_for_submission returns
 // The most descriptors one submission may carry: all its tickets must fit the ticket ring at once, or the leader
@@ -443,7 +442,7 @@ __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevS
     const uint64_t okm = __ballot(sc.w == static_cast<uint32_t>(s_g + k_of_lane + 1));
     uint32_t run = 0;
     if ((okm & 0xFull) == 0xFull) {
-      const uint32_t left = kTicketRing - (static_cast<uint32_t>(tickets_out) - tickets_done);
+      const uint32_t left = ticket_room(static_cast<uint32_t>(tickets_out), tickets_done);
       // With hundreds of submissions waiting, one of at most 32 descriptors is one ticket (see
       // ticket_size_for_submission; a fixed ticket size says so itself) -- and when the loop was armed with the entry
       // 16 x (kGroups + 1) ahead published, so is one of as many descriptors as a ticket holds: every workgroup has
@@ -538,8 +537,8 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
   // A word that workgroups count in is not one to look at all the time: reading it makes their counting wait (sixteen requests of
   // 4 MiB, looks every 0.75 us: 32.8 us with looks that read the finished tickets' count and the job slots', which share their
   // lines with those being counted in, 31.3 without; looks every 0.38 us 51 and 30.7).  So two facts are kept instead.
-  // The low word of the tickets known to be done: all of them when nothing is under way, otherwise asked for when the ticket
-  // ring may be half full.
+  // The low word of the tickets known to be done: all of them when nothing is under way, otherwise asked for as
+  // ask_what_is_done says.
   uint32_t tickets_done = static_cast<uint32_t>(tickets_out);
   // Entries below this one have job slots known to be free: what is counted there is then what has been issued.
   uint64_t free_until = s + ring_mask + 1u;
@@ -547,7 +546,8 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     tickets_done = static_cast<uint32_t>(tickets_out);
     free_until = s + ring_mask + 1u;
   };
-  auto too_many_out = [&]() { return static_cast<uint32_t>(tickets_out) - tickets_done > kTicketRing / 2; };
+  auto ask_done = [&]() { tickets_done = same_in_all_lanes32(static_cast<uint32_t>(sys_load(&st->tickets_done.value))); };
+  auto too_many_out = [&]() { return ask_what_is_done(static_cast<uint32_t>(tickets_out), tickets_done, false); };
   // The tickets of one submission of at least one descriptor, entry s_k, sixteen of them to a store instruction; false if they
   // cannot be written now.  `too_small`: see kLeaderBehind.
   auto write_tickets = [&](uint64_t s_k, u32x4 v, uint32_t count_word, uint32_t bytes, uint32_t dst_lo, uint32_t done_now, uint32_t target_prev,
@@ -570,7 +570,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     // while fewer than its size are outstanding (32-bit wrapping arithmetic).  Otherwise leave this entry
     // for a later poll.
     if (done_now != target_prev && nt != 1) return false;
-    if (static_cast<uint32_t>(tickets_out) + nt - tickets_done > kTicketRing) return false;
+    if (nt > ticket_room(static_cast<uint32_t>(tickets_out), tickets_done)) return false;
     const uint32_t target = nt == 1 ? target_prev : target_prev + nt;
     if (lane == 0) {
       sys_store_global(&job_target[slot], target);
@@ -631,7 +631,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
   const uint32_t* const jobs_completed_lo = reinterpret_cast<const uint32_t*>(&st->jobs_completed.value);
 
   for (;;) {
-    if (too_many_out()) tickets_done = same_in_all_lanes32(static_cast<uint32_t>(sys_load(&st->tickets_done.value)));
+    if (too_many_out()) ask_done();
     // (Every 64 entries it takes count as one deep poll in this launch's figures.)
     if (storm_next) {
       storm_next = false;
@@ -753,7 +753,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
           return not_whole == 0 ? kPollEntries : static_cast<uint32_t>(__builtin_ctzll(not_whole)) >> 2;
         };
         const uint32_t ready = leading(there);
-        uint32_t run = same_in_all_lanes32(std::min(leading(singles), kTicketRing - (static_cast<uint32_t>(tickets_out) - tickets_done)));
+        uint32_t run = same_in_all_lanes32(std::min(leading(singles), ticket_room(static_cast<uint32_t>(tickets_out), tickets_done)));
         if (run == 0) {
           // One of several tickets, by itself or among few, is handed out here too.
           const uint32_t count_word = lane_value(sc.y, 3);
@@ -898,7 +898,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
         const uint32_t in_flight = ev.in_flight, slot = ev.slot;
         const bool sane = ev.sane, slot_free = ev.slot_free;
         // The ticket ring has room while fewer than its size are outstanding (32-bit wrapping arithmetic).
-        const uint32_t room = kTicketRing - (static_cast<uint32_t>(tickets_out) - tickets_done);
+        const uint32_t room = ticket_room(static_cast<uint32_t>(tickets_out), tickets_done);
         const uint32_t sector = lane & 3u;
         if (__ballot(sane && n > per_ticket) == 0) {
           run = write_single_tickets(ev, sc, room);
@@ -1021,6 +1021,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
 
     // Nothing could be consumed this round.
     const bool nothing_there = (ok_mask & 0xFull) != 0xFull;
+    if (ask_what_is_done(static_cast<uint32_t>(tickets_out), tickets_done, !nothing_there)) ask_done();
     if (lane_value(aux, kAuxHostStop) != 0 && nothing_there) {
       // Stop requested and entry s not there.  The host wrote its last tail before the stop word, so a tail
       // read now bounds what is still to come.

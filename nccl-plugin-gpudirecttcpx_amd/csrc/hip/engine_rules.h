@@ -145,6 +145,17 @@ TCPXU_RULE uint32_t ticket_size_for_submission(uint32_t in_flight, uint32_t n, u
   return backlog < kDeepBacklog * workers ? kStreamTicket : kFullTicket;
 }
 
+// Room in the ticket ring.  `out` and `known_done` are low words of running counts: of the tickets written, and of those that the
+// leader knows to be done, which may be fewer than are (it does not read that count with every look, see leader_loop).
+constexpr uint32_t kTicketRing = 1u << 16;  // tickets in flight at most
+TCPXU_RULE uint32_t ticket_room(uint32_t out, uint32_t known_done) { return kTicketRing - (out - known_done); }
+// Whether to ask how many are done: whenever an entry that is there could not be handed out, however few tickets are out (one
+// entry's may need the whole ring, and nothing else would ever tell the leader that the ring has emptied), and before that
+// once the ring may be half full, so that streams hardly ever come to wait.
+TCPXU_RULE bool ask_what_is_done(uint32_t out, uint32_t known_done, bool entry_waits) {
+  return entry_waits || out - known_done > kTicketRing / 2;
+}
+
 // The leader has its compute unit to itself.  Loads seem to return to a compute unit in the order in which it issued them,
 // so the looks at the host's ring and the copy's loads wait for each other where both are under way.  A worker workgroup
 // that finds itself there claims no ticket and leaves (its place then goes to the one workgroup of the grid that found

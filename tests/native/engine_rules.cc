@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <random>
+#include <vector>
 
 using namespace tcpxu;
 
@@ -35,8 +36,42 @@ static uint32_t size_of(uint64_t in_flight, uint64_t n, uint64_t bytes, uint64_t
   return full == 48 && n <= 1024 && per_worker < 100 ? 32 : full;
 }
 
+// The leader before submissions of so many tickets each (none of more than the ring holds), workgroups finishing some of what is
+// out between two of its passes: whether all of them are handed out, and never more tickets than the ring holds.  Entries are there
+// as `there` says; when the next is not and everything is done, the leader sees that, as its looks do.
+template <class There>
+static bool all_handed_out(const std::vector<uint32_t>& tickets, uint32_t from, std::mt19937_64& rng, There there) {
+  uint32_t out = from, done = from, known = from;
+  size_t s = 0;
+  for (int waited = 0; waited < 100;) {
+    if (ask_what_is_done(out, known, false)) known = done;
+    const size_t before = s;
+    bool here = false;
+    while (s < tickets.size() && (here = there(s)) && tickets[s] <= ticket_room(out, known)) {
+      out += tickets[s++];
+      if (out - done > kTicketRing) return false;
+    }
+    if (s == tickets.size()) return true;
+    if (s == before) {
+      if (ask_what_is_done(out, known, here)) known = done;
+      if (!here && done == out) known = out;
+    }
+    waited = s == before && done == out ? waited + 1 : 0;
+    done += rng() % 4 == 0 ? out - done : static_cast<uint32_t>(rng() % (out - done + 1u));
+  }
+  return false;
+}
+
 int main() {
   std::mt19937_64 rng(1);
+  const std::vector<std::vector<uint32_t>> lists = {{37500, 37500}, {1, kTicketRing}, {kTicketRing, kTicketRing, 1, kTicketRing}, {32768, 32769}, {32768, 32768, 32768}, {1, 65535, 2, 65534}};
+  for (const auto& list : lists)
+    for (const uint32_t from : {0u, 0u - 70000u, 0u - 3u}) CHECK(all_handed_out(list, from, rng, [](size_t) { return true; }));
+  for (int i = 0; i < 3000; ++i) {
+    std::vector<uint32_t> list(1 + rng() % 200);
+    for (uint32_t& t : list) t = 1 + static_cast<uint32_t>(rng() % (rng() % 3 ? 64 : kTicketRing));
+    CHECK(all_handed_out(list, static_cast<uint32_t>(rng()), rng, [&](size_t) { return rng() % 8 != 0; }));
+  }
   for (int i = 0; i < 2000000; ++i) {
     const uint32_t n = 1 + static_cast<uint32_t>(rng() % (rng() % 2 ? 3000 : 1u << 20)), in_flight = 1 + static_cast<uint32_t>(rng() % 300);
     const uint32_t workers = 1 + static_cast<uint32_t>(rng() % 1000);
