@@ -374,11 +374,13 @@ __device__ __forceinline__ T* same_in_all_lanes_ptr(T* p) {
 //
 // A function of its own, not inlined, and called from the top of the leader's loop where little is live: with this
 // loop inside the leader's, what the compiler did with the registers around it made every poll that never sees a
-// storm 0.2 us slower.  The running count of finished tickets is read once: too few counted as done only ends the
-// storm early (after at most kTicketRing entries, which is also how long the host's stop word can go unread).
+// storm 0.2 us slower.  The running count of finished tickets is read whenever the first groups are asked for: too few
+// counted as done only ends the storm early.  It goes back to the leader with the tickets written by it: an older count
+// would be of a ring that has been gone round since.
 struct StormEnd {
   uint64_t s, tickets_out;
-  uint32_t entries;  // taken off the ring
+  uint32_t entries;       // taken off the ring
+  uint32_t tickets_done;  // low word, as last read
 };
 __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevState* st_in, uint64_t* stamps_in, uint32_t ring_mask_in,
                                                           uint32_t fixed_per_ticket_in, uint64_t s_in, uint64_t tickets_out_in) {
@@ -506,7 +508,7 @@ __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevS
     // is for the ordinary loop.
     if (feeding != 0) break;
   }
-  return StormEnd{s, tickets_out, entries};
+  return StormEnd{s, tickets_out, entries, tickets_done};
 }
 
 __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uint32_t* job_target,
@@ -631,13 +633,13 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
   const uint32_t* const jobs_completed_lo = reinterpret_cast<const uint32_t*>(&st->jobs_completed.value);
 
   for (;;) {
-    if (too_many_out()) ask_done();
     // (Every 64 entries it takes count as one deep poll in this launch's figures.)
     if (storm_next) {
       storm_next = false;
       const StormEnd end = leader_storm(ctl, st, stamps, ring_mask, fixed_per_ticket, s, tickets_out);
       s = same_in_all_lanes(end.s);
       tickets_out = same_in_all_lanes(end.tickets_out);
+      tickets_done = same_in_all_lanes32(end.tickets_done);
       const uint32_t taken = same_in_all_lanes32(end.entries);
       entries += taken;
       polls += (taken + (kDeepGroups + 1) * kPollEntries - 1) / ((kDeepGroups + 1) * kPollEntries);
@@ -651,6 +653,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     } else if (storm_backoff != 0) {
       --storm_backoff;
     }
+    if (too_many_out()) ask_done();  // (after the rolling loop, which may have filled the ring)
     // What depends on the lane is worked out afresh in every pass (the empty statement hides from the compiler that
     // the lane is the same each time): a dozen per-lane addresses kept in registers for the life of the loop are
     // what would push the kernel beyond the 80 vector registers that let two workgroups share a compute unit, and a

@@ -38,15 +38,24 @@ static uint32_t size_of(uint64_t in_flight, uint64_t n, uint64_t bytes, uint64_t
 
 // The leader before submissions of so many tickets each (none of more than the ring holds), workgroups finishing some of what is
 // out between two of its passes: whether all of them are handed out, and never more tickets than the ring holds.  Entries are there
-// as `there` says; when the next is not and everything is done, the leader sees that, as its looks do.
+// as `there` says; when the next is not and everything is done, the leader sees that, as its looks do.  Now and then it takes those
+// of one ticket in its rolling loop, which has a count of its own while tickets go on being finished.
 template <class There>
 static bool all_handed_out(const std::vector<uint32_t>& tickets, uint32_t from, std::mt19937_64& rng, There there) {
   uint32_t out = from, done = from, known = from;
   size_t s = 0;
   for (int waited = 0; waited < 100;) {
-    if (ask_what_is_done(out, known, false)) known = done;
     const size_t before = s;
     bool here = false;
+    while (rng() % 4 == 0) {
+      known = done;
+      for (; s < tickets.size() && tickets[s] == 1 && there(s) && ticket_room(out, known) != 0; ++s) {
+        ++out;
+        if (rng() % 2 == 0 && done != out) ++done;
+      }
+      if (out - done > kTicketRing) return false;
+    }
+    if (ask_what_is_done(out, known, false)) known = done;
     while (s < tickets.size() && (here = there(s)) && tickets[s] <= ticket_room(out, known)) {
       out += tickets[s++];
       if (out - done > kTicketRing) return false;
@@ -63,13 +72,18 @@ static bool all_handed_out(const std::vector<uint32_t>& tickets, uint32_t from, 
 }
 
 int main() {
+  for (const uint32_t done : {0u, 5u, 0u - 3u, 0u - kTicketRing}) {
+    CHECK(ticket_room(done, done) == kTicketRing && ticket_room(done + 1, done) == kTicketRing - 1 && ticket_room(done + kTicketRing - 1, done) == 1);
+    for (const uint32_t more : {0u, 1u, 5000u, kTicketRing, 1u << 30}) CHECK(ticket_room(done + kTicketRing + more, done) == 0);
+  }
   std::mt19937_64 rng(1);
   const std::vector<std::vector<uint32_t>> lists = {{37500, 37500}, {1, kTicketRing}, {kTicketRing, kTicketRing, 1, kTicketRing}, {32768, 32769}, {32768, 32768, 32768}, {1, 65535, 2, 65534}};
   for (const auto& list : lists)
     for (const uint32_t from : {0u, 0u - 70000u, 0u - 3u}) CHECK(all_handed_out(list, from, rng, [](size_t) { return true; }));
   for (int i = 0; i < 3000; ++i) {
-    std::vector<uint32_t> list(1 + rng() % 200);
-    for (uint32_t& t : list) t = 1 + static_cast<uint32_t>(rng() % (rng() % 3 ? 64 : kTicketRing));
+    std::vector<uint32_t> list(i % 100 == 0 ? 300000 : 1 + rng() % 200, 1u);
+    for (uint32_t& t : list)
+      if (list.size() < 300000 || rng() % 1000 == 0) t = 1 + static_cast<uint32_t>(rng() % (rng() % 3 ? 64 : kTicketRing));
     CHECK(all_handed_out(list, static_cast<uint32_t>(rng()), rng, [&](size_t) { return rng() % 8 != 0; }));
   }
   for (int i = 0; i < 2000000; ++i) {
