@@ -380,10 +380,11 @@ __device__ __forceinline__ T* same_in_all_lanes_ptr(T* p) {
 struct StormEnd {
   uint64_t s, tickets_out;
   uint32_t entries;       // taken off the ring
-  uint32_t tickets_done;  // low word, as last read
+  uint32_t tickets_done;  // known to be done, low word
 };
 __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevState* st_in, uint64_t* stamps_in, uint32_t ring_mask_in,
-                                                          uint32_t fixed_per_ticket_in, uint64_t s_in, uint64_t tickets_out_in) {
+                                                          uint32_t fixed_per_ticket_in, uint64_t s_in, uint64_t tickets_out_in,
+                                                          uint32_t tickets_done_in) {
   // Arguments arrive in vector registers.  These are the same in every lane and go back to scalar registers.
   HostCtl* ctl = same_in_all_lanes_ptr(ctl_in);
   DevState* st = same_in_all_lanes_ptr(st_in);
@@ -392,6 +393,7 @@ __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevS
   const uint32_t fixed_per_ticket = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(fixed_per_ticket_in)));
   uint64_t s = same_in_all_lanes64(s_in);
   uint64_t tickets_out = same_in_all_lanes64(tickets_out_in);
+  uint32_t tickets_done = same_in_all_lanes32(tickets_done_in);
   const uint32_t lane = threadIdx.x;
   const uint32_t k_of_lane = lane >> 2;
   uint32_t consumed = 0, entries = 0;
@@ -417,18 +419,19 @@ __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevS
   // in flight that have not gone through: kGroups - 1, ..., 1, and at 0 the storm is over.
   uint32_t feeding = kGroups;
   u32x4 sc[kGroups];
-  uint32_t ax[kGroups], tickets_done;
+  uint32_t ax[kGroups];
   bool queue_deep = false;
   // The first groups, from s on, and the running count of finished tickets: one round trip, waited for whole.
   auto arm = [&]() {
     feeding = kGroups;
 #pragma unroll
     for (uint32_t g = 0; g < kGroups; ++g) fetch_group_untracked(sc[g], ax[g], s + g * kPollEntries);
-    asm volatile("global_load_dword %0, %1, off sc0 sc1" : "=v"(tickets_done) : "v"(reinterpret_cast<const uint32_t*>(&st->tickets_done.value)) : "memory");
-    asm volatile("s_waitcnt vmcnt(0)" : "+v"(tickets_done) : : "memory");
+    uint32_t counted;
+    asm volatile("global_load_dword %0, %1, off sc0 sc1" : "=v"(counted) : "v"(reinterpret_cast<const uint32_t*>(&st->tickets_done.value)) : "memory");
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(counted) : : "memory");
 #pragma unroll
     for (uint32_t g = 0; g < kGroups; ++g) asm volatile("" : "+v"(sc[g]), "+v"(ax[g]) : : "memory");
-    tickets_done = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(tickets_done)));
+    tickets_done = known_done_after(tickets_done, same_in_all_lanes32(counted));
     // The first group's probe: the 16 x (kGroups + 1) entries from s on are published, so the queue at the leader is deep.
     queue_deep = lane_value(ax[0], 2) == static_cast<uint32_t>(s + (kGroups + 1) * kPollEntries);
   };
@@ -544,11 +547,11 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
   uint32_t tickets_done = static_cast<uint32_t>(tickets_out);
   // Entries below this one have job slots known to be free: what is counted there is then what has been issued.
   uint64_t free_until = s + ring_mask + 1u;
-  auto nothing_under_way = [&]() {  // every submission before entry s is completed, and its tickets counted
+  auto nothing_under_way = [&]() {  // every submission before entry s is completed (see known_done_after)
     tickets_done = static_cast<uint32_t>(tickets_out);
     free_until = s + ring_mask + 1u;
   };
-  auto ask_done = [&]() { tickets_done = same_in_all_lanes32(static_cast<uint32_t>(sys_load(&st->tickets_done.value))); };
+  auto ask_done = [&]() { tickets_done = known_done_after(tickets_done, same_in_all_lanes32(static_cast<uint32_t>(sys_load(&st->tickets_done.value)))); };
   auto too_many_out = [&]() { return ask_what_is_done(static_cast<uint32_t>(tickets_out), tickets_done, false); };
   // The tickets of one submission of at least one descriptor, entry s_k, sixteen of them to a store instruction; false if they
   // cannot be written now.  `too_small`: see kLeaderBehind.
@@ -636,7 +639,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     // (Every 64 entries it takes count as one deep poll in this launch's figures.)
     if (storm_next) {
       storm_next = false;
-      const StormEnd end = leader_storm(ctl, st, stamps, ring_mask, fixed_per_ticket, s, tickets_out);
+      const StormEnd end = leader_storm(ctl, st, stamps, ring_mask, fixed_per_ticket, s, tickets_out, tickets_done);
       s = same_in_all_lanes(end.s);
       tickets_out = same_in_all_lanes(end.tickets_out);
       tickets_done = same_in_all_lanes32(end.tickets_done);

@@ -39,30 +39,37 @@ static uint32_t size_of(uint64_t in_flight, uint64_t n, uint64_t bytes, uint64_t
 // The leader before submissions of so many tickets each (none of more than the ring holds), workgroups finishing some of what is
 // out between two of its passes: whether all of them are handed out, and never more tickets than the ring holds.  Entries are there
 // as `there` says; when the next is not and everything is done, the leader sees that, as its looks do.  Now and then it takes those
-// of one ticket in its rolling loop, which has a count of its own while tickets go on being finished.
+// of one ticket in its rolling loop, which has a count of its own while tickets go on being finished.  The count that is read can
+// lag behind what is done by a few tickets, also where the leader has seen that all is done: what it knows never goes back.
 template <class There>
 static bool all_handed_out(const std::vector<uint32_t>& tickets, uint32_t from, std::mt19937_64& rng, There there) {
   uint32_t out = from, done = from, known = from;
   size_t s = 0;
+  auto ask = [&] {
+    const uint32_t lag = static_cast<uint32_t>(rng() % 3 ? 0 : std::min<uint64_t>(rng() % 600, done - from));
+    const uint32_t before = known;
+    known = known_done_after(known, done - lag);
+    return known - before <= kTicketRing && done - known <= kTicketRing;
+  };
   for (int waited = 0; waited < 100;) {
     const size_t before = s;
     bool here = false;
     while (rng() % 4 == 0) {
-      known = done;
+      if (!ask()) return false;
       for (; s < tickets.size() && tickets[s] == 1 && there(s) && ticket_room(out, known) != 0; ++s) {
         ++out;
         if (rng() % 2 == 0 && done != out) ++done;
       }
       if (out - done > kTicketRing) return false;
     }
-    if (ask_what_is_done(out, known, false)) known = done;
+    if (ask_what_is_done(out, known, false) && !ask()) return false;
     while (s < tickets.size() && (here = there(s)) && tickets[s] <= ticket_room(out, known)) {
       out += tickets[s++];
       if (out - done > kTicketRing) return false;
     }
     if (s == tickets.size()) return true;
     if (s == before) {
-      if (ask_what_is_done(out, known, here)) known = done;
+      if (ask_what_is_done(out, known, here) && !ask()) return false;
       if (!here && done == out) known = out;
     }
     waited = s == before && done == out ? waited + 1 : 0;
@@ -75,6 +82,10 @@ int main() {
   for (const uint32_t done : {0u, 5u, 0u - 3u, 0u - kTicketRing}) {
     CHECK(ticket_room(done, done) == kTicketRing && ticket_room(done + 1, done) == kTicketRing - 1 && ticket_room(done + kTicketRing - 1, done) == 1);
     for (const uint32_t more : {0u, 1u, 5000u, kTicketRing, 1u << 30}) CHECK(ticket_room(done + kTicketRing + more, done) == 0);
+  }
+  for (const uint32_t known : {0u, 70000u, 0u - 2u}) {
+    for (const uint32_t less : {0u, 1u, 600u, kTicketRing}) CHECK(known_done_after(known, known - less) == known);
+    for (const uint32_t more : {1u, 600u, kTicketRing}) CHECK(known_done_after(known, known + more) == known + more);
   }
   std::mt19937_64 rng(1);
   const std::vector<std::vector<uint32_t>> lists = {{37500, 37500}, {1, kTicketRing}, {kTicketRing, kTicketRing, 1, kTicketRing}, {32768, 32769}, {32768, 32768, 32768}, {1, 65535, 2, 65534}};
