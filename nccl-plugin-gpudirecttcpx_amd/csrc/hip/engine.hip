@@ -685,6 +685,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     uint32_t aux_more[kDeepGroups] = {};
     if (direct != 0) {
       under_way = 0;  // (what has been asked for lands in LDS and is not looked at)
+      ++polls;
       sect = load_vec_sys(sect_of_lane);
       if (deep != 0 && lane == kAuxProbe) aux_addr = &ctl->ring[(s + (kDeepGroups + 1) * kPollEntries + kStormBacklog - 1) & ring_mask].w[15];
       aux = sys_load(aux_addr);
@@ -725,6 +726,7 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
           asm volatile("s_waitcnt vmcnt(%0)" : : "n"((kLooks - 1) * kLookLoads) : "memory");
           l = &looks[(look - under_way) % kLooks];
           under_way = same_in_all_lanes32(under_way - 1u);
+          ++polls;  // (a look counts when it is gone through, once, whatever becomes of its entries)
           gone = same_in_all_lanes32(static_cast<uint32_t>(s - (asked_at >> (kAskedBits * under_way))) & kAskedMask);
         }
         // Entry s sits `gone` places from the front; what lies beyond the sixteen is not in this look.
@@ -745,7 +747,6 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
           }
           idle = same_in_all_lanes32(idle + 1u);
           if (idle >= idle_limit) break;
-          ++polls;
           __builtin_amdgcn_s_sleep(kLookSleep);
           continue;
         }
@@ -806,7 +807,6 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
         lanes_together();
         entries += run;
         idle = 0;
-        ++polls;
         gone += run;
         deep = same_in_all_lanes32(ring_allows_deep && gone >= kPollEntries ? 1u : 0u);
         direct = same_in_all_lanes32(deep != 0 || run >= kManySmall ? 1u : 0u);
@@ -823,7 +823,6 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     // (After the two ways have met: a choice per lane at the end of one of them would make the compiler take everything
     // that differs between them for different from lane to lane.)
     if (k_of_lane + gone >= kPollEntries) sect.w = static_cast<uint32_t>(s + k_of_lane);
-    ++polls;
 
     const uint32_t expect = static_cast<uint32_t>(s + k_of_lane + 1);
     const uint64_t ok_mask = __ballot(sect.w == expect);

@@ -2,9 +2,15 @@
 that are one ticket always and the 32 that are while eight submissions are in flight, empty ones and ones of several tickets
 among them, one at a time and several to a call, with tickets sized by backlog and of a fixed size.  And long runs of entries
 of several tickets, which are taken 64 at a time, broken at the ends of sixteen and elsewhere by one that is not like them."""
+import ctypes
+import time
+
+import numpy as np
 import pytest
 
 import test_engine_carried_gpu as carried
+from conftest import GpuBuffers, first_difference, make_descs, oracle_expected
+from test_engine_gpu import Engine, Mapped
 
 pytestmark = pytest.mark.gpu
 
@@ -27,3 +33,34 @@ def test_long_runs_of_entries_of_several_tickets(pkg, hip, oracle, monkeypatch, 
     monkeypatch.setattr(carried, "COUNTS", counts)
     for per_call in (160, 48):
         carried.small_lists(pkg, hip, oracle, "mapped", per_call, descs_per_ticket=per_ticket)
+
+
+@pytest.mark.parametrize("counts", [[5], [100], [100, 100, 100], [100, 0, 100], [1, 1, 100, 100, 100], [1, 100, 1, 100, 100, 1]])
+def test_a_poll_of_the_ring_counts_once_whatever_it_shows(pkg, hip, oracle, counts):
+    """Everything is queued before the start, so that the first poll shows all of it; then come as many polls that show nothing
+    as it takes the kernel to leave, 7/3 of the limit."""
+    first = np.cumsum(counts) - counts
+    n = sum(counts)
+    pool = np.random.default_rng(n).integers(0, 256, 1 << 20, dtype=np.uint8)
+    descs = make_descs([((4099 * i) % ((1 << 20) - 1000), 999, 1000 * i) for i in range(n)])
+    expect = oracle_expected(oracle, pool, descs, 1000 * n)
+    g = GpuBuffers(pool, descs, 1000 * n)
+    m = Mapped(pkg, hip, descs, len(counts))
+    e = Engine(pkg, hip, spin_limit=3)
+    for i in range(len(counts)):
+        e.submit(g.pool.data_ptr(), g.dst_base, m.desc_dev(int(first[i])), counts[i], m.flag_dev(i), i + 1)
+    e.start()
+    for i in range(len(counts)):
+        m.wait(i, i + 1)
+    deadline = time.time() + 20
+    while e.running():  # (a stop would end the polls sooner)
+        assert time.time() < deadline
+    e.stop()
+    stats = pkg.EngineStats()
+    pkg.check(hip.tcpxuEngineGetStats(e.h, ctypes.byref(stats)), "tcpxuEngineGetStats")
+    got = g.result()
+    e.destroy()
+    m.free()
+    assert first_difference(got, expect) is None, repr(first_difference(got, expect))
+    assert stats.launches == 1 and stats.leader_entries == len(counts) and stats.leader_deep_polls == 0
+    assert stats.leader_polls == 1 + 7 * 3 // 3
