@@ -112,6 +112,11 @@ __device__ __forceinline__ uint32_t following(uint32_t count_word) { return (cou
 constexpr uint32_t kCarriedTicket = 1u << 28;  // in a ticket's
 constexpr uint32_t kCarriedEntries = 4;        // entries of a poll whose descriptors it fetches as well: 64 lanes' worth
 constexpr uint32_t kCarryBehind = 16;          // entries the leader is behind from which the host carries no more
+// The least submission ring.  A look or poll brings kPollEntries entries, no two of which may share a place; and the host does not
+// read the leader's position while, by the one it knows, the leader is kCarryBehind entries behind at most: a ring shorter than
+// that could be full by the known position and not by the real one, and never be found otherwise.
+constexpr uint32_t kSmallestRing = 16;
+static_assert(kPollEntries <= kSmallestRing && kCarryBehind <= kSmallestRing, "what reads or writes the ring without asking");
 // Looks at a ticket that is not there yet after which its fetcher asks for a carried list as well.  Small requests on an
 // idle engine find fetchers that have waited long, and those are the ones whose descriptors are waited for; under load a
 // ticket is there at one of the first looks, and 256 bytes more with each of those cost streams of large requests, which
@@ -1539,8 +1544,8 @@ int tcpxuEngineCreate(int device, const tcpxuEngineConfig* config, tcpxuEngine**
   tcpxuEngineConfig cfg{};
   if (config) cfg = *config;
   if (cfg.ring_entries == 0) cfg.ring_entries = 4096;
-  if ((cfg.ring_entries & (cfg.ring_entries - 1)) != 0 || cfg.ring_entries > (1u << 16) || cfg.ring_entries < 16) {
-    set_error("ring_entries %u must be a power of two in [16, 65536]", cfg.ring_entries);
+  if ((cfg.ring_entries & (cfg.ring_entries - 1)) != 0 || cfg.ring_entries > (1u << 16) || cfg.ring_entries < kSmallestRing) {
+    set_error("ring_entries %u must be a power of two in [%u, 65536]", cfg.ring_entries, kSmallestRing);
     return TCPXU_INVALID_ARGUMENT;
   }
   if (cfg.descs_per_ticket == 0) {
