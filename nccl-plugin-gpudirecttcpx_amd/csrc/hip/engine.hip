@@ -459,10 +459,8 @@ __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevS
       // work anyway, and a ticket per entry is what lets the leader keep up (1024 requests of 33 whole pages in
       // flight: 5.8 -> 33 M requests/s).  No sizing here, and a group with a larger one ends the storm and goes the
       // ordinary way.
-      EntryView more;
+      EntryView more{};  // (write_single_tickets_of_group looks at nothing but what is set here)
       more.n = quad_value<3>(sc.y) & kCountMask;  // payload word 10 sits in .y of sector 3
-      more.bytes = 0, more.per_ticket = 0, more.in_flight = 0;  // (not looked at by write_single_tickets_of_group)
-      more.target_prev = 0, more.slot_free = true;
       more.sane = ((okm >> (4 * k_of_lane)) & 0xFull) == 0xFull && more.n - 1u < kMaxDescsPerSubmission;
       more.slot = static_cast<uint32_t>(s_g + k_of_lane) & ring_mask;
       const uint32_t one_ticket = fixed_per_ticket != 0 ? fixed_per_ticket : queue_deep ? kMaxDescsPerTicket : kSmallSubmission;
@@ -1620,7 +1618,7 @@ int tcpxuEngineCreate(int device, const tcpxuEngineConfig* config, tcpxuEngine**
       break;
     }
     e->jobs_done = reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(e->st) + sizeof(DevState));
-    e->job_target = e->jobs_done + cfg.ring_entries;  // (leader_storm works the second out from the first)
+    e->job_target = e->jobs_done + cfg.ring_entries;  // (leader_loop's job_slot_word finds the second by the first)
     // Test aid: where the engine's counts of submissions and tickets start.  Records are stamped with the low 32 bits
     // of their sequence number, and a busy engine passes 2^32 submissions within the hour; a test that starts just
     // below sees the crossing in milliseconds.  (Start more than a lap of the ticket ring below: a slot of either ring
