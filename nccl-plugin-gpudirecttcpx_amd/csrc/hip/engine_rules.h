@@ -148,9 +148,11 @@ TCPXU_RULE uint32_t ticket_size_for_submission(uint32_t in_flight, uint32_t n, u
 // Room in the ticket ring.  `out` and `known_done` are low words of running counts: of the tickets written, and of those that the
 // leader knows to be done, which may be fewer than are (it does not read that count with every look, see leader_loop).
 constexpr uint32_t kTicketRing = 1u << 16;  // tickets in flight at most
-// (None, and not four billion, where the two say that more are out than the ring holds.)
+// (None, and not four billion, where the two say that more are out than the ring holds.  A signed maximum is one scalar
+// instruction; a comparison of the two counts becomes a vector subtraction and a trip back, in every look that shows an entry.)
 TCPXU_RULE uint32_t ticket_room(uint32_t out, uint32_t known_done) {
-  return out - known_done < kTicketRing ? kTicketRing - (out - known_done) : 0u;
+  const int32_t room = static_cast<int32_t>(kTicketRing - (out - known_done));
+  return room > 0 ? static_cast<uint32_t>(room) : 0u;
 }
 // Whether to ask how many are done: whenever an entry that is there could not be handed out, however few tickets are out (one
 // entry's may need the whole ring, and nothing else would ever tell the leader that the ring has emptied), and before that
