@@ -66,6 +66,7 @@ constexpr uint32_t kPollEntries = 16;  // submission entries fetched per load in
 // is what capped a storm of one-ticket requests near 9 M/s.
 constexpr uint32_t kDeepGroups = 3;    // groups of kPollEntries beyond the first in a deep poll
 constexpr uint32_t kStormBacklog = 128;  // entries published beyond a poll's 64 from which the leader takes them in a rolling loop
+constexpr uint32_t kStormMost = 1u << 24;  // entries after which that loop returns all the same (see leader_storm)
 // Lanes of the auxiliary load, among those that read nothing of an entry's own (see leader_loop).
 constexpr uint32_t kAuxHostStop = 2, kAuxJobsCompleted = 6, kAuxProbe = 10;
 constexpr uint32_t kNeverIdleOut = 0xFFFFFFFFu;
@@ -380,16 +381,16 @@ __device__ __forceinline__ T* same_in_all_lanes_ptr(T* p) {
 // A function of its own, not inlined, and called from the top of the leader's loop where little is live: with this
 // loop inside the leader's, what the compiler did with the registers around it made every poll that never sees a
 // storm 0.2 us slower.  The running count of finished tickets is read whenever the first groups are asked for: too few
-// counted as done only ends the storm early.  It goes back to the leader with the tickets written by it: an older count
-// would be of a ring that has been gone round since.
+// counted as done only ends the storm early.  The leader, whose own count of them is of before the storm, asks again once
+// so many are out by that count that the ring may be half full -- which the counts' low words tell, since no storm goes on for
+// more than kStormMost entries.  (The loop's count handed back with the rest costs a lone request 0.04 us, 2.40 -> 2.44 from its
+// descriptors staged to its last store, in copy wavefronts whose instructions are the same and lie elsewhere.)
 struct StormEnd {
   uint64_t s, tickets_out;
-  uint32_t entries;       // taken off the ring
-  uint32_t tickets_done;  // known to be done, low word
+  uint32_t entries;  // taken off the ring
 };
 __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevState* st_in, uint64_t* stamps_in, uint32_t ring_mask_in,
-                                                          uint32_t fixed_per_ticket_in, uint64_t s_in, uint64_t tickets_out_in,
-                                                          uint32_t tickets_done_in) {
+                                                          uint32_t fixed_per_ticket_in, uint64_t s_in, uint64_t tickets_out_in) {
   // Arguments arrive in vector registers.  These are the same in every lane and go back to scalar registers.
   HostCtl* ctl = same_in_all_lanes_ptr(ctl_in);
   DevState* st = same_in_all_lanes_ptr(st_in);
@@ -398,7 +399,6 @@ __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevS
   const uint32_t fixed_per_ticket = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(fixed_per_ticket_in)));
   uint64_t s = same_in_all_lanes64(s_in);
   uint64_t tickets_out = same_in_all_lanes64(tickets_out_in);
-  uint32_t tickets_done = same_in_all_lanes32(tickets_done_in);
   const uint32_t lane = threadIdx.x;
   const uint32_t k_of_lane = lane >> 2;
   uint32_t consumed = 0, entries = 0;
@@ -424,19 +424,18 @@ __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevS
   // in flight that have not gone through: kGroups - 1, ..., 1, and at 0 the storm is over.
   uint32_t feeding = kGroups;
   u32x4 sc[kGroups];
-  uint32_t ax[kGroups];
+  uint32_t ax[kGroups], tickets_done;
   bool queue_deep = false;
   // The first groups, from s on, and the running count of finished tickets: one round trip, waited for whole.
   auto arm = [&]() {
     feeding = kGroups;
 #pragma unroll
     for (uint32_t g = 0; g < kGroups; ++g) fetch_group_untracked(sc[g], ax[g], s + g * kPollEntries);
-    uint32_t counted;
-    asm volatile("global_load_dword %0, %1, off sc0 sc1" : "=v"(counted) : "v"(reinterpret_cast<const uint32_t*>(&st->tickets_done.value)) : "memory");
-    asm volatile("s_waitcnt vmcnt(0)" : "+v"(counted) : : "memory");
+    asm volatile("global_load_dword %0, %1, off sc0 sc1" : "=v"(tickets_done) : "v"(reinterpret_cast<const uint32_t*>(&st->tickets_done.value)) : "memory");
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(tickets_done) : : "memory");
 #pragma unroll
     for (uint32_t g = 0; g < kGroups; ++g) asm volatile("" : "+v"(sc[g]), "+v"(ax[g]) : : "memory");
-    tickets_done = known_done_after(tickets_done, same_in_all_lanes32(counted));
+    tickets_done = same_in_all_lanes32(tickets_done);
     // The first group's probe: the 16 x (kGroups + 1) entries from s on are published, so the queue at the leader is deep.
     queue_deep = lane_value(ax[0], 2) == static_cast<uint32_t>(s + (kGroups + 1) * kPollEntries);
   };
@@ -512,9 +511,9 @@ __device__ __attribute__((noinline)) StormEnd leader_storm(HostCtl* ctl_in, DevS
     // leaving, waiting for the ordinary loop to find 64 entries and as many again beyond them, and coming back.
     // Anything else -- a group not there whole, entries of more than one ticket, no room in the ticket ring --
     // is for the ordinary loop.
-    if (feeding != 0) break;
+    if (feeding != 0 || entries >= kStormMost) break;
   }
-  return StormEnd{s, tickets_out, entries, tickets_done};
+  return StormEnd{s, tickets_out, entries};
 }
 
 __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uint32_t* job_target,
@@ -642,10 +641,9 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
     // (Every 64 entries it takes count as one deep poll in this launch's figures.)
     if (storm_next) {
       storm_next = false;
-      const StormEnd end = leader_storm(ctl, st, stamps, ring_mask, fixed_per_ticket, s, tickets_out, tickets_done);
+      const StormEnd end = leader_storm(ctl, st, stamps, ring_mask, fixed_per_ticket, s, tickets_out);
       s = same_in_all_lanes(end.s);
       tickets_out = same_in_all_lanes(end.tickets_out);
-      tickets_done = same_in_all_lanes32(end.tickets_done);
       const uint32_t taken = same_in_all_lanes32(end.entries);
       entries += taken;
       polls += (taken + (kDeepGroups + 1) * kPollEntries - 1) / ((kDeepGroups + 1) * kPollEntries);

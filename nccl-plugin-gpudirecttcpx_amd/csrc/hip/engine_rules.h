@@ -163,7 +163,7 @@ TCPXU_RULE bool ask_what_is_done(uint32_t out, uint32_t known_done, bool entry_w
 // What is known once the count has been read.  It can say less than is known already: a workgroup counts a ticket and, where that
 // is the submission's last, the submission with two additions to different lines and waits for neither, so that the leader can
 // see all submissions completed, and take all tickets for done, before the last tickets are counted.  They are done all the same.
-// (No more than a ring of tickets is written between two readings: a difference of half the range or more is a step back.)
+// (Far less than half the range is written between two readings: a difference of that or more is a step back.)
 TCPXU_RULE uint32_t known_done_after(uint32_t known_done, uint32_t counted) {
   return static_cast<int32_t>(counted - known_done) > 0 ? counted : known_done;
 }
