@@ -1164,26 +1164,45 @@ __device__ uint32_t try_fetch_ticket(DevState* st, const uint32_t* stop_word, ui
   const uint64_t bounce = word64(0), dst = word64(2), descs_addr = word64(4);
   // One 16-byte descriptor per lane straight from where the submission keeps them (system scope: never a cached
   // copy); lanes past the end repeat the last one and write no record.
-  const uint32_t mine = lane < n ? lane : (n != 0 ? n - 1u : 0u);  // a ticket has at least one descriptor
-  if (carried) d[3] = 0;  // (the stamp's place is the high word of the destination offset)
-  else d = load_vec_sys(reinterpret_cast<const uint8_t*>(descs_addr) + 16 * mine);
-  const uint32_t so = d[0], len = d[1];
-  const uint64_t doff = (static_cast<uint64_t>(d[3]) << 32) | d[2];
-  // The descriptor before the ticket's first and the one after its last, where the submission has them (lanes 0
-  // and 1, in the same round trip): the neighbouring tickets' fetchers look at the same pairs from the other side.
+  //
+  // The descriptor before the ticket's first and the one after its last come with them, where the submission has them (the
+  // neighbouring tickets' fetchers look at the same pairs from the other side): lane l then asks for descriptor l - 1, and one
+  // move along the lanes puts them where they are worked on.  What bounds the first tickets of a burst is the number of
+  // lines that all workers read over PCIe at once, 3.1 ns each where they are a line or two apart (2.3 in longer stretches):
+  // a ticket of 32 takes five, and seven while its neighbours were asked for by themselves.  (Us a call with lists in mapped
+  // memory, before / now: 64 MiB of ragged fragments 34.8 / 34.0, 256 MiB 107.5 / 107.1, 16 MiB of wire fragments in requests of
+  // 256 KiB 18.5 / 18.2; lists in the GPU's memory as before.  One load for both kinds of ticket: with a load each in two branches
+  // small requests, which have no such neighbours, take 1.5 to 3 % longer.)
   const bool more_before = (ticket_bits & kMoreBefore) != 0, more_after = (ticket_bits & kMoreAfter) != 0;
   uint32_t before_len = 0, before_dlo = 0, before_dhi = 0, after_so = 0, after_len = 0, after_dlo = 0, after_dhi = 0;
-  if (more_before || more_after) {  // wave-uniform: a ticket without such neighbours pays nothing here
-    u32x4 outer = {0u, 0u, 0u, 0u};
-    if ((lane == 0 && more_before) || (lane == 1 && more_after)) {
-      const uint64_t at = lane == 0 ? descs_addr - sizeof(tcpxuLoadMeta) : descs_addr + sizeof(tcpxuLoadMeta) * n;
-      outer = load_vec_sys(reinterpret_cast<const uint8_t*>(at));
+  const bool outward = more_before || more_after;
+  int mine = static_cast<int>(lane < n ? lane : n - 1u);  // a ticket has at least one descriptor
+  const int last = static_cast<int>(n) - (more_after ? 0 : 1);  // (of those that a ticket with neighbours asks for)
+  if (outward) mine = std::min(std::max(static_cast<int>(lane) - 1, more_before ? -1 : 0), last);
+  if (carried) d[3] = 0;  // (the stamp's place is the high word of the destination offset)
+  else d = load_vec_sys(reinterpret_cast<const uint8_t*>(descs_addr) + 16 * mine);
+  if (outward) {  // wave-uniform: a ticket without such neighbours pays nothing here
+    auto from_lane = [](uint32_t v, uint32_t src) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(src))); };
+    const u32x4 w = d;
+    u32x4 beyond = {0u, 0u, 0u, 0u};
+    if (n >= kWaveLanes - 1)
+      beyond = load_vec_sys(reinterpret_cast<const uint8_t*>(descs_addr) + 16 * std::min(static_cast<int>(lane) + kWaveLanes - 1, last));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int wrap = __builtin_amdgcn_readfirstlane(static_cast<int>(beyond[k]));
+      d[k] = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(wrap, static_cast<int>(w[k]), kDppWaveShiftLeft1, 0xF, 0xF, false));
     }
-    auto from_lane = [](uint32_t v, int src) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), src)); };
-    before_len = from_lane(outer[1], 0), before_dlo = from_lane(outer[2], 0), before_dhi = from_lane(outer[3], 0);
-    after_so = from_lane(outer[0], 1), after_len = from_lane(outer[1], 1);
-    after_dlo = from_lane(outer[2], 1), after_dhi = from_lane(outer[3], 1);
+    if (more_before) before_len = from_lane(w[1], 0), before_dlo = from_lane(w[2], 0), before_dhi = from_lane(w[3], 0);
+    if (more_after) {
+      const bool is_beyond = n >= kWaveLanes - 1;
+      const uint32_t at = is_beyond ? n - (kWaveLanes - 1) : n + 1;
+      const u32x4 after = is_beyond ? beyond : w;
+      after_so = from_lane(after[0], at), after_len = from_lane(after[1], at);
+      after_dlo = from_lane(after[2], at), after_dhi = from_lane(after[3], at);
+    }
   }
+  const uint32_t so = d[0], len = d[1];
+  const uint64_t doff = (static_cast<uint64_t>(d[3]) << 32) | d[2];
   const uint64_t fdst = dst + doff, fsrc = bounce + so;
   uint32_t kind = kRecRounds;
   FragmentPlan plan = {0, len, 0, 0, len >> 4};
