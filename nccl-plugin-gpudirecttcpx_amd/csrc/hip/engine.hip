@@ -211,10 +211,6 @@ __device__ __forceinline__ void drain_memory_ops() { asm volatile("s_waitcnt vmc
 __device__ __forceinline__ uint32_t bcast(uint32_t v, uint32_t src_lane) {
   return __shfl(v, static_cast<int>(src_lane), kWaveLanes);
 }
-__device__ __forceinline__ uint64_t bcast64(uint64_t v, uint32_t src_lane) {
-  return (static_cast<uint64_t>(bcast(static_cast<uint32_t>(v >> 32), src_lane)) << 32) |
-         bcast(static_cast<uint32_t>(v), src_lane);
-}
 // ---- looks at the ring ----------------------------------------------------------------------------------------------
 // A look brings sixteen entries, the descriptors that travel with the first four, and what is known of the entries' job
 // slots, straight into LDS.  kLooks of them are under way at a time, so that an entry waits half the round trip to the
@@ -1089,6 +1085,13 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
 }
 
 // ---- worker -------------------------------------------------------------------------------------------------------
+// A lone request waits for every instruction and every trip to the LDS between its ticket and the first load, and between the
+// last store and its completion word.  Hence: values of other lanes by moves and masks, not by exchanges through the LDS; the
+// load of the descriptors ahead of what is left in the LDS; one word that says whether there is a ticket and what it is; a
+// fragment's record waited for once; and what the last wavefront has to say read while its stores are on their way.  (Us,
+// before / with all of these: 64 KiB of pages 7.52 / 7.42, through the plugin 6.72 / 6.55, 2048 of those 16 posted at a time 920 / 912, 300 KiB
+// of ragged fragments 9.40 / 9.06.)
+//
 // A worker workgroup is kCopyWaves copy wavefronts and one fetcher wavefront.  Towards the end of ticket i the
 // fetcher claims a number, polls that ticket's slot, pulls the ticket's descriptors over PCIe and writes their
 // records into the other LDS stage; between two tickets the copy wavefronts only meet the fetcher at one barrier.  The copy wavefront
@@ -1117,10 +1120,9 @@ static_assert(sizeof(RoundRec) == 48, "three 16-byte LDS reads");
 // In a staged ticket's word 10 (see copy_ticket), where the descriptors of a ticket of more than kFullTicket never travel.
 constexpr uint32_t kRoundsAlone = kCarriedTicket;
 static_assert(kCarriedDescs <= kFullTicket, "the bit has another meaning in tickets that bring their descriptors");
-struct Stage {
-  uint32_t payload[kPayloadWords];
-  uint32_t go;
-  uint32_t pad[3];
+constexpr int kTicketWord = 10;  // of a ticket's payload: never zero, since a ticket has descriptors
+struct alignas(16) Stage {
+  uint32_t payload[kPayloadWords];  // kTicketWord zero: no more tickets
   RoundRec rec[kMaxDescsPerTicket];
 };
 
@@ -1129,6 +1131,7 @@ struct Stage {
 typedef TCPXU_LDS Stage LdsStage;
 typedef TCPXU_LDS uint32_t lds_u32;
 
+__device__ __forceinline__ uint64_t lanes_where(bool holds) { return __builtin_amdgcn_ballot_w64(holds); }
 __device__ __forceinline__ uint32_t lane_shift(uint32_t v, uint32_t from_lane) {
   return static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(static_cast<int>((from_lane & 63u) << 2), static_cast<int>(v)));
 }
@@ -1146,18 +1149,12 @@ __device__ uint32_t try_fetch_ticket(DevState* st, const uint32_t* stop_word, ui
   u32x4 d = {0u, 0u, 0u, 0u};
   if (ask && lane < kCarriedDescs) d = load_vec_sys(reinterpret_cast<const uint8_t*>(&st->carried[ticket & (kTicketRing - 1)]) + 16 * lane);
   *stop_up = lane_value(word, 16) != 0;
-  const bool stamp_ok = (lane < 16 && (lane & 3) == 3) ? (word == expect) : true;
-  if (!__all(stamp_ok)) return 0;
-  const uint32_t ticket_bits = lane_value(word, payload_slot(10));
+  if (~lanes_where(word == expect) & 0x8888u) return 0;
+  const uint32_t ticket_bits = lane_value(word, payload_slot(kTicketWord));
   const uint32_t n = ticket_bits & 0xFFu;
   const bool carried = ask && (ticket_bits & kCarriedTicket) != 0;
-  if (carried && !__all(lane >= n || d[3] == expect)) return 0;  // its descriptors are still on their way
+  if (carried && (~lanes_where(d[3] == expect) & ((1u << n) - 1u)) != 0) return 0;  // its descriptors are still on their way
   const uint64_t fetched_at = stamps ? clock_now() : 0;
-  // Lane broadcasts need the whole wavefront: gather first, then let 12 lanes store.
-  const uint32_t pl = lane < kPayloadWords ? lane : 0u;
-  const uint32_t gathered = bcast(word, (pl / 3) * 4 + (pl % 3));
-  if (lane < kPayloadWords) stage->payload[lane] = gathered;
-  if (lane == 0) stage->go = 1;
   auto word64 = [&](int lo) {
     return (static_cast<uint64_t>(lane_value(word, payload_slot(lo + 1))) << 32) | lane_value(word, payload_slot(lo));
   };
@@ -1181,6 +1178,8 @@ __device__ uint32_t try_fetch_ticket(DevState* st, const uint32_t* stop_word, ui
   if (outward) mine = std::min(std::max(static_cast<int>(lane) - 1, more_before ? -1 : 0), last);
   if (carried) d[3] = 0;  // (the stamp's place is the high word of the destination offset)
   else d = load_vec_sys(reinterpret_cast<const uint8_t*>(descs_addr) + 16 * mine);
+  // (After the load: a wait for the LDS on the way to it is one that a request waits for.)
+  if (lane < 16 && (lane & 3u) != 3) stage->payload[3 * (lane >> 2) + (lane & 3u)] = word;
   if (outward) {  // wave-uniform: a ticket without such neighbours pays nothing here
     auto from_lane = [](uint32_t v, uint32_t src) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(src))); };
     const u32x4 w = d;
@@ -1214,14 +1213,14 @@ __device__ uint32_t try_fetch_ticket(DevState* st, const uint32_t* stop_word, ui
   // the line before taken from what the neighbour found about the line after, one round of lane exchanges less but more
   // branches, 200 requests of 256 KiB in one call took 47.4 us instead of 46.9, 32 of 2 MiB 32.8 instead of 32.4.
   const uint32_t off_line = (static_cast<uint32_t>(fdst) | len) & (kLineBytes - 1);
-  const bool off_lines = __any(lane < n && (off_line != 0 || len == 0));
+  const bool off_lines = lanes_where(lane < n && (off_line != 0 || len == 0)) != 0;
   if (lane == 0 && !off_lines && n > kBurstTicket && n <= kShortBurstTicket && (ticket_bits & kOnlyTicket) == 0)
-    stage->payload[10] = ticket_bits | kRoundsAlone;
+    stage->payload[kTicketWord] = ticket_bits | kRoundsAlone;
   if (off_lines) {
     // The neighbours' descriptors decide which destination lines are shared with them.  A fragment's neighbours are
     // the nearest descriptors of the ticket that are not empty: an empty descriptor between two fragments (a
     // zero-length control message's, a fragment cut to nothing) leaves them back to back in the destination.
-    const uint64_t live = __ballot(lane < n && len != 0);
+    const uint64_t live = lanes_where(lane < n && len != 0);
     const uint64_t below = live & ((1ull << lane) - 1ull);
     const uint64_t above = lane < 63u ? live & ~((2ull << lane) - 1ull) : 0ull;
     const bool prev_inside = below != 0, next_inside = above != 0;
@@ -1266,17 +1265,18 @@ __device__ uint32_t try_fetch_ticket(DevState* st, const uint32_t* stop_word, ui
 
 // Counts a finished ticket (all of its payload is in memory); the last ticket of a submission publishes the
 // completion word.
-__device__ void retire_ticket(DevState* st, uint32_t* jobs_done, const LdsStage* stage, uint32_t lane, uint64_t* stamps) {
+// `flag` and `rest` are the ticket's payload words 4 to 7 and 8 to 11.
+__device__ __forceinline__ void retire_ticket(DevState* st, uint32_t* jobs_done, u32x4 flag, u32x4 rest, uint32_t lane, uint64_t* stamps) {
   if (lane == 0) {
-    const uint32_t job = (stage->payload[10] >> 8) & 0xFFFFu;
-    const uint32_t target = stage->payload[11];
-    const uint64_t done_flag = (static_cast<uint64_t>(stage->payload[7]) << 32) | stage->payload[6];
-    const uint64_t done_value = (static_cast<uint64_t>(stage->payload[9]) << 32) | stage->payload[8];
-    if ((stage->payload[10] & kOnlyTicket) != 0) {
+    const uint32_t job = (rest[2] >> 8) & 0xFFFFu;
+    const uint32_t target = rest[3];
+    const uint64_t done_flag = (static_cast<uint64_t>(flag[3]) << 32) | flag[2];
+    const uint64_t done_value = (static_cast<uint64_t>(rest[1]) << 32) | rest[0];
+    if ((rest[2] & kOnlyTicket) != 0) {
       // The submission's only ticket completes it: tell the caller first, count afterwards (nobody waits for the
       // counts' round trips).  Its job slot has nothing to count.
       if (stamps) sys_store(&stamps[kStampsPerJob * job + 3], clock_now());
-      sys_store(reinterpret_cast<uint64_t*>(done_flag), done_value);
+      sys_store_global(reinterpret_cast<uint64_t*>(done_flag), done_value);
       __hip_atomic_fetch_add(&st->tickets_done.value, 1ull, __ATOMIC_RELAXED, SYS);
       __hip_atomic_fetch_add(&st->jobs_completed.value, 1ull, __ATOMIC_RELAXED, SYS);
       return;
@@ -1286,7 +1286,7 @@ __device__ void retire_ticket(DevState* st, uint32_t* jobs_done, const LdsStage*
     if (count == target) {
       // Every other ticket's payload was in memory before it was counted, and so is this one's.
       if (stamps) sys_store(&stamps[kStampsPerJob * job + 3], clock_now());
-      sys_store(reinterpret_cast<uint64_t*>(done_flag), done_value);
+      sys_store_global(reinterpret_cast<uint64_t*>(done_flag), done_value);
       __hip_atomic_fetch_add(&st->jobs_completed.value, 1ull, __ATOMIC_RELAXED, SYS);
     }
   }
@@ -1296,19 +1296,26 @@ __device__ void retire_ticket(DevState* st, uint32_t* jobs_done, const LdsStage*
 // ticket, rounded up), one round (at most 4 KiB) in flight at a time, or two.  A wavefront that writes one contiguous
 // stretch of the destination after another measured about 1 % faster end to end than fragments dealt out in turn
 // (wave, wave + kCopyWaves, ...).
-__device__ __forceinline__ void copy_ticket(const LdsStage* stage, uint32_t wave, uint32_t lane, lds_u32* waves_on_last) {
+__device__ __forceinline__ void copy_ticket(const LdsStage* stage, uint32_t ticket_word, uint32_t wave, uint32_t lane, lds_u32* waves_on_last) {
   auto uniform = [](uint32_t v) { return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(v)); };
   wave = uniform(wave);
-  const uint32_t n = uniform(stage->payload[10]) & 0xFFu;
+  const uint32_t n = ticket_word & 0xFFu;
   const uint32_t per = (n + kCopyWaves - 1) / kCopyWaves;
   uint32_t j = wave * per < n ? wave * per : n;
   const uint32_t end = j + per < n ? j + per : n;
-  // Told once, when the wavefront turns to the last fragment of its share (at once if it has none): the fetcher
-  // uses it to start fetching the next ticket.
-  auto on_last_fragment = [&] {
+  // Told once, when the wavefront has turned to the last fragment of its share (or has none left): the fetcher uses it to
+  // start fetching the next ticket.  After the fragment's record has been read, since the LDS answers a wavefront in order; ahead
+  // of its loads in a stream's tickets, where issuing them takes a microsecond while the memory system is full, and after
+  // them in a request's only ticket, whose loads are what is waited for.  (256 MiB of ragged fragments with all after their
+  // loads 108.1 us, so 107.3; 2048 requests of 64 KiB through the plugin, 16 posted at a time, with all ahead of them 936 to 954 us,
+  // so 912.)
+  bool told = false;
+  auto tell_if_on_last = [&] {
+    if (told || j < end) return;
+    told = true;
     if (lane == 0) __hip_atomic_fetch_add(waves_on_last, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    lanes_together();
   };
-  if (j >= end) on_last_fragment();
   uint32_t nvec_left = 0;
   // The next round of the share into `out`, or false when there is none; `prev` is the round before it (read only
   // while a fragment longer than one round goes on).
@@ -1325,9 +1332,9 @@ __device__ __forceinline__ void copy_ticket(const LdsStage* stage, uint32_t wave
     }
     while (j < end) {
       const lds_u32x4* words = reinterpret_cast<const lds_u32x4*>(&stage->rec[j]);
-      const u32x4 w0 = words[0], w1 = words[1], w2 = words[2];
+      u32x4 w0 = words[0], w1 = words[1], w2 = words[2];
+      asm volatile("" : "+v"(w0), "+v"(w1), "+v"(w2));  // one wait for the three, not one each where the compiler first needs it
       ++j;
-      if (j >= end) on_last_fragment();
       const uint32_t bits = uniform(w2[2]);
       const uint32_t kind = bits >> 24;
       if (kind == kRecSkip) continue;
@@ -1354,16 +1361,20 @@ __device__ __forceinline__ void copy_ticket(const LdsStage* stage, uint32_t wave
   // of 64 KiB through the plugin, 16 posted at a time, 1045 / 1000 us, 256 MiB of ragged fragments 114.2 / 107.6, of whole pages
   // 103.9 / 105.7; streams of fragments on lines, 2 KiB in tickets of 32, 5.67 / 5.38 TB/s r+w, 1 KiB in tickets of 64, 5.29 / 5.35;
   // 64 MiB of pages in tickets of 18 31.2 / 30.9 us.)
-  const bool pairs = n > kFullTicket || (uniform(stage->payload[10]) & kOnlyTicket) != 0;
-  const bool alone = n > kFullTicket && (uniform(stage->payload[10]) & kRoundsAlone) != 0;
+  const bool only = (ticket_word & kOnlyTicket) != 0;
+  const bool pairs = n > kFullTicket || only;
+  const bool alone = n > kFullTicket && (ticket_word & kRoundsAlone) != 0;
   CopyRound r, next;
   CopyRegs x, y;
   bool more = produce(r, r);
   while (more) {
+    if (!only) tell_if_on_last();
     round_load(r, x, lane);
     if (pairs) {
       const bool second = !alone && produce(next, r);
+      if (!only) tell_if_on_last();
       if (second) round_load(next, y, lane);
+      if (only) tell_if_on_last();
       rounds_wait(x, y);
       round_store_loaded(r, x, lane);
       if (second) {
@@ -1378,6 +1389,7 @@ __device__ __forceinline__ void copy_ticket(const LdsStage* stage, uint32_t wave
       r = next;
     }
   }
+  tell_if_on_last();
 }
 
 // The compute unit that the calling wavefront runs on, as an odd number; kNoPlace is none's.
@@ -1436,13 +1448,13 @@ __device__ void worker_loop(DevState* st, uint32_t* jobs_done, uint32_t flags, u
           __builtin_amdgcn_s_sleep(1);
       }
       if (not_needed()) {
-        if (lane == 0) next->go = 0;
+        if (lane == 0) next->payload[kTicketWord] = 0;
         __syncthreads();
         break;
       }
       uint64_t t = 0;
       if (lane == 0) t = __hip_atomic_fetch_add(&st->ticket_head.value, 1ull, __ATOMIC_RELAXED, SYS);
-      const uint64_t ticket = bcast64(t, 0);
+      const uint64_t ticket = same_in_all_lanes64(t);
       bool give_up = false, stop_before = false, first_look = true;
       uint32_t backoff = 1, looks = 0;
       for (;;) {
@@ -1455,7 +1467,7 @@ __device__ void worker_loop(DevState* st, uint32_t* jobs_done, uint32_t flags, u
           // The stop word was already up at the previous look and the ticket is still not there: the leader
           // publishes every ticket before any stop word, so it never will be.
           give_up = true;
-          if (lane == 0) next->go = 0;
+          if (lane == 0) next->payload[kTicketWord] = 0;
           break;
         }
         stop_before = stop_up;
@@ -1480,14 +1492,18 @@ __device__ void worker_loop(DevState* st, uint32_t* jobs_done, uint32_t flags, u
     for (uint32_t i = 0;; ++i) {
       __syncthreads();  // stage i&1 is ready
       LdsStage* stage = (LdsStage*)&stages[i & 1];
-      if (stage->go == 0) break;
-      copy_ticket(stage, wave, lane, (lds_u32*)&s_waves_on_last);
-      drain_memory_ops();  // this wavefront's write-through stores are acknowledged
+      const uint32_t ticket_word = same_in_all_lanes32(stage->payload[kTicketWord]);
+      if (ticket_word == 0) break;
+      copy_ticket(stage, ticket_word, wave, lane, (lds_u32*)&s_waves_on_last);
+      // (What the last wavefront needs, read while the stores are on their way.)
+      const lds_u32x4* words = reinterpret_cast<const lds_u32x4*>(&stage->payload[0]);
+      u32x4 flag = words[1], rest = words[2];
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : "+v"(flag), "+v"(rest) : : "memory");  // this wavefront's write-through stores are acknowledged
       uint32_t arrived = 0;
       if (lane == 0)
         arrived = __hip_atomic_fetch_add(&s_waves_done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) + 1u;
       // The wavefront that finishes last counts the ticket: every wavefront's payload is in memory by then.
-      if (bcast(arrived, 0) == (i + 1) * kCopyWaves) retire_ticket(st, jobs_done, stage, lane, stamps);
+      if (same_in_all_lanes32(arrived) == (i + 1) * kCopyWaves) retire_ticket(st, jobs_done, flag, rest, lane, stamps);
     }
   }
 }
