@@ -1088,9 +1088,10 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
 // A lone request waits for every instruction and every trip to the LDS between its ticket and the first load, and between the
 // last store and its completion word.  Hence: values of other lanes by moves and masks, not by exchanges through the LDS; the
 // load of the descriptors ahead of what is left in the LDS; one word that says whether there is a ticket and what it is; a
-// fragment's record waited for once; and what the last wavefront has to say read while its stores are on their way.  (Us,
-// before / with all of these: 64 KiB of pages 7.52 / 7.42, through the plugin 6.72 / 6.55, 2048 of those 16 posted at a time 920 / 912, 300 KiB
-// of ragged fragments 9.40 / 9.06.)
+// fragment's record waited for once; what tells the fetcher to go on a store, not an addition; and what the last wavefront has
+// to say read while its stores are on their way.  (Us, before / with all of these: 64 KiB of pages 7.60 / 7.44, through the plugin
+// 6.71 / 6.49, a page 5.73 / 5.50, 1 MiB of wire fragments 9.87 / 9.55, 2048 requests of 64 KiB through the plugin, 16 posted at a time,
+// 896 / 882; streams of 64 KiB requests, 1 / 8 / 64 / 256 in flight, 0.170 / 1.338 / 8.72 / 21.6 M/s before, 0.175 / 1.373 / 8.65 / 21.4 now.)
 //
 // A worker workgroup is kCopyWaves copy wavefronts and one fetcher wavefront.  Towards the end of ticket i the
 // fetcher claims a number, polls that ticket's slot, pulls the ticket's descriptors over PCIe and writes their
@@ -1296,26 +1297,18 @@ __device__ __forceinline__ void retire_ticket(DevState* st, uint32_t* jobs_done,
 // ticket, rounded up), one round (at most 4 KiB) in flight at a time, or two.  A wavefront that writes one contiguous
 // stretch of the destination after another measured about 1 % faster end to end than fragments dealt out in turn
 // (wave, wave + kCopyWaves, ...).
-__device__ __forceinline__ void copy_ticket(const LdsStage* stage, uint32_t ticket_word, uint32_t wave, uint32_t lane, lds_u32* waves_on_last) {
+__device__ __forceinline__ void copy_ticket(const LdsStage* stage, uint32_t ticket_word, uint32_t wave, uint32_t lane, lds_u32* on_last, uint32_t turn) {
   auto uniform = [](uint32_t v) { return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(v)); };
   wave = uniform(wave);
   const uint32_t n = ticket_word & 0xFFu;
   const uint32_t per = (n + kCopyWaves - 1) / kCopyWaves;
   uint32_t j = wave * per < n ? wave * per : n;
   const uint32_t end = j + per < n ? j + per : n;
-  // Told once, when the wavefront has turned to the last fragment of its share (or has none left): the fetcher uses it to
-  // start fetching the next ticket.  After the fragment's record has been read, since the LDS answers a wavefront in order; ahead
-  // of its loads in a stream's tickets, where issuing them takes a microsecond while the memory system is full, and after
-  // them in a request's only ticket, whose loads are what is waited for.  (256 MiB of ragged fragments with all after their
-  // loads 108.1 us, so 107.3; 2048 requests of 64 KiB through the plugin, 16 posted at a time, with all ahead of them 936 to 954 us,
-  // so 912.)
-  bool told = false;
-  auto tell_if_on_last = [&] {
-    if (told || j < end) return;
-    told = true;
-    if (lane == 0) __hip_atomic_fetch_add(waves_on_last, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    lanes_together();
-  };
+  // Told once, when the wavefront turns to the last fragment of its share (at once if it has none): the fetcher
+  // uses it to start fetching the next ticket.  Every wavefront has a word of its own for that, which all of its lanes write: a
+  // counter would cost an addition of one lane, which is a dozen instructions ahead of a lone request's loads.
+  auto on_last_fragment = [&] { __hip_atomic_store(on_last, turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+  if (j >= end) on_last_fragment();
   uint32_t nvec_left = 0;
   // The next round of the share into `out`, or false when there is none; `prev` is the round before it (read only
   // while a fragment longer than one round goes on).
@@ -1333,8 +1326,11 @@ __device__ __forceinline__ void copy_ticket(const LdsStage* stage, uint32_t tick
     while (j < end) {
       const lds_u32x4* words = reinterpret_cast<const lds_u32x4*>(&stage->rec[j]);
       u32x4 w0 = words[0], w1 = words[1], w2 = words[2];
-      asm volatile("" : "+v"(w0), "+v"(w1), "+v"(w2));  // one wait for the three, not one each where the compiler first needs it
+      // One wait for the three, not one each where the compiler first needs it, and ahead of what is added to the LDS next: it
+      // answers a wavefront in order.
+      asm volatile("" : "+v"(w0), "+v"(w1), "+v"(w2));
       ++j;
+      if (j >= end) on_last_fragment();
       const uint32_t bits = uniform(w2[2]);
       const uint32_t kind = bits >> 24;
       if (kind == kRecSkip) continue;
@@ -1361,20 +1357,16 @@ __device__ __forceinline__ void copy_ticket(const LdsStage* stage, uint32_t tick
   // of 64 KiB through the plugin, 16 posted at a time, 1045 / 1000 us, 256 MiB of ragged fragments 114.2 / 107.6, of whole pages
   // 103.9 / 105.7; streams of fragments on lines, 2 KiB in tickets of 32, 5.67 / 5.38 TB/s r+w, 1 KiB in tickets of 64, 5.29 / 5.35;
   // 64 MiB of pages in tickets of 18 31.2 / 30.9 us.)
-  const bool only = (ticket_word & kOnlyTicket) != 0;
-  const bool pairs = n > kFullTicket || only;
+  const bool pairs = n > kFullTicket || (ticket_word & kOnlyTicket) != 0;
   const bool alone = n > kFullTicket && (ticket_word & kRoundsAlone) != 0;
   CopyRound r, next;
   CopyRegs x, y;
   bool more = produce(r, r);
   while (more) {
-    if (!only) tell_if_on_last();
     round_load(r, x, lane);
     if (pairs) {
       const bool second = !alone && produce(next, r);
-      if (!only) tell_if_on_last();
       if (second) round_load(next, y, lane);
-      if (only) tell_if_on_last();
       rounds_wait(x, y);
       round_store_loaded(r, x, lane);
       if (second) {
@@ -1389,7 +1381,6 @@ __device__ __forceinline__ void copy_ticket(const LdsStage* stage, uint32_t tick
       r = next;
     }
   }
-  tell_if_on_last();
 }
 
 // The compute unit that the calling wavefront runs on, as an odd number; kNoPlace is none's.
@@ -1404,13 +1395,13 @@ __device__ __forceinline__ uint32_t compute_unit_here() {
 __device__ void worker_loop(DevState* st, uint32_t* jobs_done, uint32_t flags, uint64_t* stamps) {
   __shared__ Stage stages[2];
   __shared__ uint32_t s_waves_done;  // copy wavefronts that have finished (and drained) a ticket, running total
-  __shared__ uint32_t s_waves_on_last;  // copy wavefronts that have turned to their last fragment of a ticket, ditto
+  __shared__ uint32_t s_on_last[kCopyWaves];  // of each copy wavefront, the tickets whose last fragment it has turned to
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = tid & (kWaveLanes - 1);
   const uint32_t wave = tid / kWaveLanes;
   if (tid == 0) {
     s_waves_done = 0;
-    s_waves_on_last = 0;
+    for (uint32_t w = 0; w < kCopyWaves; ++w) s_on_last[w] = 0;
   }
   __syncthreads();
 
@@ -1438,14 +1429,17 @@ __device__ void worker_loop(DevState* st, uint32_t* jobs_done, uint32_t flags, u
     uint32_t staged = 0;
     bool eager = false;
     const bool allow_eager = (flags & 1u) != 0;
-    const uint32_t* const claim_gate = (flags & 2u) != 0 ? &s_waves_on_last : &s_waves_done;
+    const bool early = (flags & 2u) != 0;
+    auto gate_open = [&](uint32_t tickets) {
+      if (!early) return __hip_atomic_load((lds_u32*)&s_waves_done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == tickets * kCopyWaves;
+      return lanes_where(__hip_atomic_load((lds_u32*)&s_on_last[lane % kCopyWaves], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != tickets) == 0;
+    };
     const uint32_t backoff_cap = (flags >> 8) & 0xFFu;
     for (;;) {
       LdsStage* next = (LdsStage*)&stages[staged & 1];
       if (!eager) {
         // Wait for the copy of ticket staged-1 to finish (LDS only: no memory traffic while waiting).
-        while (__hip_atomic_load(claim_gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != staged * kCopyWaves)
-          __builtin_amdgcn_s_sleep(1);
+        while (!gate_open(staged)) __builtin_amdgcn_s_sleep(1);
       }
       if (not_needed()) {
         if (lane == 0) next->payload[kTicketWord] = 0;
@@ -1494,14 +1488,14 @@ __device__ void worker_loop(DevState* st, uint32_t* jobs_done, uint32_t flags, u
       LdsStage* stage = (LdsStage*)&stages[i & 1];
       const uint32_t ticket_word = same_in_all_lanes32(stage->payload[kTicketWord]);
       if (ticket_word == 0) break;
-      copy_ticket(stage, ticket_word, wave, lane, (lds_u32*)&s_waves_on_last);
+      copy_ticket(stage, ticket_word, wave, lane, (lds_u32*)&s_on_last[wave], i + 1);
       // (What the last wavefront needs, read while the stores are on their way.)
       const lds_u32x4* words = reinterpret_cast<const lds_u32x4*>(&stage->payload[0]);
       u32x4 flag = words[1], rest = words[2];
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : "+v"(flag), "+v"(rest) : : "memory");  // this wavefront's write-through stores are acknowledged
       uint32_t arrived = 0;
       if (lane == 0)
-        arrived = __hip_atomic_fetch_add(&s_waves_done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) + 1u;
+        arrived = __builtin_amdgcn_atomic_inc32((lds_u32*)&s_waves_done, 0xFFFFFFFFu, __ATOMIC_RELAXED, "workgroup") + 1u;
       // The wavefront that finishes last counts the ticket: every wavefront's payload is in memory by then.
       if (same_in_all_lanes32(arrived) == (i + 1) * kCopyWaves) retire_ticket(st, jobs_done, flag, rest, lane, stamps);
     }
