@@ -148,6 +148,9 @@ typedef struct tcpxDeviceOps {
   /* Optional (may be NULL): engine_submit with the request's size as a hint (tcpxuEngineSubmitSized). */
   int (*engine_submit_sized)(tcpxuEngine* engine, const void* bounce_base, void* dst_base, const void* descs_dev,
                              uint32_t n_descs, uint64_t payload_bytes, void* done_flag_dev, uint64_t done_value);
+  /* Optional (may be NULL): how many descriptors of a list in mapped memory a submission brings along
+   * (tcpxuEngineCarriedDescs); such a request gets no second copy while it is the only one. */
+  uint32_t (*engine_carried_descs)(void);
 } tcpxDeviceOps;
 
 /* Installs `ops` in place of the HIP layer (NULL restores the default binding).  For host-logic tests only;

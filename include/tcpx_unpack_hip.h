@@ -151,6 +151,10 @@ int tcpxuEngineSubmit(tcpxuEngine* engine, const void* bounce_base, void* dst_ba
 int tcpxuEngineSubmitSized(tcpxuEngine* engine, const void* bounce_base, void* dst_base, const void* descs_dev,
                            uint32_t n_descs, uint64_t payload_bytes, void* done_flag_dev, uint64_t done_value);
 
+/* Descriptors of a list in memory from tcpxuMappedAlloc up to which the calls above copy it beside the submission, so that
+ * the GPU need not fetch it by itself (while the engine keeps up, and for the first few of a call). */
+uint32_t tcpxuEngineCarriedDescs(void);
+
 /* Several slots published under one lock with one store of the ring's tail: what a poller that finds several
  * requests complete in one pass submits together (a storm of small requests is bound by the host's cost per
  * publish).  All `n` submissions are checked first and none is queued if one is refused (TCPXU_INVALID_ARGUMENT).

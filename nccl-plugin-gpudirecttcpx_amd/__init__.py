@@ -208,6 +208,7 @@ _HIP_PROTOTYPES = {
         ],
     ),
     "tcpxuEngineCompleted": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_uint64)]),
+    "tcpxuEngineCarriedDescs": (ctypes.c_uint32, []),
     "tcpxuEngineSubmitMany": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(Submission), ctypes.c_uint32, ctypes.POINTER(ctypes.c_uint32)]),
     "tcpxuEngineEnableStamps": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_double)]),
     "tcpxuEngineReadStamps": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_uint64, ctypes.c_uint32, ctypes.POINTER(ctypes.c_uint64)]),

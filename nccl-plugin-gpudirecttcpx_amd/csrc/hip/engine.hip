@@ -1984,6 +1984,8 @@ int tcpxuEngineGetConfig(tcpxuEngine* e, tcpxuEngineConfig* config) {
   return TCPXU_SUCCESS;
 }
 
+uint32_t tcpxuEngineCarriedDescs(void) { return kCarriedDescs; }
+
 int tcpxuEngineDevice(tcpxuEngine* e, int* device) {
   if (!e || !device) return TCPXU_INVALID_ARGUMENT;
   *device = e->device;

@@ -58,6 +58,7 @@ const tcpxDeviceOps* default_device_ops() {
   ok &= bind(&g_hip_ops.visible_alloc, "tcpxuVisibleAlloc");
   ok &= bind(&g_hip_ops.visible_free, "tcpxuVisibleFree");
   ok &= bind(&g_hip_ops.visible_flush, "tcpxuVisibleFlush");
+  ok &= bind(&g_hip_ops.engine_carried_descs, "tcpxuEngineCarriedDescs");
   if (!ok) {
     dlclose(g_hip_lib);
     g_hip_lib = nullptr;

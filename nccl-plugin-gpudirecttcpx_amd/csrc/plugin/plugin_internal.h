@@ -455,6 +455,7 @@ struct Global {
   ncclDebugLogger_t logger = nullptr;
   const tcpxDeviceOps* ops = nullptr;
   bool ops_injected = false;
+  uint32_t carried_descs = 0;  // descriptors that the engine brings along with a submission (tcpxDeviceOps::engine_carried_descs)
   int n_devices = 0;
   DeviceState devices[kMaxDevices];
   // Flags (environment, range-checked in tcpxInit like TCPX_GET_INT_FLAG, src/net_tcpx.cc:440-452).
