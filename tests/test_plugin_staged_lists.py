@@ -1,33 +1,85 @@
 """The second copy of a request's descriptors is written by whole lines of four: lists that end within a line, fill it or go one
-beyond, small ones and of a request that is alone (no GPU: the emulated device of tests/emu)."""
+beyond, small ones and of a request that is alone; and where the engine brings lists of mapped slots along, a small request that is
+alone has none (no GPU: the emulated device of tests/emu)."""
+import ctypes
+
 import numpy as np
 import pytest
 
-from test_plugin_host import ARENA_BYTES, comm, env, host_buffer  # noqa: F401  (fixtures)
+from test_plugin_host import ARENA_BYTES, comm, env, host_buffer, load_emu  # noqa: F401  (fixtures)
+
+OPS = 19  # members of tcpxDeviceOps, the last of them engine_carried_descs
+CARRIED = 16
+
+
+def receive(env, comm, sizes, seed):
+    """Posts a request for each of `sizes` (fragment counts) before any of their bytes is there; how many lists were copied."""
+    rng = np.random.default_rng(seed)
+    copies, posted, first = env.emu.emu_counter(6), [], 0
+    env.arena_np[:] = rng.integers(0, 256, len(env.arena_np), dtype=np.uint8)
+    pages = rng.permutation(sum(sizes)) % (ARENA_BYTES // 4096)
+    for n in sizes:
+        frags = np.zeros(n, dtype=env.pkg.Workload(1, shrink=6).frag_dtype)
+        frags["frag_size"] = rng.integers(1, 200, n)
+        frags["frag_token"] = pages[first : first + n]
+        frags["frag_offset"] = frags["frag_token"] * 4096 + rng.integers(0, 3896, n)
+        first += n
+        total = int(frags["frag_size"].sum())
+        buf, ptr = host_buffer(total)
+        mh = comm.reg(ptr, total)
+        rc, req = comm.irecv(ptr, total, mh)
+        assert rc == 0
+        posted.append((frags, total, buf, mh, req))
+    for frags, total, buf, mh, req in posted:
+        comm.ctrl(0, total, 0, total)
+        comm.deliver(0, frags)
+    for frags, total, buf, mh, req in posted:
+        for _ in range(100000):
+            rc, done = comm.test(req)[:2]
+            assert rc == 0
+            if done:
+                break
+        assert done
+        assert comm.consumed(req) == 0
+        comm.dereg(mh)
+        assert buf.tobytes() == b"".join(env.arena_np[int(f["frag_offset"]) :][: int(f["frag_size"])].tobytes() for f in frags)
+    return env.emu.emu_counter(6) - copies
+
+
+@pytest.fixture(scope="module")
+def carrying(env):  # noqa: F811
+    """The emulated device with an engine that brings lists along, in place of the one that does not."""
+    ops = (ctypes.c_void_p * OPS)()
+    ctypes.memmove(ops, env.emu.emu_ops(), ctypes.sizeof(ops))
+    assert ops[OPS - 2] and not ops[OPS - 1]
+    count = ctypes.CFUNCTYPE(ctypes.c_uint32)(lambda: CARRIED)
+    ops[OPS - 1] = ctypes.cast(count, ctypes.c_void_p).value
+
+    def install(table):
+        assert env.lib.tcpxFinalize() == 0
+        assert env.lib.tcpxSetDeviceOpsForTesting(table) == 0
+        assert env.lib.tcpxInit(None) == 0
+        base = ctypes.c_void_p()
+        assert env.lib.tcpxSynthArenaCreate(0, ARENA_BYTES, ctypes.byref(base)) == 0
+        env.arena = base.value
+        env.arena_np = np.frombuffer((ctypes.c_uint8 * ARENA_BYTES).from_address(base.value), dtype=np.uint8)
+
+    install(ctypes.addressof(ops))
+    yield env
+    install(env.emu.emu_ops())
 
 
 @pytest.mark.parametrize("n", [1, 3, 4, 5, 8, 13, 15, 16, 17, 19, 509, 511, 512])
 def test_a_second_copy_of_any_length(env, comm, n):  # noqa: F811
-    rng = np.random.default_rng(n)
-    frags = np.zeros(n, dtype=env.pkg.Workload(1, shrink=6).frag_dtype)
-    frags["frag_size"] = rng.integers(1, 200, n)
-    frags["frag_token"] = rng.permutation(n) % (ARENA_BYTES // 4096)
-    frags["frag_offset"] = frags["frag_token"] * 4096 + rng.integers(0, 3896, n)
-    env.arena_np[:] = rng.integers(0, 256, len(env.arena_np), dtype=np.uint8)
-    total = int(frags["frag_size"].sum())
-    buf, ptr = host_buffer(total)
-    mh = comm.reg(ptr, total)
-    copies = env.emu.emu_counter(6)
-    rc, req = comm.irecv(ptr, total, mh)
-    assert rc == 0
-    comm.ctrl(0, total, 0, total)
-    comm.deliver(0, frags)
-    for _ in range(100000):
-        rc, done = comm.test(req)[:2]
-        assert rc == 0
-        if done:
-            break
-    assert done and env.emu.emu_counter(6) == copies + 1
-    assert comm.consumed(req) == 0
-    comm.dereg(mh)
-    assert buf.tobytes() == b"".join(env.arena_np[int(f["frag_offset"]) :][: int(f["frag_size"])].tobytes() for f in frags)
+    assert receive(env, comm, [n], n) == 1
+
+
+@pytest.mark.parametrize("n", [1, 4, 15, 16, 17, 512, 513])
+def test_no_second_copy_of_a_list_that_travels(carrying, n):
+    comm = carrying.driver.RecvComm(0)  # noqa: F811
+    try:
+        assert receive(carrying, comm, [n], n) == (1 if 16 < n <= 512 else 0)
+        # Of three that are posted together the last one may find the others done.
+        assert receive(carrying, comm, [n] * 3, n + 1) >= (2 if n <= 16 else 0)
+    finally:
+        comm.close()
