@@ -645,16 +645,23 @@ inline void write_lines(union loadMeta* to, const union loadMeta* from, size_t n
 // 1078 the copy takes as long as it saves.  16 posted at a time: 8 MiB in requests of 18 84.5 / 100, four requests of 64
 // whole pages 11.6 / 11.9 with a copy of the first.)
 //
-// Not for a small one that has no other beside it, if the engine brings the lists of mapped slots along with its submissions: that
-// costs neither the host's flush nor a read of the GPU's.  (Us, copy / brought along: a request of 1 page 5.52 / 5.43, 4 5.88 / 5.60,
-// 10 6.96 / 6.72, 16 6.52 / 6.43.  For all small ones, 16 posted at a time, 256 of 1 page 95.4 / 102.3, 4 95.7 / 105.4, 8 99.8 / 108.7,
-// 16 110.7 / 111.8, since a look of the engine brings four lists and it is the flush's time that others wait for; while fewer than 3 are
-// at the GPU the same as when alone.)
+// Not for a small one that has no other beside it in its comm and fewer than kCrowd from all comms at the GPU, if the engine brings
+// the lists of mapped slots along with its submissions: that costs neither the host's flush nor a read of the GPU's.  (Us, copy /
+// brought along: a request of 1 page 5.52 / 5.43, 4 5.88 / 5.60, 10 6.96 / 6.72, 16 6.52 / 6.43.  For all small ones of a comm, 16
+// posted at a time, 256 of 1 page 95.4 / 102.3, 4 95.7 / 105.4, 8 99.8 / 108.7, 16 110.7 / 111.8.)
+//
+// The engine belongs to the device, and a look of it brings four lists: of many comms that hand over a request each, one behind
+// the other, those beyond the fourth are fetched over PCIe.  (Us from posted to done, mean over comms that post one request each
+// and wait for all.  4 / 8 / 12 / 16 comms, 1 page, copied if any other is at the GPU 4.95 / 4.98 / 4.98 / 5.08; brought along
+// while fewer than 3 are there 4.82 / 4.95 / 4.97 / 5.05, than 4 4.73 / 4.99 / 4.96 / 5.02, than 6 4.72 / 5.21 / 5.20 / 5.21, always
+// 4.72 / 5.43 / 5.74 / 6.12.  16 pages, any other 5.96 / 5.94 / 6.00 / 6.02, 4 5.80 / 6.01 / 6.01 / 6.02, always 5.79 / 6.38 / 6.73 / 7.01.
+// Comms that each post again as soon as their own is done come apart in time: 16 of them with 1 page take 8.93 a turn, 8.77 with
+// this rule and 6.99 always; 8 5.44, 5.42 and 5.19.)
 __attribute__((noinline)) const void* descriptors_for_engine(Comm* comm, const Request* r) {
   UnpackQueue* q = comm->queue;
   const bool small = r->slot.cnt_cache <= kStagedDescs;
   const bool alone = comm->slots_at_gpu == 0 && comm->to_submit == 1 && !comm->rq.has(kReqActive) && !comm->rq.has(kReqPosted);
-  const bool travels = alone && r->slot.cnt_cache <= g.carried_descs;
+  const bool travels = alone && r->slot.cnt_cache <= g.carried_descs && comm->device->at_gpu.load(std::memory_order_relaxed) < kCrowd;
   if (!q->stage || travels || (!small && (!alone || r->slot.cnt_cache > kAloneDescs))) return q->meta_dev->nccl.mem[r->slot.idx];
   const size_t at = small ? r->slot.idx * kStagedDescs : static_cast<size_t>(kStagedDescs) * kQueueDepth;
   write_lines(q->stage + at, r->slot.mem, r->slot.cnt_cache);
@@ -696,7 +703,7 @@ ncclResult_t publish_to_engine(Comm* comm, Request* r, bool* submitted) {
   r->published_ns = g.clock();
   r->unpack_watch.configure(static_cast<uint64_t>(g.timeout_threshold_ns), static_cast<uint64_t>(g.timeout_frequency_ns));
   comm->unpack_cnt++;
-  comm->slots_at_gpu++;
+  set_slots_at_gpu(comm, comm->slots_at_gpu + 1);
   comm->max_slots_at_gpu = std::max(comm->max_slots_at_gpu, comm->slots_at_gpu);
   *submitted = true;
   return ncclSuccess;
@@ -1165,7 +1172,7 @@ ncclResult_t tcpxTest(void* request, int* done, int* size) {
         }
         return ncclSuccess;
       }
-      comm->slots_at_gpu--;
+      set_slots_at_gpu(comm, comm->slots_at_gpu - 1);
       comm->unpack_ns += g.clock() - r->published_ns;
     } else {
       *r->slot.cnt = 0;  // src/net_tcpx.cc:1361
@@ -1235,6 +1242,7 @@ ncclResult_t tcpxClose(void* oComm) {
       WARN("head %lu tail %lu some pages not yet freed?", static_cast<unsigned long>(comm->queue->head),
            static_cast<unsigned long>(comm->queue->tail));
     unpack_queue_free(comm->queue);
+    set_slots_at_gpu(comm, 0);  // (what it leaves there is nobody's to wait for)
     std::lock_guard<std::mutex> lock(comm->device->mu);
     std::vector<Comm*>& open = comm->device->comms;
     open.erase(std::remove(open.begin(), open.end(), comm), open.end());

@@ -437,7 +437,21 @@ struct DeviceState {
   std::vector<Comm*> comms;           // open receive comms
   uint64_t pages_never_returned = 0;  // page references that comms still held when they were closed
   std::vector<QueueBlock> free_blocks;
+  // What all comms have at the GPU, for a comm that asks whether its one small request has others beside it there: the sum of
+  // their shares (see at_gpu_share).  On a line of its own: every comm's thread writes it.
+  alignas(64) std::atomic<uint32_t> at_gpu{0};
 };
+
+// A comm's part of DeviceState::at_gpu by the slots that it has there.  All but the first count as kCrowd at once, so that a comm that
+// keeps several there leaves the word alone.  kCrowd: the lists that a look of the engine brings along (the figures stand at
+// descriptors_for_engine).
+constexpr uint32_t kCrowd = 4;
+constexpr uint32_t at_gpu_share(uint32_t slots) { return slots < 2 ? slots : kCrowd; }
+inline void set_slots_at_gpu(Comm* comm, uint32_t slots) {
+  const uint32_t was = at_gpu_share(comm->slots_at_gpu), is = at_gpu_share(slots);
+  comm->slots_at_gpu = slots;
+  if (is != was) comm->device->at_gpu.fetch_add(is - was, std::memory_order_relaxed);
+}
 
 // Who copies.  kDeviceHost: this plugin's engine unpacks every request and test() reports done after the copy; the
 // plugin advertises an ordinary host-driven network (NCCL_NET_DEVICE_HOST), so no consumer kernel touches the

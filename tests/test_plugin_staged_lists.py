@@ -83,3 +83,83 @@ def test_no_second_copy_of_a_list_that_travels(carrying, n):
         assert receive(carrying, comm, [n] * 3, n + 1) >= (2 if n <= 16 else 0)
     finally:
         comm.close()
+
+
+class Small:
+    """A comm with small requests of 3 descriptors that the engine holds."""
+
+    def __init__(self, env, at):
+        self.env, self.comm, self.at, self.held = env, env.driver.RecvComm(0), at, []
+        self.buf, self.ptr = host_buffer(4096)
+        self.mh = self.comm.reg(self.ptr, 4096)
+
+    def post(self):
+        """Hands a request to the engine; whether its list was copied."""
+        submitted, copied = self.env.emu.emu_counter(0), self.env.emu.emu_counter(6)
+        frags = np.zeros(3, dtype=self.env.pkg.Workload(1, shrink=6).frag_dtype)
+        frags["frag_size"], frags["frag_token"] = 100, 3 * (8 * self.at + len(self.held)) + np.arange(3)
+        frags["frag_offset"] = 4096 * frags["frag_token"]
+        rc, req = self.comm.irecv(self.ptr + 300 * len(self.held), 300, self.mh)
+        assert rc == 0
+        self.held.append((frags, req))
+        self.comm.ctrl(0, 300, 0, 300)
+        self.comm.deliver(0, frags)
+        for _ in range(100000):
+            assert self.comm.test(self.held[0][1])[:2] == (0, 0)  # (only the oldest may be asked for)
+            if self.env.emu.emu_counter(0) == submitted + 1:
+                return self.env.emu.emu_counter(6) - copied
+        raise AssertionError("request never reached the engine")
+
+    def finish(self):
+        for frags, req in self.held:
+            assert self.comm.test(req)[:2] == (0, 1) and self.comm.consumed(req) == 0
+        want = b"".join(self.env.arena_np[int(f["frag_offset"]) :][:100].tobytes() for frags, _ in self.held for f in frags)
+        assert self.buf.tobytes()[: len(want)] == want
+        self.held = []
+
+
+@pytest.mark.parametrize("others", [0, 1, 3, 4, 5, 16])
+def test_lists_travel_while_few_comms_have_requests_at_the_gpu(carrying, others):
+    """The engine is the device's: a small request that is alone in its comm counts what all comms have there."""
+    env = carrying
+    env.arena_np[:] = np.random.default_rng(others).integers(0, 256, len(env.arena_np), dtype=np.uint8)
+    comms = [Small(env, i) for i in range(others + 1)]
+    env.emu.emu_set_hold(1)
+    try:
+        for _ in range(2):  # (and again once all have been reported done)
+            assert [c.post() for c in comms] == [int(i >= 4) for i in range(others + 1)]
+            assert env.emu.emu_release(1 << 20) == others + 1
+            for c in comms:
+                c.finish()
+    finally:
+        env.emu.emu_set_hold(0)
+        env.emu.emu_release(1 << 20)
+        for c in comms:
+            c.comm.close()
+
+
+def test_a_comm_with_several_at_the_gpu_is_a_crowd_until_it_is_done_or_closed(carrying):
+    env = carrying
+    env.arena_np[:] = np.random.default_rng(1).integers(0, 256, len(env.arena_np), dtype=np.uint8)
+    busy, other = Small(env, 0), Small(env, 1)
+    env.emu.emu_set_hold(1)
+    try:
+        for closed in (False, True):
+            assert [busy.post() for _ in range(3)] == [0, 1, 1]
+            assert other.post() == 1
+            assert env.emu.emu_release(4) == 4
+            other.finish()
+            assert other.post() == 1  # (done, but not reported yet)
+            assert env.emu.emu_release(1) == 1
+            other.finish()
+            if closed:
+                busy.comm.close()
+            else:
+                busy.finish()
+            assert other.post() == 0
+            assert env.emu.emu_release(1) == 1
+            other.finish()
+    finally:
+        env.emu.emu_set_hold(0)
+        env.emu.emu_release(1 << 20)
+        other.comm.close()
