@@ -149,7 +149,8 @@ typedef struct tcpxDeviceOps {
   int (*engine_submit_sized)(tcpxuEngine* engine, const void* bounce_base, void* dst_base, const void* descs_dev,
                              uint32_t n_descs, uint64_t payload_bytes, void* done_flag_dev, uint64_t done_value);
   /* Optional (may be NULL): how many descriptors of a list in mapped memory a submission brings along
-   * (tcpxuEngineCarriedDescs); such a request gets no second copy while it is the only one. */
+   * (tcpxuEngineCarriedDescs); such a request gets no second copy while it is its comm's only one and few of the
+   * device's others are at the GPU. */
   uint32_t (*engine_carried_descs)(void);
 } tcpxDeviceOps;
 

@@ -418,13 +418,14 @@ struct QueueBlock {  // mapped metadata + device handle, recycled between comms 
   QueueMeta* meta;
   QueueMeta* meta_dev;
   struct unpackNetDeviceHandle* dev_handle;
-  // Device memory the host can write, kStageDescs descriptors, or null: where the descriptors of a small request, or of one
-  // that is alone, are copied to as well, so that the GPU need not fetch them over PCIe (see publish_to_engine).
+  // Device memory the host can write, kStageDescs descriptors, or null: where the descriptors of a small request that has others
+  // beside it, or of a longer one that is alone, are copied to as well, so that the GPU need not fetch them over PCIe (which
+  // requests those are: descriptors_for_engine).
   union loadMeta* stage;
   union loadMeta* stage_dev;
 };
 constexpr uint32_t kStagedDescs = 16;   // a small request's, of which each slot has its own
-constexpr uint32_t kAloneDescs = 512;   // of a request that is alone at the GPU, behind the slots' own
+constexpr uint32_t kAloneDescs = 512;   // of a longer request that is its comm's only one, behind the slots' own
 constexpr uint32_t kStageDescs = kStagedDescs * kQueueDepth + kAloneDescs;
 
 struct DeviceState {

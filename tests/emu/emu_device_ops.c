@@ -47,6 +47,7 @@ static uint64_t g_submitted = 0, g_mapped_live = 0, g_device_live = 0, g_arenas_
 static struct { uint8_t* p; size_t bytes; } g_visible[EMU_MAX_VISIBLE];
 static uint64_t g_visible_live = 0, g_staged_submits = 0, g_visible_flushes = 0, g_last_payload_bytes = 0;
 static int g_visible_off = 0;
+static uint32_t g_carried_descs = 16; /* as the engine that ships */
 static int in_visible(const void* p);
 
 static void run_job(const emu_job* j) {
@@ -59,6 +60,7 @@ void emu_set_hold(int hold) { g_hold = hold; }
 void emu_set_skip_copy(int skip) { g_skip_copy = skip; } /* completes submissions without moving bytes: for timing the host code alone */
 void emu_set_ring_full(int full) { g_ring_full = full; }
 void emu_set_visible_off(int off) { g_visible_off = off; } /* allocations of host-visible device memory fail */
+void emu_set_carried_descs(uint32_t n) { g_carried_descs = n; } /* asked for when the plugin is initialised */
 int emu_pending(void) { return g_n_pending; }
 int emu_release(int n) { /* completes the n oldest held submissions; returns how many were completed */
   int done = 0;
@@ -174,6 +176,7 @@ static int emu_visible_free(int dev, void* host_ptr) {
   return TCPXU_INVALID_ARGUMENT;
 }
 static void emu_visible_flush(void) { ++g_visible_flushes; }
+static uint32_t emu_engine_carried_descs(void) { return g_carried_descs; }
 static int in_visible(const void* p) {
   for (int i = 0; i < EMU_MAX_VISIBLE; ++i)
     if (g_visible[i].p && (const uint8_t*)p >= g_visible[i].p && (const uint8_t*)p < g_visible[i].p + g_visible[i].bytes) return 1;
@@ -185,5 +188,6 @@ static const tcpxDeviceOps g_ops = {
     emu_device_alloc, emu_device_free,   emu_copy_to_device, emu_engine_create, emu_engine_start,
     emu_engine_stop,  emu_engine_destroy, emu_engine_submit, emu_last_error,
     emu_visible_alloc, emu_visible_free, emu_visible_flush, emu_engine_submit_sized,
+    emu_engine_carried_descs,
 };
 const tcpxDeviceOps* emu_ops(void) { return &g_ops; }

@@ -34,6 +34,7 @@ def load_emu():
     lib.emu_set_hold.argtypes = [ctypes.c_int]
     lib.emu_set_ring_full.argtypes = [ctypes.c_int]
     lib.emu_set_visible_off.argtypes = [ctypes.c_int]
+    lib.emu_set_carried_descs.argtypes = [ctypes.c_uint32]
     lib.emu_counter.restype = ctypes.c_uint64
     lib.emu_counter.argtypes = [ctypes.c_int]
     return lib

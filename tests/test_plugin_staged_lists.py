@@ -1,15 +1,10 @@
 """The second copy of a request's descriptors is written by whole lines of four: lists that end within a line, fill it or go one
 beyond, small ones and of a request that is alone; and where the engine brings lists of mapped slots along, a small request that is
 alone has none (no GPU: the emulated device of tests/emu)."""
-import ctypes
-
 import numpy as np
 import pytest
 
-from test_plugin_host import ARENA_BYTES, comm, env, host_buffer, load_emu  # noqa: F401  (fixtures)
-
-OPS = 19  # members of tcpxDeviceOps, the last of them engine_carried_descs
-CARRIED = 16
+from test_plugin_host import ARENA_BYTES, brings_no_lists, comm, env, host_buffer  # noqa: F401  (fixtures)
 
 
 def receive(env, comm, sizes, seed):
@@ -46,43 +41,16 @@ def receive(env, comm, sizes, seed):
     return env.emu.emu_counter(6) - copies
 
 
-@pytest.fixture(scope="module")
-def carrying(env):  # noqa: F811
-    """The emulated device with an engine that brings lists along, in place of the one that does not."""
-    ops = (ctypes.c_void_p * OPS)()
-    ctypes.memmove(ops, env.emu.emu_ops(), ctypes.sizeof(ops))
-    assert ops[OPS - 2] and not ops[OPS - 1]
-    count = ctypes.CFUNCTYPE(ctypes.c_uint32)(lambda: CARRIED)
-    ops[OPS - 1] = ctypes.cast(count, ctypes.c_void_p).value
-
-    def install(table):
-        assert env.lib.tcpxFinalize() == 0
-        assert env.lib.tcpxSetDeviceOpsForTesting(table) == 0
-        assert env.lib.tcpxInit(None) == 0
-        base = ctypes.c_void_p()
-        assert env.lib.tcpxSynthArenaCreate(0, ARENA_BYTES, ctypes.byref(base)) == 0
-        env.arena = base.value
-        env.arena_np = np.frombuffer((ctypes.c_uint8 * ARENA_BYTES).from_address(base.value), dtype=np.uint8)
-
-    install(ctypes.addressof(ops))
-    yield env
-    install(env.emu.emu_ops())
-
-
 @pytest.mark.parametrize("n", [1, 3, 4, 5, 8, 13, 15, 16, 17, 19, 509, 511, 512])
-def test_a_second_copy_of_any_length(env, comm, n):  # noqa: F811
+def test_a_second_copy_of_any_length(env, brings_no_lists, comm, n):  # noqa: F811
     assert receive(env, comm, [n], n) == 1
 
 
 @pytest.mark.parametrize("n", [1, 4, 15, 16, 17, 512, 513])
-def test_no_second_copy_of_a_list_that_travels(carrying, n):
-    comm = carrying.driver.RecvComm(0)  # noqa: F811
-    try:
-        assert receive(carrying, comm, [n], n) == (1 if 16 < n <= 512 else 0)
-        # Of three that are posted together the last one may find the others done.
-        assert receive(carrying, comm, [n] * 3, n + 1) >= (2 if n <= 16 else 0)
-    finally:
-        comm.close()
+def test_no_second_copy_of_a_list_that_travels(env, comm, n):  # noqa: F811
+    assert receive(env, comm, [n], n) == (1 if 16 < n <= 512 else 0)
+    # Of three that are posted together the last one may find the others done.
+    assert receive(env, comm, [n] * 3, n + 1) >= (2 if n <= 16 else 0)
 
 
 class Small:
@@ -119,9 +87,8 @@ class Small:
 
 
 @pytest.mark.parametrize("others", [0, 1, 3, 4, 5, 16])
-def test_lists_travel_while_few_comms_have_requests_at_the_gpu(carrying, others):
+def test_lists_travel_while_few_comms_have_requests_at_the_gpu(env, others):  # noqa: F811
     """The engine is the device's: a small request that is alone in its comm counts what all comms have there."""
-    env = carrying
     env.arena_np[:] = np.random.default_rng(others).integers(0, 256, len(env.arena_np), dtype=np.uint8)
     comms = [Small(env, i) for i in range(others + 1)]
     env.emu.emu_set_hold(1)
@@ -138,8 +105,7 @@ def test_lists_travel_while_few_comms_have_requests_at_the_gpu(carrying, others)
             c.comm.close()
 
 
-def test_a_comm_with_several_at_the_gpu_is_a_crowd_until_it_is_done_or_closed(carrying):
-    env = carrying
+def test_a_comm_with_several_at_the_gpu_is_a_crowd_until_it_is_done_or_closed(env):  # noqa: F811
     env.arena_np[:] = np.random.default_rng(1).integers(0, 256, len(env.arena_np), dtype=np.uint8)
     busy, other = Small(env, 0), Small(env, 1)
     env.emu.emu_set_hold(1)
