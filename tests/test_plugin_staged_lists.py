@@ -7,8 +7,9 @@ import pytest
 from test_plugin_host import ARENA_BYTES, brings_no_lists, comm, env, host_buffer  # noqa: F401  (fixtures)
 
 
-def receive(env, comm, sizes, seed):
-    """Posts a request for each of `sizes` (fragment counts) before any of their bytes is there; how many lists were copied."""
+def receive(env, comm, sizes, seed, copied):
+    """Posts a request for each of `sizes` (fragment counts) before any of their bytes is there, and lets the engine have them all
+    before it completes one; `copied` of the lists are copied."""
     rng = np.random.default_rng(seed)
     copies, posted, first = env.emu.emu_counter(6), [], 0
     env.arena_np[:] = rng.integers(0, 256, len(env.arena_np), dtype=np.uint8)
@@ -28,29 +29,30 @@ def receive(env, comm, sizes, seed):
     for frags, total, buf, mh, req in posted:
         comm.ctrl(0, total, 0, total)
         comm.deliver(0, frags)
+    submitted = env.emu.emu_counter(0)
+    env.emu.emu_set_hold(1)  # (none is done before all are at the engine)
+    for _ in range(100000):
+        assert comm.test(posted[0][4])[:2] == (0, 0)
+        if env.emu.emu_counter(0) == submitted + len(sizes):
+            break
+    assert env.emu.emu_counter(6) - copies == copied
+    assert env.emu.emu_release(1 << 20) == len(sizes)
+    env.emu.emu_set_hold(0)
     for frags, total, buf, mh, req in posted:
-        for _ in range(100000):
-            rc, done = comm.test(req)[:2]
-            assert rc == 0
-            if done:
-                break
-        assert done
-        assert comm.consumed(req) == 0
+        assert comm.test(req)[:2] == (0, 1) and comm.consumed(req) == 0
         comm.dereg(mh)
         assert buf.tobytes() == b"".join(env.arena_np[int(f["frag_offset"]) :][: int(f["frag_size"])].tobytes() for f in frags)
-    return env.emu.emu_counter(6) - copies
 
 
 @pytest.mark.parametrize("n", [1, 3, 4, 5, 8, 13, 15, 16, 17, 19, 509, 511, 512])
 def test_a_second_copy_of_any_length(env, brings_no_lists, comm, n):  # noqa: F811
-    assert receive(env, comm, [n], n) == 1
+    receive(env, comm, [n], n, 1)
 
 
 @pytest.mark.parametrize("n", [1, 4, 15, 16, 17, 512, 513])
-def test_no_second_copy_of_a_list_that_travels(env, comm, n):  # noqa: F811
-    assert receive(env, comm, [n], n) == (1 if 16 < n <= 512 else 0)
-    # Of three that are posted together the last one may find the others done.
-    assert receive(env, comm, [n] * 3, n + 1) >= (2 if n <= 16 else 0)
+def test_which_lists_are_copied_where_the_engine_brings_them_along(env, comm, n):  # noqa: F811
+    receive(env, comm, [n], n, 1 if 16 < n <= 512 else 0)
+    receive(env, comm, [n] * 3, n + 1, 3 if n <= 16 else 0)
 
 
 class Small:
