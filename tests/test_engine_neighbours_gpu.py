@@ -30,22 +30,24 @@ def test_neighbours_of_a_ticket(pkg, hip, oracle, per, beyond):
     total = int(lens.sum())
     pool = rng.integers(0, 256, PAGES * 4096, dtype=np.uint8)
     expect = oracle_expected(oracle, pool, descs, total, 3)
-    g = GpuBuffers(pool, descs, total, 3)
+    buffers = [GpuBuffers(pool, descs, total, 3) for _ in range(2)]  # one a turn: what either fails to write shows
     m = Mapped(pkg, hip, descs, COUNT)
     e = Engine(pkg, hip, workgroups=33, descs_per_ticket=per)
     subs = (pkg.Submission * COUNT)()
     print("%d submissions of %d descriptors in tickets of %d" % (COUNT, n, per), flush=True)
-    e.start()
     accepted = ctypes.c_uint32()
-    for turn in (1, 2):
-        for i in range(COUNT):
-            subs[i] = pkg.Submission(g.pool.data_ptr(), g.dst_base, m.desc_dev(i * n), m.flag_dev(i), turn, n, 400 * n)
-        assert hip.tcpxuEngineSubmitMany(e.h, subs, COUNT, ctypes.byref(accepted)) == pkg.SUCCESS, hip.tcpxuLastError()
-        assert accepted.value == COUNT
-        for i in range(COUNT):
-            m.wait(i, turn)
-    e.stop()
-    got = g.result()
-    e.destroy()
+    try:
+        e.start()
+        for turn, g in enumerate(buffers, 1):
+            for i in range(COUNT):
+                subs[i] = pkg.Submission(g.pool.data_ptr(), g.dst_base, m.desc_dev(i * n), m.flag_dev(i), turn, n, 400 * n)
+            assert hip.tcpxuEngineSubmitMany(e.h, subs, COUNT, ctypes.byref(accepted)) == pkg.SUCCESS, hip.tcpxuLastError()
+            assert accepted.value == COUNT
+            for i in range(COUNT):
+                m.wait(i, turn)
+    finally:
+        e.destroy()  # (stops it: nothing may be left running on buffers that go back to the allocator)
     m.free()
-    assert first_difference(got, expect) is None, repr(first_difference(got, expect))
+    for turn, g in enumerate(buffers, 1):
+        difference = first_difference(g.result(), expect)
+        assert difference is None, "turn %d, first (index, got, want, count): %r" % (turn, difference)
