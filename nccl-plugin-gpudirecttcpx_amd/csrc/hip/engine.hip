@@ -1089,9 +1089,10 @@ __device__ void leader_loop(HostCtl* ctl, DevState* st, uint32_t* jobs_done, uin
 // last store and its completion word.  Hence: values of other lanes by moves and masks, not by exchanges through the LDS; the
 // load of the descriptors ahead of what is left in the LDS; one word that says whether there is a ticket and what it is; a
 // fragment's record waited for once; what tells the fetcher to go on a store, not an addition; and what the last wavefront has
-// to say read while its stores are on their way.  (Us, before / with all of these: 64 KiB of pages 7.60 / 7.44, through the plugin
-// 6.71 / 6.49, a page 5.73 / 5.50, 1 MiB of wire fragments 9.87 / 9.55, 2048 requests of 64 KiB through the plugin, 16 posted at a time,
-// 896 / 882; streams of 64 KiB requests, 1 / 8 / 64 / 256 in flight, 0.170 / 1.338 / 8.72 / 21.6 M/s before, 0.175 / 1.373 / 8.65 / 21.4 now.)
+// to say read while its stores are on their way.  (Us, without / with all of these: 64 KiB of pages 7.50 / 7.42, through the plugin
+// 6.79 / 6.57, a page 5.73 / 5.50, 1 MiB of wire fragments 9.87 / 9.55, 2048 requests of 64 KiB through the plugin, 16 posted at a time,
+// 908 / 890, of which about 1 % gives back what the one load of a ticket's neighbours, below, costs those; streams of 64 KiB
+// requests, 1 / 8 / 64 / 256 in flight, 0.170 / 1.338 / 8.72 / 21.6 M/s without, 0.175 / 1.373 / 8.65 / 21.4 with.)
 //
 // A worker workgroup is kCopyWaves copy wavefronts and one fetcher wavefront.  Towards the end of ticket i the
 // fetcher claims a number, polls that ticket's slot, pulls the ticket's descriptors over PCIe and writes their
@@ -1167,8 +1168,8 @@ __device__ uint32_t try_fetch_ticket(DevState* st, const uint32_t* stop_word, ui
   // neighbouring tickets' fetchers look at the same pairs from the other side): lane l then asks for descriptor l - 1, and one
   // move along the lanes puts them where they are worked on.  What bounds the first tickets of a burst is the number of
   // lines that all workers read over PCIe at once, 3.1 ns each where they are a line or two apart (2.3 in longer stretches):
-  // a ticket of 32 takes five, and seven while its neighbours were asked for by themselves.  (Us a call with lists in mapped
-  // memory, before / now: 64 MiB of ragged fragments 34.8 / 34.0, 256 MiB 107.5 / 107.1, 16 MiB of wire fragments in requests of
+  // a ticket of 32 whose list starts off a line of 128 bytes takes five, and seven while its neighbours were asked for by
+  // themselves (on a line, as in the plugin's slots, it takes six both ways).  (Us a call with lists in mapped memory, before / now: 64 MiB of ragged fragments 34.8 / 34.0, 256 MiB 107.5 / 107.1, 16 MiB of wire fragments in requests of
   // 256 KiB 18.5 / 18.2; lists in the GPU's memory as before.  One load for both kinds of ticket: with a load each in two branches
   // small requests, which have no such neighbours, take 1.5 to 3 % longer.)
   const bool more_before = (ticket_bits & kMoreBefore) != 0, more_after = (ticket_bits & kMoreAfter) != 0;
@@ -1180,9 +1181,11 @@ __device__ uint32_t try_fetch_ticket(DevState* st, const uint32_t* stop_word, ui
   if (one_load) mine = std::min(std::max(static_cast<int>(lane) - 1, first), last);
   if (carried) d[3] = 0;  // (the stamp's place is the high word of the destination offset)
   else d = load_vec_sys(reinterpret_cast<const uint8_t*>(descs_addr) + 16 * mine);
-  // The neighbours, where they are more than lanes are left: by themselves, in the same trip.  (With one load of 64 descriptors from
-  // the one before on and a second of two, a full ticket is eleven lines instead of ten: streams of 1 KiB fragments 0.665 -> 0.605 of
-  // the roofline.  The empty statement: in other tickets nothing of it is used.)
+  // The neighbours, where they are more than lanes are left: by themselves, in the same trip.  (Us a call of 64 lists of 2048
+  // fragments in tickets of 64, so / with one load of 64 descriptors from the one before on and a second of two.  1 KiB each: lists on
+  // a line, where that is ten lines / eleven, 63.5 / 72.3; one descriptor off it, eleven / nine and the long load on lines, 67.9 / 67.2; two, four
+  // or seven off, eleven / ten, 67.8 / 70.3.  512 to 1535 bytes: 66.9 / 76.4, 70.7 / 70.9, 70.5 / 74.3.  The empty statement: in other
+  // tickets nothing of it is used.)
   u32x4 outer;
   asm volatile("" : "=v"(outer));
   if (outward && !one_load && lane < 2) outer = load_vec_sys(reinterpret_cast<const uint8_t*>(descs_addr) + 16 * (lane == 0 ? first : last));

@@ -624,8 +624,8 @@ ncclResult_t ensure_engine(DeviceState* ds) {
 
 // Descriptors into host-visible device memory, which the host writes through write-combining buffers of 64 bytes: by whole
 // lines, front to back, each line written once (the rest of the last one is whatever the slot holds there).  What memcpy makes of
-// other sizes than 128 and 256 bytes -- two stores that overlap -- leaves a line in several pieces, and the flush behind it waits for
-// each.  (256 requests of so many descriptors, 16 posted at a time, us by memcpy / so: 1 96.5 / 95.4, 4 121 / 95.7, 6 122 / 96.9,
+// 64, 96, 160, 192 and 224 bytes -- stores that overlap -- leaves a line in several pieces, and the flush behind it waits for each; of 16, 128
+// and 256 bytes it does not.  (256 requests of so many descriptors, 16 posted at a time, us by memcpy / so: 1 96.5 / 95.4, 4 121 / 95.7, 6 122 / 96.9,
 // 8 99.6 / 99.8, 10 129.7 / 104.5, 12 134.2 / 107.6, 14 134.9 / 108.6, 16 110.7 / 110.7; of 10 KB in fragments of any length 150.8 / 123.5.)
 inline void write_lines(union loadMeta* to, const union loadMeta* from, size_t n) {
   constexpr size_t kLine = 4;
